@@ -163,7 +163,8 @@ int matmul_host(smx_ctx* c, const char* key, const float* xs, size_t m, size_t i
                         force_gemm, nullptr, nullptr);
     if (rc != SMX_OK) return rc;
     if (!y_direct) SMX_HIP(c, hipMemcpyAsync(pinned ? (void*)c->hy.p : (void*)y, c->yf32.p, yb, hipMemcpyDeviceToHost, c->stream));
-    SMX_HIP(c, hipStreamSynchronize(c->stream));
+    if (!pinned) SMX_HIP(c, hipStreamSynchronize(c->stream));
+    else if ((rc = stream_wait(c)) != SMX_OK) return rc;
     if (pinned) memcpy(y, c->hy.p, yb);
     return SMX_OK;
 }
@@ -284,7 +285,9 @@ static int gemv_batch_host(smx_ctx* c, size_t n, const char* const* keys, const 
             if (ws[i] && status[i] == SMX_OK)
                 SMX_HIP(c, hipMemcpyAsync(ys[i], c->yf32.p + yoff[i], ws[i]->N * 4, hipMemcpyDeviceToHost, c->stream));
     }
-    SMX_HIP(c, hipStreamSynchronize(c->stream));  // the batch's single sync (decode.rs:3247)
+    // the batch's single sync (decode.rs:3247)
+    if (!pinned) SMX_HIP(c, hipStreamSynchronize(c->stream));
+    else if ((rc = stream_wait(c)) != SMX_OK) return rc;
     if (pinned)
         for (size_t i = 0; i < n; i++)
             if (ws[i] && status[i] == SMX_OK) memcpy(ys[i], c->hy.p + yoff[i], ws[i]->N * 4);
@@ -313,15 +316,23 @@ int smx_lm_head_argmax_rows(smx_ctx* c, const char* key, const float* xs, size_t
     int rc;
     if ((rc = ensure(c, c->xf32, m * w->K * 4)) != SMX_OK) return rc;
     if ((rc = ensure(c, c->yf32, m * w->N * 4)) != SMX_OK) return rc;
-    const size_t ids_bytes = (m * 4 + 255) & ~size_t(255);   // ids, then the chunk candidates
-    if ((rc = ensure(c, c->tab, ids_bytes + argmax_scratch_bytes(m, w->N))) != SMX_OK) return rc;
-    SMX_HIP(c, hipMemcpyAsync(c->xf32.p, xs, m * w->K * 4, hipMemcpyHostToDevice, c->stream));
+    if ((rc = ensure(c, c->tab, argmax_scratch_bytes(m, w->N))) != SMX_OK) return rc;   // the chunk candidates
+    // rows of up to 8 MiB in all travel through the pinned staging (a copy from pageable memory has the host wait for it),
+    // and the last kernel writes the indices into pinned memory itself
+    const size_t xb = m * w->K * 4;
+    const bool pinned = xb <= (size_t(8) << 20);
+    if (pinned) {
+        if ((rc = ensure_host(c, c->hx, xb)) != SMX_OK) return rc;
+        memcpy(c->hx.p, xs, xb);
+    }
+    if ((rc = ensure_host(c, c->hy, m * 4)) != SMX_OK) return rc;
+    SMX_HIP(c, hipMemcpyAsync(c->xf32.p, pinned ? (const void*)c->hx.p : (const void*)xs, xb, hipMemcpyHostToDevice, c->stream));
     rc = run_matmul_dev(c, *w, (const float*)c->xf32.p, m, (float*)c->yf32.p, false, nullptr, nullptr);
     if (rc != SMX_OK) return rc;
-    rc = launch_argmax_rows(c, (const float*)c->yf32.p, m, w->N, (char*)c->tab.p + ids_bytes, (unsigned*)c->tab.p);
+    rc = launch_argmax_rows(c, (const float*)c->yf32.p, m, w->N, c->tab.p, (unsigned*)c->hy.p);
     if (rc != SMX_OK) return rc;
-    SMX_HIP(c, hipMemcpyAsync(out, c->tab.p, m * 4, hipMemcpyDeviceToHost, c->stream));
-    SMX_HIP(c, hipStreamSynchronize(c->stream));
+    if ((rc = stream_wait(c)) != SMX_OK) return rc;
+    memcpy(out, c->hy.p, m * 4);
     return SMX_OK;
 }
 
@@ -451,7 +462,7 @@ int smx_gemv_fused(smx_ctx* c, const char* key, int act, const float* a, const f
     const ActProd prod = {act, b_dev, eps};
     if ((rc = launch_gemv_group(c, &w, xs, ys, 1, nullptr, &prod)) != SMX_OK) return rc;
     if (!y_direct) SMX_HIP(c, hipMemcpyAsync(c->hy.p, c->yf32.p, yb, hipMemcpyDeviceToHost, c->stream));
-    SMX_HIP(c, hipStreamSynchronize(c->stream));
+    if ((rc = stream_wait(c)) != SMX_OK) return rc;
     memcpy(y, c->hy.p, yb);
     return SMX_OK;
 }

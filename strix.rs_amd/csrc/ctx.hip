@@ -1,4 +1,6 @@
 // Context, weight residency (upload + repack to planar HBM layout), scratch and profiling.
+#include <atomic>
+#include <chrono>
 #include <cstring>
 
 #include "smx_internal.h"
@@ -73,6 +75,34 @@ int ensure_host(smx_ctx* c, DevBuf& b, size_t bytes) {
         return fail(c, SMX_ERR_NOMEM, "pinned host allocation of %zu bytes failed: %s", cap, hipGetErrorString(e));
     }
     b.cap = cap;
+    return SMX_OK;
+}
+
+__global__ __launch_bounds__(64) void stream_flag_kernel(unsigned* flag, unsigned value) {
+    if (threadIdx.x == 0) __hip_atomic_store(flag, value, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// hipStreamSynchronize has the runtime put a barrier packet with a completion signal behind the last kernel and wait for
+// that signal: 9.4 us for an empty kernel.  One word in pinned host memory written by a kernel of its own is seen by a
+// polling host 6.4 us after the same start (the stream runs the word's kernel after everything in front of it has
+// completed and written its results; 14.0 -> 10.0 us with a 256-workgroup kernel that reads and writes pinned memory).
+// The poll is bounded: work of more than kSpinUs, or a failed launch, goes through the runtime's own wait.
+int stream_wait(smx_ctx* c) {
+    constexpr double kSpinUs = 2000.0;
+    const unsigned want = ++c->flag_seq;
+    hipLaunchKernelGGL(stream_flag_kernel, dim3(1), dim3(64), 0, c->stream, c->hflag, want);
+    SMX_HIP(c, hipGetLastError());
+    const volatile unsigned* flag = c->hflag;
+    const auto t0 = std::chrono::steady_clock::now();
+    for (unsigned i = 1;; i++) {
+        if (*flag == want) {
+            std::atomic_thread_fence(std::memory_order_acquire);
+            return SMX_OK;
+        }
+        __builtin_ia32_pause();
+        if (i % 64 == 0 && std::chrono::duration<double, std::micro>(std::chrono::steady_clock::now() - t0).count() > kSpinUs) break;
+    }
+    SMX_HIP(c, hipStreamSynchronize(c->stream));
     return SMX_OK;
 }
 
@@ -310,8 +340,18 @@ int smx_create(int device, smx_ctx** out) {
         delete c;
         return fail(nullptr, SMX_ERR_HIP, "smx_create: hipEventCreate failed");
     }
+    e = hipHostMalloc((void**)&c->hflag, 64, hipHostMallocDefault);
+    if (e != hipSuccess) {
+        (void)hipEventDestroy(c->t0);
+        (void)hipEventDestroy(c->t1);
+        (void)hipStreamDestroy(c->stream);
+        delete c;
+        return hip_fail(nullptr, e, "hipHostMalloc");
+    }
+    *c->hflag = 0;
     if (noalloc_init(c) != SMX_OK) {   // the static scratch array of the allocation-free entry point, on this device
         g_create_err = c->err;
+        (void)hipHostFree(c->hflag);
         (void)hipEventDestroy(c->t0);
         (void)hipEventDestroy(c->t1);
         (void)hipStreamDestroy(c->stream);
@@ -337,6 +377,7 @@ void smx_destroy(smx_ctx* c) {
     for (char* p : c->retired) (void)hipFree(p);
     for (DevBuf* b : {&c->hx, &c->hy, &c->htab})
         if (b->p) (void)hipHostFree(b->p);
+    (void)hipHostFree(c->hflag);
     if (c->htab_done) (void)hipEventDestroy(c->htab_done);
     for (auto& r : c->prof) {
         (void)hipEventDestroy(r.e0);

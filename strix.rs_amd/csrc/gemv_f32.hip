@@ -410,7 +410,7 @@ int smx_gemv_f32(smx_ctx* c, const char* key, const float* x, size_t in_len, flo
         if ((rc = launch_gemv_f32(c, w, x_direct ? (const float*)c->hx.p : (const float*)c->xf32.p,
                                   y_direct ? (float*)c->hy.p : (float*)c->yf32.p)) != SMX_OK) return rc;
         if (!y_direct) SMX_HIP(c, hipMemcpyAsync(c->hy.p, c->yf32.p, yb, hipMemcpyDeviceToHost, c->stream));
-        SMX_HIP(c, hipStreamSynchronize(c->stream));
+        if ((rc = stream_wait(c)) != SMX_OK) return rc;
         std::memcpy(y, c->hy.p, yb);
         return SMX_OK;
     });

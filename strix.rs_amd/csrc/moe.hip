@@ -823,7 +823,8 @@ static int moe_ffn_host(smx_ctx* c, size_t layer, const int32_t* ids, const floa
     }
     if (aq) SMX_HIP(c, hipMemcpyAsync(aq, s.aq, k * L.eff, hipMemcpyDeviceToHost, c->stream));
     if (ad) SMX_HIP(c, hipMemcpyAsync(ad, s.ad, k * (L.eff / 32) * 4, hipMemcpyDeviceToHost, c->stream));
-    SMX_HIP(c, hipStreamSynchronize(c->stream));
+    if (gu || aq || ad) SMX_HIP(c, hipStreamSynchronize(c->stream));   // (the stage copies go to pageable memory)
+    else if ((rc = stream_wait(c)) != SMX_OK) return rc;
     memcpy(y, c->hy.p, hb);
     return SMX_OK;
     });

@@ -76,6 +76,8 @@ struct smx_ctx {
     smx::DevBuf raw;    // upload staging: the raw GGUF blocks of the tensor being repacked (kept up to kRawKeepBytes between uploads)
     smx::DevBuf hx, hy; // pinned HOST staging of the host-pointer calls' activations and results
     smx::DevBuf htab;   // pinned HOST staging of the small tables of enqueue-only calls
+    unsigned* hflag = nullptr;   // pinned HOST word that stream_wait's last kernel writes
+    unsigned flag_seq = 0;       // what it writes next
     hipEvent_t htab_done = nullptr;  // recorded after the last copy out of htab (null: htab is free)
 
     // tuning overrides (0 = automatic)
@@ -136,6 +138,8 @@ int ensure(smx_ctx* c, DevBuf& b, size_t bytes);
 void release_device(smx_ctx* c, char* p);
 // the same for a pinned host buffer (hipHostMalloc)
 int ensure_host(smx_ctx* c, DevBuf& b, size_t bytes);
+// Waits until everything enqueued on the context's stream has run (the one synchronisation of a host-pointer call).
+int stream_wait(smx_ctx* c);
 
 // Raises a kernel's dynamic-LDS limit when it asks for more than the 48 KB default (remembered per
 // context and kernel so that replays and captured launches do not repeat the call).
