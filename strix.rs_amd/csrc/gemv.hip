@@ -103,6 +103,13 @@ __global__ __launch_bounds__(1024) void gemv_flat_kernel(const GemvJobs J, int* 
                                                blockIdx.x, jb.n_wgs, jb.magic_u, dump, dump_per_row);
 }
 
+// The same for a launch of ONE job: two lines of arguments instead of the group's 2.3 KB, which the runtime writes into device
+// memory over the bus at every launch (an empty kernel: 2.5 us per launch with 16 or 256 bytes of arguments, 3.1 with 2300).
+template <class Ops, int MT, int PRE, int GL, int FQ>
+__global__ __launch_bounds__(1024) void gemv_flat1_kernel(const GemvJob jb) {
+    gemv_body_flat<Ops, MT, PRE, GL, FQ, false>(jb.W, jb.X(), jb.y, jb.N, jb.nblk, jb.N, MT == 1 ? 1 : jb.m, blockIdx.x, jb.n_wgs, jb.magic_u);
+}
+
 // Paired form: workgroup (x, p) serves jobs 2p (gate) and 2p + 1 (up) over the same rows and writes the product of the
 // activated gate dot and the up dot (gemv_body_flat, DUAL).
 // IND: 0 = the jobs' weights as given, 1 = experts read from device memory (J.ids), 2 = experts routed here: every workgroup
@@ -208,21 +215,36 @@ int launch_one(smx_ctx* c, const Geom& g, const GemvJobs& J, int njobs, int nblk
 template <class Ops, int MT, int PRE, int GL, int FQ, bool DUMP = false>
 int launch_flat_fq(smx_ctx* c, const Geom& g, const GemvJobs& J, int njobs, int nblk, int m, int* dump = nullptr,
                    int dump_per_row = 0) {
-    auto k = gemv_flat_kernel<Ops, MT, PRE, GL, FQ, DUMP>;
-    if (J.ids) {   // experts chosen on the device: one fp32 activation row per job, no dump
-        if constexpr (MT == 1 && FQ != 0 && !DUMP) k = gemv_flat_kernel<Ops, MT, PRE, GL, FQ, DUMP, true>;
-        else return fail(c, SMX_ERR_ARG, "gemv: device-routed experts take one fp32 activation row per job");
-    }
-    int rc = set_dyn_lds(c, k, g.lds);
-    if (rc != SMX_OK) return rc;
     const unsigned upb = std::is_same<Ops, OpsQ6_K>::value ? 4u : (std::is_same<Ops, OpsQ8_0>::value ? 2u : 1u);
     const unsigned units = (unsigned)nblk * upb;                             // units per row
     const unsigned magic = (unsigned)(((1ull << 32) + units - 1) / units);   // floor(f * magic / 2^32) = f / units for f < 2^16
-    GemvJobs JJ = J;
-    for (int i = 0; i < njobs; i++) { JJ.job[i].nblk = nblk; JJ.job[i].m = m; JJ.job[i].n_wgs = (int)g.grid; JJ.job[i].magic_u = magic; }
-    hipLaunchKernelGGL(k, dim3(g.grid, (unsigned)njobs), dim3(1024), g.lds, c->stream, JJ, dump, dump_per_row);
-    SMX_HIP(c, hipGetLastError());
-    return SMX_OK;
+    if constexpr (!DUMP) {
+        if (njobs == 1 && !J.ids) {
+            auto k1 = gemv_flat1_kernel<Ops, MT, PRE, GL, FQ>;
+            int rc = set_dyn_lds(c, k1, g.lds);
+            if (rc != SMX_OK) return rc;
+            GemvJob j1 = J.job[0];
+            j1.nblk = nblk; j1.m = m; j1.n_wgs = (int)g.grid; j1.magic_u = magic;
+            hipLaunchKernelGGL(k1, dim3(g.grid), dim3(1024), g.lds, c->stream, j1);
+            SMX_HIP(c, hipGetLastError());
+            return SMX_OK;
+        }
+    }
+    if constexpr (MT == 1) {
+        auto k = gemv_flat_kernel<Ops, MT, PRE, GL, FQ, DUMP>;
+        if (J.ids) {   // experts chosen on the device: one fp32 activation row per job, no dump
+            if constexpr (FQ != 0 && !DUMP) k = gemv_flat_kernel<Ops, MT, PRE, GL, FQ, DUMP, true>;
+            else return fail(c, SMX_ERR_ARG, "gemv: device-routed experts take one fp32 activation row per job");
+        }
+        int rc = set_dyn_lds(c, k, g.lds);
+        if (rc != SMX_OK) return rc;
+        GemvJobs JJ = J;
+        for (int i = 0; i < njobs; i++) { JJ.job[i].nblk = nblk; JJ.job[i].m = m; JJ.job[i].n_wgs = (int)g.grid; JJ.job[i].magic_u = magic; }
+        hipLaunchKernelGGL(k, dim3(g.grid, (unsigned)njobs), dim3(1024), g.lds, c->stream, JJ, dump, dump_per_row);
+        SMX_HIP(c, hipGetLastError());
+        return SMX_OK;
+    }
+    return fail(c, SMX_ERR_ARG, "gemv: several activation rows take one job per launch");
 }
 
 template <class Ops, int MT>
