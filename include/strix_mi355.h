@@ -112,7 +112,7 @@ int smx_gemv_rows(smx_ctx* ctx, const char* key, const float* xs, size_t m, size
 int smx_gemv_batch(smx_ctx* ctx, size_t n, const char* const* keys, const float* const* xs,
                    const size_t* in_lens, float* const* ys, const size_t* out_caps, int* status);
 /* The same batch in the arithmetic of smx_gemv_f32 (what the reference's gemv_batch launches,
- * decode.rs:3227-3255 over the fp32-activation kernels): one launch per item, back to back, one sync. */
+ * decode.rs:3227-3255 over the fp32-activation kernels): consecutive items of one format and in_dim share a launch, one sync. */
 int smx_gemv_f32_batch(smx_ctx* ctx, size_t n, const char* const* keys, const float* const* xs,
                        const size_t* in_lens, float* const* ys, const size_t* out_caps, int* status);
 

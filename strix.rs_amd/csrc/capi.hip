@@ -186,8 +186,8 @@ int smx_gemm(smx_ctx* c, const char* key, const float* xs, size_t m, size_t in_d
     return matmul_host(c, key, xs, m, in_dim, y, y_cap, true, "gemm");
 }
 
-// One device job and one synchronisation for n host-pointer GEMVs.  f32: every item runs the fp32-activation kernel
-// (one launch per item, back to back); otherwise consecutive items of one format and row length share a launch.
+// One device job and one synchronisation for n host-pointer GEMVs; consecutive items of one format and row length share a
+// launch.  f32: in the fp32-activation arithmetic.
 static int gemv_batch_host(smx_ctx* c, size_t n, const char* const* keys, const float* const* xs, const size_t* in_lens,
                            float* const* ys, const size_t* out_caps, int* status, bool f32) {
     if (!c) return SMX_ERR_ARG;
@@ -256,25 +256,20 @@ static int gemv_batch_host(smx_ctx* c, size_t n, const char* const* keys, const 
         if (y_direct) ydev[i] = (float*)(c->hy.p + yoff[i]);
     }
     if (pinned && xo && !x_direct) SMX_HIP(c, hipMemcpyAsync(c->xf32.p, c->hx.p, xo, hipMemcpyHostToDevice, c->stream));
-    // consecutive items of one format and row length share a launch (up to 8 per launch)
+    // consecutive items of one format and row length share a launch
     for (size_t i = 0; i < n;) {
         if (!ws[i]) { i++; continue; }
-        if (f32) {
-            status[i] = launch_gemv_f32(c, *ws[i], xdev[i], ydev[i]);
-            i++;
-            continue;
-        }
-        const Weight* gw[8];
-        const float* gx[8];
-        float* gy[8];
-        size_t idx[8];
+        const Weight* gw[SMX_GEMV_GROUP_MAX];
+        const float* gx[SMX_GEMV_GROUP_MAX];
+        float* gy[SMX_GEMV_GROUP_MAX];
+        size_t idx[SMX_GEMV_GROUP_MAX];
         int g = 0;
         size_t j = i;
-        while (j < n && g < 8 && ws[j] && ws[j]->type == ws[i]->type && ws[j]->K == ws[i]->K) {
+        while (j < n && g < SMX_GEMV_GROUP_MAX && ws[j] && ws[j]->type == ws[i]->type && ws[j]->K == ws[i]->K) {
             gw[g] = ws[j]; gx[g] = xdev[j]; gy[g] = ydev[j]; idx[g] = j;
             g++; j++;
         }
-        rc = launch_gemv_group(c, gw, gx, gy, g);
+        rc = f32 ? launch_gemv_f32_group(c, gw, gx, gy, g) : launch_gemv_group(c, gw, gx, gy, g);
         for (int k = 0; k < g; k++) status[idx[k]] = rc;
         i = j;
     }

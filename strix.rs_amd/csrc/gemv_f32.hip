@@ -15,6 +15,7 @@
 // in flight, DPP reduction per row.
 // HBM-bound by bytes.
 #include <algorithm>
+#include <cstddef>
 #include <cstring>
 #include <type_traits>
 
@@ -208,13 +209,12 @@ __device__ __forceinline__ float unit_dot_flat(OpsQ6_K, const OpsQ6_K::Regs& r, 
     return h2f(r.d) * acc;
 }
 
-// blockIdx.x of n_wgs workgroups share the rows; magic_u = ceil(2^32 / units per row).  Every argument lies in the
-// first 64-byte line of the kernel-argument segment.
+// Workgroup wg of n_wgs that share the rows; magic_u = ceil(2^32 / units per row).
 template <class Ops, int PRE, int GL>
-__global__ __launch_bounds__(1024) void gemv_f32_flat_kernel(const GemvW W, const float* __restrict__ x, float* __restrict__ y,
-                                                             int nblk, int N, int n_wgs, unsigned magic_u) {
+__device__ __forceinline__ void f32_flat_body(const GemvW W, const float* __restrict__ x, float* __restrict__ y, int nblk, int N, int wg,
+                                              int n_wgs, unsigned magic_u) {
     extern __shared__ __align__(16) char smem[];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, wg = blockIdx.x;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int U = Ops::units_per_row(nblk), nb32 = Ops::nb32(nblk);
     float* xs = (float*)smem;
     float* hs = xs + nb32 * 36;
@@ -287,6 +287,42 @@ __global__ __launch_bounds__(1024) void gemv_f32_flat_kernel(const GemvW W, cons
     }
 }
 
+// Every argument lies in the first 64-byte line of the kernel-argument segment.
+template <class Ops, int PRE, int GL>
+__global__ __launch_bounds__(1024) void gemv_f32_flat_kernel(const GemvW W, const float* __restrict__ x, float* __restrict__ y,
+                                                             int nblk, int N, int n_wgs, unsigned magic_u) {
+    f32_flat_body<Ops, PRE, GL>(W, x, y, nblk, N, blockIdx.x, n_wgs, magic_u);
+}
+
+// Several weights of one format and row length in one launch (the items of a gemv_batch: q, k and v, gate and up).  Job j has
+// the workgroups first[j] .. first[j + 1] - 1, as many as its share of all rows asks for, so that a group of unequal weights
+// (grouped key/value heads) still gives every CU the same number of rows.  A row's sum does not depend on the split: same
+// bits as a launch per item.
+struct F32Job {
+    GemvW W;
+    const float* x;
+    float* y;
+    int N;
+    int pad[3];
+};
+struct F32Jobs {
+    int first[SMX_GEMV_GROUP_MAX];   // unused entries: 0x7fffffff
+    int n_total, nblk;
+    unsigned magic_u;
+    int pad[13];
+    F32Job job[SMX_GEMV_GROUP_MAX];
+};
+static_assert(sizeof(F32Job) == 64 && offsetof(F32Jobs, job) % 64 == 0, "a job is one line of the kernel-argument segment");
+template <class Ops, int PRE, int GL>
+__global__ __launch_bounds__(1024) void gemv_f32_group_kernel(const F32Jobs J) {
+    int j = 0;
+#pragma unroll
+    for (int i = 1; i < SMX_GEMV_GROUP_MAX; i++) j += (int)blockIdx.x >= J.first[i] ? 1 : 0;
+    const F32Job& jb = J.job[j];
+    const int w0 = J.first[j], w1 = min(j + 1 < SMX_GEMV_GROUP_MAX ? J.first[j + 1] : J.n_total, J.n_total);
+    f32_flat_body<Ops, PRE, GL>(jb.W, jb.x, jb.y, J.nblk, jb.N, blockIdx.x - w0, w1 - w0, J.magic_u);
+}
+
 // The flat form's geometry (as for the Q8-activation GEMV): whole further rounds of workgroups when a CU's share of
 // the rows is too large for the 16-bit unit index or for LDS.  Returns false when the shape is not served.
 struct F32Flat { int gl; unsigned grid, magic; size_t lds; };
@@ -331,6 +367,23 @@ static int launch_f32_flat(smx_ctx* c, const Weight& w, const float* x, float* y
     return fail(c, SMX_ERR_ARG, "gemv_f32: no flat variant for %d-unit groups", g.gl);
 }
 
+template <class Ops, int PRE>
+static int launch_f32_group_type(smx_ctx* c, const F32Jobs& J, int gl, size_t lds) {
+    auto go = [&](auto kern) -> int {
+        int rc = set_dyn_lds(c, kern, lds);
+        if (rc != SMX_OK) return rc;
+        hipLaunchKernelGGL(kern, dim3((unsigned)J.n_total), dim3(1024), lds, c->stream, J);
+        SMX_HIP(c, hipGetLastError());
+        return SMX_OK;
+    };
+    if (gl == 16) return go(gemv_f32_group_kernel<Ops, PRE, 16>);
+    if (gl == 8) return go(gemv_f32_group_kernel<Ops, PRE, 8>);
+    if constexpr (std::is_same<Ops, OpsQ6_K>::value) {
+        if (gl == 4) return go(gemv_f32_group_kernel<Ops, PRE, 4>);
+    }
+    return fail(c, SMX_ERR_ARG, "gemv_f32: no group variant for %d-unit groups", gl);
+}
+
 template <class Ops>
 static int launch_f32_type(smx_ctx* c, const Weight& w, const float* x, float* y) {
     const GemvW W = {w.scales, (const uint4*)w.quants, (const uint4*)w.qh, (const uint2*)w.sc};
@@ -368,6 +421,64 @@ int launch_gemv_f32(smx_ctx* c, const Weight& w, const float* x, float* y) {
     }
     ProfScope ps(c, "gemv_f32_q6_k");
     return flat ? launch_f32_flat<OpsQ6_K, 1>(c, w, x, y, fg) : launch_f32_type<OpsQ6_K>(c, w, x, y);
+}
+
+// n weights of one format and row length: one launch where the flat form serves them all, otherwise one per item.
+// Three Q8_0 weights (2560, 640 and 640 rows of 2560): 3 launches of 5.1 / 3.3 / 3.3 us in a row -> one of 5.5 us.
+int launch_gemv_f32_group(smx_ctx* c, const Weight* const* ws, const float* const* xs, float* const* ys, int n) {
+    if (n < 1 || n > SMX_GEMV_GROUP_MAX) return fail(c, SMX_ERR_ARG, "gemv_f32 group of %d", n);
+    F32Flat g = {};
+    bool flat = n > 1;
+    size_t rows_total = 0, max_n = 0;
+    for (int i = 0; i < n && flat; i++) {
+        if (ws[i]->type != ws[0]->type || ws[i]->K != ws[0]->K) return fail(c, SMX_ERR_ARG, "gemv_f32 group mixes formats or row lengths");
+        flat = ws[i]->N <= 0x7fffffffu / 4 && f32_flat_geom(c, *ws[i], g);
+        rows_total += ws[i]->N;
+        max_n = std::max(max_n, ws[i]->N);
+    }
+    F32Jobs J = {};
+    size_t lds = 0;
+    if (flat) {
+        const Weight& w = *ws[0];
+        const size_t units = w.nblk * (w.type == kQ6_K ? 4 : (w.type == kQ8_0 ? 2 : 1)), xbytes = (w.K / 32) * (36 + 2) * 4;
+        const size_t cus = (size_t)c->num_cu;
+        flat = false;
+        for (size_t rounds = 1; rounds <= 64 && !flat; rounds++) {   // whole rounds of workgroups, as in f32_flat_geom
+            size_t rows = (rows_total + cus * rounds - 1) / (cus * rounds), total;
+            for (;; rows++) {   // the items' workgroups round up: rows per workgroup such that they still fit
+                total = 0;
+                for (int i = 0; i < n; i++) total += (ws[i]->N + rows - 1) / rows;
+                if (total <= cus * rounds || rows >= max_n) break;
+            }
+            lds = xbytes + rows * units / g.gl * 4;
+            if (rows * units >= 60000 || lds > 128 * 1024) continue;
+            flat = true;
+            J.n_total = 0;
+            for (int i = 0; i < SMX_GEMV_GROUP_MAX; i++) J.first[i] = 0x7fffffff;
+            for (int i = 0; i < n; i++) {
+                J.first[i] = J.n_total;
+                J.n_total += (int)((ws[i]->N + rows - 1) / rows);
+                J.job[i].W = {ws[i]->scales, (const uint4*)ws[i]->quants, (const uint4*)ws[i]->qh, (const uint2*)ws[i]->sc};
+                J.job[i].x = xs[i];
+                J.job[i].y = ys[i];
+                J.job[i].N = (int)ws[i]->N;
+            }
+            J.nblk = (int)w.nblk;
+            J.magic_u = (unsigned)(((1ull << 32) + units - 1) / units);
+        }
+    }
+    if (!flat) {
+        for (int i = 0; i < n; i++) {
+            int rc = launch_gemv_f32(c, *ws[i], xs[i], ys[i]);
+            if (rc != SMX_OK) return rc;
+        }
+        return SMX_OK;
+    }
+    const QType type = ws[0]->type;
+    ProfScope ps(c, type == kQ4_0 ? "gemv_f32_q4_0" : type == kQ8_0 ? "gemv_f32_q8_0" : "gemv_f32_q6_k");
+    if (type == kQ4_0) return launch_f32_group_type<OpsQ4_0, 3>(c, J, g.gl, lds);
+    if (type == kQ8_0) return launch_f32_group_type<OpsQ8_0, 3>(c, J, g.gl, lds);
+    return launch_f32_group_type<OpsQ6_K, 1>(c, J, g.gl, lds);
 }
 
 }  // namespace smx

@@ -226,6 +226,8 @@ int launch_gemv(smx_ctx* c, const Weight& w, const float* x, size_t m, float* y,
                 const ActScratch* sc = nullptr);
 // y[N] = dequant(W) . x with fp32 activations (no quantiser): the arithmetic of the reference's per-weight gemv.
 int launch_gemv_f32(smx_ctx* c, const Weight& w, const float* x, float* y);
+// n <= SMX_GEMV_GROUP_MAX of them, of one format and row length, in one launch (one each where the shape does not allow it).
+int launch_gemv_f32_group(smx_ctx* c, const Weight* const* ws, const float* const* xs, float* const* ys, int n);
 // Quantise m device rows and run the kernel that serves this (weight, m): the dot4 GEMV, the small-batch MFMA
 // kernel or the tiled GEMM (force_gemm: never the GEMV).  sc: caller-provided room for the quantised rows.
 int run_matmul_dev(smx_ctx* c, const Weight& w, const float* xs_dev, size_t m, float* y_dev, bool force_gemm, int32_t* dump,
