@@ -12,12 +12,14 @@ The directory name contains a dot, so load this package by path, e.g.
                                            submodule_search_locations=[".../strix.rs_amd"])
 """
 import ctypes as C
+import importlib.util
 import os
 
 import numpy as np
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libstrix_mi355.so")
+NATIVE_PATH = os.path.join(_HERE, "_smx_native.so")
 
 SMX_OK, SMX_NOT_RESIDENT = 1, 0
 GEMV_MAX_M = 8
@@ -150,6 +152,23 @@ def load_library():
     return L
 
 
+_native = None
+
+
+def load_native():
+    """The extension module with the hot calls (host/pybind.cpp; same library, no ctypes conversions)."""
+    global _native
+    if _native is None:
+        load_library()
+        if not os.path.exists(NATIVE_PATH):
+            raise FileNotFoundError(f"{NATIVE_PATH} is missing: build it with `python strix.rs_amd/build.py`")
+        spec = importlib.util.spec_from_file_location("_smx_native", NATIVE_PATH)
+        mod = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(mod)
+        _native = mod
+    return _native
+
+
 def _p(a):
     return None if a is None else a.ctypes.data_as(C.c_void_p)
 
@@ -251,17 +270,19 @@ class Mi355WeightAccel:
     """One device, one stream, resident quantized weights (WeightAccel, accel.rs:147)."""
 
     def __init__(self, device=0):
-        self._L = load_library()
+        self._L, self._n = load_library(), load_native()
+        self._a = None   # the context's address, for the native calls
         h = C.c_void_p()
         rc = self._L.smx_create(device, C.byref(h))
         if rc != SMX_OK:
             raise SmxError(rc, self._L.smx_last_error(None).decode())
         self._h = h
+        self._a = h.value
 
     def close(self):
         if getattr(self, "_h", None):
             self._L.smx_destroy(self._h)
-            self._h = None
+            self._h = self._a = None
 
     def __del__(self):
         self.close()
@@ -337,20 +358,22 @@ class Mi355WeightAccel:
         return (i.value, o.value) if ok else None
 
     def gemv(self, key, x, out_dim):
-        x = _c(x, np.float32).reshape(-1)
         y = np.empty(out_dim, np.float32)
-        ok = self._check(self._L.smx_gemv(self._h, key.encode(), _p(x), x.size, _p(y), y.size))
-        return y if ok else None
+        rc = self._n.gemv(self._a, key, x, y)
+        if rc is None:   # not a contiguous float32 array
+            rc = self._n.gemv(self._a, key, _c(x, np.float32), y)
+        return y if rc == SMX_OK or self._check(rc) else None
 
     def gemv_f32(self, key, x, out_dim):
         """gemv with fp32 activations (the arithmetic of the reference's per-weight gemv and of its CPU path)."""
-        x = _c(x, np.float32).reshape(-1)
         y = np.empty(out_dim, np.float32)
-        ok = self._check(self._L.smx_gemv_f32(self._h, key.encode(), _p(x), x.size, _p(y), y.size))
-        return y if ok else None
+        rc = self._n.gemv_f32(self._a, key, x, y)
+        if rc is None:
+            rc = self._n.gemv_f32(self._a, key, _c(x, np.float32), y)
+        return y if rc == SMX_OK or self._check(rc) else None
 
     def gemv_f32_dev(self, key, x_dev, y_dev):
-        return self._check(self._L.smx_gemv_f32_dev(self._h, key.encode(), x_dev, y_dev))
+        return self._check(self._n.gemv_f32_dev(self._a, key, x_dev, y_dev))
 
     def gemv_fused(self, key, act, a, b, out_dim, eps=0.0):
         """GEMV of producer(a, b): rmsnorm(a)*b, silu(a)*b or gelu_tanh(a)*b (kernels.rs:101-226), one launch."""
@@ -365,14 +388,19 @@ class Mi355WeightAccel:
         xs = _c(xs, np.float32)
         m, k = xs.shape
         y = np.empty((m, out_dim), np.float32)
-        ok = self._check(self._L.smx_gemv_rows(self._h, key.encode(), _p(xs), m, k, _p(y), y.size))
-        return y if ok else None
+        rc = self._n.gemv_rows(self._a, key, xs, m, y)
+        if rc is None:   # no rows: the library's own argument error
+            rc = self._L.smx_gemv_rows(self._h, key.encode(), _p(xs), m, k, _p(y), y.size)
+        return y if rc == SMX_OK or self._check(rc) else None
 
     def gemv_batch(self, calls, out_dims, f32=False):
         """calls: [(key, x)], out_dims: [out_dim]; returns [array | None] (accel.rs:397).  f32: the arithmetic of gemv_f32."""
         n = len(calls)
-        xs = [_c(x, np.float32).reshape(-1) for _, x in calls]
         ys = [np.empty(d, np.float32) for d in out_dims]
+        rc = self._n.gemv_batch(self._a, 1 if f32 else 0, calls, ys)
+        if rc == SMX_OK:
+            return ys
+        xs = [_c(x, np.float32).reshape(-1) for _, x in calls]   # a decline, an error or an array to convert: item by item
         keys = (C.c_char_p * n)(*[k.encode() for k, _ in calls])
         xp = (C.c_void_p * n)(*[x.ctypes.data for x in xs])
         yp = (C.c_void_p * n)(*[y.ctypes.data for y in ys])
@@ -390,32 +418,39 @@ class Mi355WeightAccel:
 
     def prefill_q8_gemm(self, key, xs, m, out_dim):
         """y[m][out_dim] token-major (accel.rs:213)."""
-        xs = _c(xs, np.float32).reshape(m, -1)
         y = np.empty((m, out_dim), np.float32)
-        ok = self._check(self._L.smx_gemm(self._h, key.encode(), _p(xs), m, xs.shape[1], _p(y), y.size))
-        return y if ok else None
+        rc = self._n.gemm(self._a, key, xs, m, y)
+        if rc is None:
+            xs = _c(xs, np.float32).reshape(m, -1)
+            rc = self._L.smx_gemm(self._h, key.encode(), _p(xs), m, xs.shape[1], _p(y), y.size)
+        return y if rc == SMX_OK or self._check(rc) else None
 
     def lm_head_argmax_rows(self, key, xs, m):
-        xs = _c(xs, np.float32).reshape(m, -1)
         out = np.empty(m, np.uint32)
-        ok = self._check(self._L.smx_lm_head_argmax_rows(self._h, key.encode(), _p(xs), m, xs.shape[1], _p(out)))
-        return out if ok else None
+        rc = self._n.lm_head_argmax_rows(self._a, key, xs, m, out)
+        if rc is None:
+            xs = _c(xs, np.float32).reshape(m, -1)
+            rc = self._L.smx_lm_head_argmax_rows(self._h, key.encode(), _p(xs), m, xs.shape[1], _p(out))
+        return out if rc == SMX_OK or self._check(rc) else None
 
     def moe_ffn(self, layer, ids, wexp, x, sgate=0.0):
-        ids, wexp, x = _c(ids, np.int32), _c(wexp, np.float32), _c(x, np.float32).reshape(-1)
-        y = np.empty(x.size, np.float32)
-        ok = self._check(self._L.smx_moe_ffn(self._h, layer, _p(ids), _p(wexp), ids.size, _p(x), x.size,
-                                             sgate, _p(y), y.size))
-        return y if ok else None
+        y = np.empty(np.size(x), np.float32)
+        rc = self._n.moe_ffn(self._a, layer, ids, wexp, x, sgate, y)
+        if rc is None:
+            ids, wexp, x = _c(ids, np.int32), _c(wexp, np.float32), _c(x, np.float32).reshape(-1)
+            rc = self._L.smx_moe_ffn(self._h, layer, _p(ids), _p(wexp), ids.size, _p(x), x.size, sgate, _p(y), y.size)
+        return y if rc == SMX_OK or self._check(rc) else None
 
     def moe_layer_q8_dev(self, layer, xs, m, plan, slot_tok, wslot):
         xs = _c(xs, np.float32).reshape(m, -1)
-        plan = _c(plan, np.uint64).reshape(-1, 3)
-        slot_tok, wslot = _c(slot_tok, np.int32), _c(wslot, np.float32)
         y = np.empty_like(xs)
-        ok = self._check(self._L.smx_moe_layer(self._h, layer, _p(xs), m, _p(plan), plan.shape[0],
-                                               _p(slot_tok), _p(wslot), slot_tok.size, _p(y), y.size))
-        return y if ok else None
+        rc = self._n.moe_layer(self._a, layer, xs, m, plan, slot_tok, wslot, y)
+        if rc is None:
+            plan = _c(plan, np.uint64).reshape(-1, 3)
+            slot_tok, wslot = _c(slot_tok, np.int32), _c(wslot, np.float32)
+            rc = self._L.smx_moe_layer(self._h, layer, _p(xs), m, _p(plan), plan.shape[0], _p(slot_tok), _p(wslot), slot_tok.size,
+                                       _p(y), y.size)
+        return y if rc == SMX_OK or self._check(rc) else None
 
     def moe_layer_ffn(self, layer, plan, xs, rows):
         """plan: (expert, rows) pairs; xs[rows][hidden] expert-major; returns dy[rows][hidden] (accel.rs:238-246)."""
@@ -433,10 +468,12 @@ class Mi355WeightAccel:
 
     def moe_layer_resident(self, layer, xs_dev, m, plan, slot_tok, wslot, y_dev):
         """moe_layer_q8_dev with activations and result already on the device (enqueue only)."""
-        plan = _c(plan, np.uint64).reshape(-1, 3)
-        slot_tok, wslot = _c(slot_tok, np.int32), _c(wslot, np.float32)
-        return self._check(self._L.smx_moe_layer_dev(self._h, layer, xs_dev, m, _p(plan), plan.shape[0],
-                                                     _p(slot_tok), _p(wslot), slot_tok.size, y_dev))
+        rc = self._n.moe_layer_dev(self._a, layer, xs_dev, m, plan, slot_tok, wslot, y_dev)
+        if rc is None:
+            plan = _c(plan, np.uint64).reshape(-1, 3)
+            slot_tok, wslot = _c(slot_tok, np.int32), _c(wslot, np.float32)
+            rc = self._L.smx_moe_layer_dev(self._h, layer, xs_dev, m, _p(plan), plan.shape[0], _p(slot_tok), _p(wslot), slot_tok.size, y_dev)
+        return self._check(rc)
 
     # -- parity instrumentation
     def quantize(self, x, k):
@@ -511,40 +548,35 @@ class Mi355WeightAccel:
         self._check(self._L.smx_sync(self._h))
 
     def gemv_dev(self, key, xs_dev, m, y_dev):
-        return self._check(self._L.smx_gemv_dev(self._h, key.encode(), xs_dev, m, y_dev))
+        return self._check(self._n.gemv_dev(self._a, key, xs_dev, m, y_dev))
 
     def gemv_noalloc_dev(self, key, xs_dev, m, y_dev):
         """gemv_dev that allocates nothing (static device scratch; m <= 8, in_dim <= 16384)."""
-        return self._check(self._L.smx_gemv_noalloc_dev(self._h, key.encode(), xs_dev, m, y_dev))
+        return self._check(self._n.gemv_noalloc_dev(self._a, key, xs_dev, m, y_dev))
 
     def gemv_batch_dev(self, keys, xs_dev, ys_dev):
-        n = len(keys)
-        k = (C.c_char_p * n)(*[s.encode() for s in keys])
-        xp = (C.c_void_p * n)(*xs_dev)
-        yp = (C.c_void_p * n)(*ys_dev)
-        return self._check(self._L.smx_gemv_batch_dev(self._h, n, k, xp, yp))
+        return self._check(self._n.gemv_batch_dev(self._a, keys, xs_dev, ys_dev))
 
     def gemv_fused_dev(self, keys, act, a_dev, b_dev, ys_dev, eps=0.0):
-        n = len(keys)
-        k = (C.c_char_p * n)(*[s.encode() for s in keys])
-        yp = (C.c_void_p * n)(*ys_dev)
-        return self._check(self._L.smx_gemv_fused_dev(self._h, n, k, int(act), a_dev, b_dev, float(eps), yp))
+        return self._check(self._n.gemv_fused_dev(self._a, keys, act, a_dev, b_dev, eps, ys_dev))
 
     def ffn_gate_up_dev(self, gate_key, up_key, act, x_dev, h_dev, norm=False, norm_w_dev=None, eps=0.0):
         """h = act(gate . x') * (up . x') in one launch, x' = x or rmsnorm(x) * norm_w (see smx_ffn_gate_up_dev)."""
-        return self._check(self._L.smx_ffn_gate_up_dev(self._h, gate_key.encode(), up_key.encode(), int(act), x_dev,
-                                                       1 if norm else 0, norm_w_dev, float(eps), h_dev))
+        return self._check(self._n.ffn_gate_up_dev(self._a, gate_key, up_key, act, x_dev, 1 if norm else 0, norm_w_dev, eps, h_dev))
 
     def gemm_fused_dev(self, key, act, a_dev, b_dev, m, y_dev, eps=0.0):
         """Prefill rows through a producer + quantiser + int8 GEMM (see smx_gemm_fused_dev)."""
-        return self._check(self._L.smx_gemm_fused_dev(self._h, key.encode(), int(act), a_dev, b_dev, m, float(eps), y_dev))
+        return self._check(self._n.gemm_fused_dev(self._a, key, act, a_dev, b_dev, m, eps, y_dev))
 
     def gemm_dev(self, key, xs_dev, m, y_dev):
-        return self._check(self._L.smx_gemm_dev(self._h, key.encode(), xs_dev, m, y_dev))
+        return self._check(self._n.gemm_dev(self._a, key, xs_dev, m, y_dev))
 
     def moe_ffn_dev(self, layer, ids, wexp, x_dev, y_dev):
-        ids, wexp = _c(ids, np.int32), _c(wexp, np.float32)
-        return self._check(self._L.smx_moe_ffn_dev(self._h, layer, _p(ids), _p(wexp), ids.size, x_dev, y_dev))
+        rc = self._n.moe_ffn_dev(self._a, layer, ids, wexp, x_dev, y_dev)
+        if rc is None:
+            ids, wexp = _c(ids, np.int32), _c(wexp, np.float32)
+            rc = self._L.smx_moe_ffn_dev(self._h, layer, _p(ids), _p(wexp), ids.size, x_dev, y_dev)
+        return self._check(rc)
 
     def moe_route(self, logits, k):
         """Router on the device (topk_router, kernels.rs:1846-1872): (ids[k] i32, w[k] f32)."""
@@ -554,7 +586,7 @@ class Mi355WeightAccel:
         return ids, w
 
     def moe_route_dev(self, logits_dev, ne, k, ids_dev, w_dev):
-        return self._check(self._L.smx_moe_route_dev(self._h, logits_dev, ne, k, ids_dev, w_dev))
+        return self._check(self._n.moe_route_dev(self._a, logits_dev, ne, k, ids_dev, w_dev))
 
     def moe_router_dev(self, key, x_dev, k, ids_dev, w_dev, logits_dev=None):
         """Router logits (GEMV of the resident router weight) + softmax + top-k in one call."""
@@ -562,11 +594,11 @@ class Mi355WeightAccel:
 
     def moe_ffn_logits_dev(self, layer, logits_dev, k, x_dev, y_dev, ids_dev, w_dev):
         """Routed expert FFN of a decode token from the router logits (routing inside the gate/up launch where it serves)."""
-        return self._check(self._L.smx_moe_ffn_logits_dev(self._h, layer, logits_dev, k, x_dev, y_dev, ids_dev, w_dev))
+        return self._check(self._n.moe_ffn_logits_dev(self._a, layer, logits_dev, k, x_dev, y_dev, ids_dev, w_dev))
 
     def moe_ffn_routed_dev(self, layer, ids_dev, w_dev, k, x_dev, y_dev):
         """moe_ffn_dev reading the routing from device memory at run time (capturable with new routing)."""
-        return self._check(self._L.smx_moe_ffn_routed_dev(self._h, layer, ids_dev, w_dev, k, x_dev, y_dev))
+        return self._check(self._n.moe_ffn_routed_dev(self._a, layer, ids_dev, w_dev, k, x_dev, y_dev))
 
     def moe_shexp_dev(self, layer, sgate, x_dev, y_dev):
         """y_dev += sgate * shared_expert(x_dev) (decode.rs:1820-1855)."""
@@ -581,7 +613,7 @@ class Mi355WeightAccel:
         return g
 
     def graph_launch(self, g):
-        self._check(self._L.smx_graph_launch(self._h, g))
+        self._check(self._n.graph_launch(self._a, g))
 
     def graph_destroy(self, g):
         self._L.smx_graph_destroy(self._h, g)

@@ -4,6 +4,7 @@ import glob
 import os
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
@@ -55,8 +56,18 @@ def build(verbose=False, extra=(), incremental=False):
     _run([HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", LIB, *objs[:n]], "link " + LIB)
     if BENCH_SRC:
         _run([HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", BENCH_LIB, *objs[n:]], "link " + BENCH_LIB)
+    build_pybind()
     build_selftest()
     return LIB
+
+
+def build_pybind():
+    """The CPython extension module with the hot calls (host compiler only); it links to the library beside it."""
+    out = os.path.join(HERE, "_smx_native.so")
+    cmd = ["g++", "-std=c++17", "-O2", "-Wall", "-shared", "-fPIC", "-I" + sysconfig.get_paths()["include"],
+           os.path.join(HERE, "host", "pybind.cpp"), "-o", out, "-L" + HERE, "-lstrix_mi355", "-Wl,-rpath,$ORIGIN"]
+    _run(cmd, "g++ host/pybind.cpp")
+    return out
 
 
 def build_selftest():
