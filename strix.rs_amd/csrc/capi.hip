@@ -4,6 +4,7 @@
 #include <cstring>
 
 #include "detmath.h"
+#include "hostpipe.h"
 #include "smx_internal.h"
 
 using namespace smx;
@@ -127,6 +128,31 @@ int run_matmul_dev(smx_ctx* c, const Weight& w, const float* xs_dev, size_t m, f
 
 namespace {
 
+// A matmul whose rows and results are large: groups of rows pass through copy in, kernels and copy out one behind the other,
+// so that the bus carries both directions while the device computes.  A group is 256 rows (two token tiles of the GEMM:
+// smaller ones lose more in the kernel than they bring) and at least 4 MB of transfers; the first one of several is 128 rows,
+// so that the copy out starts earlier.
+int matmul_host_large(smx_ctx* c, const Weight& w, const float* xs, size_t m, float* y, bool force_gemm) {
+    HostPipe* hp;
+    int rc = host_pipe(c, &hp);
+    if (rc != SMX_OK) return rc;
+    const size_t per_row = (w.K + w.N) * 4;
+    size_t group = std::max<size_t>(256, ((size_t(4) << 20) / per_row + 255) & ~size_t(255));
+    rc = hp->begin(c);
+    for (size_t r = 0; r < m && rc == SMX_OK;) {
+        const size_t n = r == 0 && group == 256 && m >= 384 ? 128 : m - r < 2 * group ? m - r : group;
+        float* xd = (float*)c->xf32.p + r * w.K;
+        float* yd = (float*)c->yf32.p + r * w.N;
+        rc = hp->in(c, xd, xs + r * w.K, n * w.K * 4);
+        if (rc == SMX_OK) rc = hp->in_done(c);
+        hp->populate(y + r * w.N, n * w.N * 4);   // behind this group's rows, in front of the next one's
+        if (rc == SMX_OK) rc = run_matmul_dev(c, w, xd, n, yd, force_gemm, nullptr, nullptr);
+        if (rc == SMX_OK) rc = hp->out(c, y + r * w.N, yd, n * w.N * 4);
+        r += n;
+    }
+    return hp->end(c, rc);
+}
+
 int matmul_host(smx_ctx* c, const char* key, const float* xs, size_t m, size_t in_dim, float* y, size_t y_cap,
                 bool force_gemm, const char* who) {
     if (!c) return SMX_ERR_ARG;
@@ -141,31 +167,38 @@ int matmul_host(smx_ctx* c, const char* key, const float* xs, size_t m, size_t i
     int rc;
     if ((rc = ensure(c, c->xf32, m * w->K * 4)) != SMX_OK) return rc;
     if ((rc = ensure(c, c->yf32, m * w->N * 4)) != SMX_OK) return rc;
-    // small transfers go through pinned staging: a pageable hipMemcpyAsync costs ~10 us each way
     const size_t xb = m * w->K * 4, yb = m * w->N * 4;
-    const bool pinned = xb + yb <= (size_t(8) << 20);
-    if (pinned) {
-        if ((rc = ensure_host(c, c->hx, xb)) != SMX_OK) return rc;
-        if ((rc = ensure_host(c, c->hy, yb)) != SMX_OK) return rc;
-        memcpy(c->hx.p, xs, xb);
-    }
+    if (xb + yb >= kHostPipeBytes) return matmul_host_large(c, *w, xs, m, y, force_gemm);
     // Up to 4 rows on the GEMV kernels (plain loads of x, plain stores of y): the kernel reads the pinned staging and writes the
     // pinned result itself.  A copy command each way costs more than the kernel (measured per call with one synchronisation:
     // kernel alone 13 us, + host-to-device copy 16, + device-to-host copy 25; kernel on the pinned buffers 17).
     const bool gemv_path = m <= 4 && !force_gemm && !skinny_serves(*w, m);
+    if (!gemv_path && c->tune_host_io == 0) {
+        HostPipe* hp;
+        const float* x;
+        if ((rc = host_send(c, c->xf32.p, xs, xb, true, y, yb, &hp, &x)) != SMX_OK) return rc;   // (the quantiser reads a row once)
+        rc = run_matmul_dev(c, *w, x, m, (float*)c->yf32.p, force_gemm, nullptr, nullptr);
+        return host_receive(c, y, c->yf32.p, yb, hp, rc);
+    }
+    // small transfers go through pinned staging: a pageable hipMemcpyAsync costs ~10 us each way
+    if ((rc = ensure_host(c, c->hx, xb)) != SMX_OK) return rc;
+    if ((rc = ensure_host(c, c->hy, yb)) != SMX_OK) return rc;
+    memcpy(c->hx.p, xs, xb);
     // (x: one row of up to 64 KB; every workgroup reads the whole row, and several long rows read over the bus by 256
     // workgroups cost more than the copy command: Q8_0 2560 x 9728, 3 rows, 39 - 45 us against 34)
-    const bool x_direct = pinned && gemv_path && m == 1 && xb <= (size_t(64) << 10) && c->tune_host_io != 1 && c->tune_host_io != 2;
-    const bool y_direct = pinned && gemv_path && c->tune_host_io != 1;
-    if (!x_direct)
-        SMX_HIP(c, hipMemcpyAsync(c->xf32.p, pinned ? (const void*)c->hx.p : (const void*)xs, xb, hipMemcpyHostToDevice, c->stream));
+    const bool x_direct = gemv_path && m == 1 && xb <= (size_t(64) << 10) && c->tune_host_io != 1 && c->tune_host_io != 2;
+    const bool y_direct = gemv_path && c->tune_host_io != 1;
+    if (!x_direct && c->tune_host_io == 0) {
+        if ((rc = staged_to_device(c, c->xf32.p, c->hx.p, xb)) != SMX_OK) return rc;
+    } else if (!x_direct) {
+        SMX_HIP(c, hipMemcpyAsync(c->xf32.p, c->hx.p, xb, hipMemcpyHostToDevice, c->stream));
+    }
     rc = run_matmul_dev(c, *w, x_direct ? (const float*)c->hx.p : (const float*)c->xf32.p, m, y_direct ? (float*)c->hy.p : (float*)c->yf32.p,
                         force_gemm, nullptr, nullptr);
     if (rc != SMX_OK) return rc;
-    if (!y_direct) SMX_HIP(c, hipMemcpyAsync(pinned ? (void*)c->hy.p : (void*)y, c->yf32.p, yb, hipMemcpyDeviceToHost, c->stream));
-    if (!pinned) SMX_HIP(c, hipStreamSynchronize(c->stream));
-    else if ((rc = stream_wait(c)) != SMX_OK) return rc;
-    if (pinned) memcpy(y, c->hy.p, yb);
+    if (!y_direct) SMX_HIP(c, hipMemcpyAsync(c->hy.p, c->yf32.p, yb, hipMemcpyDeviceToHost, c->stream));
+    if ((rc = stream_wait(c)) != SMX_OK) return rc;
+    memcpy(y, c->hy.p, yb);
     return SMX_OK;
 }
 
@@ -321,8 +354,11 @@ int smx_lm_head_argmax_rows(smx_ctx* c, const char* key, const float* xs, size_t
         memcpy(c->hx.p, xs, xb);
     }
     if ((rc = ensure_host(c, c->hy, m * 4)) != SMX_OK) return rc;
-    SMX_HIP(c, hipMemcpyAsync(c->xf32.p, pinned ? (const void*)c->hx.p : (const void*)xs, xb, hipMemcpyHostToDevice, c->stream));
-    rc = run_matmul_dev(c, *w, (const float*)c->xf32.p, m, (float*)c->yf32.p, false, nullptr, nullptr);
+    // (kernels that read a row once take it from the staging)
+    const bool direct = pinned && !(m <= 4 && !skinny_serves(*w, m));
+    if (!pinned) SMX_HIP(c, hipMemcpyAsync(c->xf32.p, xs, xb, hipMemcpyHostToDevice, c->stream));
+    else if (!direct && (rc = staged_to_device(c, c->xf32.p, c->hx.p, xb)) != SMX_OK) return rc;
+    rc = run_matmul_dev(c, *w, direct ? (const float*)c->hx.p : (const float*)c->xf32.p, m, (float*)c->yf32.p, false, nullptr, nullptr);
     if (rc != SMX_OK) return rc;
     rc = launch_argmax_rows(c, (const float*)c->yf32.p, m, w->N, c->tab.p, (unsigned*)c->hy.p);
     if (rc != SMX_OK) return rc;

@@ -3,6 +3,7 @@
 #include <chrono>
 #include <cstring>
 
+#include "hostpipe.h"
 #include "smx_internal.h"
 
 namespace smx {
@@ -340,7 +341,7 @@ int smx_create(int device, smx_ctx** out) {
         delete c;
         return fail(nullptr, SMX_ERR_HIP, "smx_create: hipEventCreate failed");
     }
-    e = hipHostMalloc((void**)&c->hflag, 64, hipHostMallocDefault);
+    e = hipHostMalloc((void**)&c->hflag, kHostFlags * 4, hipHostMallocDefault);
     if (e != hipSuccess) {
         (void)hipEventDestroy(c->t0);
         (void)hipEventDestroy(c->t1);
@@ -348,7 +349,7 @@ int smx_create(int device, smx_ctx** out) {
         delete c;
         return hip_fail(nullptr, e, "hipHostMalloc");
     }
-    *c->hflag = 0;
+    memset(c->hflag, 0, kHostFlags * 4);   // sequence numbers start at 1
     if (noalloc_init(c) != SMX_OK) {   // the static scratch array of the allocation-free entry point, on this device
         g_create_err = c->err;
         (void)hipHostFree(c->hflag);
@@ -366,6 +367,7 @@ void smx_destroy(smx_ctx* c) {
     if (!c) return;
     (void)hipSetDevice(c->device);
     (void)hipStreamSynchronize(c->stream);
+    delete c->pipe;
     for (auto& kv : c->weights) free_weight(kv.second);
     for (auto& kv : c->moe) {
         free_weight(kv.second.gate);

@@ -1115,7 +1115,7 @@ static int moe_layer_impl(smx_ctx* c, size_t layer, const float* xs, size_t m, c
         if ((rc = ensure(c, c->xf32, m * hidden * 4)) != SMX_OK) return rc;
         if ((rc = ensure(c, c->yf32, m * hidden * 4)) != SMX_OK) return rc;
     }
-    const float* x_dev = on_device ? xs : (const float*)c->xf32.p;
+    const float* x_dev = xs;
     float* y_dev = on_device ? y : (float*)c->yf32.p;
     std::vector<GemmTile> tiles_gu, tiles_dn;
     build_tiles(plan, nplan, L.eff, &tiles_gu);
@@ -1124,22 +1124,26 @@ static int moe_layer_impl(smx_ctx* c, size_t layer, const float* xs, size_t m, c
     const size_t o_st = tb.add(slot_tok, slots * 4), o_ws = tb.add(wslot, slots * 4), o_tp = tb.add(tok_ptr.data(), (m + 1) * 4),
                  o_ts = tb.add(tok_slots.data(), slots * 4), o_t1 = tb.add(tiles_gu.data(), tiles_gu.size() * sizeof(GemmTile)),
                  o_t2 = tb.add(tiles_dn.data(), tiles_dn.size() * sizeof(GemmTile));
-    if (!on_device) SMX_HIP(c, hipMemcpyAsync(c->xf32.p, xs, m * hidden * 4, hipMemcpyHostToDevice, c->stream));
-    if ((rc = tb.upload(c)) != SMX_OK) return rc;
+    HostPipe* hp = nullptr;
+    if (!on_device && (rc = host_send(c, c->xf32.p, xs, m * hidden * 4, true, y, m * hidden * 4, &hp, &x_dev)) != SMX_OK) return rc;
     SlotScratch ss;
-    rc = moe_slots_enqueue(c, L, x_dev, m, (const int*)(c->tab.p + o_st), slots, (const GemmTile*)(c->tab.p + o_t1), tiles_gu.size(),
-                           (const GemmTile*)(c->tab.p + o_t2), tiles_dn.size(), &ss);
-    if (rc != SMX_OK) return rc;
-    float* dy = ss.dy;
-    {
+    const auto compute = [&]() -> int {
+        int rc = tb.upload(c);
+        if (rc != SMX_OK) return rc;
+        rc = moe_slots_enqueue(c, L, x_dev, m, (const int*)(c->tab.p + o_st), slots, (const GemmTile*)(c->tab.p + o_t1), tiles_gu.size(),
+                               (const GemmTile*)(c->tab.p + o_t2), tiles_dn.size(), &ss);
+        if (rc != SMX_OK) return rc;
+        float* dy = ss.dy;
         ProfScope ps(c, "moe_combine");
         hipLaunchKernelGGL(moe_combine_kernel, dim3((unsigned)((hidden / 4 + 255) / 256), (unsigned)m), dim3(256), 0, c->stream,
                            dy, (const int*)(c->tab.p + o_tp), (const int*)(c->tab.p + o_ts),
                            (const float*)(c->tab.p + o_ws), y_dev, (int)hidden, ((uintptr_t)y_dev & 15) == 0);
         SMX_HIP(c, hipGetLastError());
-    }
+        return SMX_OK;
+    };
+    rc = compute();
     if (!on_device) {
-        SMX_HIP(c, hipMemcpyAsync(y, c->yf32.p, m * hidden * 4, hipMemcpyDeviceToHost, c->stream));
+        if ((rc = host_receive(c, y, c->yf32.p, m * hidden * 4, hp, rc)) != SMX_OK) return rc;
         if (stages) {
             const size_t eff = L.eff;
             if (stages->gu) {   // g and u are separate [slots][eff] planes on the device
@@ -1149,10 +1153,10 @@ static int moe_layer_impl(smx_ctx* c, size_t layer, const float* xs, size_t m, c
             if (stages->aq) SMX_HIP(c, hipMemcpyAsync(stages->aq, ss.aq, slots * eff, hipMemcpyDeviceToHost, c->stream));
             if (stages->ad) SMX_HIP(c, hipMemcpyAsync(stages->ad, ss.ad, slots * (eff / 32) * 4, hipMemcpyDeviceToHost, c->stream));
             if (stages->dy) SMX_HIP(c, hipMemcpyAsync(stages->dy, ss.dy, slots * hidden * 4, hipMemcpyDeviceToHost, c->stream));
+            SMX_HIP(c, hipStreamSynchronize(c->stream));
         }
-        SMX_HIP(c, hipStreamSynchronize(c->stream));
     }
-    return SMX_OK;
+    return rc;
     });
 }
 
@@ -1191,14 +1195,13 @@ int smx_moe_layer_ffn(smx_ctx* c, size_t layer, const int32_t* plan, size_t npla
     const size_t o_t1 = tb.add(tiles_gu.data(), tiles_gu.size() * sizeof(GemmTile)),
                  o_t2 = tb.add(tiles_dn.data(), tiles_dn.size() * sizeof(GemmTile));
     if ((rc = tb.upload(c)) != SMX_OK) return rc;
-    SMX_HIP(c, hipMemcpyAsync(c->xf32.p, xs, rows * hidden * 4, hipMemcpyHostToDevice, c->stream));
-    SlotScratch ss;
-    rc = moe_slots_enqueue(c, L, (const float*)c->xf32.p, rows, nullptr, rows, (const GemmTile*)(c->tab.p + o_t1), tiles_gu.size(),
+    HostPipe* hp = nullptr;
+    const float* x_dev;
+    if ((rc = host_send(c, c->xf32.p, xs, rows * hidden * 4, true, dy, rows * hidden * 4, &hp, &x_dev)) != SMX_OK) return rc;
+    SlotScratch ss = {};
+    rc = moe_slots_enqueue(c, L, x_dev, rows, nullptr, rows, (const GemmTile*)(c->tab.p + o_t1), tiles_gu.size(),
                            (const GemmTile*)(c->tab.p + o_t2), tiles_dn.size(), &ss);
-    if (rc != SMX_OK) return rc;
-    SMX_HIP(c, hipMemcpyAsync(dy, ss.dy, rows * hidden * 4, hipMemcpyDeviceToHost, c->stream));
-    SMX_HIP(c, hipStreamSynchronize(c->stream));
-    return SMX_OK;
+    return host_receive(c, dy, ss.dy, rows * hidden * 4, hp, rc);
     });
 }
 

@@ -15,6 +15,8 @@
 
 namespace smx {
 
+class HostPipe;
+
 enum QType { kQ4_0 = 2, kQ8_0 = 8, kQ6_K = 14 };
 
 // A resident weight: one device allocation, planes at 256-byte aligned offsets,
@@ -76,8 +78,9 @@ struct smx_ctx {
     smx::DevBuf raw;    // upload staging: the raw GGUF blocks of the tensor being repacked (kept up to kRawKeepBytes between uploads)
     smx::DevBuf hx, hy; // pinned HOST staging of the host-pointer calls' activations and results
     smx::DevBuf htab;   // pinned HOST staging of the small tables of enqueue-only calls
-    unsigned* hflag = nullptr;   // pinned HOST word that stream_wait's last kernel writes
-    unsigned flag_seq = 0;       // what it writes next
+    unsigned* hflag = nullptr;   // pinned HOST words: [0] stream_wait's, [64 ..] one per part of a result on its way (host_receive)
+    unsigned flag_seq = 0;       // what is written there next
+    smx::HostPipe* pipe = nullptr;   // transfers of large host-pointer calls (made by the first of them)
     hipEvent_t htab_done = nullptr;  // recorded after the last copy out of htab (null: htab is free)
 
     // tuning overrides (0 = automatic)
@@ -140,6 +143,20 @@ void release_device(smx_ctx* c, char* p);
 int ensure_host(smx_ctx* c, DevBuf& b, size_t bytes);
 // Waits until everything enqueued on the context's stream has run (the one synchronisation of a host-pointer call).
 int stream_wait(smx_ctx* c);
+// The context's HostPipe, and the size of a host-pointer call (bytes in + out) from which it pays.
+int host_pipe(smx_ctx* c, HostPipe** out);
+constexpr size_t kHostFlags = 1024;   // words at hflag
+constexpr size_t kHostPipeBytes = size_t(3) << 20;
+// One transfer in and one out around the kernels of a call: through the pinned staging buffers, or from kHostPipeBytes on
+// through the HostPipe (*hp, null otherwise).  *src is where the kernels find the rows: `dev`, or the pinned staging itself
+// when each of them is read once (read_once).  After a host_send that returned SMX_OK the call ends with host_receive,
+// which takes the error of what lies between and waits for everything.
+int host_send(smx_ctx* c, void* dev, const void* host, size_t bytes, bool read_once, void* result, size_t result_bytes, HostPipe** hp,
+              const float** src);
+// Pinned staging -> device by a kernel (whole floats): a copy command runs on another engine, whose signal the kernels
+// behind it wait for (lm_head_argmax_rows of three rows 228 -> 222 us).
+int staged_to_device(smx_ctx* c, void* dev, const void* staged, size_t bytes);
+int host_receive(smx_ctx* c, void* host, const void* dev, size_t bytes, HostPipe* hp, int rc);
 
 // Raises a kernel's dynamic-LDS limit when it asks for more than the 48 KB default (remembered per
 // context and kernel so that replays and captured launches do not repeat the call).

@@ -43,3 +43,44 @@ def test_arrays_of_other_layouts(accel, synth):
     assert np.array_equal(accel.lm_head_argmax_rows("hl", wide[:, ::2], 3), ids)
     batch = accel.gemv_batch([("hl", x1), ("absent", x1), ("hl", wide[1, ::2])], [N, N, N])
     assert np.array_equal(batch[0], accel.gemv("hl", x1, N)) and batch[1] is None and np.array_equal(batch[2], accel.gemv("hl", x[1], N))
+
+
+def _dev_gemm(accel, key, xs, N):
+    m, K = xs.shape
+    xd, yd = accel.dev_alloc(xs.nbytes), accel.dev_alloc(m * N * 4)
+    accel.h2d(xd, xs)
+    assert accel.gemm_dev(key, xd, m, yd)
+    y = accel.d2h(np.empty((m, N), np.float32), yd)
+    accel.dev_free(xd)
+    accel.dev_free(yd)
+    return y
+
+
+@pytest.mark.parametrize("ty,m,N,K", [(8, 5, 33, 96), (2, 40, 1001, 256), (8, 64, 4096, 2048), (8, 128, 4097, 1024), (14, 383, 999, 2560), (2, 513, 777, 1024),
+                                      (8, 900, 4096, 512), (8, 1500, 9001, 256), (8, 300, 256, 15360)])
+def test_large_transfers_equal_the_device_call(accel, synth, ty, m, N, K):
+    """Every route of a host call: the staging with whole and ragged 16 KB parts, one and several row groups through the ring, more
+    results than the ring holds (54 MB), inputs larger than it.  (Row groups may take another split-K: 1e-6 instead of equal bits.)"""
+    assert _up(accel, ty)("hp", synth.make_weight(ty, N, K, seed=N), K, N)
+    xs = synth.make_acts(m, K, seed=m)
+    want = _dev_gemm(accel, "hp", xs, N)
+    for _ in range(2):
+        got = accel.prefill_q8_gemm("hp", xs, m, N)
+        assert np.abs(got - want).max() <= 1e-6 * np.abs(want).max()
+
+
+@pytest.mark.parametrize("m,hidden", [(3, 256), (150, 512), (700, 1024)])
+def test_moe_layer_host_rows_equal_resident_rows(accel, synth, m, hidden):
+    ne, eff, k = 8, 256, 3
+    gate, up, down = synth.make_moe_q8(ne, hidden, eff, seed=hidden)
+    assert accel.upload_moe_q8(7, gate, up, down, hidden, eff, ne)
+    ids, w = synth.zipf_routing(m, ne, k, seed=m)
+    plan, tok, wslot = synth.group_by_expert(ids, w, ne)
+    xs = synth.make_acts(m, hidden, seed=3)
+    xd, yd = accel.dev_alloc(xs.nbytes), accel.dev_alloc(xs.nbytes)
+    accel.h2d(xd, xs)
+    assert accel.moe_layer_resident(7, xd, m, plan, tok, wslot, yd)
+    want = accel.d2h(np.empty_like(xs), yd)
+    accel.dev_free(xd)
+    accel.dev_free(yd)
+    assert np.array_equal(accel.moe_layer_q8_dev(7, xs, m, plan, tok, wslot), want)
