@@ -19,8 +19,8 @@ const Weight* find_weight(smx_ctx* c, const char* key) {
 // Scratch for m quantised rows of length K.
 int ensure_act(smx_ctx* c, size_t m, size_t K) {
     int rc;
-    if ((rc = ensure(c, c->xq, m * K)) != SMX_OK) return rc;
-    if ((rc = ensure(c, c->xd, m * (K / 32) * 4)) != SMX_OK) return rc;
+    if ((rc = ensure(c, c->xq, m * K + kReadSlack)) != SMX_OK) return rc;
+    if ((rc = ensure(c, c->xd, m * (K / 32) * 4 + kReadSlack)) != SMX_OK) return rc;
     return ensure(c, c->xs, m * (K / 32) * 4);
 }
 

@@ -229,7 +229,7 @@ static int build_weight(smx_ctx* c, QType type, const uint8_t* bytes, size_t nby
             c->raw.cap = 0;
         }
     };
-    hipError_t e = hipMalloc((void**)&w.base, w.bytes);
+    hipError_t e = hipMalloc((void**)&w.base, w.bytes + kReadSlack);
     if (e != hipSuccess) {
         (void)hipGetLastError();
         drop_raw();

@@ -13,71 +13,38 @@
 //     0x4B400000 so its i32 result, read as a float, is 12582912 + I exactly; one FMA with the
 //     exactly representable -dw*12582912 (dw is an f16 value) gives fl(dw*I) with no int->float
 //     conversion, a second FMA applies dx and accumulates: two VALU operations per output per block;
-//   * Q6_K weights (kernels.rs:1688-1735 q6_gemm_moe keeps them in their 210-byte form too): the 6-bit
-//     quants are widened to signed int8 (q - 32) while being staged, and because the format scales
-//     16-element sub-blocks each 32-block takes two v_mfma_i32_32x32x16_i8, one exact i32 per
-//     sub-block, each rescaled by its own d * sc (four VALU operations per output per 32-block);
+//   * Q6_K weights have a kernel of their own (gemm_q6.h);
 //   * split-K: grid.z slices of whole stages write fp32 partials that a second kernel sums in slice
 //     order (deterministic, unlike the reference's atomicAdd, kernels.rs:597).
-// Bound: dense int8 MFMA, 2*M*N*K operations.
+// Bound: 2*M*N*K int8 operations on the matrix cores plus 32 FMAs per MFMA; the two add up (a SIMD runs both at one power
+// budget: 17 ns per MFMA, 21 ns per 16 FMAs measured alone, 60 ns per MFMA with its 32 FMAs), which puts the exact rescale's
+// ceiling at 1.1 POPS.  What is left is every other instruction a wave issues, so the loop holds no bounds test, no 64-bit
+// address and no branch per row tile (see main_loop).  2048 tokens x 15360 x 3840: Q8_0 340 -> 303 us, Q4_0 350 -> 316 us with
+// row tiles counted at compile time, scalar stage offsets and the MFMAs issued one row tile ahead.
 #include <algorithm>
+#include <type_traits>
 
+#include "gemm_dev.h"
+#include "gemm_q6.h"
 #include "mfma_dev.h"
-#include "smx_internal.h"
 
 namespace smx {
 
-constexpr int BN = 128, KB = 4;
-constexpr int GRP = 1024;                   // 8 rows x 128 B of one stage: row r at r * 128, its 16-byte chunk c at slot (c + r) % 8
-constexpr int B_BYTES = 16 * GRP;           // 128 weight rows
-// A workgroup of NW waves covers 32 * NW tokens x 128 weight rows (NW = 8: 256 x 128, one workgroup
-// per CU; NW = 4: 128 x 128, two per CU).  The larger tile reads 25 % fewer operand bytes per
-// operation through L2, which is what bounds the kernel after the epilogue FMAs.
-constexpr int a_bytes(int NW) { return 4 * NW * GRP; }
-constexpr int stage_bytes(int NW, bool q6 = false) { return a_bytes(NW) + B_BYTES + (q6 ? 2 : 1) * KB * 128 * 4 + KB * 32 * NW * 4; }
-// four 6-bit quants (low nibbles in lo4, the two high bits in hi2) -> four signed bytes q - 32
-__device__ __forceinline__ unsigned q6_bytes(unsigned lo4, unsigned hi2) {
-    return (((lo4 & 0x0f0f0f0fu) | ((hi2 & 0x03030303u) << 4) | 0x80808080u) - 0x20202020u) ^ 0x80808080u;
-}
+constexpr int STAGE_BYTES = A_BYTES + B_BYTES + KB * 128 * 4 + KB * BM * 4;
 
-// Operand fragments of one 32-block.  SUB = 1: one K = 32 MFMA per row tile, a lane holds 16 k of
-// its row; SUB = 2 (Q6_K): two K = 16 MFMAs, a lane holds 8 k of each 16-element sub-block.
-template <int SUB>
+// Operand fragments on their way from LDS to the matrix cores.  The weight fragments of several row tiles are not
+// double-buffered: a row tile's registers are refilled for the next block as soon as its MFMA has been issued (a single row
+// tile's MFMA comes too soon after that: it takes b[0] and b[1] in turn).
 struct GemmFrag {
-    v4i a;           // this wave's 32 tokens x 32 k
-    v4i b[4];        // 4 x (32 weight rows x 32 k)
-    float4 dx[4];    // SUB = 1: activation scales of the 16 tokens this lane accumulates
-    float dxv;       // SUB = 2: one scale per lane: lane n of each 16-lane row holds the scale of the token of accumulator n
-    float dw[4][SUB];  // weight scale of this lane's row in each of the 4 row tiles (per sub-block)
+    v4i a[2];         // this wave's 32 tokens x 32 k, two blocks in turn; a lane holds 16 k of its token
+    float4 dx[2][4];  // activation scales of the 16 tokens this lane accumulates
+    v4i b[4];         // 4 x (32 weight rows x 32 k)
+    float4 dw[4];     // weight scales of this lane's row in each row tile, the four blocks of the stage
 };
 
-constexpr int FMT_Q8 = 0, FMT_Q4 = 1, FMT_Q6 = 2;
-
-// Optional per-workgroup timeline (development builds only: -DSMX_GEMM_TRACE; compiled out of the library): start and end of
-// every workgroup of a launch on the constant 100 MHz clock, with its live tokens and the hardware unit it ran on.
-#ifdef SMX_GEMM_TRACE
-__device__ unsigned long long* g_gemm_trace = nullptr;   // [(grouped gate/up launch: 4096) + workgroup][4]
-#define SMX_GEMM_T0 const unsigned long long smx_t0 = wall_clock64()
-#define SMX_GEMM_T1(LIVE, OP)                                                                                                  \
-    do {                                                                                                                        \
-        if (threadIdx.x == 0 && g_gemm_trace && blockIdx.x < 4096) {                                                            \
-            unsigned long long* o_ = g_gemm_trace + ((size_t)(p.nops > 1 ? 4096 : 0) + blockIdx.x) * 4;                         \
-            o_[0] = smx_t0; o_[1] = wall_clock64(); o_[2] = (unsigned long long)(LIVE) | ((unsigned long long)(OP) << 32);      \
-            o_[3] = (unsigned long long)__builtin_amdgcn_s_getreg(63492) | ((unsigned long long)__builtin_amdgcn_s_getreg(63508) << 32); \
-        }                                                                                                                       \
-    } while (0)
-#else
-#define SMX_GEMM_T0 do { } while (0)
-#define SMX_GEMM_T1(LIVE, OP) do { } while (0)
-#endif
-
-template <int FMT, bool DUMP, int NW>
-__global__ __launch_bounds__(64 * NW, NW == 8 ? 1 : 2) void gemm_i8_kernel(GemmArgs p) {
+template <bool Q4, bool DUMP>
+__global__ __launch_bounds__(64 * NW, 2) void gemm_i8_kernel(GemmArgs p) {
     SMX_GEMM_T0;
-    constexpr bool Q4 = FMT == FMT_Q4, Q6 = FMT == FMT_Q6;
-    static_assert(!Q6 || NW == 4, "the Q6_K staging map is written for 256 threads");
-    constexpr int SUB = Q6 ? 2 : 1;  // scaled sub-blocks per 32-block
-    constexpr int BM = 32 * NW, A_BYTES = a_bytes(NW), STAGE_BYTES = stage_bytes(NW, Q6);
     constexpr int BG = 16 / NW;  // 8-row groups of B each wave stages
     extern __shared__ __align__(16) char smem[];
     const int tid = threadIdx.x, lane = tid & 63;
@@ -85,48 +52,11 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? 1 : 2) void gemm_i8_kernel(GemmA
     const int K = p.nb * 32;
     const unsigned smem_base = lds_addr(smem);
 
-    // tile coordinates; consecutive logical tiles share a weight strip, and each XCD (blockIdx % 8)
-    // gets a contiguous range of logical tiles so its L2 holds few strips
-    int t = blockIdx.x;
-    int tok0, row0, col0, M_end, N_end;
-    int op_i = blockIdx.y;
-    if (p.tiles) {  // grouped (MoE): tile table, A rows are slots of one expert, B rows that expert's rows
-        // the operands (gate, up) of a tile are neighbours in the launch order, so that the table's order
-        // (longest tiles first) holds for all of them
-        op_i = t % p.nops;
-        t /= p.nops;
-        const GemmTile tl = p.tiles[t];
-        tok0 = tl.tok0; M_end = tl.tok_end; row0 = tl.row0; N_end = tl.row_end; col0 = tl.col0;
-    } else {
-        // The first `narrow` strips of N are 96 rows high and dispatched last (see launch_gemm); each part (128-row strips,
-        // 96-row strips) is walked on its own.
-        const int full_strips = p.tiles_n - p.narrow;
-        const int t_full = full_strips * p.tiles_m;
-        const bool nar = t >= t_full;   // never without narrow strips
-        if (nar) t -= t_full;
-        const int ns = nar ? p.narrow : full_strips;
-        const int T = ns * p.tiles_m;
-        if (p.xcd_remap & (nar ? 2 : 1)) t = (t & 7) * (T >> 3) + (t >> 3);
-        // logical order: token-tile group (walk_gm token tiles), weight strip, token tile inside the group
-        const int per_group = p.walk_gm * ns;
-        const int grp = t / per_group, in_grp = t - grp * per_group;
-        const int tn = in_grp / p.walk_gm, tm = grp * p.walk_gm + (in_grp - tn * p.walk_gm);
-        tok0 = tm * p.tile_m; M_end = min(p.M, tok0 + p.tile_m);
-        row0 = nar ? tn * 96 : p.narrow * 96 + tn * BN;
-        N_end = nar ? row0 + 96 : p.N;
-        col0 = row0;
-    }
-    const GemmOperand op = p.op[op_i];
-    // Wave roles.  A full tile gives each wave 32 tokens x 128 rows (4 row tiles).  A tile with few live
-    // tokens (the tail of M, a small expert group) would leave three of the four waves idle, so its waves
-    // share the token sub-tiles that are live and split the rows: <= 32 tokens: every wave takes the first
-    // 32 tokens and ONE row tile; <= 64 tokens: two waves per token half, two row tiles each.
-    const int live_tok = M_end - tok0;
-    const int tw = NW == 4 ? (live_tok <= 32 ? 0 : live_tok <= 64 ? (wave & 1) : wave) : wave;   // token sub-tile
-    const int live_rows = min(N_end - row0, BN);
-    const int full_cnt = (live_rows + 31) >> 5;   // a tile at the end of N, or a 96-row strip: only the row tiles that exist
-    const int nt_cnt = NW == 4 ? (live_tok <= 32 ? 1 : live_tok <= 64 ? 2 : full_cnt) : full_cnt;   // row tiles of this wave
-    const int nt_base = NW == 4 ? (live_tok <= 32 ? wave : live_tok <= 64 ? (wave >> 1) * 2 : 0) : 0;
+    const TileAt at = gemm_tile_at(p);
+    const WaveRole role = gemm_wave_role(at, wave);
+    const int tok0 = at.tok0, row0 = at.row0, M_end = at.M_end, N_end = at.N_end;
+    const int live_tok = role.live_tok, live_rows = role.live_rows, tw = role.tw, nt_cnt = role.nt_cnt, nt_base = role.nt_base;
+    const GemmOperand op = p.op[at.op_i];
 
     const int nstage_total = (p.nb + KB - 1) / KB;
     const int s_begin = blockIdx.z * p.stages_per_slice;
@@ -137,129 +67,78 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? 1 : 2) void gemm_i8_kernel(GemmA
     //      (scattered 16-byte fetches run at a fraction of the L2 -> CU rate), and lane (r, slot)
     //      fetches chunk (slot - r) % 8, so that chunk c of the 8 rows of a group lies in 8 different
     //      bank groups and every MFMA fragment read below is a conflict-free 128-bit load.
-    //      Rows past the tile's end and blocks past K re-read valid memory (clamped addresses) and
-    //      are neutralised by zero scales.  Q4_0 weights pass through registers to be widened. ----
+    //      Rows past the tile's end re-read its last one (clamped addresses), blocks past K read whatever follows the row
+    //      (up to 96 bytes of quants behind the last one: weights and activation buffers carry kReadSlack bytes more), and
+    //      both are neutralised by zero scales.  Q4_0 weights pass through registers to be widened. ----
     const int g_rowlo = lane >> 3, g_chunk = ((lane & 7) - g_rowlo) & 7;
     const int q_bi = lane & 3, q_rowlo = lane >> 2;   // Q4_0 B: lane = [row:4][block:2], 64 contiguous bytes per row
-    constexpr int QG = Q4 ? 8 / NW : 1;  // Q4_0 B: 16-byte blocks per thread per stage
-    // Q6_K B: thread = [row:7][p:1]; per stage (one half of a superblock) it reads ql[16p..], ql[32 + 16p..]
-    // and qh[16p..] of that half and makes the four 16-byte chunks 2j + p, j = 0..3 (ggml_quant.rs:417-426)
-    const int q6_row = tid >> 1, q6_p = tid & 1;
-    unsigned a_off[4], b_off[Q4 ? QG : BG];  // element offsets; the launcher keeps M*K and N*K below 2^31
+    constexpr int QG = 8 / NW;  // Q4_0 B: 16-byte blocks per thread per stage
+    // byte offsets (of this lane's 16-byte chunk of a row's first stage for the LDS-direct operands; the launcher keeps M*K and
+    // N*K below 2^31); a stage's own offset is added to the scalar base
+    unsigned a_off[4], b_off[Q4 ? QG : BG];
 #pragma unroll
     for (int ps = 0; ps < 4; ps++) {
         const int ti = min(tok0 + (ps * NW + wave) * 8 + g_rowlo, M_end - 1);
-        a_off[ps] = (unsigned)(p.a_rowmap ? p.a_rowmap[ti] : ti) * (unsigned)K;
+        a_off[ps] = (unsigned)(p.a_rowmap ? p.a_rowmap[ti] : ti) * (unsigned)K + g_chunk * 16;
     }
-    if (Q6) {
-        b_off[0] = (unsigned)min(row0 + q6_row, N_end - 1) * (unsigned)(p.nb >> 3);  // first superblock of the row
-    } else if (!Q4) {
-#pragma unroll
-        for (int ps = 0; ps < BG; ps++)
-            b_off[ps] = (unsigned)min(row0 + (ps * NW + wave) * 8 + g_rowlo, N_end - 1) * (unsigned)K;
-    } else {
+    if constexpr (Q4) {
 #pragma unroll
         for (int ps = 0; ps < QG; ps++)
-            b_off[ps] = (unsigned)min(row0 + (ps * NW + wave) * 16 + q_rowlo, N_end - 1) * (unsigned)p.nb;
+            b_off[ps] = ((unsigned)min(row0 + (ps * NW + wave) * 16 + q_rowlo, N_end - 1) * (unsigned)p.nb + q_bi) * 16u;
+    } else {
+#pragma unroll
+        for (int ps = 0; ps < BG; ps++)
+            b_off[ps] = (unsigned)min(row0 + (ps * NW + wave) * 8 + g_rowlo, N_end - 1) * (unsigned)K + g_chunk * 16;
     }
     // scales of a stage (4 blocks): threads 0..127 carry the four f16 scales of weight row tid (8
-    // contiguous bytes), threads 128..128+BM-1 the four fp32 scales of token tid - 128 (16 contiguous
-    // bytes): one load per thread when rows are 4-block aligned (nb % 4 == 0), four clamped loads otherwise.
-    // Q6_K weight scales: thread (wr, wh) carries d and the sub-block scales 4*wh .. 4*wh+3 of row wr.
-    const bool role_w = tid < 128, role_x = !role_w && tid - 128 < BM;   // wave-uniform
-    const int role_r = role_w ? tid : tid - 128;
-    const bool vec_sc = (p.nb & 3) == 0;
-    const int wr = tid & 127, wh = tid >> 7;
-    const bool w_valid = row0 + wr < N_end, x_valid = tok0 + role_r < M_end;
-    const size_t scw_base = (size_t)min(row0 + wr, N_end - 1) * (Q6 ? p.nb >> 3 : p.nb);
-    size_t scx_base;
+    // contiguous bytes), threads 128..255 the four fp32 scales of token tid - 128 (16 contiguous bytes): one load per thread.
+    const bool role_w = wave < 2, role_x = !role_w;   // scalar: waves 0, 1 carry the weights' scales, 2, 3 the activations'
+    const int role_r = tid & 127;
+    const bool w_valid = row0 + role_r < N_end, x_valid = tok0 + role_r < M_end;
+    const unsigned scw_base = (unsigned)min(row0 + role_r, N_end - 1) * (unsigned)p.nb;   // below 2^26
+    unsigned scx_base;
     {
         const int ti = min(tok0 + role_r, M_end - 1);
-        scx_base = (size_t)(p.a_rowmap ? p.a_rowmap[ti] : ti) * p.nb;
+        scx_base = (unsigned)(p.a_rowmap ? p.a_rowmap[ti] : ti) * (unsigned)p.nb;
     }
-    uint4 rb[Q6 ? 3 : QG];  // Q4_0 / Q6_K quants on their way through registers
+    uint4 rb[Q4 ? QG : 1];     // Q4_0 quants on their way through registers
     uint4 rsv = {0, 0, 0, 0};  // the thread's four raw scales: f16 pairs in .x .y (weights) or four fp32 (activations)
-    uint16_t rsd = 0;   // Q6_K: d of the superblock, row wr
-    unsigned rsc = 0;   // Q6_K: the four sub-block scales 4 * wh .. 4 * wh + 3 of the stage, row wr
 
-    // issue every global read of stage s; the register-staged parts are written by finish_stage
-    // all global reads of stage s (issuing them piecemeal between the blocks measures slower)
-    auto issue_stage = [&](int buf, int s) {
+    // all global reads of stage s (issuing them piecemeal between the blocks measures slower); the register-staged parts are
+    // written by finish_stage.  full: more than 64 live tokens, every 8-row group is fetched
+    auto issue_stage = [&](auto full, int buf, int s) __attribute__((always_inline)) {
         const unsigned sA = __builtin_amdgcn_readfirstlane(smem_base + buf * STAGE_BYTES + wave * GRP);
-        const unsigned sB = sA + A_BYTES;
         const int blk0 = s * KB;
-        const int koff = min(blk0 * 32 + g_chunk * 16, K - 16);
         // 8-token groups wholly past the tile's end are not fetched (nothing reads their LDS rows)
+        const int8_t* xa = p.xq + (size_t)blk0 * 32;
 #pragma unroll
         for (int ps = 0; ps < 4; ps++)
-            if ((ps * NW + wave) * 8 < live_tok) load_to_lds16(p.xq, a_off[ps] + koff, sA + ps * NW * GRP);
-        if (Q6) {
-            const size_t sbi = (size_t)b_off[0] + (s >> 1);
-            const char* ql = (const char*)op.wquants + sbi * 128 + (s & 1) * 64 + q6_p * 16;
-            rb[0] = *(const uint4*)ql;
-            rb[1] = *(const uint4*)(ql + 32);
-            rb[2] = *(const uint4*)((const char*)op.wqh + sbi * 64 + (s & 1) * 32 + q6_p * 16);
-        } else if (!Q4) {
+            if (decltype(full)::value || (ps * NW + wave) * 8 < live_tok) load_to_lds16(xa, a_off[ps], sA, ps * NW * GRP);
+        if constexpr (Q4) {
+            const char* wb = (const char*)op.wquants + (size_t)blk0 * 16;
+#pragma unroll
+            for (int ps = 0; ps < QG; ps++) rb[ps] = *(const uint4*)(wb + b_off[ps]);
+        } else {
+            const int8_t* wb = (const int8_t*)op.wquants + (size_t)blk0 * 32;
 #pragma unroll
             for (int ps = 0; ps < BG; ps++)
-                if ((ps * NW + wave) * 8 < live_rows) load_to_lds16(op.wquants, b_off[ps] + koff, sB + ps * NW * GRP);
-        } else {
-            const int bq = min(blk0 + q_bi, p.nb - 1);
-#pragma unroll
-            for (int ps = 0; ps < QG; ps++) rb[ps] = ((const uint4*)op.wquants)[b_off[ps] + bq];
+                if (decltype(full)::value || (ps * NW + wave) * 8 < live_rows) load_to_lds16(wb, b_off[ps], sA, A_BYTES + ps * NW * GRP);
         }
-        // branch-free and unconverted, so that nothing here waits for a load before the MFMA work
-        if (Q6) {
-            rsd = op.wscales[scw_base + (s >> 1)];
-            rsc = *(const unsigned*)(op.wsc + (scw_base + (s >> 1)) * 16 + (s & 1) * 8 + wh * 4);
-        } else if (role_w) {
-            const uint16_t* ws = op.wscales + scw_base;
-            if (vec_sc) {
-                const uint2 v = *(const uint2*)(ws + blk0);
-                rsv.x = v.x; rsv.y = v.y;
-            } else {
-                const int last = p.nb - 1;
-                rsv.x = (unsigned)ws[min(blk0, last)] | ((unsigned)ws[min(blk0 + 1, last)] << 16);
-                rsv.y = (unsigned)ws[min(blk0 + 2, last)] | ((unsigned)ws[min(blk0 + 3, last)] << 16);
-            }
+        // unconverted, so that nothing here waits for a load before the MFMA work
+        if (role_w) {
+            uint2 v;
+            __builtin_memcpy(&v, (const char*)(op.wscales + blk0) + scw_base * 2u, 8);   // 2-byte aligned where rows are not whole stages
+            rsv.x = v.x; rsv.y = v.y;
         }
-        if (role_x) {
-            const unsigned* xs = (const unsigned*)p.xd + scx_base;
-            if (vec_sc) {
-                rsv = *(const uint4*)(xs + blk0);
-            } else {
-                const int last = p.nb - 1;
-                rsv.x = xs[min(blk0, last)]; rsv.y = xs[min(blk0 + 1, last)];
-                rsv.z = xs[min(blk0 + 2, last)]; rsv.w = xs[min(blk0 + 3, last)];
-            }
-        }
+        if (role_x) __builtin_memcpy(&rsv, (const char*)(p.xd + blk0) + scx_base * 4u, 16);
     };
 
-    auto finish_stage = [&](int buf, int s) {
+    auto finish_stage = [&](int buf, int s) __attribute__((always_inline)) {
         char* sB = smem + buf * STAGE_BYTES + A_BYTES;
         float* sdw = (float*)(sB + B_BYTES);
-        float* sdx = sdw + SUB * KB * 128;
+        float* sdx = sdw + KB * 128;
         const int blk0 = s * KB;
-        if (Q6) {
-            const int r = q6_row;
-            const int off = (r >> 3) * GRP + (r & 7) * 128;
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-                const uint4 q = rb[j & 1], h = rb[2];
-                const int ls = (j >> 1) * 4, hs = 2 * j;
-                uint4 o;
-                o.x = q6_bytes(q.x >> ls, h.x >> hs);
-                o.y = q6_bytes(q.y >> ls, h.y >> hs);
-                o.z = q6_bytes(q.z >> ls, h.z >> hs);
-                o.w = q6_bytes(q.w >> ls, h.w >> hs);
-                *(uint4*)(sB + off + ((2 * j + q6_p + r) & 7) * 16) = o;  // elements 32j + 16p .. + 15 of the stage
-            }
-            const float d = w_valid ? h2f_(rsd) : 0.f;
-#pragma unroll
-            for (int j = 0; j < 4; j++)  // d * sc is exact in fp32 (11 x 8 significant bits)
-                sdw[(wh * 4 + j) * 128 + wr] = d * (float)(int)(signed char)(rsc >> (8 * j));
-        }
-        if (Q4) {
+        if constexpr (Q4) {
 #pragma unroll
             for (int ps = 0; ps < QG; ps++) {
                 const int r = (ps * NW + wave) * 16 + q_rowlo;
@@ -274,12 +153,12 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? 1 : 2) void gemm_i8_kernel(GemmA
                 *(uint4*)(sB + off + ((2 * q_bi + 1 + r) & 7) * 16) = hi;  // elements 16..31
             }
         }
-        if (!Q6 && role_w) {   // the four block scales of a row side by side: one 16-byte write here, one 16-byte read per row tile and stage
+        if (role_w) {   // the four block scales of a row side by side: one 16-byte write here, one 16-byte read per row tile and stage
             const unsigned h[4] = {rsv.x & 0xffffu, rsv.x >> 16, rsv.y & 0xffffu, rsv.y >> 16};
             float v[KB];
 #pragma unroll
             for (int j = 0; j < KB; j++) v[j] = (w_valid && blk0 + j < p.nb) ? h2f_((uint16_t)h[j]) : 0.f;
-            *(float4*)(sdw + wr * 4) = make_float4(v[0], v[1], v[2], v[3]);
+            *(float4*)(sdw + role_r * 4) = make_float4(v[0], v[1], v[2], v[3]);
         }
         if (role_x) {
             const unsigned v[4] = {rsv.x, rsv.y, rsv.z, rsv.w};
@@ -303,164 +182,133 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? 1 : 2) void gemm_i8_kernel(GemmA
     int frag_lane[KB];
 #pragma unroll
     for (int bi = 0; bi < KB; bi++) frag_lane[bi] = (col >> 3) * GRP + (col & 7) * 128 + ((2 * bi + half + col) & 7) * 16;
-    // Q6_K: a lane takes bytes 8 * half .. + 7 of BOTH 16-byte chunks of the block (the order of k
-    // inside an MFMA does not matter as long as both operands use the same one)
-    const int dx_tok = ((lane & 15) >> 2) * 8 + half * 4 + (lane & 3);  // token of accumulator lane % 16 in this lane's half
-    const int frag6 = (col >> 3) * GRP + (col & 7) * 128 + half * 8;
-
-    float4 stage_dw[4];   // Q8_0 / Q4_0: the weight scales of this lane's row in each row tile, four blocks of the stage
-    auto read_stage_scales = [&](int buf) {
-        if (Q6) return;
-        const float* sdw = (const float*)(smem + buf * STAGE_BYTES + A_BYTES + B_BYTES);
+    GemmFrag f;
+    // of block bi of the stage in `buf`: the tokens' fragment and scales into slot `slot`
+    auto read_tokens = [&](int slot, int buf, int bi) __attribute__((always_inline)) {
+        const char* sA = smem + buf * STAGE_BYTES + tw * 4 * GRP;
+        const float* sdx = (const float*)(smem + buf * STAGE_BYTES + A_BYTES + B_BYTES) + KB * 128 + bi * BM + tw * 32;
 #pragma unroll
-        for (int nt = 0; nt < 4; nt++) {
-            if (nt >= nt_cnt) break;
-            stage_dw[nt] = *(const float4*)(sdw + ((nt_base + nt) * 32 + col) * 4);
-        }
+        for (int g = 0; g < 4; g++) f.dx[slot][g] = *(const float4*)(sdx + g * 8 + half * 4);
+        f.a[slot] = *(const v4i*)(sA + frag_lane[bi]);
     };
-    auto read_frag = [&](GemmFrag<SUB>& f, int buf, int bi) {
-        const char* sA = smem + buf * STAGE_BYTES;
-        const char* sB = sA + A_BYTES;
-        const float* sdw = (const float*)(sB + B_BYTES);
-        const float* sdx = sdw + SUB * KB * 128;
-        if (Q6) {
-            f.dxv = sdx[bi * BM + tw * 32 + dx_tok];
-        } else {
-#pragma unroll
-            for (int g = 0; g < 4; g++) f.dx[g] = *(const float4*)(sdx + bi * BM + tw * 32 + g * 8 + half * 4);
-        }
-        const char* sBw = sB + nt_base * 4 * GRP;   // this wave's row tiles
-        const float* sdww = sdw + nt_base * 32;
-        if (Q6) {
-            const int o0 = frag6 + ((2 * bi + col) & 7) * 16, o1 = frag6 + ((2 * bi + 1 + col) & 7) * 16;
-            const int2 a0 = *(const int2*)(sA + tw * 4 * GRP + o0), a1 = *(const int2*)(sA + tw * 4 * GRP + o1);
-            f.a = v4i{a0.x, a0.y, a1.x, a1.y};
-#pragma unroll
-            for (int nt = 0; nt < 4; nt++) {
-                if (nt >= nt_cnt) break;
-                const int2 b0 = *(const int2*)(sBw + nt * 4 * GRP + o0), b1 = *(const int2*)(sBw + nt * 4 * GRP + o1);
-                f.b[nt] = v4i{b0.x, b0.y, b1.x, b1.y};
-#pragma unroll
-                for (int jj = 0; jj < SUB; jj++) f.dw[nt][jj] = sdww[(2 * bi + jj) * 128 + nt * 32 + col];
-            }
-        } else {
-            f.a = *(const v4i*)(sA + tw * 4 * GRP + frag_lane[bi]);
-#pragma unroll
-            for (int nt = 0; nt < 4; nt++) {
-                if (nt >= nt_cnt) break;
-                f.b[nt] = *(const v4i*)(sBw + nt * 4 * GRP + frag_lane[bi]);
-                f.dw[nt][0] = bi == 0 ? stage_dw[nt].x : (bi == 1 ? stage_dw[nt].y : (bi == 2 ? stage_dw[nt].z : stage_dw[nt].w));
-            }
-        }
+    // the fragment of row tile nt into f.b[idx]
+    auto read_rows = [&](int idx, int nt, int buf, int bi) __attribute__((always_inline)) {
+        f.b[idx] = *(const v4i*)(smem + buf * STAGE_BYTES + A_BYTES + (nt_base + nt) * 4 * GRP + frag_lane[bi]);
     };
-
-    // One block: 4 MFMAs, each followed by its 32 epilogue FMAs; MFMA nt + 1 is issued before the
-    // FMAs of nt so that the matrix pipe and the vector ALU overlap within the wave.  The empty asm
-    // statements pin the order: without them the FMAs of a whole stage sink below its 16 MFMAs,
-    // whose results (256 registers) then spill.
-    // unit u = row tile u / SUB, sub-block u % SUB
-    auto mfma_unit = [&](const GemmFrag<SUB>& f, int u) -> v16i {
-        if (Q6) {
-            const int nt = u >> 1, jj = u & 1;
-            const long a = ((long)(unsigned)f.a[2 * jj]) | ((long)f.a[2 * jj + 1] << 32);
-            const long b = ((long)(unsigned)f.b[nt][2 * jj]) | ((long)f.b[nt][2 * jj + 1] << 32);
-            return __builtin_amdgcn_mfma_i32_32x32x16_i8(a, b, cmagic, 0, 0, 0);
-        }
-        return __builtin_amdgcn_mfma_i32_32x32x32_i8(f.a, f.b[u], cmagic, 0, 0, 0);
+    auto read_scales = [&](int nt, int buf) __attribute__((always_inline)) {
+        f.dw[nt] = *(const float4*)((const float*)(smem + buf * STAGE_BYTES + A_BYTES + B_BYTES) + ((nt_base + nt) * 32 + col) * 4);
     };
-    auto compute = [&](const GemmFrag<SUB>& f, int blk) {
-        const float dxr[16] = {f.dx[0].x, f.dx[0].y, f.dx[0].z, f.dx[0].w, f.dx[1].x, f.dx[1].y, f.dx[1].z, f.dx[1].w,
-                               f.dx[2].x, f.dx[2].y, f.dx[2].z, f.dx[2].w, f.dx[3].x, f.dx[3].y, f.dx[3].z, f.dx[3].w};
-        v16i d[2];
-        d[0] = mfma_unit(f, 0);
+    auto mfma_tile = [&](auto ntc, int slot, int nt) __attribute__((always_inline)) -> v16i {
+        return __builtin_amdgcn_mfma_i32_32x32x32_i8(f.a[slot], f.b[decltype(ntc)::value == 1 ? slot : nt], cmagic, 0, 0, 0);
+    };
+    using T = std::true_type;
+    using F = std::false_type;
+    v16i d[2];
+    // One block (bi of the stage in `buf`) of the wave's NT row tiles.  The MFMA of a row tile is issued in front of the FMAs of
+    // the tile before it, across the blocks too: a result is read 32 FMAs after its MFMA was issued, and the fragments of the
+    // next block (nbi of nbuf) are requested a block ahead.  The scheduling barriers hold that order; left to itself the
+    // compiler issues an MFMA right in front of the FMAs that need it and pads the wait with s_nop.
+    auto compute = [&](auto ntc, auto blki, auto last, int s, int nbuf) __attribute__((always_inline)) {
+        constexpr int NT = decltype(ntc)::value, bi = decltype(blki)::value, slot = bi & 1, nbi = (bi + 1) & 3;
+        constexpr bool LAST = decltype(last)::value;   // the last block of all
+        if (!LAST) read_tokens(slot ^ 1, nbuf, nbi);
+        if (!LAST && NT == 1) read_rows(slot ^ 1, 0, nbuf, nbi);
+        const float dxr[16] = {f.dx[slot][0].x, f.dx[slot][0].y, f.dx[slot][0].z, f.dx[slot][0].w, f.dx[slot][1].x, f.dx[slot][1].y,
+                               f.dx[slot][1].z, f.dx[slot][1].w, f.dx[slot][2].x, f.dx[slot][2].y, f.dx[slot][2].z, f.dx[slot][2].w,
+                               f.dx[slot][3].x, f.dx[slot][3].y, f.dx[slot][3].z, f.dx[slot][3].w};
 #pragma unroll
-        for (int u = 0; u < 4 * SUB; u++) {
-            const int nt = u / SUB, jj = u % SUB;
-            if (nt >= nt_cnt) break;
-            if (u + 1 < 4 * SUB && (u + 1) / SUB < nt_cnt) {
-                d[(u + 1) & 1] = mfma_unit(f, u + 1);
-                asm volatile("" : "+v"(d[(u + 1) & 1]));
-            }
-            const v16i dn = d[u & 1];
-            const float dw = f.dw[nt][jj];
-            const float ndw = -dw * MAGIC_F;  // exact: dw has at most 18 significant bits (f16, or f16 x int8)
-            if (Q6) {
-                scale_accumulate(acc[nt], dn, dw, ndw, f.dxv);
-            } else {
+        for (int nt = 0; nt < NT; nt++) {
+            const int cur = (bi * NT + nt) & 1;
+            if (nt + 1 < NT) d[cur ^ 1] = mfma_tile(ntc, slot, nt + 1);
+            else if (!LAST) d[cur ^ 1] = mfma_tile(ntc, slot ^ 1, 0);
+            if (nt + 1 < NT || !LAST) asm volatile("" : "+v"(d[cur ^ 1]));
+            if (!LAST && NT > 1) read_rows(nt, nt, nbuf, nbi);   // the MFMA of the tile's old fragment has been issued
+            __builtin_amdgcn_sched_barrier(0);
+            const v16i dn = d[cur];
+            const float dw = bi == 0 ? f.dw[nt].x : bi == 1 ? f.dw[nt].y : bi == 2 ? f.dw[nt].z : f.dw[nt].w;
+            const float ndw = -dw * MAGIC_F;  // exact: dw has 11 significant bits
 #pragma unroll
-                for (int i = 0; i < 16; i++) acc[nt][i] = fmaf(dxr[i], fmaf(dw, __int_as_float(dn[i]), ndw), acc[nt][i]);
-            }
+            for (int i = 0; i < 16; i++) acc[nt][i] = fmaf(dxr[i], fmaf(dw, __int_as_float(dn[i]), ndw), acc[nt][i]);
             asm volatile("" : "+v"(acc[nt][0]), "+v"(acc[nt][1]), "+v"(acc[nt][2]), "+v"(acc[nt][3]), "+v"(acc[nt][4]),
                               "+v"(acc[nt][5]), "+v"(acc[nt][6]), "+v"(acc[nt][7]), "+v"(acc[nt][8]), "+v"(acc[nt][9]),
                               "+v"(acc[nt][10]), "+v"(acc[nt][11]), "+v"(acc[nt][12]), "+v"(acc[nt][13]),
                               "+v"(acc[nt][14]), "+v"(acc[nt][15]));
-            if (DUMP) {
+            if constexpr (DUMP) {
+                const int blk = s * KB + bi;
                 const int row = row0 + (nt_base + nt) * 32 + col;
 #pragma unroll
                 for (int i = 0; i < 16; i++) {
                     const int tok = tok0 + tw * 32 + (i >> 2) * 8 + half * 4 + (i & 3);
-                    if (tok < M_end && row < N_end && blk < p.nb)
-                        p.dump[((size_t)tok * p.N + row) * (SUB * p.nb) + SUB * blk + jj] = dn[i] - MAGIC_I;
+                    if (tok < M_end && row < N_end && blk < p.nb) p.dump[((size_t)tok * p.N + row) * p.nb + blk] = dn[i] - MAGIC_I;
                 }
             }
+            if (!LAST && bi == 3) read_scales(nt, nbuf);
+            __builtin_amdgcn_sched_barrier(0);
         }
     };
 
-    if (s_begin < s_end) {
-        issue_stage(0, s_begin);
+    // The stages, for a number of row tiles known at compile time (tested at run time in front of every row tile it cost a
+    // stage of 16 MFMAs some 60 branches and 140 scalar instructions, and a wave issues one instruction at a time);
+    // 0: a wave whose 32 tokens all lie past the tile's end (ragged expert groups, M tails) only helps with the staging, its
+    // SIMD time goes to the other workgroup on the CU.
+    // One barrier per stage, in front of its last block: there every wave holds that block's fragments in registers and
+    // its own loads of the next stage have landed (they were requested four blocks earlier), so behind the barrier the
+    // stage's buffer takes the loads of the stage after next, and the next stage's first fragments are read under the last
+    // block's arithmetic.
+    auto main_loop = [&](auto ntc, auto full) __attribute__((always_inline)) {
+        constexpr int NT = decltype(ntc)::value;
+        using I0 = std::integral_constant<int, 0>;
+        using I1 = std::integral_constant<int, 1>;
+        using I2 = std::integral_constant<int, 2>;
+        using I3 = std::integral_constant<int, 3>;
+        if (s_begin >= s_end) return;   // (an empty K slice)
+        issue_stage(full, 0, s_begin);
         finish_stage(0, s_begin);
-    }
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-    // a wave whose 32 tokens all lie past the tile's end (ragged expert groups, M tails) only helps
-    // with the staging: its SIMD time goes to the other workgroup on the CU
-    const bool wave_live = tw * 32 < live_tok;
-    // The waves of a workgroup leave the barrier together, and 8 KB of loads per wave queue up in the
-    // CU's one address unit (20 cycles per 1 KB load alone, 64 behind three other waves): even waves
-    // issue the next stage's loads before block 0, odd waves after it (measured +4 %; spreading them
-    // over all four blocks leaves the last ones too little time to land: +1 %).
-    const int my_slot = wave & 1;
-    for (int s = s_begin; s < s_end; s++) {
-        const int buf = (s - s_begin) & 1;
-        const bool more = s + 1 < s_end;
-        if (more && (my_slot == 0 || !wave_live)) issue_stage(buf ^ 1, s + 1);
-        if (wave_live) {
-        GemmFrag<SUB> f0, f1;
-        read_stage_scales(buf);
-        read_frag(f0, buf, 0);
-        read_frag(f1, buf, 1);
-        __builtin_amdgcn_sched_barrier(0);
-        compute(f0, s * KB + 0);
-        __builtin_amdgcn_sched_barrier(0);
-        if (more && my_slot == 1) issue_stage(buf ^ 1, s + 1);
-        read_frag(f0, buf, 2);
-        __builtin_amdgcn_sched_barrier(0);
-        compute(f1, s * KB + 1);
-        __builtin_amdgcn_sched_barrier(0);
-        read_frag(f1, buf, 3);
-        __builtin_amdgcn_sched_barrier(0);
-        compute(f0, s * KB + 2);
-        __builtin_amdgcn_sched_barrier(0);
-        compute(f1, s * KB + 3);
-        __builtin_amdgcn_sched_barrier(0);
-        }
-        if (more) finish_stage(buf ^ 1, s + 1);
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
-    }
-
-    float* out = op.out + (size_t)blockIdx.z * p.M * p.ldo;
+        if (s_begin + 1 < s_end) issue_stage(full, 1, s_begin + 1);
+        if constexpr (NT > 0) {
+            read_tokens(0, 0, 0);
 #pragma unroll
-    for (int nt = 0; nt < 4; nt++) {
-        if (nt >= nt_cnt) break;
-        const int row = row0 + (nt_base + nt) * 32 + col;
-#pragma unroll
-        for (int i = 0; i < 16; i++) {
-            const int tok = tok0 + tw * 32 + (i >> 2) * 8 + half * 4 + (i & 3);
-            if (tok < M_end && row < N_end) out[(size_t)tok * p.ldo + col0 + (nt_base + nt) * 32 + col] = acc[nt][i];
+            for (int nt = 0; nt < NT; nt++) {
+                read_rows(nt, nt, 0, 0);
+                read_scales(nt, 0);
+            }
+            d[0] = mfma_tile(ntc, 0, 0);
+            asm volatile("" : "+v"(d[0]));
         }
-    }
-    SMX_GEMM_T1(live_tok, op_i);
+        // The waves of a workgroup leave the barrier together, and 8 KB of loads per wave queue up in the CU's one address
+        // unit (20 cycles per 1 KB load alone, 64 behind three other waves): even waves issue the stage after next's loads
+        // right behind the barrier, odd waves one block later.
+        const int my_slot = NT > 0 ? wave & 1 : 0;
+        for (int s = s_begin; s < s_end; s++) {
+            const int buf = (s - s_begin) & 1;
+            if constexpr (NT > 0) {
+                compute(ntc, I0(), F(), s, buf);
+                compute(ntc, I1(), F(), s, buf);
+                compute(ntc, I2(), F(), s, buf);
+            }
+            if (s + 1 == s_end) break;
+            finish_stage(buf ^ 1, s + 1);
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            __syncthreads();
+            const bool more = s + 2 < s_end;
+            if (more && my_slot == 0) issue_stage(full, buf, s + 2);
+            if constexpr (NT > 0) {
+                compute(ntc, I3(), F(), s, buf ^ 1);
+                if (more && my_slot == 1) issue_stage(full, buf, s + 2);
+            }
+        }
+        if constexpr (NT > 0) compute(ntc, I3(), T(), s_end - 1, 0);
+    };
+    if (tw * 32 >= live_tok) main_loop(std::integral_constant<int, 0>(), F());
+    else if (nt_cnt == 4) main_loop(std::integral_constant<int, 4>(), T());
+    else if (nt_cnt == 2) main_loop(std::integral_constant<int, 2>(), F());
+    else if (nt_cnt == 1) main_loop(std::integral_constant<int, 1>(), F());
+    else main_loop(std::integral_constant<int, 4>(), F());   // three, or the end of N: what is past it is not written
+
+    gemm_store(p, op, at, role, acc, lane);
+    SMX_GEMM_T1(live_tok, at.op_i);
 }
 
 #ifdef SMX_GEMM_TRACE
@@ -492,15 +340,18 @@ static int pick_splitk(int slots, int tiles, int nstages) {
     return std::max(1, std::min(z, 16));
 }
 
-template <int FMT, bool DUMP, int NW>
-static int launch_gemm_variant(smx_ctx* c, const GemmArgs& p, dim3 grid) {
-    auto k = gemm_i8_kernel<FMT, DUMP, NW>;
-    const size_t lds = 2 * stage_bytes(NW, FMT == FMT_Q6);
+template <class Kernel>
+static int launch_gemm_variant(smx_ctx* c, Kernel k, size_t lds, const GemmArgs& p, dim3 grid) {
     int rc = set_dyn_lds(c, k, lds);
     if (rc != SMX_OK) return rc;
     hipLaunchKernelGGL(k, grid, dim3(64 * NW), lds, c->stream, p);
     SMX_HIP(c, hipGetLastError());
     return SMX_OK;
+}
+static int launch_gemm_type(smx_ctx* c, QType type, bool dump, const GemmArgs& p, dim3 grid) {
+    if (type == kQ6_K) return launch_gemm_variant(c, dump ? gemm_q6_kernel<true> : gemm_q6_kernel<false>, Q6_LDS_BYTES, p, grid);
+    if (type == kQ4_0) return launch_gemm_variant(c, dump ? gemm_i8_kernel<true, true> : gemm_i8_kernel<true, false>, 2 * STAGE_BYTES, p, grid);
+    return launch_gemm_variant(c, dump ? gemm_i8_kernel<false, true> : gemm_i8_kernel<false, false>, 2 * STAGE_BYTES, p, grid);
 }
 
 GemmOperand gemm_operand(const Weight& w, float* out) {
@@ -621,14 +472,7 @@ int launch_gemm(smx_ctx* c, const Weight& w, const int8_t* xq, const float* xd, 
     const dim3 grid((unsigned)T_launch, 1, (unsigned)Z);
     {
         ProfScope ps(c, w.type == kQ4_0 ? "gemm_i8_q4_0" : w.type == kQ6_K ? "gemm_i8_q6_k" : "gemm_i8_q8_0");
-        int rc;
-        if (w.type == kQ6_K) {
-            rc = dump ? launch_gemm_variant<FMT_Q6, true, 4>(c, p, grid) : launch_gemm_variant<FMT_Q6, false, 4>(c, p, grid);
-        } else if (w.type == kQ4_0) {
-            rc = dump ? launch_gemm_variant<FMT_Q4, true, 4>(c, p, grid) : launch_gemm_variant<FMT_Q4, false, 4>(c, p, grid);
-        } else {
-            rc = dump ? launch_gemm_variant<FMT_Q8, true, 4>(c, p, grid) : launch_gemm_variant<FMT_Q8, false, 4>(c, p, grid);
-        }
+        int rc = launch_gemm_type(c, w.type, dump != nullptr, p, grid);
         if (rc != SMX_OK) return rc;
     }
     if (Z > 1) {
@@ -650,8 +494,7 @@ int launch_gemm_grouped(smx_ctx* c, QType type, const GemmArgs& args, int ntiles
     GemmArgs p = args;   // one K slice: every stage
     p.nops = nops;
     p.stages_per_slice = (p.nb + KB - 1) / KB;
-    if (type == kQ6_K) return launch_gemm_variant<FMT_Q6, false, 4>(c, p, grid);
-    if (type == kQ8_0) return launch_gemm_variant<FMT_Q8, false, 4>(c, p, grid);
+    if (type == kQ6_K || type == kQ8_0) return launch_gemm_type(c, type, false, p, grid);
     return fail(c, SMX_ERR_ARG, "grouped gemm: weight type %d not supported", (int)type);
 }
 

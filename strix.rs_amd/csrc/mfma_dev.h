@@ -30,6 +30,14 @@ __device__ __forceinline__ void load_to_lds16(const void* g, unsigned lds_base) 
                  : "s"(__builtin_amdgcn_readfirstlane(lds_base)), "v"(g)
                  : "memory", "m0");
 }
+// The same with a wave-uniform base pointer, a 32-bit per-lane byte offset (no 64-bit address arithmetic) and a constant
+// added to the LDS base.
+__device__ __forceinline__ void load_to_lds16(const void* sbase, unsigned voff, unsigned lds_base, int lds_off) {
+    asm volatile("s_add_i32 m0, %0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+                 :
+                 : "s"(lds_base), "v"(voff), "s"(sbase), "i"(lds_off)
+                 : "memory", "m0", "scc");
+}
 // The same with a wave-uniform base pointer and a 32-bit per-lane byte offset (no 64-bit address arithmetic).
 __device__ __forceinline__ void load_to_lds16(const void* sbase, unsigned voff, unsigned lds_base) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
@@ -41,7 +49,7 @@ __device__ __forceinline__ unsigned lds_addr(const void* p) {
     return (unsigned)(uintptr_t)(const __attribute__((address_space(3))) char*)p;
 }
 
-// acc[I] += dx(token of accumulator I) * fl(dw * dot I).  In the 32x32 MFMA output, accumulator i of
+// acc[I] += dx(token of accumulator I) * t[I].  In the 32x32 MFMA output, accumulator i of
 // lane half h is token (i/4)*8 + h*4 + i%4, so the 16 activation scales a lane needs differ between the
 // two halves; they are kept ONE per lane -- lane n of every 16-lane row holds the scale of accumulator n
 // for that row's half -- and the multiply-add reads it through a row broadcast (DPP row_newbcast:n):
@@ -50,10 +58,7 @@ __device__ __forceinline__ unsigned lds_addr(const void* p) {
     asm("v_fmac_f32_dpp %0, %1, %2 row_newbcast:" #I " row_mask:0xf bank_mask:0xf"        \
         : "+v"(accv[I])                                                                     \
         : "v"(dxv), "v"(t[I]))
-__device__ __forceinline__ void scale_accumulate(float (&accv)[16], const v16i& dn, float dw, float ndw, float dxv) {
-    float t[16];
-#pragma unroll
-    for (int i = 0; i < 16; i++) t[i] = fmaf(dw, __int_as_float(dn[i]), ndw);
+__device__ __forceinline__ void bcast_accumulate(float (&accv)[16], const float (&t)[16], float dxv) {
     SMX_FMAC_BC(0); SMX_FMAC_BC(1); SMX_FMAC_BC(2); SMX_FMAC_BC(3); SMX_FMAC_BC(4); SMX_FMAC_BC(5); SMX_FMAC_BC(6);
     SMX_FMAC_BC(7); SMX_FMAC_BC(8); SMX_FMAC_BC(9); SMX_FMAC_BC(10); SMX_FMAC_BC(11); SMX_FMAC_BC(12);
     SMX_FMAC_BC(13); SMX_FMAC_BC(14); SMX_FMAC_BC(15);

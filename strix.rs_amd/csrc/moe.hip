@@ -983,8 +983,8 @@ static int moe_slots_enqueue(smx_ctx* c, const MoeLayer& L, const float* x_dev, 
                              const GemmTile* tiles_gu, size_t n_gu, const GemmTile* tiles_dn, size_t n_dn, SlotScratch* out) {
     const size_t hidden = L.hidden, eff = L.eff, nb = hidden / 32, enb = eff / 32;
     int rc;
-    if ((rc = ensure(c, c->xq, m * hidden)) != SMX_OK) return rc;
-    if ((rc = ensure(c, c->xd, m * nb * 4)) != SMX_OK) return rc;
+    if ((rc = ensure(c, c->xq, m * hidden + kReadSlack)) != SMX_OK) return rc;
+    if ((rc = ensure(c, c->xd, m * nb * 4 + kReadSlack)) != SMX_OK) return rc;
     if ((rc = ensure(c, c->xs, m * nb * 4)) != SMX_OK) return rc;
     Carver cv;
     const size_t o_g = cv.take(slots * eff * 4), o_u = cv.take(slots * eff * 4), o_aq = cv.take(slots * eff),

@@ -189,6 +189,9 @@ struct ProfScope {
     ~ProfScope();
 };
 
+// Bytes that the tiled GEMM may read behind the last row of its operands (a last stage of 4 blocks that ends inside the row).
+constexpr size_t kReadSlack = 256;
+
 // One weight/output pair of a GEMM launch.
 struct GemmOperand {
     const uint16_t* wscales;  // f16 [rows][nb]; Q6_K: the superblock scale d, [rows][nb / 8]

@@ -101,6 +101,29 @@ def test_gemm_96_row_strips(accel, orc, synth, relerr, ty, M, N, K):
     accel.evict("t.n96")
 
 
+@pytest.mark.parametrize("ty", [2, 8, 14])
+@pytest.mark.parametrize("M,N", [(1, 33), (33, 128), (65, 97), (97, 31), (129, 160)])
+def test_gemm_pipeline_edges(accel, orc, synth, relerr, ty, M, N):
+    """One, two, three and five stages of four blocks (Q6_K: two, four and six), the last one whole or cut, for waves of one
+    to four row tiles and waves without live tokens; and every K slice a single stage.  The largest operands: all-equal
+    rows reach the extremes of x and q, whose dots must be exact in whatever type the products are summed."""
+    for K in (256, 512, 768) if ty == 14 else (32, 128, 160, 384, 608):
+        raw = synth.make_weight(ty, N, K, seed=M + N + K)
+        xs = synth.make_acts(M, K, seed=K)
+        xs[0] = np.where(np.arange(K) // 32 % 2, 1.0, -1.0)
+        assert getattr(accel, UPLOAD[ty])("t.edge", raw, K, N)
+        ref = orc.matmul_q8_from_f32(ty, raw, K, N, xs)
+        for splitk in (1, 0, 16):
+            accel.tune("gemm_splitk", splitk)
+            assert relerr(accel.prefill_q8_gemm("t.edge", xs, M, N), ref) <= TOL, (K, splitk)
+        accel.tune("gemm_splitk", 0)
+        xq, _, _ = orc.actquant(xs, K)
+        dots = accel.gemm_block_dots("t.edge", xs, M, N, K // (16 if ty == 14 else 32))
+        for t in sorted({0, M // 2, M - 1}):
+            assert np.array_equal(dots[t], orc.block_dots(ty, raw, K, N, xq[t])), (K, t)
+    accel.evict("t.edge")
+
+
 def test_gemm_declines_and_errors(accel, synth, pkg):
     assert accel.prefill_q8_gemm("t.absent", np.zeros((2, 64), np.float32), 2, 8) is None
     raw = synth.make_weight(8, 8, 256, seed=1)
