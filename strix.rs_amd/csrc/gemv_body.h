@@ -47,14 +47,15 @@ extern __device__ unsigned long long* g_smx_trace;
 __device__ __forceinline__ float h2f(uint16_t h) { return __half2float(__ushort_as_half(h)); }
 __device__ __forceinline__ int dot4(int a, int b, int c) { return __builtin_amdgcn_sdot4(a, b, c, false); }
 // value of the neighbouring lane (lane ^ 1)
-__device__ __forceinline__ int swap1(int v) { return __builtin_amdgcn_update_dpp(0, v, 0xB1, 0xf, 0xf, false); }
+// (bound_ctrl: the compiler then folds the move into the addition behind it)
+__device__ __forceinline__ int swap1(int v) { return __builtin_amdgcn_update_dpp(0, v, 0xB1, 0xf, 0xf, true); }
 
 // Cross-lane moves on the DPP path (no LDS round trip).  CTRL: 0xB1 = lane^1, 0x4E = lane^2 (quad
 // permutes), 0x141 = mirror within 8 lanes, 0x140 = mirror within a 16-lane row, 0x142 / 0x143 =
 // broadcast of lane 15 / 31 into the following row(s).
 template <int CTRL, int ROW_MASK = 0xf>
 __device__ __forceinline__ int dpp_i(int v) {
-    return __builtin_amdgcn_update_dpp(0, v, CTRL, ROW_MASK, 0xf, false);
+    return __builtin_amdgcn_update_dpp(0, v, CTRL, ROW_MASK, 0xf, ROW_MASK == 0xf);
 }
 template <int CTRL, int ROW_MASK = 0xf>
 __device__ __forceinline__ float dpp_f(float v) {
@@ -338,7 +339,13 @@ __device__ __forceinline__ void compute_unit(OpsQ6_K, const OpsQ6_K::Regs& r, co
         q[3][i] = ((b4[i] >> 4) & 0x0f0f0f0fu) | ((h4[i] >> 2) & 0x30303030u);
     }
     const float d = (act && c == 0) ? h2f(r.d) : 0.f;  // even lane carries the 32-blocks
-    const unsigned long long scw = ((unsigned long long)r.sc.y << 32) | r.sc.x;
+    int s8[4], s8m[4];   // sub-block scale 2j + c, and -32 times it
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        s8[j] = __builtin_amdgcn_sbfe(j < 2 ? r.sc.x : r.sc.y, 16 * (j & 1) + 8 * c, 8);
+        s8m[j] = -32 * s8[j];
+        asm("" : "+v"(s8m[j]));   // opaque: the compiler would merge the two products below into one of 32 bits
+    }
 #pragma unroll
     for (int t = 0; t < MT; t++) {
         const char* tok = smem + t * tokb;
@@ -354,13 +361,14 @@ __device__ __forceinline__ void compute_unit(OpsQ6_K, const OpsQ6_K::Regs& r, co
             is = dot4((int)q[j][1], (int)xv.y, is);
             is = dot4((int)q[j][2], (int)xv.z, is);
             is = dot4((int)q[j][3], (int)xv.w, is);
-            const int xs16 = c ? (sps[j] >> 16) : (int)(short)(sps[j] & 0xffff);
-            const int isum = is - 32 * xs16;  // sum((q-32)x) = sum(qx) - 32 sum(x)
+            const int xs16 = __builtin_amdgcn_sbfe(sps[j], c * 16, 16);
             if (DUMP) {
-                if (act && t == 0 && dump_row) dump_row[(u >> 2) * 16 + ((u >> 1) & 1) * 8 + 2 * j + c] = isum;
+                if (act && t == 0 && dump_row) dump_row[(u >> 2) * 16 + ((u >> 1) & 1) * 8 + 2 * j + c] = is - 32 * xs16;
             }
-            const int s8 = (int)(signed char)((scw >> (8 * (2 * j + c))) & 0xff);
-            int tj = s8 * isum;
+            // sc * sum((q - 32) x) = sc * sum(qx) - 32 sc * sum(x); 24-bit factors (at most 16 * 63 * 127 beside sc, 16 * 127 beside
+            // 32 sc): a 32-bit multiplication takes four times as long.  With it and a variant for three rows of its own
+            // 262144 x 3840 takes 164 us at three rows (212 before) and 195 at four (223); up to two are bound by HBM (146, 152)
+            int tj = __mul24(s8[j], is) + __mul24(s8m[j], xs16);
             tj += swap1(tj);
             acc[t] += (d * dxs[j]) * (float)tj;
         }

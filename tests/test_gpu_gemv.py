@@ -171,6 +171,34 @@ def test_gemv_rows_quantised_in_kernel(accel, orc, synth, relerr, ty, N, K):
     accel.evict("t.rq")
 
 
+# rows per workgroup of one, ragged shares, the longest rows the kernel quantises for three rows (16384), longer ones and rows that
+# are no whole number of unit groups (both through the four-row variants)
+@pytest.mark.parametrize("ty,N,K", [(2, 1, 256), (8, 257, 512), (14, 300, 256), (2, 700, 16384), (8, 70, 16384), (14, 33, 16384),
+                                    (2, 40, 16640), (8, 50, 96), (14, 3000, 3840)])
+def test_gemv_three_rows(accel, orc, synth, relerr, ty, N, K):
+    raw = synth.make_weight(ty, N, K, seed=N + K)
+    _up(accel, ty, "t.r3", raw, K, N)
+    xs = synth.make_acts(3, K, seed=K)
+    assert relerr(accel.gemv_rows("t.r3", xs, N), orc.matmul_q8_from_f32(ty, raw, K, N, xs)) <= 1e-5
+    accel.evict("t.r3")
+
+
+@pytest.mark.parametrize("bits", [0x00, 0xff])
+@pytest.mark.parametrize("m", [1, 3, 4])
+def test_q6k_largest_integers(accel, orc, relerr, m, bits):
+    """Quants of -32 or 31 throughout, sub-block scales of -128 and 127, activations that all quantise to +-127: the largest
+    factors of the 24-bit products."""
+    N, K = 6, 512
+    raw = np.full((N * K // 256, 210), bits, np.uint8)
+    raw[:, 192:208] = np.where(np.arange(16) % 3 == 0, 127, 128).astype(np.uint8)
+    raw[:, 208:] = np.frombuffer(np.float16(0.01).tobytes(), np.uint8)
+    xs = np.where(np.arange(m * K).reshape(m, K) // 64 % 4 == 0, 3.0, -3.0).astype(np.float32)   # (unequal shares: the sums do not cancel)
+    _up(accel, 14, "t.big", raw.reshape(-1), K, N)
+    assert np.array_equal(accel.gemv_block_dots("t.big", xs[0], N, K // 16), orc.block_dots(14, raw.reshape(-1), K, N, orc.actquant(xs[0], K)[0][0]))
+    assert relerr(accel.gemv_rows("t.big", xs, N), orc.matmul_q8_from_f32(14, raw.reshape(-1), K, N, xs)) <= 1e-5
+    accel.evict("t.big")
+
+
 def test_gemv_rows_long_k_batched(accel, orc, synth, relerr):
     # the batched verify shape: Q8_0 2560 x 9728, M = 8 (large LDS staging, 16-wave groups)
     N, K, m = 2560, 9728, 8
