@@ -301,6 +301,68 @@ __global__ __launch_bounds__(64 * NW, 2) void gemm_i8_kernel(GemmArgs p) {
         }
         if constexpr (NT > 0) compute(ntc, I3(), T(), s_end - 1, 0);
     };
+    // Up to 32 live tokens of a Q8_0 weight in whole stages: the tile is bound by its weight stream (a wave has one MFMA per block), and
+    // one stage on its way at a time, 1.6 us per 16 KB, is the trip to memory.  A stage without the empty token slots fits three
+    // times, so two are on their way while one is computed; its scales go to LDS directly too (their load through registers would
+    // have the compiler wait for everything behind it), the activations' as one per lane, read through a row broadcast.
+    // MoE layer, 512 tokens over 64 experts (half the tiles are such): 157.6 -> 149.6 us, 64 tokens 111 -> 98; 150 tokens x 15360 x
+    // 3840: 54.9 -> 49.5.  For 33..64 tokens the loop below is ahead (161 us on the first): their tiles are bound by the arithmetic.
+    auto sparse_loop = [&]() __attribute__((always_inline)) {
+        constexpr int W_AT = 4 * GRP, DW_AT = W_AT + B_BYTES, DX_AT = DW_AT + 128 * 8, BUF = DX_AT + 32 * 16;
+        constexpr int LOADS = 7;   // of a wave and stage
+        static_assert(3 * BUF <= 2 * STAGE_BYTES, "three stages of 32 tokens");
+        unsigned w_off[4];   // this wave's 32 weight rows; of the tokens, a_off[0]
+#pragma unroll
+        for (int j = 0; j < 4; j++) w_off[j] = (unsigned)min(row0 + wave * 32 + j * 8 + g_rowlo, N_end - 1) * (unsigned)K + g_chunk * 16;
+        const unsigned dw_off = (unsigned)min(row0 + wave * 32 + (lane >> 1), N_end - 1) * (unsigned)p.nb * 2u + (lane & 1) * 4;
+        const int dt = min(tok0 + (wave & 1) * 16 + (lane >> 2), M_end - 1);   // (waves 2 and 3 write what 0 and 1 write)
+        const unsigned dx_off = ((unsigned)(p.a_rowmap ? p.a_rowmap[dt] : dt) * (unsigned)p.nb + (lane & 3)) * 4u;
+        auto issue = [&](int buf, int s) __attribute__((always_inline)) {
+            const unsigned sb = __builtin_amdgcn_readfirstlane(smem_base + buf * BUF);
+            load_to_lds16(p.xq + (size_t)s * (KB * 32), a_off[0], sb + wave * GRP);
+            const int8_t* wb = (const int8_t*)op.wquants + (size_t)s * (KB * 32);
+#pragma unroll
+            for (int j = 0; j < 4; j++) load_to_lds16(wb, w_off[j], sb + W_AT + (wave * 4 + j) * GRP);
+            load_to_lds4(op.wscales + s * KB, dw_off, sb + DW_AT + wave * 256);
+            load_to_lds4(p.xd + s * KB, dx_off, sb + DX_AT + (wave & 1) * 256);
+        };
+        const int dx_slot = ((lane & 15) >> 2) * 8 + half * 4 + (lane & 3);   // token of accumulator lane % 16 in this lane half
+        if (s_begin >= s_end) return;
+        issue(0, s_begin);
+        if (s_begin + 1 < s_end) issue(1, s_begin + 1);
+        int buf = 0;
+        for (int s = s_begin; s < s_end; s++) {
+            if (s + 1 < s_end) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"i"(LOADS) : "memory");
+            else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+            __builtin_amdgcn_s_barrier();   // every wave's part of the stage has landed, and the stage before it has been read
+            asm volatile("" ::: "memory");
+            if (s + 2 < s_end) issue(buf == 0 ? 2 : buf - 1, s + 2);
+            const char* sb = smem + buf * BUF;
+            const uint2 dwr = *(const uint2*)(sb + DW_AT + (wave * 32 + col) * 8);
+            const float4 dx4 = *(const float4*)(sb + DX_AT + dx_slot * 16);
+            const unsigned dwh[KB] = {dwr.x & 0xffffu, dwr.x >> 16, dwr.y & 0xffffu, dwr.y >> 16};
+            const float dxv[KB] = {dx4.x, dx4.y, dx4.z, dx4.w};
+#pragma unroll
+            for (int bi = 0; bi < KB; bi++) {
+                const v4i fa = *(const v4i*)(sb + frag_lane[bi]), fb = *(const v4i*)(sb + W_AT + wave * 4 * GRP + frag_lane[bi]);
+                const v16i dn = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa, fb, cmagic, 0, 0, 0);
+                const float dw = h2f_((uint16_t)dwh[bi]), ndw = -dw * MAGIC_F;
+                float t[16];
+#pragma unroll
+                for (int i = 0; i < 16; i++) t[i] = fmaf(dw, __int_as_float(dn[i]), ndw);
+                bcast_accumulate(acc[0], t, dxv[bi]);
+            }
+            buf = buf == 2 ? 0 : buf + 1;
+        }
+    };
+    if constexpr (!Q4 && !DUMP) {
+        if (live_tok <= 32 && (p.nb & (KB - 1)) == 0) {   // workgroup-uniform
+            sparse_loop();
+            gemm_store(p, op, at, role, acc, lane);
+            SMX_GEMM_T1(live_tok, at.op_i);
+            return;
+        }
+    }
     if (tw * 32 >= live_tok) main_loop(std::integral_constant<int, 0>(), F());
     else if (nt_cnt == 4) main_loop(std::integral_constant<int, 4>(), T());
     else if (nt_cnt == 2) main_loop(std::integral_constant<int, 2>(), F());

@@ -45,6 +45,13 @@ __device__ __forceinline__ void load_to_lds16(const void* sbase, unsigned voff, 
                  : "s"(__builtin_amdgcn_readfirstlane(lds_base)), "v"(voff), "s"(sbase)
                  : "memory", "m0");
 }
+// The same with 4 bytes per lane: lane i's land at lds_base + 4 * i.
+__device__ __forceinline__ void load_to_lds4(const void* sbase, unsigned voff, unsigned lds_base) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2"
+                 :
+                 : "s"(__builtin_amdgcn_readfirstlane(lds_base)), "v"(voff), "s"(sbase)
+                 : "memory", "m0");
+}
 __device__ __forceinline__ unsigned lds_addr(const void* p) {
     return (unsigned)(uintptr_t)(const __attribute__((address_space(3))) char*)p;
 }

@@ -198,3 +198,18 @@ def test_small_batch_rows_equal_single_rows(accel, synth, relerr):
     with pytest.raises(Exception):
         accel.gemv_rows("t.sbr", synth.make_acts(33, K, seed=1), N)   # gemv_rows takes up to 32 rows
     accel.evict("t.sbr")
+
+
+@pytest.mark.parametrize("N,K", [(1, 128), (100, 256), (129, 384), (300, 512), (2560, 1280), (520, 9728), (128, 160)])
+@pytest.mark.parametrize("m", [129, 143, 160])
+def test_gemm_tail_tile_of_few_tokens(accel, orc, synth, relerr, m, N, K):
+    """A last tile of 1, 15 and 32 tokens has a loop of its own (one, two and more stages; rows in part of a tile; K = 160: no whole
+    stages, the general loop).  Its tokens repeat the first ones, which run in a full tile: the same bits."""
+    raw = synth.make_weight(8, N, K, seed=N)
+    xs = synth.make_acts(m, K, seed=m)
+    xs[128:] = xs[:m - 128]
+    assert accel.upload_q8_0("t.tail", raw, K, N)
+    y = accel.prefill_q8_gemm("t.tail", xs, m, N)
+    assert np.array_equal(y[128:], y[:m - 128])
+    assert relerr(y, orc.matmul_q8_from_f32(8, raw, K, N, xs)) <= TOL
+    accel.evict("t.tail")
