@@ -402,6 +402,23 @@ static int pick_splitk(int slots, int tiles, int nstages) {
     return std::max(1, std::min(z, 16));
 }
 
+// Whether 64-token tiles beat 128-token ones for more than 128 tokens of a Q8_0 / Q4_0 weight: twice the workgroups, each stage
+// 0.54 of the time, fewer K slices to add up, and a last tile that is less empty.  Estimated from what either launch needs when it
+// fits one round of the chip's slots (beyond that a partly filled round decides, and 128 tokens stay): stages one after the other,
+// and the reduction's 5 MB of partials per us against 2.7 us per 128-token stage; the two share a fixed part of about 3 stages.
+// Measured 128 -> 64: Q8_0 200 x 2560 x 2560 23.5 -> 19.1 us, 260 x 4096 x 4096 32.5 -> 28.9, 300 x 9728 x 2560 41.2 -> 36.8, 333 x 2560 x
+// 9728 43.8 -> 41.2 (Q4_0 44.5 -> 42.9), Q4_0 150 x 3840 x 15360 52.3 -> 49.0; where the estimate stays: Q8_0 500 x 2560 x 9728 52.1 / 52.8,
+// Q4_0 700 67.8 / 73.8, Q8_0 1000 87.4 / 109.
+static bool short_tiles_pay(int slots, int M, int N, int nstages) {
+    const auto cost = [&](int bm, double per_stage) -> double {
+        const int T = (M + bm - 1) / bm * ((N + BN - 1) / BN);
+        if (T > slots) return 1e30;
+        const int z = pick_splitk(slots, T, nstages), stages = (nstages + z - 1) / z;
+        return 3.0 + stages * per_stage + (z > 1 ? (double)z * M * N * 4 / 5e6 / 2.7 : 0.0);
+    };
+    return cost(64, 0.54) < 0.97 * cost(128, 1.0);
+}
+
 template <class Kernel>
 static int launch_gemm_variant(smx_ctx* c, Kernel k, size_t lds, const GemmArgs& p, dim3 grid) {
     int rc = set_dyn_lds(c, k, lds);
@@ -453,8 +470,9 @@ int launch_gemm(smx_ctx* c, const Weight& w, const int8_t* xq, const float* xd, 
     // the K slices are long; as two rows of 64-token tiles (the waves pair up on two row tiles each) the launch has twice
     // the workgroups at half the work each: Q8_0 2560 x 9728 and 9728 x 2560 at 96 / 128 tokens 28.2 / 29.4 -> 25.4 /
     // 26.7 us and 25.9 / 27.3 -> 22.9 / 24.7 us, 15360 x 3840 -2..4 %, the long-K shapes and Q6_K unchanged within 2 %.
-    // From 129 tokens on the gain is erratic (-10 .. +20 % with the shape and the split-K factor it meets): 128-token tiles.
-    const int bm = (c->tune_gemm_tile_m == 64 || (c->tune_gemm_tile_m == 0 && p.M > 64 && p.M <= 128 && w.type != kQ6_K)) ? 64 : 128;
+    // From 129 tokens on: see short_tiles_pay.
+    const int bm = (c->tune_gemm_tile_m == 64 || (c->tune_gemm_tile_m == 0 && p.M > 64 && w.type != kQ6_K &&
+                                                  (p.M <= 128 || short_tiles_pay(slots, p.M, p.N, (p.nb + KB - 1) / KB)))) ? 64 : 128;
     p.tile_m = bm;
     p.tiles_m = (p.M + bm - 1) / bm;
     const int T = p.tiles_m * p.tiles_n;

@@ -213,3 +213,20 @@ def test_gemm_tail_tile_of_few_tokens(accel, orc, synth, relerr, m, N, K):
     assert np.array_equal(y[128:], y[:m - 128])
     assert relerr(y, orc.matmul_q8_from_f32(8, raw, K, N, xs)) <= TOL
     accel.evict("t.tail")
+
+
+@pytest.mark.parametrize("ty", [8, 2])
+@pytest.mark.parametrize("m,N,K", [(129, 300, 640), (191, 512, 2048), (257, 1000, 96), (384, 260, 4224), (640, 1030, 256)])
+def test_gemm_tile_heights_agree(accel, orc, synth, relerr, ty, m, N, K):
+    """More than 128 tokens in 64- or 128-token tiles, as the rule on sizes picks and either one forced."""
+    raw = synth.make_weight(ty, N, K, seed=N)
+    xs = synth.make_acts(m, K, seed=m)
+    ref = orc.matmul_q8_from_f32(ty, raw, K, N, xs)
+    assert getattr(accel, UPLOAD[ty])("t.th", raw, K, N)
+    try:
+        for height in (0, 64, 128):
+            accel.tune("gemm_tile_m", height)
+            assert relerr(accel.prefill_q8_gemm("t.th", xs, m, N), ref) <= TOL, height
+    finally:
+        accel.tune("gemm_tile_m", 0)
+    accel.evict("t.th")
