@@ -393,30 +393,37 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float4* __rest
     y[i] = s;
 }
 
-// Split-K factor: the reference splits only the long-K shapes (in_dim >= 12288, decode.rs:5658) to
-// fill its grid; here: as many K slices as still fit the chip's workgroup slots in ONE round
-// (a second, partly filled round costs more than the shorter slices save), whole stages, at least
-// 6 stages per slice.  Measured on M = 64..1024 of both FFN shapes.
-static int pick_splitk(int slots, int tiles, int nstages) {
-    const int z = std::min(slots / std::max(tiles, 1), std::max(1, nstages / 6));
-    return std::max(1, std::min(z, 16));
-}
-
-// Whether 64-token tiles beat 128-token ones for more than 128 tokens of a Q8_0 / Q4_0 weight: twice the workgroups, each stage
-// 0.54 of the time, fewer K slices to add up, and a last tile that is less empty.  Estimated from what either launch needs when it
-// fits one round of the chip's slots (beyond that a partly filled round decides, and 128 tokens stay): stages one after the other,
-// and the reduction's 5 MB of partials per us against 2.7 us per 128-token stage; the two share a fixed part of about 3 stages.
-// Measured 128 -> 64: Q8_0 200 x 2560 x 2560 23.5 -> 19.1 us, 260 x 4096 x 4096 32.5 -> 28.9, 300 x 9728 x 2560 41.2 -> 36.8, 333 x 2560 x
-// 9728 43.8 -> 41.2 (Q4_0 44.5 -> 42.9), Q4_0 150 x 3840 x 15360 52.3 -> 49.0; where the estimate stays: Q8_0 500 x 2560 x 9728 52.1 / 52.8,
-// Q4_0 700 67.8 / 73.8, Q8_0 1000 87.4 / 109.
-static bool short_tiles_pay(int slots, int M, int N, int nstages) {
-    const auto cost = [&](int bm, double per_stage) -> double {
+// Tile height and K slices.  The reference splits only the long-K shapes (in_dim >= 12288, decode.rs:5658) to fill its grid.  Here the
+// launch that is estimated to take least, among tiles of 64 (Q8_0, Q4_0) and 128 tokens and every number of whole-stage slices
+// whose workgroups fit the chip's slots in ONE round (a second, partly filled round costs more than shorter slices save): a
+// workgroup's stages one after the other, at the time a stage takes with the CU to itself or shared with a second
+// workgroup, plus the launch that adds up the slices' partials, 3.5 us and 5 MB of them per us.  Tiles that need several rounds: 128 tokens, one slice.
+// The stage times are measured (us): 64 tokens 1.05 alone / 1.46 shared, 128 tokens 1.55 / 2.7, Q6_K 2.75 / 4.3.  Per call against a
+// rule of at least 6 stages per slice and 128-token tiles: Q8_0 200 x 2560 x 2560 23.5 -> 19 us, 300 x 9728 x 2560 41.2 -> 36.8,
+// 333 x 2560 x 9728 43.8 -> 41.2 (Q4_0 44.5 -> 42.9), Q4_0 103 x 1088 x 1024 15.5 -> 12.0, Q6_K 72 x 2208 x 3328 28.9 -> 21.2, 600 x 2560 x
+// 2560 44.0 -> 37.5; Q8_0 500 and 1000 x 2560 x 9728 keep 128-token tiles (64: 52.8 for 52.1, 109 for 87.4).
+struct Tiling { int bm, slices; };
+static Tiling pick_tiling(int num_cu, int slots, bool q6, int M, int N, int nstages, bool split) {
+    Tiling best = {128, 1};
+    double least = 1e30;
+    for (int bm : {64, 128}) {
+        if ((bm == 64) ? q6 || M <= 64 : !q6 && M > 64 && M <= 128) continue;   // (65..128 tokens: as two rows of tiles)
         const int T = (M + bm - 1) / bm * ((N + BN - 1) / BN);
-        if (T > slots) return 1e30;
-        const int z = pick_splitk(slots, T, nstages), stages = (nstages + z - 1) / z;
-        return 3.0 + stages * per_stage + (z > 1 ? (double)z * M * N * 4 / 5e6 / 2.7 : 0.0);
-    };
-    return cost(64, 0.54) < 0.97 * cost(128, 1.0);
+        if (T > slots) continue;
+        const bool low = bm == 64 || M <= 64;
+        const double alone = q6 ? 2.75 : low ? 1.05 : 1.55, shared = q6 ? 4.3 : low ? 1.46 : 2.7;
+        const int zmax = split ? std::min(std::min(slots / T, nstages), 16) : 1;
+        for (int z = 1; z <= zmax; z++) {
+            const int stages = (nstages + z - 1) / z;
+            if (z > 1 && stages == (nstages + z - 2) / (z - 1)) continue;   // the same slices as with one fewer
+            const double us = stages * (T * z > num_cu ? shared : alone) + (z > 1 ? 3.5 + (double)z * M * N * 4 / 5e6 : 0.0);
+            if (us < least) {
+                least = us;
+                best = {bm, z};
+            }
+        }
+    }
+    return best;
 }
 
 template <class Kernel>
@@ -466,13 +473,14 @@ int launch_gemm(smx_ctx* c, const Weight& w, const int8_t* xq, const float* xd, 
     // and the clock the chip sustains drops by as much).
     const int slots = c->num_cu * 2;
     p.tiles_n = (p.N + BN - 1) / BN;
-    // Tokens per tile.  65..128 tokens make one row of 128-token tiles in which half the waves of a workgroup may idle and
-    // the K slices are long; as two rows of 64-token tiles (the waves pair up on two row tiles each) the launch has twice
-    // the workgroups at half the work each: Q8_0 2560 x 9728 and 9728 x 2560 at 96 / 128 tokens 28.2 / 29.4 -> 25.4 /
-    // 26.7 us and 25.9 / 27.3 -> 22.9 / 24.7 us, 15360 x 3840 -2..4 %, the long-K shapes and Q6_K unchanged within 2 %.
-    // From 129 tokens on: see short_tiles_pay.
-    const int bm = (c->tune_gemm_tile_m == 64 || (c->tune_gemm_tile_m == 0 && p.M > 64 && w.type != kQ6_K &&
-                                                  (p.M <= 128 || short_tiles_pay(slots, p.M, p.N, (p.nb + KB - 1) / KB)))) ? 64 : 128;
+    const int nstages = (p.nb + KB - 1) / KB;
+    const bool may_split = dump == nullptr && (m * w.N) % 4 == 0;
+    const Tiling tiling = pick_tiling(c->num_cu, slots, w.type == kQ6_K, p.M, p.N, nstages, may_split && c->tune_gemm_splitk == 0);
+    // 65..128 tokens are always two rows of 64-token tiles (in one row of 128 half the waves of a workgroup may idle): Q8_0
+    // 2560 x 9728 and 9728 x 2560 at 96 / 128 tokens 28.2 / 29.4 -> 25.4 / 26.7 us and 25.9 / 27.3 -> 22.9 / 24.7 us.
+    int bm = tiling.bm;
+    if (p.M > 64 && p.M <= 128 && w.type != kQ6_K) bm = 64;   // (also when they need several rounds)
+    if (c->tune_gemm_tile_m != 0) bm = c->tune_gemm_tile_m;
     p.tile_m = bm;
     p.tiles_m = (p.M + bm - 1) / bm;
     const int T = p.tiles_m * p.tiles_n;
@@ -490,8 +498,7 @@ int launch_gemm(smx_ctx* c, const Weight& w, const int8_t* xq, const float* xd, 
         while (p.tiles_m % gm != 0) gm--;   // whole groups
         p.walk_gm = gm;
     }
-    const int nstages = (p.nb + KB - 1) / KB;
-    int Z = (dump || (m * w.N) % 4 != 0) ? 1 : (c->tune_gemm_splitk > 0 ? std::min(c->tune_gemm_splitk, nstages) : pick_splitk(slots, T, nstages));
+    int Z = !may_split ? 1 : c->tune_gemm_splitk > 0 ? std::min(c->tune_gemm_splitk, nstages) : T <= slots ? std::min(tiling.slices, std::max(1, slots / T)) : 1;
     p.stages_per_slice = (nstages + Z - 1) / Z;
     Z = (nstages + p.stages_per_slice - 1) / p.stages_per_slice;
     // Mixed strips.  When the tiles need several rounds of the chip's workgroup slots and the last round is partly filled,
