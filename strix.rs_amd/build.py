@@ -61,11 +61,11 @@ def build(verbose=False, extra=(), incremental=False):
     return LIB
 
 
-def build_pybind():
+def build_pybind(out_dir=HERE, lib="strix_mi355"):
     """The CPython extension module with the hot calls (host compiler only); it links to the library beside it."""
-    out = os.path.join(HERE, "_smx_native.so")
+    out = os.path.join(out_dir, "_smx_native.so")
     cmd = ["g++", "-std=c++17", "-O2", "-Wall", "-shared", "-fPIC", "-I" + sysconfig.get_paths()["include"],
-           os.path.join(HERE, "host", "pybind.cpp"), "-o", out, "-L" + HERE, "-lstrix_mi355", "-Wl,-rpath,$ORIGIN"]
+           os.path.join(HERE, "host", "pybind.cpp"), "-o", out, "-L" + out_dir, "-l" + lib, "-Wl,-rpath,$ORIGIN"]
     _run(cmd, "g++ host/pybind.cpp")
     return out
 

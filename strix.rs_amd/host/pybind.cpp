@@ -124,36 +124,54 @@ FN(ffn_gate_up_dev) {
         !to_int(a[5], &norm) || !to_ptr(a[6], &w) || !to_float(a[7], &eps) || !to_ptr(a[8], &h)) return nullptr;
     ALLOW(smx_ffn_gate_up_dev(c, g, u, act, x, norm, w, eps, h));
 }
-// keys / addresses of a group (up to the ABI's limit; more are counted and refused there)
-bool to_keys(PyObject* seq, const char** out, Py_ssize_t* count) {
-    PyObject* f = PySequence_Fast(seq, "a sequence of keys");
-    if (!f) return false;
-    *count = PySequence_Fast_GET_SIZE(f);
-    bool ok = true;
-    for (Py_ssize_t i = 0; ok && i < *count && i < kMaxGroup; i++) ok = to_key(PySequence_Fast_GET_ITEM(f, i), &out[i]);
-    Py_DECREF(f);   // the caller's sequence keeps the strings alive
-    return ok;
+// A caller's sequence, its items held until the call has returned: the library reads the keys with the interpreter lock
+// released, when nothing else need keep them alive (a sequence that makes its items when asked, as a numpy array of strings
+// does; a list that another thread changes).
+struct Items {
+    PyObject* t = nullptr;
+    bool take(PyObject* iterable) {
+        t = PySequence_Tuple(iterable);
+        return t != nullptr;
+    }
+    Py_ssize_t count() const { return PyTuple_GET_SIZE(t); }
+    PyObject* operator[](Py_ssize_t i) const { return PyTuple_GET_ITEM(t, i); }
+    Items() = default;
+    Items(const Items&) = delete;
+    Items& operator=(const Items&) = delete;
+    ~Items() { Py_XDECREF(t); }
+};
+// keys (anything of known length) / addresses of a group (up to the ABI's limit; more are counted and refused there)
+bool to_keys(PyObject* seq, Items* held, const char** out, Py_ssize_t* count) {
+    if (PyObject_Size(seq) < 0 || !held->take(seq)) return false;
+    *count = held->count();
+    for (Py_ssize_t i = 0; i < *count && i < kMaxGroup; i++)
+        if (!to_key((*held)[i], &out[i])) return false;
+    return true;
 }
 template <class T>
 bool to_ptrs(PyObject* seq, T** out, Py_ssize_t want) {
-    PyObject* f = PySequence_Fast(seq, "a sequence of addresses");
-    if (!f) return false;
-    bool ok = PySequence_Fast_GET_SIZE(f) == want;
-    if (!ok) PyErr_SetString(PyExc_ValueError, "one address per key");
-    for (Py_ssize_t i = 0; ok && i < want && i < kMaxGroup; i++) ok = to_ptr(PySequence_Fast_GET_ITEM(f, i), &out[i]);
-    Py_DECREF(f);
-    return ok;
+    Items f;
+    if (!f.take(seq)) return false;
+    if (f.count() != want) {
+        PyErr_SetString(PyExc_ValueError, "one address per key");
+        return false;
+    }
+    for (Py_ssize_t i = 0; i < want && i < kMaxGroup; i++)
+        if (!to_ptr(f[i], &out[i])) return false;
+    return true;
 }
 // (ctx, keys, xs_dev, ys_dev)
 FN(gemv_batch_dev) {
     smx_ctx* c; const char* keys[kMaxGroup] = {}; const float* xs[kMaxGroup] = {}; float* ys[kMaxGroup] = {}; Py_ssize_t k;
-    if (!argc_is(n, 4) || !to_ptr(a[0], &c) || !to_keys(a[1], keys, &k) || !to_ptrs(a[2], xs, k) || !to_ptrs(a[3], ys, k)) return nullptr;
+    Items held;
+    if (!argc_is(n, 4) || !to_ptr(a[0], &c) || !to_keys(a[1], &held, keys, &k) || !to_ptrs(a[2], xs, k) || !to_ptrs(a[3], ys, k)) return nullptr;
     ALLOW(smx_gemv_batch_dev(c, (size_t)k, keys, xs, ys));
 }
 // (ctx, keys, act, a_dev, b_dev, eps, ys_dev)
 FN(gemv_fused_dev) {
     smx_ctx* c; const char* keys[kMaxGroup] = {}; int act; const float *x, *b; float eps; float* ys[kMaxGroup] = {}; Py_ssize_t k;
-    if (!argc_is(n, 7) || !to_ptr(a[0], &c) || !to_keys(a[1], keys, &k) || !to_int(a[2], &act) || !to_ptr(a[3], &x) || !to_ptr(a[4], &b) ||
+    Items held;
+    if (!argc_is(n, 7) || !to_ptr(a[0], &c) || !to_keys(a[1], &held, keys, &k) || !to_int(a[2], &act) || !to_ptr(a[3], &x) || !to_ptr(a[4], &b) ||
         !to_float(a[5], &eps) || !to_ptrs(a[6], ys, k)) return nullptr;
     ALLOW(smx_gemv_fused_dev(c, (size_t)k, keys, act, x, b, eps, ys));
 }
@@ -213,15 +231,17 @@ FN(gemv_batch) {
     smx_ctx* c; int f32;
     if (!argc_is(n, 4) || !to_ptr(a[0], &c) || !to_int(a[1], &f32)) return nullptr;
     if (!PyList_Check(a[2]) || !PyList_Check(a[3])) Py_RETURN_NONE;
-    const Py_ssize_t k = PyList_GET_SIZE(a[2]);
-    if (k > kMaxGroup || PyList_GET_SIZE(a[3]) != k) Py_RETURN_NONE;
+    Items calls, outs;
+    if (!calls.take(a[2]) || !outs.take(a[3])) return nullptr;
+    const Py_ssize_t k = calls.count();
+    if (k > kMaxGroup || outs.count() != k) Py_RETURN_NONE;
     const char* keys[kMaxGroup]; const float* xs[kMaxGroup]; float* ys[kMaxGroup]; size_t il[kMaxGroup], oc[kMaxGroup]; int st[kMaxGroup];
     Array x[kMaxGroup], y[kMaxGroup];
     for (Py_ssize_t i = 0; i < k; i++) {
-        PyObject* t = PyList_GET_ITEM(a[2], i);
+        PyObject* t = calls[i];
         if (!PyTuple_Check(t) || PyTuple_GET_SIZE(t) != 2) Py_RETURN_NONE;
         if (!to_key(PyTuple_GET_ITEM(t, 0), &keys[i])) return nullptr;
-        if (!x[i].get(PyTuple_GET_ITEM(t, 1), "f", 4) || !y[i].get(PyList_GET_ITEM(a[3], i), "f", 4, true)) Py_RETURN_NONE;
+        if (!x[i].get(PyTuple_GET_ITEM(t, 1), "f", 4) || !y[i].get(outs[i], "f", 4, true)) Py_RETURN_NONE;
         xs[i] = (const float*)x[i].b.buf; il[i] = x[i].count();
         ys[i] = (float*)y[i].b.buf; oc[i] = y[i].count();
         st[i] = 0;
