@@ -395,12 +395,24 @@ class Mi355WeightAccel:
 
     def gemv_batch(self, calls, out_dims, f32=False):
         """calls: [(key, x)], out_dims: [out_dim]; returns [array | None] (accel.rs:397).  f32: the arithmetic of gemv_f32."""
-        n = len(calls)
         ys = [np.empty(d, np.float32) for d in out_dims]
-        rc = self._n.gemv_batch(self._a, 1 if f32 else 0, calls, ys)
-        if rc == SMX_OK:
+        st = self._n.gemv_batch(self._a, 1 if f32 else 0, calls, ys)
+        if st == SMX_OK:
             return ys
-        xs = [_c(x, np.float32).reshape(-1) for _, x in calls]   # a decline, an error or an array to convert: item by item
+        if st is None:   # an array to convert, or more items than the extension takes: nothing has run
+            st = self._gemv_batch_ctypes(calls, ys, f32)
+        elif not isinstance(st, list):
+            self._check(st)
+        out = []
+        for s, y in zip(st, ys):   # the items' own codes
+            if s < 0:
+                raise SmxError(s, self.last_error())
+            out.append(y if s == SMX_OK else None)
+        return out
+
+    def _gemv_batch_ctypes(self, calls, ys, f32):
+        n = len(calls)
+        xs = [_c(x, np.float32).reshape(-1) for _, x in calls]
         keys = (C.c_char_p * n)(*[k.encode() for k, _ in calls])
         xp = (C.c_void_p * n)(*[x.ctypes.data for x in xs])
         yp = (C.c_void_p * n)(*[y.ctypes.data for y in ys])
@@ -409,12 +421,7 @@ class Mi355WeightAccel:
         st = (C.c_int * n)()
         fn = self._L.smx_gemv_f32_batch if f32 else self._L.smx_gemv_batch
         self._check(fn(self._h, n, keys, xp, il, yp, oc, st))
-        out = []
-        for i in range(n):
-            if st[i] < 0:
-                raise SmxError(st[i], self.last_error())
-            out.append(ys[i] if st[i] == SMX_OK else None)
-        return out
+        return list(st)
 
     def prefill_q8_gemm(self, key, xs, m, out_dim):
         """y[m][out_dim] token-major (accel.rs:213)."""

@@ -15,7 +15,7 @@ from conftest import PKG_DIR, _load_by_path
 RECORDER = r"""
 #include <stddef.h>
 static int (*seen)(size_t, const char* const*);
-static int statuses[64], batch_calls, batch_rc = 1;
+static int statuses[80], batch_calls, batch_rc = 1;
 void rec_set(int (*f)(size_t, const char* const*)) { seen = f; }
 void rec_status(int rc, const int* st, size_t n) { batch_rc = rc; for (size_t i = 0; i < n; i++) statuses[i] = st[i]; }
 int rec_batch_calls(void) { return batch_calls; }
@@ -138,3 +138,51 @@ def test_refused_key_sequences(rec):
         mod.gemv_batch_dev(16, [b"a"], [256], [512])
     with pytest.raises(ValueError):
         mod.gemv_batch_dev(16, NAMES, [256], [512] * 5)
+
+
+@pytest.fixture
+def recorded(rec, pkg):
+    """An accelerator object over the recorder (nothing is created or destroyed)."""
+    mod, L = rec
+    L.smx_last_error.restype = C.c_char_p
+    a = pkg.Mi355WeightAccel.__new__(pkg.Mi355WeightAccel)
+    a._L, a._n, a._a, a._h = L, mod, 16, C.c_void_p(16)
+    yield a
+    a._h = None
+
+
+@pytest.mark.parametrize("status", [(1, 1, 1), (1, 0, 1), (0, 0, 0), (1, -1, 0)])
+@pytest.mark.parametrize("layout", ["float32", "float64"])
+def test_a_batch_runs_once_whatever_its_items_return(recorded, rec, pkg, status, layout):
+    """A declined item is the ordinary case (a weight that is not resident): its batch must not be computed a second time."""
+    L = rec[1]
+    L.rec_status(1, (C.c_int * 3)(*status), 3)
+    calls = [(f"k{i}", np.full(4, 10 * i, layout)) for i in range(3)]
+    before = L.rec_batch_calls()
+    if min(status) < 0:
+        with pytest.raises(pkg.SmxError, match="recorded"):
+            recorded.gemv_batch(calls, [2, 2, 2])
+    else:
+        got = recorded.gemv_batch(calls, [2, 2, 2])
+        assert [g is not None for g in got] == [s == 1 for s in status]
+        assert all(g is None or g[0] == 11 * i for i, g in enumerate(got))
+    assert L.rec_batch_calls() == before + 1
+
+
+def test_a_failed_batch_raises_and_runs_once(recorded, rec, pkg):
+    L = rec[1]
+    L.rec_status(-2, (C.c_int * 1)(1), 1)
+    before = L.rec_batch_calls()
+    with pytest.raises(pkg.SmxError, match="smx error -2"):
+        recorded.gemv_batch([("k", np.zeros(4, np.float32))], [2])
+    assert L.rec_batch_calls() == before + 1
+    L.rec_status(1, (C.c_int * 1)(1), 1)
+
+
+def test_a_batch_of_more_items_than_the_extension_takes(recorded, rec):
+    L = rec[1]
+    n = 64 + 1
+    L.rec_status(1, (C.c_int * n)(*[1] * n), n)
+    before = L.rec_batch_calls()
+    got = recorded.gemv_batch([(f"k{i}", np.zeros(4, np.float32)) for i in range(n)], [2] * n)
+    assert len(got) == n and L.rec_batch_calls() == before + 1
