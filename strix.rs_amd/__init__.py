@@ -1,4 +1,4 @@
-"""Python binding of libstrix_mi355.so (ctypes over the C ABI in include/strix_mi355.h).
+"""Python binding of libstrix_mi355.so (the C ABI in include/strix_mi355.h; hot calls through a CPython extension, the rest ctypes).
 
 `Mi355WeightAccel` mirrors the method names, argument meaning and decline
 behaviour of the reference's `WeightAccel` trait
@@ -14,6 +14,7 @@ The directory name contains a dot, so load this package by path, e.g.
 import ctypes as C
 import importlib.util
 import os
+import warnings
 
 import numpy as np
 
@@ -155,13 +156,89 @@ def load_library():
 _native = None
 
 
+class CtypesCalls:
+    """The functions of the extension module over ctypes, for an interpreter without the headers to build it with: the same
+    library calls, the same arguments and codes, 2..5 us more around each."""
+
+    def __init__(self, lib):
+        self._L = lib
+
+    @staticmethod
+    def _keys(keys):
+        n = len(keys)
+        return n, (C.c_char_p * n)(*[k.encode() for k in keys])
+
+    @staticmethod
+    def _ptrs(ptrs, n):
+        ptrs = list(ptrs)
+        if len(ptrs) != n:
+            raise ValueError("one address per key")
+        return (C.c_void_p * n)(*ptrs)
+
+    def gemv_dev(self, c, key, x, m, y):
+        return self._L.smx_gemv_dev(c, key.encode(), x, int(m), y)
+
+    def gemm_dev(self, c, key, x, m, y):
+        return self._L.smx_gemm_dev(c, key.encode(), x, int(m), y)
+
+    def gemv_noalloc_dev(self, c, key, x, m, y):
+        return self._L.smx_gemv_noalloc_dev(c, key.encode(), x, int(m), y)
+
+    def gemv_f32_dev(self, c, key, x, y):
+        return self._L.smx_gemv_f32_dev(c, key.encode(), x, y)
+
+    def gemm_fused_dev(self, c, key, act, a, b, m, eps, y):
+        return self._L.smx_gemm_fused_dev(c, key.encode(), int(act), a, b, int(m), float(eps), y)
+
+    def ffn_gate_up_dev(self, c, gate, up, act, x, norm, w, eps, h):
+        return self._L.smx_ffn_gate_up_dev(c, gate.encode(), up.encode(), int(act), x, int(norm), w, float(eps), h)
+
+    def gemv_batch_dev(self, c, keys, xs, ys):
+        n, k = self._keys(keys)
+        return self._L.smx_gemv_batch_dev(c, n, k, self._ptrs(xs, n), self._ptrs(ys, n))
+
+    def gemv_fused_dev(self, c, keys, act, a, b, eps, ys):
+        n, k = self._keys(keys)
+        return self._L.smx_gemv_fused_dev(c, n, k, int(act), a, b, float(eps), self._ptrs(ys, n))
+
+    def moe_route_dev(self, c, logits, ne, k, ids, w):
+        return self._L.smx_moe_route_dev(c, logits, int(ne), int(k), ids, w)
+
+    def moe_ffn_logits_dev(self, c, layer, logits, k, x, y, ids, w):
+        return self._L.smx_moe_ffn_logits_dev(c, int(layer), logits, int(k), x, y, ids, w)
+
+    def moe_ffn_routed_dev(self, c, layer, ids, w, k, x, y):
+        return self._L.smx_moe_ffn_routed_dev(c, int(layer), ids, w, int(k), x, y)
+
+    def graph_launch(self, c, g):
+        return self._L.smx_graph_launch(c, g)
+
+    def gemv(self, c, key, x, y):
+        x = _c(x, np.float32)
+        return self._L.smx_gemv(c, key.encode(), _p(x), x.size, _p(y), y.size)
+
+    def gemv_f32(self, c, key, x, y):
+        x = _c(x, np.float32)
+        return self._L.smx_gemv_f32(c, key.encode(), _p(x), x.size, _p(y), y.size)
+
+    # the callers convert what these do not take, and call the library themselves
+    def _by_caller(self, *a):
+        return None
+
+    gemv_rows = gemm = lm_head_argmax_rows = gemv_batch = moe_ffn = moe_ffn_dev = moe_layer = moe_layer_dev = _by_caller
+
+
 def load_native():
-    """The extension module with the hot calls (host/pybind.cpp; same library, no ctypes conversions)."""
+    """The extension module with the hot calls (host/pybind.cpp; same library, no ctypes conversions), or CtypesCalls where it
+    has not been built."""
     global _native
     if _native is None:
-        load_library()
+        lib = load_library()
         if not os.path.exists(NATIVE_PATH):
-            raise FileNotFoundError(f"{NATIVE_PATH} is missing: build it with `python strix.rs_amd/build.py`")
+            warnings.warn(f"{NATIVE_PATH} is missing (`python strix.rs_amd/build.py` builds it where Python.h is installed): "
+                          "calls go through ctypes, 2..5 us more each", RuntimeWarning, stacklevel=3)
+            _native = CtypesCalls(lib)
+            return _native
         spec = importlib.util.spec_from_file_location("_smx_native", NATIVE_PATH)
         mod = importlib.util.module_from_spec(spec)
         spec.loader.exec_module(mod)

@@ -62,9 +62,16 @@ def build(verbose=False, extra=(), incremental=False):
 
 
 def build_pybind(out_dir=HERE, lib="strix_mi355"):
-    """The CPython extension module with the hot calls (host compiler only); it links to the library beside it."""
+    """The CPython extension module with the hot calls (host compiler only); it links to the library beside it.  Without the
+    interpreter's headers there is none, and the package makes the same calls through ctypes."""
     out = os.path.join(out_dir, "_smx_native.so")
-    cmd = ["g++", "-std=c++17", "-O2", "-Wall", "-shared", "-fPIC", "-I" + sysconfig.get_paths()["include"],
+    include = sysconfig.get_paths()["include"]
+    if not os.path.exists(os.path.join(include, "Python.h")):
+        print(f"no Python.h in {include}: the package will call the library through ctypes")
+        if os.path.exists(out):
+            os.remove(out)   # one of an older build
+        return None
+    cmd = ["g++", "-std=c++17", "-O2", "-Wall", "-shared", "-fPIC", "-I" + include,
            os.path.join(HERE, "host", "pybind.cpp"), "-o", out, "-L" + out_dir, "-l" + lib, "-Wl,-rpath,$ORIGIN"]
     _run(cmd, "g++ host/pybind.cpp")
     return out
