@@ -17,7 +17,8 @@
  * serialised by the caller (the reference is driven the same way,
  * crates/strix-backend-rocm/src/decode.rs:559-562); distinct contexts are
  * independent.  Host-pointer entry points copy in, run, copy out and
- * synchronise; `_dev` entry points take device pointers, enqueue on the
+ * synchronise (every input has been read before a result is written, so the
+ * caller's buffers may overlap); `_dev` entry points take device pointers, enqueue on the
  * context's stream and return without synchronising.
  */
 #ifndef STRIX_MI355_H

@@ -131,20 +131,23 @@ namespace {
 // A matmul whose rows and results are large: groups of rows pass through copy in, kernels and copy out one behind the other,
 // so that the bus carries both directions while the device computes.  A group is 256 rows (two token tiles of the GEMM:
 // smaller ones lose more in the kernel than they bring) and at least 4 MB of transfers; the first one of several is 128 rows,
-// so that the copy out starts earlier.
+// so that the copy out starts earlier.  Rows that the results overlap are all copied in first.
 int matmul_host_large(smx_ctx* c, const Weight& w, const float* xs, size_t m, float* y, bool force_gemm) {
     HostPipe* hp;
     int rc = host_pipe(c, &hp);
     if (rc != SMX_OK) return rc;
     const size_t per_row = (w.K + w.N) * 4;
     size_t group = std::max<size_t>(256, ((size_t(4) << 20) / per_row + 255) & ~size_t(255));
+    const bool overlap = (uintptr_t)xs < (uintptr_t)(y + m * w.N) && (uintptr_t)y < (uintptr_t)(xs + m * w.K);
     rc = hp->begin(c);
+    if (overlap && rc == SMX_OK) rc = hp->in(c, c->xf32.p, xs, m * w.K * 4);
+    if (overlap && rc == SMX_OK) rc = hp->in_done(c);
     for (size_t r = 0; r < m && rc == SMX_OK;) {
         const size_t n = r == 0 && group == 256 && m >= 384 ? 128 : m - r < 2 * group ? m - r : group;
         float* xd = (float*)c->xf32.p + r * w.K;
         float* yd = (float*)c->yf32.p + r * w.N;
-        rc = hp->in(c, xd, xs + r * w.K, n * w.K * 4);
-        if (rc == SMX_OK) rc = hp->in_done(c);
+        if (!overlap) rc = hp->in(c, xd, xs + r * w.K, n * w.K * 4);
+        if (!overlap && rc == SMX_OK) rc = hp->in_done(c);
         hp->populate(y + r * w.N, n * w.N * 4);   // behind this group's rows, in front of the next one's
         if (rc == SMX_OK) rc = run_matmul_dev(c, w, xd, n, yd, force_gemm, nullptr, nullptr);
         if (rc == SMX_OK) rc = hp->out(c, y + r * w.N, yd, n * w.N * 4);
