@@ -166,8 +166,9 @@ int matmul_host(smx_ctx* c, const char* key, const float* xs, size_t m, size_t i
     if (in_dim != w->K) return fail(c, SMX_ERR_ARG, "%s: activation length %zu, weight in_dim %zu", who, in_dim, w->K);
     if (m == 0) return fail(c, SMX_ERR_ARG, "%s: zero rows", who);
     if (y_cap < m * w->N) return fail(c, SMX_ERR_ARG, "%s: output capacity %zu < %zu", who, y_cap, m * w->N);
-    SMX_HIP(c, hipSetDevice(c->device));
     int rc;
+    if ((rc = refuse_capture(c, who)) != SMX_OK) return rc;
+    SMX_HIP(c, hipSetDevice(c->device));
     if ((rc = ensure(c, c->xf32, m * w->K * 4)) != SMX_OK) return rc;
     if ((rc = ensure(c, c->yf32, m * w->N * 4)) != SMX_OK) return rc;
     const size_t xb = m * w->K * 4, yb = m * w->N * 4;
@@ -229,6 +230,8 @@ static int gemv_batch_host(smx_ctx* c, size_t n, const char* const* keys, const 
     if (!c) return SMX_ERR_ARG;
     if (!keys || !xs || !in_lens || !ys || !out_caps || !status) return fail(c, SMX_ERR_ARG, "gemv_batch: null argument");
     return guarded(c, "gemv_batch", [&]() -> int {
+    int rc;
+    if ((rc = refuse_capture(c, "gemv_batch")) != SMX_OK) return rc;
     SMX_HIP(c, hipSetDevice(c->device));
     // Pass 1: validate and size one scratch region per item so the whole batch is one device job.
     std::vector<const Weight*> ws(n, nullptr);
@@ -255,7 +258,6 @@ static int gemv_batch_host(smx_ctx* c, size_t n, const char* const* keys, const 
         qbytes += (w->K + 255) & ~size_t(255);
         dbytes += ((w->K / 32) * 4 + 255) & ~size_t(255);
     }
-    int rc;
     if ((rc = ensure(c, c->xf32, xbytes)) != SMX_OK) return rc;
     if ((rc = ensure(c, c->yf32, ybytes)) != SMX_OK) return rc;
     (void)qbytes; (void)dbytes;
@@ -343,8 +345,9 @@ int smx_lm_head_argmax_rows(smx_ctx* c, const char* key, const float* xs, size_t
     if (!w) return SMX_NOT_RESIDENT;
     if (in_dim != w->K) return fail(c, SMX_ERR_ARG, "lm_head_argmax_rows: activation length %zu, in_dim %zu", in_dim, w->K);
     if (m == 0) return fail(c, SMX_ERR_ARG, "lm_head_argmax_rows: zero rows");
-    SMX_HIP(c, hipSetDevice(c->device));
     int rc;
+    if ((rc = refuse_capture(c, "lm_head_argmax_rows")) != SMX_OK) return rc;
+    SMX_HIP(c, hipSetDevice(c->device));
     if ((rc = ensure(c, c->xf32, m * w->K * 4)) != SMX_OK) return rc;
     if ((rc = ensure(c, c->yf32, m * w->N * 4)) != SMX_OK) return rc;
     if ((rc = ensure(c, c->tab, argmax_scratch_bytes(m, w->N))) != SMX_OK) return rc;   // the chunk candidates
@@ -473,6 +476,7 @@ int smx_gemv_fused(smx_ctx* c, const char* key, int act, const float* a, const f
     if (rc != SMX_OK) return rc;
     if (in_len != w->K) return fail(c, SMX_ERR_ARG, "gemv_fused: activation length %zu, weight in_dim %zu", in_len, w->K);
     if (out_cap < w->N) return fail(c, SMX_ERR_ARG, "gemv_fused: output capacity %zu < %zu", out_cap, w->N);
+    if ((rc = refuse_capture(c, "gemv_fused")) != SMX_OK) return rc;
     SMX_HIP(c, hipSetDevice(c->device));
     if ((rc = ensure(c, c->xf32, 2 * w->K * 4)) != SMX_OK) return rc;
     if ((rc = ensure(c, c->yf32, w->N * 4)) != SMX_OK) return rc;
@@ -531,8 +535,9 @@ int smx_quantize(smx_ctx* c, const float* x, size_t m, size_t k, int8_t* xq, flo
     if (!c) return SMX_ERR_ARG;
     if (!x || !xq || !xd) return fail(c, SMX_ERR_ARG, "quantize: null argument");
     if (m == 0 || k == 0 || k % 32 != 0) return fail(c, SMX_ERR_ARG, "quantize: bad shape %zu x %zu", m, k);
-    SMX_HIP(c, hipSetDevice(c->device));
     int rc;
+    if ((rc = refuse_capture(c, "quantize")) != SMX_OK) return rc;
+    SMX_HIP(c, hipSetDevice(c->device));
     if ((rc = ensure(c, c->xf32, m * k * 4)) != SMX_OK) return rc;
     if ((rc = ensure_act(c, m, k)) != SMX_OK) return rc;
     SMX_HIP(c, hipMemcpyAsync(c->xf32.p, x, m * k * 4, hipMemcpyHostToDevice, c->stream));
@@ -556,8 +561,9 @@ static int block_dots(smx_ctx* c, const char* key, const float* xs, size_t m, si
     const size_t per = w->type == kQ6_K ? w->K / 16 : w->K / 32;
     const size_t need = m * w->N * per;
     if (out_cap < need) return fail(c, SMX_ERR_ARG, "%s: output capacity %zu < %zu", who, out_cap, need);
-    SMX_HIP(c, hipSetDevice(c->device));
     int rc;
+    if ((rc = refuse_capture(c, who)) != SMX_OK) return rc;
+    SMX_HIP(c, hipSetDevice(c->device));
     if ((rc = ensure(c, c->xf32, m * w->K * 4)) != SMX_OK) return rc;
     if ((rc = ensure(c, c->yf32, m * w->N * 4)) != SMX_OK) return rc;
     if ((rc = ensure(c, c->work, need * 4)) != SMX_OK) return rc;

@@ -507,8 +507,9 @@ int smx_gemv_f32(smx_ctx* c, const char* key, const float* x, size_t in_len, flo
         if (!x || !y) return fail(c, SMX_ERR_ARG, "gemv_f32: null argument");
         if (in_len != w.K) return fail(c, SMX_ERR_ARG, "gemv_f32: activation length %zu, weight in_dim %zu", in_len, w.K);
         if (out_cap < w.N) return fail(c, SMX_ERR_ARG, "gemv_f32: output capacity %zu < %zu", out_cap, w.N);
-        SMX_HIP(c, hipSetDevice(c->device));
         int rc;
+        if ((rc = refuse_capture(c, "gemv_f32")) != SMX_OK) return rc;
+        SMX_HIP(c, hipSetDevice(c->device));
         const size_t xb = w.K * 4, yb = w.N * 4;
         if ((rc = ensure(c, c->xf32, xb)) != SMX_OK) return rc;
         if ((rc = ensure(c, c->yf32, yb)) != SMX_OK) return rc;

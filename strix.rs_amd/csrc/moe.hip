@@ -790,8 +790,9 @@ static int moe_ffn_host(smx_ctx* c, size_t layer, const int32_t* ids, const floa
     const MoeLayer& L = it->second;
     if (x_len != L.hidden) return fail(c, SMX_ERR_ARG, "moe_ffn: activation length %zu, hidden %zu", x_len, L.hidden);
     if (y_cap < L.hidden) return fail(c, SMX_ERR_ARG, "moe_ffn: output capacity %zu < %zu", y_cap, L.hidden);
-    SMX_HIP(c, hipSetDevice(c->device));
     int rc;
+    if ((rc = refuse_capture(c, "moe_ffn")) != SMX_OK) return rc;
+    SMX_HIP(c, hipSetDevice(c->device));
     if ((rc = ensure(c, c->xf32, L.hidden * 4)) != SMX_OK) return rc;
     if ((rc = ensure(c, c->yf32, L.hidden * 4)) != SMX_OK) return rc;
     // The token's row and the result travel through the context's pinned staging; the kernels read the row there themselves
@@ -921,8 +922,9 @@ int smx_moe_route(smx_ctx* c, const float* logits, size_t ne, size_t k, int32_t*
     if (!c) return SMX_ERR_ARG;
     if (!logits || !ids || !w) return fail(c, SMX_ERR_ARG, "moe_route: null argument");
     if (ne == 0 || k == 0 || k > 64) return fail(c, SMX_ERR_LIMIT, "moe_route: %zu experts, top %zu", ne, k);
-    SMX_HIP(c, hipSetDevice(c->device));
     int rc;
+    if ((rc = refuse_capture(c, "moe_route")) != SMX_OK) return rc;
+    SMX_HIP(c, hipSetDevice(c->device));
     if ((rc = ensure(c, c->xf32, ne * 4)) != SMX_OK) return rc;
     if ((rc = ensure(c, c->tab, 2 * 64 * 4)) != SMX_OK) return rc;
     SMX_HIP(c, hipMemcpyAsync(c->xf32.p, logits, ne * 4, hipMemcpyHostToDevice, c->stream));
@@ -1110,6 +1112,7 @@ static int moe_layer_impl(smx_ctx* c, size_t layer, const float* xs, size_t m, c
         std::vector<int> fill(tok_ptr.begin(), tok_ptr.end() - 1);
         for (size_t s = 0; s < slots; s++) tok_slots[fill[slot_tok[s]]++] = (int)s;  // ascending slot order per token
     }
+    if (!on_device && (rc = refuse_capture(c, "moe_layer")) != SMX_OK) return rc;
     SMX_HIP(c, hipSetDevice(c->device));
     if (!on_device) {
         if ((rc = ensure(c, c->xf32, m * hidden * 4)) != SMX_OK) return rc;
@@ -1186,6 +1189,7 @@ int smx_moe_layer_ffn(smx_ctx* c, size_t layer, const int32_t* plan, size_t npla
         off += (size_t)cnt;
     }
     if (off != rows) return fail(c, SMX_ERR_ARG, "moe_layer_ffn: the groups hold %zu rows, the call says %zu", off, rows);
+    if ((rc = refuse_capture(c, "moe_layer_ffn")) != SMX_OK) return rc;
     SMX_HIP(c, hipSetDevice(c->device));
     if ((rc = ensure(c, c->xf32, rows * hidden * 4)) != SMX_OK) return rc;
     std::vector<GemmTile> tiles_gu, tiles_dn;

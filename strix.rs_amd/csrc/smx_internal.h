@@ -135,6 +135,13 @@ int guarded(smx_ctx* c, const char* who, F&& body) {
     }
 }
 
+// Host-pointer calls wait for the device and use streams of their own: refused between graph_begin and graph_end, before they
+// touch the capture.
+inline int refuse_capture(smx_ctx* c, const char* who) {
+    if (!c->capturing) return SMX_OK;
+    return fail(c, SMX_ERR_ARG, "%s: host-pointer calls cannot be captured (use the device-pointer form)", who);
+}
+
 int ensure(smx_ctx* c, DevBuf& b, size_t bytes);
 // Frees a device allocation that kernels of the context may name, or, while a captured graph of the
 // context is alive, keeps it until the context closes (a replay may still read it).

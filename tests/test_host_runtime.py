@@ -79,3 +79,38 @@ def test_rows_and_results_that_overlap(run, m, K, N, behind):
         if got.size:                          # (a small call's kernels read the staging itself)
             assert np.array_equal(got, want)
     """, m=m, K=K, N=N, behind=behind)
+
+
+def test_host_calls_are_refused_during_capture(run):
+    """At once, without a wait and without pulling further streams into the capture, which goes on."""
+    run("""
+        a = accel()
+        K, N, ne, hidden, eff = 256, 4096, 4, 256, 256
+        assert a.upload_moe_q8(0, *synth.make_moe_q8(ne, hidden, eff, seed=1), hidden, eff, ne)
+        x, xs = synth.make_acts(1, K, seed=1)[0], synth.make_acts(300, K, seed=1)
+        ids, w = synth.zipf_routing(300, ne, 2, seed=3)
+        plan, tok, wslot = synth.group_by_expert(ids, w, ne)
+        calls = [lambda: a.gemv("w", x, N), lambda: a.gemv_f32("w", x, N), lambda: a.gemv_rows("w", xs[:7], N), lambda: a.prefill_q8_gemm("w", xs, 300, N),
+                 lambda: a.gemv_batch([("w", x)] * 2, [N] * 2), lambda: a.gemv_fused("w", 1, x, x, N), lambda: a.lm_head_argmax_rows("w", xs[:3], 3),
+                 lambda: a.quantize(xs, K), lambda: a.gemv_block_dots("w", x, N, K // 32), lambda: a.moe_ffn(0, ids[0], w[0], x),
+                 lambda: a.moe_route(x[:64], 8), lambda: a.moe_layer_q8_dev(0, xs, 300, plan, tok, wslot),
+                 lambda: a.moe_layer_ffn(0, [(1, 300)], xs, 300)]
+        for call in calls[:3]:       # (a context that has made no large call yet)
+            call()
+        streams = F.fake_streams()
+        a.graph_begin()
+        for i, call in enumerate(calls):
+            t0 = time.perf_counter()
+            try:
+                call()
+            except pkg.SmxError as e:
+                assert e.code == -1 and "captured" in str(e), (i, e)
+            else:
+                raise AssertionError(i)
+            assert time.perf_counter() - t0 < 1.0, i
+        assert a.gemv("absent", x, N) is None       # a decline comes first, as ever
+        assert F.fake_streams() == streams
+        a.graph_end()
+        for call in calls:
+            call()
+    """)
