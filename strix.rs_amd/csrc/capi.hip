@@ -192,6 +192,7 @@ int matmul_host(smx_ctx* c, const char* key, const float* xs, size_t m, size_t i
     // workgroups cost more than the copy command: Q8_0 2560 x 9728, 3 rows, 39 - 45 us against 34)
     const bool x_direct = gemv_path && m == 1 && xb <= (size_t(64) << 10) && c->tune_host_io != 1 && c->tune_host_io != 2;
     const bool y_direct = gemv_path && c->tune_host_io != 1;
+    HostCall call(c);
     if (!x_direct && c->tune_host_io == 0) {
         if ((rc = staged_to_device(c, c->xf32.p, c->hx.p, xb)) != SMX_OK) return rc;
     } else if (!x_direct) {
@@ -203,7 +204,7 @@ int matmul_host(smx_ctx* c, const char* key, const float* xs, size_t m, size_t i
     if (!y_direct) SMX_HIP(c, hipMemcpyAsync(c->hy.p, c->yf32.p, yb, hipMemcpyDeviceToHost, c->stream));
     if ((rc = stream_wait(c)) != SMX_OK) return rc;
     memcpy(y, c->hy.p, yb);
-    return SMX_OK;
+    return call.done();
 }
 
 }  // namespace
@@ -270,6 +271,7 @@ static int gemv_batch_host(smx_ctx* c, size_t n, const char* const* keys, const 
     size_t xo = 0, yo = 0;
     std::vector<size_t> yoff(n, 0);
     std::vector<float*> xdev(n, nullptr), ydev(n, nullptr);
+    HostCall call(c);
     for (size_t i = 0; i < n; i++) {
         const Weight* w = ws[i];
         if (!w) continue;
@@ -324,7 +326,7 @@ static int gemv_batch_host(smx_ctx* c, size_t n, const char* const* keys, const 
     if (pinned)
         for (size_t i = 0; i < n; i++)
             if (ws[i] && status[i] == SMX_OK) memcpy(ys[i], c->hy.p + yoff[i], ws[i]->N * 4);
-    return SMX_OK;
+    return call.done();
     });
 }
 
@@ -361,6 +363,7 @@ int smx_lm_head_argmax_rows(smx_ctx* c, const char* key, const float* xs, size_t
     }
     if ((rc = ensure_host(c, c->hy, m * 4)) != SMX_OK) return rc;
     // (kernels that read a row once take it from the staging)
+    HostCall call(c);
     const bool direct = pinned && !(m <= 4 && !skinny_serves(*w, m));
     if (!pinned) SMX_HIP(c, hipMemcpyAsync(c->xf32.p, xs, xb, hipMemcpyHostToDevice, c->stream));
     else if (!direct && (rc = staged_to_device(c, c->xf32.p, c->hx.p, xb)) != SMX_OK) return rc;
@@ -370,7 +373,7 @@ int smx_lm_head_argmax_rows(smx_ctx* c, const char* key, const float* xs, size_t
     if (rc != SMX_OK) return rc;
     if ((rc = stream_wait(c)) != SMX_OK) return rc;
     memcpy(out, c->hy.p, m * 4);
-    return SMX_OK;
+    return call.done();
 }
 
 int smx_gemv_dev(smx_ctx* c, const char* key, const float* xs_dev, size_t m, float* y_dev) {
@@ -487,6 +490,7 @@ int smx_gemv_fused(smx_ctx* c, const char* key, int act, const float* a, const f
     if ((rc = ensure_host(c, c->hy, yb)) != SMX_OK) return rc;
     memcpy(c->hx.p, a, w->K * 4);
     if (b) memcpy(c->hx.p + w->K * 4, b, w->K * 4);
+    HostCall call(c);
     // the kernel reads the pinned staging and writes the pinned result itself (see matmul_host)
     const bool x_direct = xb <= (size_t(64) << 10) && c->tune_host_io != 1 && c->tune_host_io != 2, y_direct = c->tune_host_io != 1;
     if (x_direct) {
@@ -502,7 +506,7 @@ int smx_gemv_fused(smx_ctx* c, const char* key, int act, const float* a, const f
     if (!y_direct) SMX_HIP(c, hipMemcpyAsync(c->hy.p, c->yf32.p, yb, hipMemcpyDeviceToHost, c->stream));
     if ((rc = stream_wait(c)) != SMX_OK) return rc;
     memcpy(y, c->hy.p, yb);
-    return SMX_OK;
+    return call.done();
 }
 
 // Prefill form of smx_gemv_fused_dev: the producer runs over m rows in the quantiser launch.
@@ -540,6 +544,7 @@ int smx_quantize(smx_ctx* c, const float* x, size_t m, size_t k, int8_t* xq, flo
     SMX_HIP(c, hipSetDevice(c->device));
     if ((rc = ensure(c, c->xf32, m * k * 4)) != SMX_OK) return rc;
     if ((rc = ensure_act(c, m, k)) != SMX_OK) return rc;
+    HostCall call(c);
     SMX_HIP(c, hipMemcpyAsync(c->xf32.p, x, m * k * 4, hipMemcpyHostToDevice, c->stream));
     rc = launch_actquant(c, (const float*)c->xf32.p, m, k, (int8_t*)c->xq.p, (float*)c->xd.p, (int32_t*)c->xs.p);
     if (rc != SMX_OK) return rc;
@@ -548,7 +553,7 @@ int smx_quantize(smx_ctx* c, const float* x, size_t m, size_t k, int8_t* xq, flo
     // the packed dword (lo16 | hi16 << 16) is two consecutive little-endian i16: xs16[m][k/16]
     if (xs16) SMX_HIP(c, hipMemcpyAsync(xs16, c->xs.p, m * (k / 32) * 4, hipMemcpyDeviceToHost, c->stream));
     SMX_HIP(c, hipStreamSynchronize(c->stream));
-    return SMX_OK;
+    return call.done();
 }
 
 static int block_dots(smx_ctx* c, const char* key, const float* xs, size_t m, size_t in_dim, int32_t* out,
@@ -567,12 +572,13 @@ static int block_dots(smx_ctx* c, const char* key, const float* xs, size_t m, si
     if ((rc = ensure(c, c->xf32, m * w->K * 4)) != SMX_OK) return rc;
     if ((rc = ensure(c, c->yf32, m * w->N * 4)) != SMX_OK) return rc;
     if ((rc = ensure(c, c->work, need * 4)) != SMX_OK) return rc;
+    HostCall call(c);
     SMX_HIP(c, hipMemcpyAsync(c->xf32.p, xs, m * w->K * 4, hipMemcpyHostToDevice, c->stream));
     rc = run_matmul_dev(c, *w, (const float*)c->xf32.p, m, (float*)c->yf32.p, gemm, (int32_t*)c->work.p, nullptr);
     if (rc != SMX_OK) return rc;
     SMX_HIP(c, hipMemcpyAsync(out, c->work.p, need * 4, hipMemcpyDeviceToHost, c->stream));
     SMX_HIP(c, hipStreamSynchronize(c->stream));
-    return SMX_OK;
+    return call.done();
 }
 
 int smx_gemv_block_dots(smx_ctx* c, const char* key, const float* x, size_t in_len, int32_t* out, size_t out_cap) {

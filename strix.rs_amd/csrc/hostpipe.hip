@@ -359,6 +359,7 @@ int host_receive(smx_ctx* c, void* host, const void* dev, size_t bytes, HostPipe
         if (rc == SMX_OK) rc = hp->out(c, host, dev, bytes);
         return hp->end(c, rc);
     }
+    HostCall call(c);
     if (rc != SMX_OK) return rc;
     // The result crosses as parts that report themselves (span_out_kernel), each copied on while the next ones are on the
     // bus.  (A copy command and a wait: the wait alone is 8 us dearer behind a copy than behind a kernel.)
@@ -389,7 +390,7 @@ int host_receive(smx_ctx* c, void* host, const void* dev, size_t bytes, HostPipe
             break;
         }
     }
-    return SMX_OK;
+    return call.done();
 }
 
 int host_pipe(smx_ctx* c, HostPipe** out) {

@@ -802,6 +802,7 @@ static int moe_ffn_host(smx_ctx* c, size_t layer, const int32_t* ids, const floa
     if ((rc = ensure_host(c, c->hx, hb)) != SMX_OK) return rc;
     if ((rc = ensure_host(c, c->hy, hb)) != SMX_OK) return rc;
     memcpy(c->hx.p, x, hb);
+    HostCall call(c);
     const bool x_direct = hb <= (size_t(64) << 10) && c->tune_host_io == 0, y_direct = sgate == 0.0f && c->tune_host_io != 1;
     if (!x_direct) SMX_HIP(c, hipMemcpyAsync(c->xf32.p, c->hx.p, hb, hipMemcpyHostToDevice, c->stream));
     const float* x_dev = x_direct ? (const float*)c->hx.p : (const float*)c->xf32.p;
@@ -810,10 +811,7 @@ static int moe_ffn_host(smx_ctx* c, size_t layer, const int32_t* ids, const floa
     if (rc != SMX_OK) return rc;
     if (sgate != 0.0f) {  // decode.rs:2850, 2865: no shared expert resident -> the whole call declines
         rc = shexp_enqueue(c, layer, L.hidden, sgate, x_dev, (float*)c->yf32.p);
-        if (rc != SMX_OK) {
-            (void)hipStreamSynchronize(c->stream);
-            return rc;
-        }
+        if (rc != SMX_OK) return rc;
     }
     if (!y_direct) SMX_HIP(c, hipMemcpyAsync(c->hy.p, c->yf32.p, hb, hipMemcpyDeviceToHost, c->stream));
     if (gu) {
@@ -827,7 +825,7 @@ static int moe_ffn_host(smx_ctx* c, size_t layer, const int32_t* ids, const floa
     if (gu || aq || ad) SMX_HIP(c, hipStreamSynchronize(c->stream));   // (the stage copies go to pageable memory)
     else if ((rc = stream_wait(c)) != SMX_OK) return rc;
     memcpy(y, c->hy.p, hb);
-    return SMX_OK;
+    return call.done();
     });
 }
 
@@ -927,13 +925,14 @@ int smx_moe_route(smx_ctx* c, const float* logits, size_t ne, size_t k, int32_t*
     SMX_HIP(c, hipSetDevice(c->device));
     if ((rc = ensure(c, c->xf32, ne * 4)) != SMX_OK) return rc;
     if ((rc = ensure(c, c->tab, 2 * 64 * 4)) != SMX_OK) return rc;
+    HostCall call(c);
     SMX_HIP(c, hipMemcpyAsync(c->xf32.p, logits, ne * 4, hipMemcpyHostToDevice, c->stream));
     rc = smx_moe_route_dev(c, (const float*)c->xf32.p, ne, k, (int32_t*)c->tab.p, (float*)(c->tab.p + 256));
     if (rc != SMX_OK) return rc;
     SMX_HIP(c, hipMemcpyAsync(ids, c->tab.p, k * 4, hipMemcpyDeviceToHost, c->stream));
     SMX_HIP(c, hipMemcpyAsync(w, c->tab.p + 256, k * 4, hipMemcpyDeviceToHost, c->stream));
     SMX_HIP(c, hipStreamSynchronize(c->stream));
-    return SMX_OK;
+    return call.done();
 }
 
 int smx_moe_ffn_routed_dev(smx_ctx* c, size_t layer, const int32_t* ids_dev, const float* w_dev, size_t k, const float* x_dev,
@@ -1148,6 +1147,7 @@ static int moe_layer_impl(smx_ctx* c, size_t layer, const float* xs, size_t m, c
     if (!on_device) {
         if ((rc = host_receive(c, y, c->yf32.p, m * hidden * 4, hp, rc)) != SMX_OK) return rc;
         if (stages) {
+            HostCall call(c);   // (the copies go to the caller's memory)
             const size_t eff = L.eff;
             if (stages->gu) {   // g and u are separate [slots][eff] planes on the device
                 SMX_HIP(c, hipMemcpy2DAsync(stages->gu, 2 * eff * 4, ss.g, eff * 4, eff * 4, slots, hipMemcpyDeviceToHost, c->stream));
@@ -1157,6 +1157,7 @@ static int moe_layer_impl(smx_ctx* c, size_t layer, const float* xs, size_t m, c
             if (stages->ad) SMX_HIP(c, hipMemcpyAsync(stages->ad, ss.ad, slots * (eff / 32) * 4, hipMemcpyDeviceToHost, c->stream));
             if (stages->dy) SMX_HIP(c, hipMemcpyAsync(stages->dy, ss.dy, slots * hidden * 4, hipMemcpyDeviceToHost, c->stream));
             SMX_HIP(c, hipStreamSynchronize(c->stream));
+            (void)call.done();
         }
     }
     return rc;

@@ -142,6 +142,22 @@ inline int refuse_capture(smx_ctx* c, const char* who) {
     return fail(c, SMX_ERR_ARG, "%s: host-pointer calls cannot be captured (use the device-pointer form)", who);
 }
 
+// Stands in a host-pointer call from its first enqueued command on: however the call ends before done(), nothing that it
+// has enqueued still runs when it returns (reading the staging that the next call fills, say).
+struct HostCall {
+    smx_ctx* c;
+    explicit HostCall(smx_ctx* c_) : c(c_) {}
+    HostCall(const HostCall&) = delete;
+    HostCall& operator=(const HostCall&) = delete;
+    ~HostCall() {
+        if (c) (void)hipStreamSynchronize(c->stream);
+    }
+    int done() {
+        c = nullptr;
+        return SMX_OK;
+    }
+};
+
 int ensure(smx_ctx* c, DevBuf& b, size_t bytes);
 // Frees a device allocation that kernels of the context may name, or, while a captured graph of the
 // context is alive, keeps it until the context closes (a replay may still read it).
@@ -157,7 +173,7 @@ constexpr size_t kHostPipeBytes = size_t(3) << 20;
 // One transfer in and one out around the kernels of a call: through the pinned staging buffers, or from kHostPipeBytes on
 // through the HostPipe (*hp, null otherwise).  *src is where the kernels find the rows: `dev`, or the pinned staging itself
 // when each of them is read once (read_once).  After a host_send that returned SMX_OK the call ends with host_receive,
-// which takes the error of what lies between and waits for everything.
+// which takes the error of what lies between and waits for everything, after an error too.
 int host_send(smx_ctx* c, void* dev, const void* host, size_t bytes, bool read_once, void* result, size_t result_bytes, HostPipe** hp,
               const float** src);
 // Pinned staging -> device by a kernel (whole floats): a copy command runs on another engine, whose signal the kernels

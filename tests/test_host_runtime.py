@@ -114,3 +114,43 @@ def test_host_calls_are_refused_during_capture(run):
         for call in calls:
             call()
     """)
+
+
+@pytest.mark.parametrize("call,slow,failing", [
+    ("a.prefill_q8_gemm('w', xs[:70], 70, N)", "actquant", "gemm_i8"), ("a.prefill_q8_gemm('w', xs[:70], 70, N)", "gemm_i8", "span_out"),
+    ("a.prefill_q8_gemm('w', xs, 300, N)", "actquant", "gemm_i8"), ("a.prefill_q8_gemm('w', xs, 300, N)", "gemm_i8", "span_out"),
+    ("a.gemv('w', xs[:1], N)", "gemv_flat", "stream_flag"), ("a.gemv_f32('w', xs[:1], N)", "gemv_f32", "stream_flag"),
+    ("a.gemv_rows('w', xs[:3], N)", "span_in", "gemv_"), ("a.gemv_rows('w', xs[:9], N)", "skinny_quant", "skinny_kernel"),
+    ("a.gemv_batch([('w', xs[0])] * 2, [N] * 2)", "gemv_", "stream_flag"), ("a.gemv_fused('w', 1, xs[0], xs[0], N)", "gemv_", "stream_flag"),
+    ("a.lm_head_argmax_rows('w', xs[:3], 3)", "gemv_", "argmax_final"), ("a.gemm_block_dots('w', xs[:70], 70, N, K // 32)", "actquant", "gemm_i8"),
+    ("a.moe_ffn(0, ids[0], w[0], xs[0])", "dual", "moe_down"), ("a.moe_ffn(0, ids[0], w[0], xs[0], 0.5)", "moe_down", "shexp_add"),
+    ("a.moe_layer_q8_dev(0, xs, 300, plan, tok, wslot)", "gemm_i8", "moe_combine"),
+    ("a.moe_layer_ffn(0, [(1, 300)], xs, 300)", "actquant", "silu_mul")])
+def test_a_failed_call_leaves_nothing_running(run, call, slow, failing):
+    run("""
+        a = accel()
+        K, N, ne, hidden, eff = 256, 4096, 4, 256, 256
+        assert a.upload_moe_q8(0, *synth.make_moe_q8(ne, hidden, eff, seed=1), hidden, eff, ne)
+        for part in ("gate", "up", "down"):
+            assert a.upload_q8_0(f"blk.0.ffn_{part}_shexp.weight", synth.make_q8_0(hidden, eff, 1), eff, hidden)
+        xs = synth.make_acts(300, K, seed=1)
+        ids, w = synth.zipf_routing(300, ne, 2, seed=3)
+        plan, tok, wslot = synth.group_by_expert(ids, w, ne)
+        eval(call)
+        F.fake_slow_kernel(slow.encode(), 100000)
+        F.fake_failing_kernel(failing.encode())
+        t0 = time.perf_counter()
+        try:
+            eval(call)
+        except pkg.SmxError as e:
+            pending = F.fake_pending()
+            assert e.code == -2 and "HIP error" in str(e), e
+        else:
+            raise AssertionError("no error")
+        assert F.fake_failed_launches() > 0
+        assert time.perf_counter() - t0 > 0.09      # the slow kernel did run
+        assert pending == 0
+        F.fake_failing_kernel(b"")
+        F.fake_slow_kernel(b"", 0)
+        eval(call)                                  # and the next call is an ordinary one
+    """, call=call, slow=slow, failing=failing)
