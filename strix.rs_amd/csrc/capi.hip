@@ -132,14 +132,11 @@ namespace {
 // so that the bus carries both directions while the device computes.  A group is 256 rows (two token tiles of the GEMM:
 // smaller ones lose more in the kernel than they bring) and at least 4 MB of transfers; the first one of several is 128 rows,
 // so that the copy out starts earlier.  Rows that the results overlap are all copied in first.
-int matmul_host_large(smx_ctx* c, const Weight& w, const float* xs, size_t m, float* y, bool force_gemm) {
-    HostPipe* hp;
-    int rc = host_pipe(c, &hp);
-    if (rc != SMX_OK) return rc;
+int matmul_host_large(smx_ctx* c, HostPipe* hp, const Weight& w, const float* xs, size_t m, float* y, bool force_gemm) {
     const size_t per_row = (w.K + w.N) * 4;
     size_t group = std::max<size_t>(256, ((size_t(4) << 20) / per_row + 255) & ~size_t(255));
     const bool overlap = (uintptr_t)xs < (uintptr_t)(y + m * w.N) && (uintptr_t)y < (uintptr_t)(xs + m * w.K);
-    rc = hp->begin(c);
+    int rc = hp->begin(c);
     if (overlap && rc == SMX_OK) rc = hp->in(c, c->xf32.p, xs, m * w.K * 4);
     if (overlap && rc == SMX_OK) rc = hp->in_done(c);
     for (size_t r = 0; r < m && rc == SMX_OK;) {
@@ -172,7 +169,15 @@ int matmul_host(smx_ctx* c, const char* key, const float* xs, size_t m, size_t i
     if ((rc = ensure(c, c->xf32, m * w->K * 4)) != SMX_OK) return rc;
     if ((rc = ensure(c, c->yf32, m * w->N * 4)) != SMX_OK) return rc;
     const size_t xb = m * w->K * 4, yb = m * w->N * 4;
-    if (xb + yb >= kHostPipeBytes) return matmul_host_large(c, *w, xs, m, y, force_gemm);
+    if (xb + yb >= kHostPipeBytes) {
+        if (HostPipe* hp = host_pipe(c)) return matmul_host_large(c, hp, *w, xs, m, y, force_gemm);
+        HostCall call(c);
+        SMX_HIP(c, hipMemcpyAsync(c->xf32.p, xs, xb, hipMemcpyHostToDevice, c->stream));
+        if ((rc = run_matmul_dev(c, *w, (const float*)c->xf32.p, m, (float*)c->yf32.p, force_gemm, nullptr, nullptr)) != SMX_OK) return rc;
+        SMX_HIP(c, hipMemcpyAsync(y, c->yf32.p, yb, hipMemcpyDeviceToHost, c->stream));
+        SMX_HIP(c, hipStreamSynchronize(c->stream));
+        return call.done();
+    }
     // Up to 4 rows on the GEMV kernels (plain loads of x, plain stores of y): the kernel reads the pinned staging and writes the
     // pinned result itself.  A copy command each way costs more than the kernel (measured per call with one synchronisation:
     // kernel alone 13 us, + host-to-device copy 16, + device-to-host copy 25; kernel on the pinned buffers 17).

@@ -7,6 +7,7 @@
 
 #include <algorithm>
 #include <cstring>
+#include <system_error>
 
 #include "smx_internal.h"
 
@@ -92,7 +93,11 @@ int HostPipe::open(smx_ctx* c) {
     cpu_set_t set;
     int cores = 1;
     if (sched_getaffinity(0, sizeof set, &set) == 0) cores = CPU_COUNT(&set);
-    for (int i = 0; i < std::min(kMaxWorkers, cores - 1); i++) threads.emplace_back([this] { worker(); });
+    try {
+        for (int i = 0; i < std::min(kMaxWorkers, cores - 1); i++) threads.emplace_back([this] { worker(); });
+    } catch (const std::system_error&) {
+        // no further thread to be had: with those there are (the calling thread takes part in any case)
+    }
     return SMX_OK;
 }
 
@@ -345,7 +350,10 @@ int host_send(smx_ctx* c, void* dev, const void* host, size_t bytes, bool read_o
         }
         return staged_to_device(c, dev, c->hx.p, bytes);
     }
-    if ((rc = host_pipe(c, hp)) != SMX_OK) return rc;
+    if (!(*hp = host_pipe(c))) {
+        SMX_HIP(c, hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, c->stream));
+        return SMX_OK;
+    }
     rc = (*hp)->begin(c);
     if (rc == SMX_OK) rc = (*hp)->in(c, dev, host, bytes);
     if (rc == SMX_OK) rc = (*hp)->in_done(c);
@@ -361,6 +369,11 @@ int host_receive(smx_ctx* c, void* host, const void* dev, size_t bytes, HostPipe
     }
     HostCall call(c);
     if (rc != SMX_OK) return rc;
+    if (bytes >= kHostPipeBytes) {   // (no pipe)
+        SMX_HIP(c, hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, c->stream));
+        SMX_HIP(c, hipStreamSynchronize(c->stream));
+        return call.done();
+    }
     // The result crosses as parts that report themselves (span_out_kernel), each copied on while the next ones are on the
     // bus.  (A copy command and a wait: the wait alone is 8 us dearer behind a copy than behind a kernel.)
     constexpr size_t kPart = HostPipe::kPart;
@@ -393,24 +406,18 @@ int host_receive(smx_ctx* c, void* host, const void* dev, size_t bytes, HostPipe
     return call.done();
 }
 
-int host_pipe(smx_ctx* c, HostPipe** out) {
-    if (!c->pipe) {
-        HostPipe* p = new (std::nothrow) HostPipe();
-        if (!p) return fail(c, SMX_ERR_NOMEM, "out of host memory");
-        int rc;
-        try {
-            rc = p->open(c);
-        } catch (const std::exception& e) {   // a thread could not be started
-            rc = fail(c, SMX_ERR_NOMEM, "host transfer threads: %s", e.what());
-        }
-        if (rc != SMX_OK) {
-            delete p;
-            return rc;
-        }
-        c->pipe = p;
+HostPipe* host_pipe(smx_ctx* c) {
+    if (c->pipe || c->pipe_refused) return c->pipe;
+    HostPipe* p = new (std::nothrow) HostPipe();
+    int rc = SMX_ERR_NOMEM;
+    try {
+        if (p) rc = p->open(c);
+    } catch (const std::exception&) {   // out of host memory
     }
-    *out = c->pipe;
-    return SMX_OK;
+    if (rc == SMX_OK) c->pipe = p;
+    else delete p;
+    c->pipe_refused = rc != SMX_OK;
+    return c->pipe;
 }
 
 }  // namespace smx

@@ -81,6 +81,7 @@ struct smx_ctx {
     unsigned* hflag = nullptr;   // pinned HOST words: [0] stream_wait's, [64 ..] one per part of a result on its way (host_receive)
     unsigned flag_seq = 0;       // what is written there next
     smx::HostPipe* pipe = nullptr;   // transfers of large host-pointer calls (made by the first of them)
+    bool pipe_refused = false;       // it could not be made: those calls copy from and to the caller's memory directly
     hipEvent_t htab_done = nullptr;  // recorded after the last copy out of htab (null: htab is free)
 
     // tuning overrides (0 = automatic)
@@ -166,12 +167,13 @@ void release_device(smx_ctx* c, char* p);
 int ensure_host(smx_ctx* c, DevBuf& b, size_t bytes);
 // Waits until everything enqueued on the context's stream has run (the one synchronisation of a host-pointer call).
 int stream_wait(smx_ctx* c);
-// The context's HostPipe, and the size of a host-pointer call (bytes in + out) from which it pays.
-int host_pipe(smx_ctx* c, HostPipe** out);
+// The context's HostPipe (null where it could not be made: tried once), and the size of a host-pointer call (bytes in + out)
+// from which it pays.
+HostPipe* host_pipe(smx_ctx* c);
 constexpr size_t kHostFlags = 1024;   // words at hflag
 constexpr size_t kHostPipeBytes = size_t(3) << 20;
 // One transfer in and one out around the kernels of a call: through the pinned staging buffers, or from kHostPipeBytes on
-// through the HostPipe (*hp, null otherwise).  *src is where the kernels find the rows: `dev`, or the pinned staging itself
+// through the HostPipe (*hp, null otherwise; without one, copy commands on the caller's memory).  *src is where the kernels find the rows: `dev`, or the pinned staging itself
 // when each of them is read once (read_once).  After a host_send that returned SMX_OK the call ends with host_receive,
 // which takes the error of what lies between and waits for everything, after an error too.
 int host_send(smx_ctx* c, void* dev, const void* host, size_t bytes, bool read_once, void* result, size_t result_bytes, HostPipe** hp,

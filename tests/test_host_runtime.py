@@ -154,3 +154,34 @@ def test_a_failed_call_leaves_nothing_running(run, call, slow, failing):
         F.fake_slow_kernel(b"", 0)
         eval(call)                                  # and the next call is an ordinary one
     """, call=call, slow=slow, failing=failing)
+
+
+@pytest.mark.parametrize("refuse", [False, True])
+def test_large_calls_without_the_pipe(run, refuse):
+    """Where 64 MB of pinned memory are not to be had the large calls copy from and to the caller's memory; it is asked for once."""
+    run("""
+        a = accel()
+        K, N, ne, hidden, eff = 256, 4096, 4, 1024, 256
+        assert a.upload_moe_q8(0, *synth.make_moe_q8(ne, hidden, eff, seed=1), hidden, eff, ne)
+        xs, xh = synth.make_acts(700, K, seed=1), synth.make_acts(700, hidden, seed=2)
+        ids, w = synth.zipf_routing(700, ne, 2, seed=3)
+        plan, tok, wslot = synth.group_by_expert(ids, w, ne)
+        if refuse:
+            F.fake_host_limit(C.c_size_t(8 << 20))
+        for _ in range(2):
+            F.fake_keep_inbound(1)
+            assert untouched(a.prefill_q8_gemm("w", xs, 700, N)) and np.array_equal(inbound(), xs.ravel())
+            F.fake_keep_inbound(1)
+            assert untouched(a.moe_layer_q8_dev(0, xh, 700, plan, tok, wslot)) 
+            assert xh.tobytes() in inbound().tobytes()
+            F.fake_keep_inbound(1)
+            y = a.moe_layer_ffn(0, [(1, 300), (2, 400)], xh, 700)
+            assert np.array_equal(np.diff(y.reshape(-1).view(np.uint32)), np.ones(y.size - 1))
+            assert xh.tobytes() in inbound().tobytes()
+        assert F.fake_host_refused() == (1 if refuse else 0)
+        assert F.fake_streams() == (1 if refuse else 3)
+        if refuse:
+            assert F.fake_host_live() < 8 << 20
+        a.close()
+        assert F.fake_host_live() == 0 and F.fake_streams() == 0
+    """, refuse=refuse)
