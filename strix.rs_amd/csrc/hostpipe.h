@@ -11,7 +11,8 @@
 // Bound: the bus (1024 x 9728 results of a 2560-long GEMM: 40 MB out = 0.74 of the call's 1.08 ms; 4.4 ms with pageable copies).
 //
 // Owned by one context, made by its first large call, given back with it: at most kMaxWorkers threads (asleep between
-// calls) and kInSlots * kPiece + kOutRing bytes of pinned memory.
+// calls, and within one when they have found no work for kSpinUs: the device computes) and kInSlots * kPiece + kOutRing bytes
+// of pinned memory.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -38,6 +39,7 @@ public:
     static constexpr int kMaxSpans = 64;
     static constexpr unsigned kOutWgs = 32;
     static constexpr int kMaxWorkers = 5;                 // more bring nothing: the bus is the bound
+    static constexpr double kSpinUs = 50.0;               // (waking a sleeping thread costs about as much)
     static constexpr int kQueue = 4096;
 
     ~HostPipe();
@@ -71,6 +73,7 @@ private:
         std::atomic<size_t> head{0}, tail{0}, done{0};
     };
     void worker();
+    bool waiting(const Queue& q) const { return q.head.load() < q.tail.load(); }
     bool run_one(Queue& q);
     void push(Queue& q, char* dst, const char* src, size_t n, std::atomic<int>* left);
     void push_copies(char* dst, const char* src, size_t n, std::atomic<int>* left);
@@ -92,7 +95,9 @@ private:
     std::chrono::steady_clock::time_point last_progress;
 
     Queue copies, pages;   // pages (populate) are taken when no copy waits, and never by the calling thread before the end
-    std::atomic<bool> active{false}, quit{false};
+    std::atomic<int> sleepers{0};
+    unsigned calls = 0;              // under mu, as quit: what a sleeping worker also wakes for
+    bool quit = false;
     std::mutex mu;
     std::condition_variable cv;
     std::vector<std::thread> threads;

@@ -53,15 +53,22 @@ bool HostPipe::run_one(Queue& q) {
 }
 
 void HostPipe::worker() {
+    unsigned seen = 0;
+    auto idle = std::chrono::steady_clock::now();
     for (;;) {
-        if (!active.load(std::memory_order_acquire)) {
-            std::unique_lock<std::mutex> l(mu);
-            cv.wait(l, [&] { return active.load() || quit.load(); });
+        if (run_one(copies) || run_one(pages)) {
+            idle = std::chrono::steady_clock::now();
+            continue;
         }
-        if (quit.load()) return;
-        if (!run_one(copies) && !run_one(pages)) {   // within a call the next task is microseconds away
-            for (int i = 0; i < 32; i++) __builtin_ia32_pause();
-        }
+        for (int i = 0; i < 32; i++) __builtin_ia32_pause();   // while transfers run the next task is microseconds away
+        if (std::chrono::duration<double, std::micro>(std::chrono::steady_clock::now() - idle).count() < kSpinUs) continue;
+        std::unique_lock<std::mutex> l(mu);
+        sleepers.fetch_add(1);   // in front of the look at the queues: a push either is seen there or sees the sleeper
+        cv.wait(l, [&] { return quit || calls != seen || waiting(copies) || waiting(pages); });
+        sleepers.fetch_sub(1);
+        if (quit) return;
+        seen = calls;
+        idle = std::chrono::steady_clock::now();
     }
 }
 
@@ -69,7 +76,11 @@ void HostPipe::push(Queue& q, char* dst, const char* src, size_t n, std::atomic<
     const size_t t = q.tail.load(std::memory_order_relaxed);
     while (t - q.done.load(std::memory_order_acquire) >= kQueue) run_one(q);
     q.task[t % kQueue] = Task{dst, src, n, left};
-    q.tail.store(t + 1, std::memory_order_release);
+    q.tail.store(t + 1);
+    if (sleepers.load() > 0) {
+        { std::lock_guard<std::mutex> l(mu); }   // (not between a sleeper's look at the queues and its sleep)
+        cv.notify_one();
+    }
 }
 
 void HostPipe::push_copies(char* dst, const char* src, size_t n, std::atomic<int>* left) {
@@ -104,7 +115,7 @@ int HostPipe::open(smx_ctx* c) {
 HostPipe::~HostPipe() {
     {
         std::lock_guard<std::mutex> l(mu);
-        quit.store(true);
+        quit = true;
     }
     cv.notify_all();
     for (auto& t : threads) t.join();
@@ -127,9 +138,9 @@ int HostPipe::begin(smx_ctx* c) {
     for (bool& u : in_used) u = false;
     {
         std::lock_guard<std::mutex> l(mu);
-        active.store(true);
+        calls++;
     }
-    cv.notify_all();
+    cv.notify_all();   // the first pieces are being queued by the time the workers are up
     SMX_HIP(c, hipEventRecord(ev_mark, c->stream));
     SMX_HIP(c, hipStreamWaitEvent(s_in, ev_mark, 0));
     return SMX_OK;
@@ -315,7 +326,6 @@ int HostPipe::end(smx_ctx* c, int rc) {
     while (rc == SMX_OK && span_handing < span_end) rc = wait_progress(c);
     for (Queue* q : {&copies, &pages})
         while (q->done.load(std::memory_order_acquire) < q->tail.load(std::memory_order_relaxed)) run_one(*q);
-    active.store(false);
     if (rc != SMX_OK) {   // whatever is still queued ends before the call returns
         (void)hipStreamSynchronize(s_in);
         (void)hipStreamSynchronize(c->stream);

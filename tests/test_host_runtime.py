@@ -185,3 +185,21 @@ def test_large_calls_without_the_pipe(run, refuse):
         a.close()
         assert F.fake_host_live() == 0 and F.fake_streams() == 0
     """, refuse=refuse)
+
+
+def test_workers_sleep_while_the_device_computes(run):
+    """During a long kernel a large call occupies the calling thread's core (it polls) and not the workers' too."""
+    run("""
+        a = accel()
+        xs = synth.make_acts(300, 256, seed=1)
+        assert untouched(a.prefill_q8_gemm("w", xs, 300, 4096))
+        F.fake_slow_kernel(b"gemm_i8", 500000)
+        cpu, wall = time.process_time(), time.perf_counter()
+        assert untouched(a.prefill_q8_gemm("w", xs, 300, 4096))
+        cpu, wall = time.process_time() - cpu, time.perf_counter() - wall
+        assert wall > 0.5 and cpu < 1.5 * wall, (cpu, wall)
+        F.fake_slow_kernel(b"", 0)
+        for _ in range(200):                        # asleep or not, each call's transfers are whole
+            F.fake_keep_inbound(1)
+            assert untouched(a.prefill_q8_gemm("w", xs, 300, 4096)) and np.array_equal(inbound(), xs.ravel())
+    """)
