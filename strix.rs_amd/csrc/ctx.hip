@@ -69,7 +69,7 @@ int ensure_host(smx_ctx* c, DevBuf& b, size_t bytes) {
         b.cap = 0;
     }
     const size_t cap = (bytes + (size_t(1) << 16) - 1) & ~((size_t(1) << 16) - 1);
-    hipError_t e = hipHostMalloc((void**)&b.p, cap, hipHostMallocDefault);
+    hipError_t e = hipHostMalloc((void**)&b.p, cap, kHostMemory);
     if (e != hipSuccess) {
         (void)hipGetLastError();
         b.p = nullptr;
@@ -85,8 +85,10 @@ __global__ __launch_bounds__(64) void stream_flag_kernel(unsigned* flag, unsigne
 
 // hipStreamSynchronize has the runtime put a barrier packet with a completion signal behind the last kernel and wait for
 // that signal: 9.4 us for an empty kernel.  One word in pinned host memory written by a kernel of its own is seen by a
-// polling host 6.4 us after the same start (the stream runs the word's kernel after everything in front of it has
-// completed and written its results; 14.0 -> 10.0 us with a 256-workgroup kernel that reads and writes pinned memory).
+// polling host 6.4 us after the same start (14.0 -> 10.0 us with a 256-workgroup kernel that reads and writes pinned memory).
+// What makes the results visible with the word: the memory is coherent (kHostMemory), so that a kernel's plain stores to it are
+// not held back in the device's caches once they have completed; a kernel ends after its stores have; and the stream starts the
+// word's kernel after everything in front of it has ended.  The host reads the results behind an acquire fence on the word.
 // The poll is bounded: work of more than kSpinUs, or a failed launch, goes through the runtime's own wait.
 int stream_wait(smx_ctx* c) {
     constexpr double kSpinUs = 2000.0;
@@ -341,7 +343,7 @@ int smx_create(int device, smx_ctx** out) {
         delete c;
         return fail(nullptr, SMX_ERR_HIP, "smx_create: hipEventCreate failed");
     }
-    e = hipHostMalloc((void**)&c->hflag, kHostFlags * 4, hipHostMallocDefault);
+    e = hipHostMalloc((void**)&c->hflag, kHostFlags * 4, kHostMemory);
     if (e != hipSuccess) {
         (void)hipEventDestroy(c->t0);
         (void)hipEventDestroy(c->t1);

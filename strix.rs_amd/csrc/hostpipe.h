@@ -39,7 +39,7 @@ public:
     static constexpr int kMaxSpans = 64;
     static constexpr unsigned kOutWgs = 32;
     static constexpr int kMaxWorkers = 5;                 // more bring nothing: the bus is the bound
-    static constexpr double kSpinUs = 250.0;              // (waking a sleeping thread costs about as much)
+    static constexpr double kSpinUs = 250.0;              // a call's own gaps are shorter (50: 1024 x 9728 results 2 % slower; 250: as without sleep)
     static constexpr int kQueue = 4096;
 
     ~HostPipe();

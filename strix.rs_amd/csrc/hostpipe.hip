@@ -94,9 +94,9 @@ int HostPipe::open(smx_ctx* c) {
     SMX_HIP(c, hipStreamCreateWithFlags(&s_out, hipStreamNonBlocking));
     for (int i = 0; i < kInSlots; i++) SMX_HIP(c, hipEventCreateWithFlags(&ev_in[i], hipEventDisableTiming));
     SMX_HIP(c, hipEventCreateWithFlags(&ev_mark, hipEventDisableTiming));
-    SMX_HIP(c, hipHostMalloc((void**)&ring_in, kInSlots * kPiece, hipHostMallocDefault));
-    SMX_HIP(c, hipHostMalloc((void**)&ring_out, kOutRing, hipHostMallocDefault));
-    SMX_HIP(c, hipHostMalloc((void**)&flags, kOutRing / kPart * 4, hipHostMallocDefault));
+    SMX_HIP(c, hipHostMalloc((void**)&ring_in, kInSlots * kPiece, kHostMemory));
+    SMX_HIP(c, hipHostMalloc((void**)&ring_out, kOutRing, kHostMemory));
+    SMX_HIP(c, hipHostMalloc((void**)&flags, kOutRing / kPart * 4, kHostMemory));
     std::memset(flags, 0, kOutRing / kPart * 4);   // sequence numbers start at 1
     copies.task.resize(kQueue);
     pages.task.resize(kQueue);

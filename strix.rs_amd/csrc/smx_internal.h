@@ -171,6 +171,9 @@ int stream_wait(smx_ctx* c);
 // from which it pays.
 HostPipe* host_pipe(smx_ctx* c);
 constexpr size_t kHostFlags = 1024;   // words at hflag
+// Pinned memory that kernels read and write themselves, asked for as coherent: without the flag it is up to the environment
+// (HIP_HOST_COHERENT), and what a polling host sees of a result rests on it (see stream_wait).
+constexpr unsigned kHostMemory = hipHostMallocCoherent;
 constexpr size_t kHostPipeBytes = size_t(3) << 20;
 // One transfer in and one out around the kernels of a call: through the pinned staging buffers, or from kHostPipeBytes on
 // through the HostPipe (*hp, null otherwise; without one, copy commands on the caller's memory).  *src is where the kernels find the rows: `dev`, or the pinned staging itself

@@ -203,3 +203,15 @@ def test_workers_sleep_while_the_device_computes(run):
             F.fake_keep_inbound(1)
             assert untouched(a.prefill_q8_gemm("w", xs, 300, 4096)) and np.array_equal(inbound(), xs.ravel())
     """)
+
+
+def test_pinned_memory_is_asked_for_as_coherent(run):
+    """Whatever HIP_HOST_COHERENT says: polled words and results that kernels write with plain stores rest on it."""
+    run("""
+        a = accel()
+        xs = synth.make_acts(300, 256, seed=1)
+        a.gemv("w", xs[0], 4096)
+        a.prefill_q8_gemm("w", xs[:70], 70, 4096)
+        a.prefill_q8_gemm("w", xs, 300, 4096)
+        assert F.fake_host_live() > 64 << 20 and F.fake_host_noncoherent() == 0
+    """)
