@@ -73,8 +73,8 @@ __global__ __launch_bounds__(64 * NW, 2) void gemm_i8_kernel(GemmArgs p) {
     const int g_rowlo = lane >> 3, g_chunk = ((lane & 7) - g_rowlo) & 7;
     const int q_bi = lane & 3, q_rowlo = lane >> 2;   // Q4_0 B: lane = [row:4][block:2], 64 contiguous bytes per row
     constexpr int QG = 8 / NW;  // Q4_0 B: 16-byte blocks per thread per stage
-    // byte offsets (of this lane's 16-byte chunk of a row's first stage for the LDS-direct operands; the launcher keeps M*K and
-    // N*K below 2^31); a stage's own offset is added to the scalar base
+    // byte offsets (of this lane's 16-byte chunk of a row's first stage for the LDS-direct operands; M*K and N*K are below 2^31:
+    // launch_gemm, for expert tensors moe_check_shape); a stage's own offset is added to the scalar base
     unsigned a_off[4], b_off[Q4 ? QG : BG];
 #pragma unroll
     for (int ps = 0; ps < 4; ps++) {
@@ -572,8 +572,9 @@ int launch_gemm(smx_ctx* c, const Weight& w, const int8_t* xq, const float* xd, 
     return SMX_OK;
 }
 
-// Grouped GEMM over a tile table (MoE prefill): one launch covers every expert; grid.y selects
-// one of `nops` weight/output pairs that share the activation rows (gate and up).
+// Grouped GEMM over a tile table (MoE prefill): one launch covers every expert; a tile's workgroups serve
+// one of `nops` weight/output pairs each that share the activation rows (gate and up).  The caller has
+// checked the shape (moe_check_shape: the kernels' offsets into the expert tensors are 32 bits wide).
 int launch_gemm_grouped(smx_ctx* c, QType type, const GemmArgs& args, int ntiles, int nops, const char* name) {
     if (ntiles <= 0) return SMX_OK;
     ProfScope ps(c, name);

@@ -58,7 +58,7 @@ __global__ __launch_bounds__(64 * NW, 2) void gemm_q6_kernel(GemmArgs p) {
     // its four blocks (ggml_quant.rs:417-426).  Scales: thread (row sr, half sh) carries d and the sub-block scales
     // 4 * sh .. 4 * sh + 3 of weight row sr; waves 2 and 3 also the four activation scales of token sr.
     const int q_row = tid >> 1, q_p = tid & 1, sr = tid & 127, sh = tid >> 7;
-    const unsigned nsb = (unsigned)(p.nb >> 3);   // superblocks of a row; the launcher keeps M*K and N*K below 2^31
+    const unsigned nsb = (unsigned)(p.nb >> 3);   // superblocks of a row (M*K and N*K are below 2^31: launch_gemm, moe_check_shape)
     unsigned q_sb = (unsigned)min(row0 + q_row, N_end - 1) * nsb, s_sb = (unsigned)min(row0 + sr, N_end - 1) * nsb, x_b;
     {
         const int ti = min(tok0 + sr, M_end - 1);

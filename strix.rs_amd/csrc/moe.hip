@@ -1068,6 +1068,7 @@ struct TableBlob {
     }
 };
 
+// What the grouped kernels' 32-bit offsets can address, for the rows and for the whole expert tensors.
 static int moe_check_shape(smx_ctx* c, const MoeLayer& L, size_t m, size_t slots) {
     if (slots > (size_t(1) << 24) || m > (size_t(1) << 24) || m * L.hidden >= (size_t(1) << 31) || slots * L.eff >= (size_t(1) << 31) ||
         slots * L.hidden >= (size_t(1) << 31) || L.ne * L.eff * L.hidden >= (size_t(1) << 31))

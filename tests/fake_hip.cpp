@@ -1,7 +1,7 @@
 // Test double of the HIP runtime functions that libstrix_mi355.so calls, for its host side on a machine without a GPU: memory
 // is malloc'ed, every stream is a thread that runs its commands in order, and of the kernels only those that move bytes or
 // report to the host do anything.  Fresh device memory holds word i = i, so that a result copied out of memory no kernel has
-// written tells where it comes from.
+// written tells where it comes from; allocations and copies of more than a gigabyte are not filled or made.
 #include <hip/hip_runtime_api.h>
 
 #include <atomic>
@@ -83,6 +83,7 @@ struct ihipEvent_t {
 };
 
 namespace {
+constexpr size_t kGigabyte = size_t(1) << 30;
 std::mutex g_mu;
 std::map<const void*, std::string> g_kernels;
 std::vector<ihipStream_t*> g_streams;
@@ -247,7 +248,7 @@ hipError_t hipMalloc(void** p, size_t n) {
     const size_t words = (n + 3) / 4;
     unsigned* w = (unsigned*)std::aligned_alloc(4096, (words * 4 + 4095) & ~size_t(4095));
     if (!w) return done(hipErrorOutOfMemory);
-    for (size_t i = 0; i < words; i++) w[i] = (unsigned)i;
+    for (size_t i = 0; n <= kGigabyte && i < words; i++) w[i] = (unsigned)i;
     *p = w;
     return hipSuccess;
 }
@@ -286,10 +287,10 @@ hipError_t hipMemcpyAsync(void* dst, const void* src, size_t n, hipMemcpyKind ki
         pinned = in(src) || in(dst);
     }
     s->add([=] {
-        std::memcpy(dst, src, n);
+        if (n <= kGigabyte) std::memcpy(dst, src, n);
         if (kind == hipMemcpyHostToDevice) {
             std::lock_guard<std::mutex> l(g_mu);
-            if (g_keep_inbound) g_inbound.append((const char*)dst, n);
+            if (g_keep_inbound && n <= kGigabyte) g_inbound.append((const char*)dst, n);
         }
     });
     if (!pinned && kind == hipMemcpyHostToDevice && !s->capturing) s->drain();   // pageable memory: staged before the call returns

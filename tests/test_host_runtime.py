@@ -215,3 +215,29 @@ def test_pinned_memory_is_asked_for_as_coherent(run):
         a.prefill_q8_gemm("w", xs, 300, 4096)
         assert F.fake_host_live() > 64 << 20 and F.fake_host_noncoherent() == 0
     """)
+
+
+@pytest.mark.parametrize("ty,eff,refused", [(8, 8192, True), (8, 8160, False), (14, 8192, True), (14, 7936, False)])
+def test_expert_tensors_beyond_the_grouped_kernels_range(run, ty, eff, refused):
+    """The grouped GEMMs address an expert tensor with 32-bit offsets: 64 experts x 8192 x 4096 = 2^31 elements are refused by
+    every grouped call, and one step less is served."""
+    run("""
+        a = pkg.Mi355WeightAccel(0)
+        ne, hidden = 64, 4096
+        n = ne * eff * hidden // (256 if ty == 14 else 32) * (210 if ty == 14 else 34)
+        raw = np.zeros(n, np.uint8)
+        assert (a.upload_moe_q6 if ty == 14 else a.upload_moe_q8)(0, raw, raw, raw, hidden, eff, ne)
+        xs = np.ones((70, hidden), np.float32)
+        ids, w = synth.zipf_routing(70, ne, 2, seed=3)
+        plan, tok, wslot = synth.group_by_expert(ids, w, ne)
+        xd, yd = a.dev_alloc(xs.nbytes), a.dev_alloc(xs.nbytes)
+        for call in (lambda: a.moe_layer_q8_dev(0, xs, 70, plan, tok, wslot), lambda: a.moe_layer_ffn(0, [(63, 70)], xs, 70),
+                     lambda: a.moe_expert_ffn(0, 1, xs, 70), lambda: a.moe_layer_resident(0, xd, 70, plan, tok, wslot, yd),
+                     lambda: a.moe_layer_stages(0, xs, 70, plan, tok, wslot, eff)):
+            try:
+                call()
+            except pkg.SmxError as e:
+                assert refused and e.code == -3, e
+            else:
+                assert not refused
+    """, ty=ty, eff=eff, refused=refused)
