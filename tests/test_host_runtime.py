@@ -241,3 +241,42 @@ def test_expert_tensors_beyond_the_grouped_kernels_range(run, ty, eff, refused):
             else:
                 assert not refused
     """, ty=ty, eff=eff, refused=refused)
+
+
+@pytest.mark.parametrize("cores", [1, 2, 8])
+@pytest.mark.parametrize("shift_in,shift_out", [(0, 0), (4, 0), (0, 4), (8, 12)])
+def test_workers_and_alignments(run, cores, shift_in, shift_out):
+    """Transfers whole with no worker besides the calling thread, with one and with several, from and to memory of any float
+    alignment; more results than the outbound ring holds (54 MB), ragged last parts."""
+    run("""
+        os.sched_setaffinity(0, set(sorted(os.sched_getaffinity(0))[:cores]))
+        K, N = 256, 4096
+        a = accel(K, N)
+        for m in (300, 3301):
+            xs, y = floats(m * K, shift_in), floats(m * N - 5, shift_out)
+            xs[:] = np.random.default_rng(m).random(m * K, dtype=np.float32)
+            F.fake_keep_inbound(1)
+            assert L.smx_gemm(a._h, b"w", p(xs), m, K, p(y), m * N - 1) == -1          # one result short: refused, nothing moved
+            assert inbound().size == 0 and not y.any()
+            y = floats(m * N, shift_out)
+            assert L.smx_gemm(a._h, b"w", p(xs), m, K, p(y), y.size) == 1
+            assert untouched(y) and np.array_equal(inbound(), xs)
+    """, cores=cores, shift_in=shift_in, shift_out=shift_out)
+
+
+@pytest.mark.parametrize("call,slow", [("a.gemv('w', xs[0], N)", "gemv_flat"), ("a.gemv_rows('w', xs[:3], N)", "gemv_"), ("a.prefill_q8_gemm('w', xs[:70], 70, N)", "gemm_i8"),
+                                       ("a.prefill_q8_gemm('w', xs, 300, N)", "gemm_i8")])
+def test_work_longer_than_the_polls(run, call, slow):
+    """Beyond the polled 2 ms a call waits in the runtime, and its result is whole."""
+    run("""
+        K, N = 256, 4096
+        a = accel(K, N)
+        xs = synth.make_acts(300, K, seed=1)
+        F.fake_slow_kernel(slow.encode(), 50000)
+        for _ in range(3):
+            t0 = time.perf_counter()
+            y = eval(call)
+            assert time.perf_counter() - t0 > 0.05
+            # (a result written by the kernel itself is the pinned buffer's filling here, one copied out the device memory's)
+            assert untouched(y) or (y.view(np.uint32) == 0xeeeeeeee).all()
+    """, call=call, slow=slow)
