@@ -12,7 +12,8 @@
 //
 // Owned by one context, made by its first large call, given back with it: at most kMaxWorkers threads (asleep between
 // calls, and within one when they have found no work for kSpinUs: the device computes) and kInSlots * kPiece + kOutRing bytes
-// of pinned memory.
+// of pinned memory, whatever the call's size.  Making it costs that first call: 190 x 4096 results of 256-long rows 7.8 ms in a
+// fresh process and 1.3 - 1.6 ms in a later context, where the second call takes 0.22 - 0.5; 700 rows 2.7 - 3.4 ms against 0.6.
 #pragma once
 #include <hip/hip_runtime.h>
 
