@@ -9,7 +9,8 @@
 //                      Infinity Cache), one xor and one store per wave: the floor of a GEMV of that size
 //   sbk_copy           plain copy, the streaming rate of the box
 //   sbk_mfma_valu      the int8 GEMM's compute phase alone (MFMA 32x32x32 i8 + the two FMAs per output
-//                      of exact per-block rescaling), with and without its LDS reads: the kernel's ceiling
+//                      of exact per-block rescaling), with and without its LDS reads: the kernel's ceiling;
+//                      and the Q6_K GEMM's (two f16 MFMAs + three vector operations per output)
 #include <hip/hip_fp16.h>
 #include <hip/hip_runtime.h>
 
@@ -108,24 +109,30 @@ typedef int v16i __attribute__((ext_vector_type(16)));
 //           activations: one coalesced 1 KB load per wave and block), the 16 activation scales of a block
 //           as ONE dword per lane read through a DPP row broadcast in the second FMA
 //   MODE 5: as 4 with the activation scales as four 16-byte LDS reads (16 registers)
+//   MODE 6: Q6_K arithmetic on integer MFMAs: two K = 16 MFMAs and four vector operations per output per 32-block
+//   MODE 7: Q6_K arithmetic as the Q6_K GEMM has it: two K = 16 f16 MFMAs, whose float results take three
+typedef _Float16 v8h __attribute__((ext_vector_type(8)));
+typedef float v16f __attribute__((ext_vector_type(16)));
 constexpr int kMagicI = 0x4B400000;
 constexpr float kMagicF = 12582912.f;
 
 #define SBK_FMAC_BC(I)                                                                     \
     asm("v_fmac_f32_dpp %0, %1, %2 row_newbcast:" #I " row_mask:0xf bank_mask:0xf" : "+v"(accv[I]) : "v"(dxv), "v"(t[I]))
+__device__ __forceinline__ void accumulate_dpp(float (&accv)[16], const float (&t)[16], float dxv) {
+    SBK_FMAC_BC(0); SBK_FMAC_BC(1); SBK_FMAC_BC(2); SBK_FMAC_BC(3); SBK_FMAC_BC(4); SBK_FMAC_BC(5); SBK_FMAC_BC(6); SBK_FMAC_BC(7);
+    SBK_FMAC_BC(8); SBK_FMAC_BC(9); SBK_FMAC_BC(10); SBK_FMAC_BC(11); SBK_FMAC_BC(12); SBK_FMAC_BC(13); SBK_FMAC_BC(14); SBK_FMAC_BC(15);
+}
 __device__ __forceinline__ void scale_accumulate_dpp(float (&accv)[16], const v16i& dn, float dw, float ndw, float dxv) {
     float t[16];
 #pragma unroll
     for (int i = 0; i < 16; i++) t[i] = fmaf(dw, __int_as_float(dn[i]), ndw);
-    SBK_FMAC_BC(0); SBK_FMAC_BC(1); SBK_FMAC_BC(2); SBK_FMAC_BC(3); SBK_FMAC_BC(4); SBK_FMAC_BC(5); SBK_FMAC_BC(6); SBK_FMAC_BC(7);
-    SBK_FMAC_BC(8); SBK_FMAC_BC(9); SBK_FMAC_BC(10); SBK_FMAC_BC(11); SBK_FMAC_BC(12); SBK_FMAC_BC(13); SBK_FMAC_BC(14); SBK_FMAC_BC(15);
+    accumulate_dpp(accv, t, dxv);
 }
 
 template <int MODE, int NT, int OCC>
 __global__ __launch_bounds__(256, OCC) void mfma_valu_kernel(const float* __restrict__ scales, int nblocks, float* __restrict__ out,
                                                            unsigned long long* __restrict__ cycles, const v4i* __restrict__ aglob) {
     extern __shared__ __align__(16) char smem[];
-    // LDS: 32 KB of operand bytes (what one stage of the GEMM holds) + 64 blocks of scales
     // LDS: 32 KB of operand bytes (what one stage of the GEMM holds) + 16 blocks of scales
     float* sdx = (float*)(smem + 32768);            // [16][128 tokens]
     float* sdw = sdx + 16 * 128;                    // [16][128 rows]
@@ -151,6 +158,37 @@ __global__ __launch_bounds__(256, OCC) void mfma_valu_kernel(const float* __rest
     v16i d[2];
 #pragma unroll
     for (int i = 0; i < 16; i++) d[0][i] = d[1][i] = kMagicI + lane + i;
+    // MODE 7: activations -128 .. 127 and weights -32 .. 31 as f16, one fragment per 16-element sub-block
+    v8h ha[2], hb[NT][2];
+    if constexpr (MODE == 7) {
+        const signed char* q = (const signed char*)smem + lane * 16;
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+#pragma unroll
+            for (int i = 0; i < 8; i++) {
+                ha[j][i] = (_Float16)(float)q[wave * 4096 + j * 8 + i];
+#pragma unroll
+                for (int nt = 0; nt < NT; nt++) hb[nt][j][i] = (_Float16)(float)(q[16384 + nt * 4096 + j * 8 + i] >> 2);
+            }
+    }
+    const v16f zero = {0.f};
+    v16f df[2][2];
+    auto issue_h = [&](int nt) {
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            df[nt & 1][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ha[j], hb[nt][j], zero, 0, 0, 0);
+            asm volatile("" : "+v"(df[nt & 1][j]));
+        }
+    };
+    if constexpr (MODE == 7) issue_h(0);
+    // MODE 6: 16-element sub-block v & 1 of row tile v >> 1
+    auto unit = [&](int v) -> v16i {
+        const int nt = v >> 1, jj = v & 1;
+        const long a = ((long)(unsigned)fa[2 * jj]) | ((long)fa[2 * jj + 1] << 32);
+        const long bq = ((long)(unsigned)fb[nt][2 * jj]) | ((long)fb[nt][2 * jj + 1] << 32);
+        return __builtin_amdgcn_mfma_i32_32x32x16_i8(a, bq, cmagic, 0, 0, 0);
+    };
+    if constexpr (MODE == 6) d[0] = unit(0);
     const unsigned long long t0 = clock64();
     // MODE 4: lane n of each 16-lane row holds the scale of accumulator n of that row's lane half
     const int dx_tok = ((lane & 15) >> 2) * 8 + half * 4 + (lane & 3);
@@ -161,7 +199,7 @@ __global__ __launch_bounds__(256, OCC) void mfma_valu_kernel(const float* __rest
         const int bs = b & 15;
         float dxr[16], dw[NT];
         float dxv = 0.f;
-        if (MODE != 0 && MODE != 6) {
+        if (MODE != 0 && MODE < 6) {
             if (MODE == 4) {
                 dxv = sdx[bs * 128 + wave * 32 + dx_tok];
             } else {
@@ -174,6 +212,26 @@ __global__ __launch_bounds__(256, OCC) void mfma_valu_kernel(const float* __rest
 #pragma unroll
             for (int nt = 0; nt < NT; nt++) dw[nt] = sdw[bs * 128 + nt * 32 + col];
         }
+        if constexpr (MODE == 7) {
+            dxv = sdx[bs * 128 + wave * 32 + dx_tok];
+            float dw2[NT];
+#pragma unroll
+            for (int nt = 0; nt < NT; nt++) {
+                dw[nt] = sdw[bs * 128 + nt * 32 + col];
+                dw2[nt] = sdw[((bs + 1) & 15) * 128 + nt * 32 + col];
+            }
+#pragma unroll
+            for (int nt = 0; nt < NT; nt++) {
+                issue_h((nt + 1) % NT);   // (the next block's first unit under this one's last FMAs)
+                __builtin_amdgcn_sched_barrier(0);
+                float t[16];
+#pragma unroll
+                for (int i = 0; i < 16; i++) t[i] = fmaf(dw[nt], df[nt & 1][0][i], dw2[nt] * df[nt & 1][1][i]);
+                accumulate_dpp(acc[nt], t, dxv);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            continue;
+        }
         if constexpr (MODE == 6) {
             // Q6_K arithmetic: the format scales 16-element sub-blocks, so a 32-block of a row tile is two K = 16 MFMAs, each
             // rescaled by its own weight scale: four vector operations per output per 32-block (the activation scale through a
@@ -185,19 +243,11 @@ __global__ __launch_bounds__(256, OCC) void mfma_valu_kernel(const float* __rest
                 dw[nt] = sdw[bs * 128 + nt * 32 + col];
                 dw2[nt] = sdw[((bs + 1) & 15) * 128 + nt * 32 + col];
             }
-            auto unit = [&](int v) -> v16i {
-                const int nt = v >> 1, jj = v & 1;
-                const long a = ((long)(unsigned)fa[2 * jj]) | ((long)fa[2 * jj + 1] << 32);
-                const long bq = ((long)(unsigned)fb[nt][2 * jj]) | ((long)fb[nt][2 * jj + 1] << 32);
-                return __builtin_amdgcn_mfma_i32_32x32x16_i8(a, bq, cmagic, 0, 0, 0);
-            };
-            d[0] = unit(0);
 #pragma unroll
             for (int v = 0; v < 2 * NT; v++) {
-                if (v + 1 < 2 * NT) {
-                    d[(v + 1) & 1] = unit(v + 1);
-                    asm volatile("" : "+v"(d[(v + 1) & 1]));
-                }
+                d[(v + 1) & 1] = unit((v + 1) % (2 * NT));
+                asm volatile("" : "+v"(d[(v + 1) & 1]));
+                __builtin_amdgcn_sched_barrier(0);
                 const int u = v >> 1;
                 const float dwv = (v & 1) ? dw2[u] : dw[u];
                 scale_accumulate_dpp(acc[u], d[v & 1], dwv, -dwv * kMagicF, dxv);
@@ -435,7 +485,7 @@ int sbk_copy(size_t bytes, int launches, double* us_per_launch) {
 // `warm_launches` untimed launches come first: under matrix load the chip takes some 20 ms to settle at the clock it
 // then sustains (the first launches after idle run 15 % slower), and a prefill is hundreds of such launches.
 int sbk_mfma_valu(int mode, int row_tiles, int wgs_per_cu, int nblocks, int warm_launches, double* us, double* tops, double* cycles_per_unit) {
-    if (!us || !tops || !cycles_per_unit || mode < 0 || mode > 6 || wgs_per_cu < 1 || wgs_per_cu > 4 || nblocks <= 0 || warm_launches < 1) return SBK_ERR;
+    if (!us || !tops || !cycles_per_unit || mode < 0 || mode > 7 || wgs_per_cu < 1 || wgs_per_cu > 4 || nblocks <= 0 || warm_launches < 1) return SBK_ERR;
     if ((row_tiles != 4 && row_tiles != 2) || (row_tiles == 4 && wgs_per_cu > 3)) return SBK_ERR;
     Timer t;
     if (!t.ok) return SBK_ERR;
@@ -456,12 +506,12 @@ int sbk_mfma_valu(int mode, int row_tiles, int wgs_per_cu, int nblocks, int warm
         (void)hipMemcpy(scales, h.data(), 1024 * 4, hipMemcpyHostToDevice);
         typedef void (*kern_t)(const float*, int, float*, unsigned long long*, const v4i*);
         // [mode][tile 4/2][occupancy class: waves per SIMD the register budget is set for]
-        static const kern_t k4lo[7] = {mfma_valu_kernel<0, 4, 2>, mfma_valu_kernel<1, 4, 2>, mfma_valu_kernel<2, 4, 2>, mfma_valu_kernel<3, 4, 2>,
-                                       mfma_valu_kernel<4, 4, 2>, mfma_valu_kernel<5, 4, 2>, mfma_valu_kernel<6, 4, 2>};
-        static const kern_t k4hi[7] = {mfma_valu_kernel<0, 4, 3>, mfma_valu_kernel<1, 4, 3>, mfma_valu_kernel<2, 4, 3>, mfma_valu_kernel<3, 4, 3>,
-                                       mfma_valu_kernel<4, 4, 3>, mfma_valu_kernel<5, 4, 3>, mfma_valu_kernel<6, 4, 3>};
-        static const kern_t k2[7] = {mfma_valu_kernel<0, 2, 4>, mfma_valu_kernel<1, 2, 4>, mfma_valu_kernel<2, 2, 4>, mfma_valu_kernel<3, 2, 4>,
-                                     mfma_valu_kernel<4, 2, 4>, mfma_valu_kernel<5, 2, 4>, mfma_valu_kernel<6, 2, 4>};
+        static const kern_t k4lo[8] = {mfma_valu_kernel<0, 4, 2>, mfma_valu_kernel<1, 4, 2>, mfma_valu_kernel<2, 4, 2>, mfma_valu_kernel<3, 4, 2>,
+                                       mfma_valu_kernel<4, 4, 2>, mfma_valu_kernel<5, 4, 2>, mfma_valu_kernel<6, 4, 2>, mfma_valu_kernel<7, 4, 2>};
+        static const kern_t k4hi[8] = {mfma_valu_kernel<0, 4, 3>, mfma_valu_kernel<1, 4, 3>, mfma_valu_kernel<2, 4, 3>, mfma_valu_kernel<3, 4, 3>,
+                                       mfma_valu_kernel<4, 4, 3>, mfma_valu_kernel<5, 4, 3>, mfma_valu_kernel<6, 4, 3>, mfma_valu_kernel<7, 4, 3>};
+        static const kern_t k2[8] = {mfma_valu_kernel<0, 2, 4>, mfma_valu_kernel<1, 2, 4>, mfma_valu_kernel<2, 2, 4>, mfma_valu_kernel<3, 2, 4>,
+                                     mfma_valu_kernel<4, 2, 4>, mfma_valu_kernel<5, 2, 4>, mfma_valu_kernel<6, 2, 4>, mfma_valu_kernel<7, 2, 4>};
         const kern_t kern = row_tiles == 2 ? k2[mode] : (wgs_per_cu <= 2 ? k4lo[mode] : k4hi[mode]);
         auto launch = [&]() { hipLaunchKernelGGL(kern, dim3(grid), dim3(256), lds, t.s, (const float*)scales, nblocks, out, cyc, (const v4i*)aglob); };
         if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess) rc = SBK_ERR;

@@ -6,7 +6,7 @@
 //   * v_mfma_f32_32x32x16_f16: K = 16 is one sub-block, its result the exact dot as a float, and
 //     acc += dx * (dw0 * I0 + dw1 * I1) takes three VALU operations per output and 32-block.  Bound: these, with the MFMAs
 //     (they add up: a SIMD runs both at one power budget).  v_mfma_i32_32x32x16_i8 has the same rate but an integer result,
-//     whose exact rescale takes four: 617 against 781 TOPS in a loop of nothing else.
+//     whose exact rescale takes four: 536 against 725 TOPS in a loop of nothing else (the machine floors of bench.py).
 //   * The weights are widened to f16 once per workgroup, on their way into LDS (two blocks of a row = 128 bytes); a wave
 //     reads its own 32 tokens only, as int8, and widens them itself: 20 operations per block next to 192.
 //   * A stage is 4 blocks (half a superblock).  The activations and the scales of a stage are double-buffered, the widened
