@@ -1200,6 +1200,7 @@ int smx_moe_layer_ffn(smx_ctx* c, size_t layer, const int32_t* plan, size_t npla
     TableBlob tb;
     const size_t o_t1 = tb.add(tiles_gu.data(), tiles_gu.size() * sizeof(GemmTile)),
                  o_t2 = tb.add(tiles_dn.data(), tiles_dn.size() * sizeof(GemmTile));
+    HostCall call(c);
     if ((rc = tb.upload(c)) != SMX_OK) return rc;
     HostPipe* hp = nullptr;
     const float* x_dev;
@@ -1207,7 +1208,8 @@ int smx_moe_layer_ffn(smx_ctx* c, size_t layer, const int32_t* plan, size_t npla
     SlotScratch ss = {};
     rc = moe_slots_enqueue(c, L, x_dev, rows, nullptr, rows, (const GemmTile*)(c->tab.p + o_t1), tiles_gu.size(),
                            (const GemmTile*)(c->tab.p + o_t2), tiles_dn.size(), &ss);
-    return host_receive(c, dy, ss.dy, rows * hidden * 4, hp, rc);
+    rc = host_receive(c, dy, ss.dy, rows * hidden * 4, hp, rc);
+    return rc == SMX_OK ? call.done() : rc;
     });
 }
 
