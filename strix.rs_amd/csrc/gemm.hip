@@ -397,21 +397,31 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float4* __rest
 // launch that is estimated to take least, among tiles of 64 (Q8_0, Q4_0) and 128 tokens and every number of whole-stage slices
 // whose workgroups fit the chip's slots in ONE round (a second, partly filled round costs more than shorter slices save): a
 // workgroup's stages one after the other, at the time a stage takes with the CU to itself or shared with a second
-// workgroup, plus the launch that adds up the slices' partials, 3.5 us and 5 MB of them per us.  Tiles that need several rounds: 128 tokens, one slice.
-// The stage times are measured (us): 64 tokens 1.05 alone / 1.46 shared, 128 tokens 1.55 / 2.7, Q6_K 2.75 / 4.3.  Per call against a
+// workgroup, plus the launch that adds up the slices' partials, 3.5 us and 5 MB of them per us.  Tiles that need several rounds: one slice, 128
+// tokens or (Q6_K) 256, whichever's rounds take less.
+// The stage times are measured (us): 64 tokens 1.05 alone / 1.46 shared, 128 tokens 1.55 / 2.7, Q6_K 2.75 / 4.3, its 256-token tiles (one
+// workgroup per CU) 3.9.  Per call against a
 // rule of at least 6 stages per slice and 128-token tiles: Q8_0 200 x 2560 x 2560 23.5 -> 19 us, 300 x 9728 x 2560 41.2 -> 36.8,
 // 333 x 2560 x 9728 43.8 -> 41.2 (Q4_0 44.5 -> 42.9), Q4_0 103 x 1088 x 1024 15.5 -> 12.0, Q6_K 72 x 2208 x 3328 28.9 -> 21.2, 600 x 2560 x
 // 2560 44.0 -> 37.5; Q8_0 500 and 1000 x 2560 x 9728 keep 128-token tiles (64: 52.8 for 52.1, 109 for 87.4).
 struct Tiling { int bm, slices; };
-static Tiling pick_tiling(int num_cu, int slots, bool q6, int M, int N, int nstages, bool split) {
+static Tiling pick_tiling(int num_cu, bool q6, int M, int N, int nstages, bool split, bool dump) {
     Tiling best = {128, 1};
     double least = 1e30;
-    for (int bm : {64, 128}) {
-        if ((bm == 64) ? q6 || M <= 64 : !q6 && M > 64 && M <= 128) continue;   // (65..128 tokens: as two rows of tiles)
-        const int T = (M + bm - 1) / bm * ((N + BN - 1) / BN);
-        if (T > slots) continue;
+    for (int bm : {64, 128, 256}) {
+        if (bm == 64 ? q6 || M <= 64 : bm == 128 ? !q6 && M > 64 && M <= 128 : !q6 || M <= 128 || dump) continue;   // (65..128 tokens: as two rows of tiles)
+        const int T = (M + bm - 1) / bm * ((N + BN - 1) / BN), slots = bm == 256 ? num_cu : 2 * num_cu;
         const bool low = bm == 64 || M <= 64;
-        const double alone = q6 ? 2.75 : low ? 1.05 : 1.55, shared = q6 ? 4.3 : low ? 1.46 : 2.7;
+        const double alone = bm == 256 ? 3.9 : q6 ? 2.75 : low ? 1.05 : 1.55, shared = bm == 256 ? 3.9 : q6 ? 4.3 : low ? 1.46 : 2.7;
+        if (T > slots) {   // whole rounds and the rest
+            const int rest = T % slots;
+            const double us = nstages * (T / slots * shared + (rest > num_cu ? shared : rest > 0 ? alone : 0.0));
+            if (bm >= 128 && us < least) {
+                least = us;
+                best = {bm, 1};
+            }
+            continue;
+        }
         const int zmax = split ? std::min(std::min(slots / T, nstages), 16) : 1;
         for (int z = 1; z <= zmax; z++) {
             const int stages = (nstages + z - 1) / z;
@@ -427,15 +437,16 @@ static Tiling pick_tiling(int num_cu, int slots, bool q6, int M, int N, int nsta
 }
 
 template <class Kernel>
-static int launch_gemm_variant(smx_ctx* c, Kernel k, size_t lds, const GemmArgs& p, dim3 grid) {
+static int launch_gemm_variant(smx_ctx* c, Kernel k, size_t lds, const GemmArgs& p, dim3 grid, int nw = NW) {
     int rc = set_dyn_lds(c, k, lds);
     if (rc != SMX_OK) return rc;
-    hipLaunchKernelGGL(k, grid, dim3(64 * NW), lds, c->stream, p);
+    hipLaunchKernelGGL(k, grid, dim3(64 * nw), lds, c->stream, p);
     SMX_HIP(c, hipGetLastError());
     return SMX_OK;
 }
 static int launch_gemm_type(smx_ctx* c, QType type, bool dump, const GemmArgs& p, dim3 grid) {
-    if (type == kQ6_K) return launch_gemm_variant(c, dump ? gemm_q6_kernel<true> : gemm_q6_kernel<false>, Q6_LDS_BYTES, p, grid);
+    if (type == kQ6_K && p.tile_m == 256) return launch_gemm_variant(c, gemm_q6_kernel<false, 8>, q6_lds_bytes(8), p, grid, 8);
+    if (type == kQ6_K) return launch_gemm_variant(c, dump ? gemm_q6_kernel<true, NW> : gemm_q6_kernel<false, NW>, q6_lds_bytes(NW), p, grid);
     if (type == kQ4_0) return launch_gemm_variant(c, dump ? gemm_i8_kernel<true, true> : gemm_i8_kernel<true, false>, 2 * STAGE_BYTES, p, grid);
     return launch_gemm_variant(c, dump ? gemm_i8_kernel<false, true> : gemm_i8_kernel<false, false>, 2 * STAGE_BYTES, p, grid);
 }
@@ -466,21 +477,21 @@ int launch_gemm(smx_ctx* c, const Weight& w, const int8_t* xq, const float* xd, 
     p.N = (int)w.N;
     p.ldo = (int)w.N;
     p.nb = (int)(w.K / 32);
-    // 128 x 128 tiles, two 4-wave workgroups per CU.  Measured alternatives, all slower on every shape tried
-    // (M 512..4096 of both FFN shapes, grouped MoE tiles): 256 x 128 tiles with one 8-wave workgroup per CU
+    // 128 x 128 tiles, two 4-wave workgroups per CU (Q6_K from 129 tokens on also 256 x 128, gemm_q6.h).  Measured alternatives for
+    // Q8_0 and Q4_0, all slower on every shape tried (M 512..4096 of both FFN shapes, grouped MoE tiles): 256 x 128 tiles with one 8-wave workgroup per CU
     // (-7 %); three workgroups per CU with 2-block stages, every operand and scale staged LDS-direct and the
     // LDS reads software-pipelined (-5..-10 %: the third wave per SIMD raises the instruction issue rate,
     // and the clock the chip sustains drops by as much).
-    const int slots = c->num_cu * 2;
     p.tiles_n = (p.N + BN - 1) / BN;
     const int nstages = (p.nb + KB - 1) / KB;
     const bool may_split = dump == nullptr && (m * w.N) % 4 == 0;
-    const Tiling tiling = pick_tiling(c->num_cu, slots, w.type == kQ6_K, p.M, p.N, nstages, may_split && c->tune_gemm_splitk == 0);
+    const Tiling tiling = pick_tiling(c->num_cu, w.type == kQ6_K, p.M, p.N, nstages, may_split && c->tune_gemm_splitk == 0, dump != nullptr);
     // 65..128 tokens are always two rows of 64-token tiles (in one row of 128 half the waves of a workgroup may idle): Q8_0
     // 2560 x 9728 and 9728 x 2560 at 96 / 128 tokens 28.2 / 29.4 -> 25.4 / 26.7 us and 25.9 / 27.3 -> 22.9 / 24.7 us.
     int bm = tiling.bm;
     if (p.M > 64 && p.M <= 128 && w.type != kQ6_K) bm = 64;   // (also when they need several rounds)
-    if (c->tune_gemm_tile_m != 0) bm = c->tune_gemm_tile_m;
+    if (c->tune_gemm_tile_m != 0) bm = c->tune_gemm_tile_m == 256 && (w.type != kQ6_K || dump) ? 128 : c->tune_gemm_tile_m;
+    const int slots = c->num_cu * (bm == 256 ? 1 : 2);   // workgroups the chip holds
     p.tile_m = bm;
     p.tiles_m = (p.M + bm - 1) / bm;
     const int T = p.tiles_m * p.tiles_n;
@@ -509,7 +520,7 @@ int launch_gemm(smx_ctx* c, const Weight& w, const int8_t* xq, const float* xd, 
     // Q6_K weights only: measured at that shape Q6_K 598 -> 575 us per launch, Q8_0 339.6 -> 337 and Q4_0 350.7 -> 349 (inside
     // the spread between machines, with 2.5 % more vector instructions per launch: a partly filled round runs faster
     // already, a workgroup alone on a CU has its SIMDs to itself).  The knob forces any number of strips for any format.
-    if (Z == 1 && bm == 128 && !dump && c->tune_gemm_narrow != 1) {
+    if (Z == 1 && bm >= 128 && !dump && c->tune_gemm_narrow != 1) {
         const auto makespan = [&](int b) -> double {   // in 128-row tile times; -1: N does not split that way
             if (96 * b > p.N) return -1.0;
             const int a = (p.N - 96 * b + BN - 1) / BN;

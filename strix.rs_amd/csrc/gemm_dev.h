@@ -76,10 +76,17 @@ struct WaveRole {
     int nt_cnt;    // row tiles of this wave; a tile at the end of N, or a 96-row strip: only the row tiles that exist
     int nt_base;
 };
-__device__ __forceinline__ WaveRole gemm_wave_role(const TileAt& t, int wave) {
+// A workgroup of eight waves (256 tokens): 32 tokens a wave, all of the row tiles.
+__device__ __forceinline__ WaveRole gemm_wave_role(const TileAt& t, int wave, int nw = NW) {
     WaveRole r;
     r.live_tok = t.M_end - t.tok0;
     r.live_rows = min(t.N_end - t.row0, BN);
+    if (nw > NW) {
+        r.tw = wave;
+        r.nt_cnt = (r.live_rows + 31) >> 5;
+        r.nt_base = 0;
+        return r;
+    }
     r.tw = r.live_tok <= 32 ? 0 : r.live_tok <= 64 ? (wave & 1) : wave;
     r.nt_cnt = r.live_tok <= 32 ? 1 : r.live_tok <= 64 ? 2 : (r.live_rows + 31) >> 5;
     r.nt_base = r.live_tok <= 32 ? wave : r.live_tok <= 64 ? (wave >> 1) * 2 : 0;

@@ -11,7 +11,12 @@
 //     reads its own 32 tokens only, as int8, and widens them itself: 20 operations per block next to 192.
 //   * A stage is 4 blocks (half a superblock).  The activations and the scales of a stage are double-buffered, the widened
 //     weights by halves of a stage (low nibbles = blocks 0 and 1, high nibbles = 2 and 3), so that two workgroups fit a CU.
+//   * NW = 8: a workgroup of 256 tokens, one per CU.  What a stage costs besides its arithmetic is weights: loading, widening and
+//     scaling them takes 30 % of the time of the two 128-token workgroups that share a CU (each repeats it), and half as
+//     much here.  The barriers cost more (all eight waves meet), most of it given back by the waves' priorities below.
 // 2048 tokens x 15360 x 3840: 573 -> 485 us against the integer form, 1000 tokens 318 -> 270 us, 300 tokens x 2560 x 2560 35 -> 29 us.
+// 256-token tiles against 128-token ones (same bits): 2048 x 15360 x 3840 501 -> 475 us, 2048 x 3840 x 15360 549 -> 490, 1000 x 15360 x
+// 3840 265 -> 241, 512 tokens 138.5 -> 123, 400 x 9728 x 2560 94.4 -> 82; without the priorities 2 % more.
 #pragma once
 #include "gemm_dev.h"
 
@@ -21,8 +26,8 @@ typedef _Float16 v2h __attribute__((ext_vector_type(2)));
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 typedef float v16f __attribute__((ext_vector_type(16)));
 
-constexpr int Q6_W_BYTES = KB * 128 * 8, Q6_X_BYTES = KB * BM * 4;   // scales of a stage: two floats per row and block, one per token and block
-constexpr int Q6_LDS_BYTES = 2 * (A_BYTES + B_BYTES + Q6_W_BYTES + Q6_X_BYTES);
+constexpr int Q6_W_BYTES = KB * 128 * 8;   // weight scales of a stage: two floats per row and block
+constexpr int q6_lds_bytes(int nw) { return 2 * (nw * 4 * GRP + B_BYTES + Q6_W_BYTES + KB * 32 * nw * 4); }
 
 // four bytes 0..255 -> two pairs of f16 with `off` taken off: 0x6400 | v is the f16 1024 + v
 __device__ __forceinline__ void widen_h(unsigned v, _Float16 off, unsigned& lo, unsigned& hi) {
@@ -31,15 +36,16 @@ __device__ __forceinline__ void widen_h(unsigned v, _Float16 off, unsigned& lo, 
     hi = __builtin_bit_cast(unsigned, __builtin_bit_cast(v2h, __builtin_amdgcn_perm(0x64646464u, v, 0x04030402u)) - o);
 }
 
-template <bool DUMP>
+template <bool DUMP, int NW>
 __global__ __launch_bounds__(64 * NW, 2) void gemm_q6_kernel(GemmArgs p) {
     SMX_GEMM_T0;
+    constexpr int BM = 32 * NW, A_BYTES = 4 * NW * GRP, Q6_X_BYTES = KB * BM * 4;   // NW 8: a workgroup of 256 tokens, one per CU
     extern __shared__ __align__(16) char smem[];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const unsigned smem_base = lds_addr(smem);
     const TileAt at = gemm_tile_at(p);
-    const WaveRole role = gemm_wave_role(at, wave);
+    const WaveRole role = gemm_wave_role(at, wave, NW);
     const int tok0 = at.tok0, row0 = at.row0, M_end = at.M_end, N_end = at.N_end, nt_base = role.nt_base;
     const GemmOperand op = p.op[at.op_i];
     const int s_begin = blockIdx.z * p.stages_per_slice;
@@ -57,14 +63,16 @@ __global__ __launch_bounds__(64 * NW, 2) void gemm_q6_kernel(GemmArgs p) {
     // quants: thread = [row:7][q:1] reads ql[16q..], ql[32 + 16q..] and qh[16q..] of the stage's half superblock: sub-block q of
     // its four blocks (ggml_quant.rs:417-426).  Scales: thread (row sr, half sh) carries d and the sub-block scales
     // 4 * sh .. 4 * sh + 3 of weight row sr; waves 2 and 3 also the four activation scales of token sr.
-    const int q_row = tid >> 1, q_p = tid & 1, sr = tid & 127, sh = tid >> 7;
+    constexpr int QI = 8 / NW;   // 16-byte pieces of ql per thread and stage; blocks of weight scales
+    const int q_row = tid / (2 * (NW / 4)), q_p = tid & 1, q_i = NW == 8 ? (tid >> 1) & 1 : 0, sr = tid & 127, sh = tid >> 7;
+    const int xr = tid & (BM - 1);
     const unsigned nsb = (unsigned)(p.nb >> 3);   // superblocks of a row (M*K and N*K are below 2^31: launch_gemm, moe_check_shape)
     unsigned q_sb = (unsigned)min(row0 + q_row, N_end - 1) * nsb, s_sb = (unsigned)min(row0 + sr, N_end - 1) * nsb, x_b;
     {
-        const int ti = min(tok0 + sr, M_end - 1);
+        const int ti = min(tok0 + xr, M_end - 1);
         x_b = (unsigned)(p.a_rowmap ? p.a_rowmap[ti] : ti) * (unsigned)p.nb;
     }
-    const bool w_valid = row0 + sr < N_end, x_valid = tok0 + sr < M_end, role_x = wave >= 2;
+    const bool w_valid = row0 + sr < N_end, x_valid = tok0 + xr < M_end, role_x = wave >= NW / 2;
     uint4 rq0, rq1, rqh, rsx = {0, 0, 0, 0};
     unsigned rsc;
     uint16_t rsd;
@@ -79,12 +87,14 @@ __global__ __launch_bounds__(64 * NW, 2) void gemm_q6_kernel(GemmArgs p) {
         asm volatile("" : "+v"(q_sb), "+v"(s_sb), "+v"(x_b));   // not hoisted: the address arithmetic is cheaper than registers held across the loop
         const int sb = s >> 1, h = s & 1;
         const char* ql = (const char*)op.wquants + (size_t)sb * 128 + h * 64;
-        const unsigned o = q_sb * 128u + q_p * 16;
+        const unsigned o = q_sb * 128u + q_p * 16 + q_i * 32;
         rq0 = *(const uint4*)(ql + o);
-        rq1 = *(const uint4*)(ql + (o + 32u));
+        if constexpr (QI == 2) rq1 = *(const uint4*)(ql + (o + 32u));
         rqh = *(const uint4*)((const char*)op.wqh + (size_t)sb * 64 + h * 32 + (q_sb * 64u + q_p * 16));
         rsd = *(const uint16_t*)((const char*)(op.wscales + sb) + s_sb * 2u);
-        rsc = *(const unsigned*)((const char*)op.wsc + (size_t)sb * 16 + h * 8 + (s_sb * 16u + sh * 4));
+        const char* psc = (const char*)op.wsc + (size_t)sb * 16 + h * 8 + (s_sb * 16u + sh * (2 * QI));
+        if constexpr (QI == 2) rsc = *(const unsigned*)psc;
+        else rsc = *(const uint16_t*)psc;
         if (role_x) rsx = *(const uint4*)((const char*)(p.xd + (size_t)s * KB) + x_b * 4u);
     };
     // blocks 2 * h and 2 * h + 1 of the stage, widened; 16-byte chunk c (= block 1b, sub-block 1b, half 1b) of row r at slot (c + r) % 8
@@ -92,14 +102,18 @@ __global__ __launch_bounds__(64 * NW, 2) void gemm_q6_kernel(GemmArgs p) {
         constexpr int h = decltype(hc)::value;
         char* b = smem + 2 * A_BYTES + h * B_BYTES + (q_row >> 3) * GRP + (q_row & 7) * 128;
 #pragma unroll
-        for (int i = 0; i < 2; i++) {
-            const uint4 q = i ? rq1 : rq0;
+        for (int ii = 0; ii < QI; ii++) {
+            const int i = QI == 2 ? ii : q_i;
+            const uint4 q = ii ? rq1 : rq0;
             const unsigned v[4] = {q.x, q.y, q.z, q.w}, g[4] = {rqh.x, rqh.y, rqh.z, rqh.w};
 #pragma unroll
             for (int e = 0; e < 2; e++) {
                 uint4 o;
                 const int hs = 2 * (2 * h + i);
-                const auto bits = [&](int k) { return ((v[k] >> (4 * h)) & 0x0f0f0f0fu) | ((hs < 4 ? g[k] << (4 - hs) : g[k] >> (hs - 4)) & 0x30303030u); };
+                const auto bits = [&](int k) {
+                    const unsigned hi = QI == 1 ? ((g[k] >> (2 * i)) >> (4 * h)) << 4 : hs < 4 ? g[k] << (4 - hs) : g[k] >> (hs - 4);
+                    return ((v[k] >> (4 * h)) & 0x0f0f0f0fu) | (hi & 0x30303030u);
+                };
                 widen_h(bits(2 * e), (_Float16)1056.f, o.x, o.y);
                 widen_h(bits(2 * e + 1), (_Float16)1056.f, o.z, o.w);
                 *(uint4*)(b + ((i * 4 + q_p * 2 + e + q_row) & 7) * 16) = o;
@@ -110,20 +124,19 @@ __global__ __launch_bounds__(64 * NW, 2) void gemm_q6_kernel(GemmArgs p) {
         float2* sdw = (float2*)(smem + 2 * (A_BYTES + B_BYTES) + buf * Q6_W_BYTES);
         const float d = w_valid ? h2f_(rsd) : 0.f;   // d * sc is exact in fp32 (11 x 8 significant bits)
         const auto sc = [&](int j) { return d * (float)(int)(signed char)(rsc >> (8 * j)); };
-        sdw[(2 * sh) * 128 + sr] = make_float2(sc(0), sc(1));
-        sdw[(2 * sh + 1) * 128 + sr] = make_float2(sc(2), sc(3));
+#pragma unroll
+        for (int j = 0; j < QI; j++) sdw[(QI * sh + j) * 128 + sr] = make_float2(sc(2 * j), sc(2 * j + 1));
         if (role_x) {
             float* sdx = (float*)(smem + 2 * (A_BYTES + B_BYTES + Q6_W_BYTES) + buf * Q6_X_BYTES);
             const unsigned v[4] = {rsx.x, rsx.y, rsx.z, rsx.w};
 #pragma unroll
-            for (int j = 0; j < KB; j++) sdx[j * BM + sr] = x_valid ? __uint_as_float(v[j]) : 0.f;
+            for (int j = 0; j < KB; j++) sdx[j * BM + xr] = x_valid ? __uint_as_float(v[j]) : 0.f;
         }
     };
 
     // ---- arithmetic ----
     const int half = lane >> 5, col = lane & 31;
     const int row_off = (col >> 3) * GRP + (col & 7) * 128;
-    const int dx_tok = role.tw * 32 + ((lane & 15) >> 2) * 8 + half * 4 + (lane & 3);  // token of accumulator lane % 16 in this lane's half
     float acc[4][16];
 #pragma unroll
     for (int nt = 0; nt < 4; nt++)
@@ -131,7 +144,10 @@ __global__ __launch_bounds__(64 * NW, 2) void gemm_q6_kernel(GemmArgs p) {
         for (int i = 0; i < 16; i++) acc[nt][i] = 0.f;
     v8h af[2];       // the tokens' fragments of the block whose MFMAs are being issued, per sub-block
     int2 araw[2];    // the next block's, before widening
-    float dxv[4];    // per block: lane n of each 16-lane row holds the scale of the token of accumulator n
+    // Activation scales of the 16 tokens this lane accumulates, of the block whose products are being scaled.  (As one per lane,
+    // read through a row broadcast, they cost a register and one read instead of four; but a broadcast multiply-add takes a SIMD
+    // 4 cycles and keeps the other wave's from issuing beside it, where a plain one takes 2: 1000 x 15360 x 3840 261 -> 254 us.)
+    float4 dx[4];
     v4i bf[2][2];    // weight fragments, two units in turn, per sub-block
     float2 dw[4];    // weight scales of this lane's row, four units in turn
     v16f d[2][2];    // products, two units in turn, per sub-block
@@ -141,7 +157,6 @@ __global__ __launch_bounds__(64 * NW, 2) void gemm_q6_kernel(GemmArgs p) {
         const int bi = (g / NT) & 3, nt = g % NT;
         if (nt == 0) {
             const char* sA = smem + buf * A_BYTES + role.tw * 4 * GRP + row_off + half * 8;
-            dxv[bi] = ((const float*)(smem + 2 * (A_BYTES + B_BYTES + Q6_W_BYTES) + buf * Q6_X_BYTES))[bi * BM + dx_tok];
             araw[0] = *(const int2*)(sA + ((2 * bi + col) & 7) * 16);
             araw[1] = *(const int2*)(sA + ((2 * bi + 1 + col) & 7) * 16);
         }
@@ -149,6 +164,11 @@ __global__ __launch_bounds__(64 * NW, 2) void gemm_q6_kernel(GemmArgs p) {
         bf[g & 1][0] = *(const v4i*)(sB + (((bi & 1) * 4 + half + col) & 7) * 16);
         bf[g & 1][1] = *(const v4i*)(sB + (((bi & 1) * 4 + 2 + half + col) & 7) * 16);
         dw[g & 3] = ((const float2*)(smem + 2 * (A_BYTES + B_BYTES) + buf * Q6_W_BYTES))[bi * 128 + (nt_base + nt) * 32 + col];
+    };
+    auto read_dx = [&](int bi, int buf) __attribute__((always_inline)) {
+        const float* sdx = (const float*)(smem + 2 * (A_BYTES + B_BYTES + Q6_W_BYTES) + buf * Q6_X_BYTES) + bi * BM + role.tw * 32 + half * 4;
+#pragma unroll
+        for (int g = 0; g < 4; g++) dx[g] = *(const float4*)(sdx + g * 8);
     };
     auto widen_tokens = [&]() __attribute__((always_inline)) {
 #pragma unroll
@@ -204,6 +224,15 @@ __global__ __launch_bounds__(64 * NW, 2) void gemm_q6_kernel(GemmArgs p) {
             } else {
 #pragma unroll
                 for (int g = 0; g < U; g++) {
+                    if constexpr (NW == 8) {
+                        // The two waves of a SIMD meet at every stage's barriers; the elder would issue whenever it can and then
+                        // wait there while the other goes on alone, at two thirds of the rate of both.  Priority falls with the way.
+                        if (g == 0) __builtin_amdgcn_s_setprio(3);
+                        else if (g == U / 4) __builtin_amdgcn_s_setprio(2);
+                        else if (g == U / 2) __builtin_amdgcn_s_setprio(1);
+                        else if (g == 3 * U / 4) __builtin_amdgcn_s_setprio(0);
+                    }
+                    if (g % NT == 0) read_dx(g / NT, buf);
                     if ((g + 1) % NT == 0) widen_tokens();
                     mfma_unit(g + 1);   // (behind the last stage: of stale operands, never used)
                     if (g + 2 == U / 2) __syncthreads();
@@ -216,7 +245,12 @@ __global__ __launch_bounds__(64 * NW, 2) void gemm_q6_kernel(GemmArgs p) {
                     float t[16];
 #pragma unroll
                     for (int i = 0; i < 16; i++) t[i] = fmaf(w.x, d0[i], w.y * d1[i]);
-                    bcast_accumulate(acc[nt], t, dxv[bi]);
+                    const float dxr[16] = {dx[0].x, dx[0].y, dx[0].z, dx[0].w, dx[1].x, dx[1].y, dx[1].z, dx[1].w,
+                                           dx[2].x, dx[2].y, dx[2].z, dx[2].w, dx[3].x, dx[3].y, dx[3].z, dx[3].w};
+#pragma unroll
+                    for (int i = 0; i < 16; i++) acc[nt][i] = fmaf(dxr[i], t[i], acc[nt][i]);
+#pragma unroll
+                    for (int i = 0; i < 16; i++) asm volatile("" : "+v"(acc[nt][i]));   // (not moved between units: they would spill)
                     if constexpr (DUMP) {
                         const int row = row0 + (nt_base + nt) * 32 + col;
 #pragma unroll

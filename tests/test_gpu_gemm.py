@@ -230,3 +230,31 @@ def test_gemm_tile_heights_agree(accel, orc, synth, relerr, ty, m, N, K):
     finally:
         accel.tune("gemm_tile_m", 0)
     accel.evict("t.th")
+
+
+@pytest.mark.parametrize("m,N,K", [(129, 130, 256), (257, 300, 768), (290, 96, 2560), (511, 1000, 512), (640, 15000, 256), (1000, 416, 4096)])
+def test_gemm_q6_k_wide_tiles(accel, orc, synth, relerr, m, N, K):
+    """256-token tiles of a Q6_K weight: last tiles of 1, 34, 128 and all but one tokens, strips that end inside a row tile, one
+    stage pair and many, several rounds of workgroups, K slices.  Unsplit they give the bits of 128-token tiles."""
+    raw = synth.make_weight(14, N, K, seed=N)
+    xs = synth.make_acts(m, K, seed=m)
+    assert accel.upload_q6_k("t.wide", raw, K, N)
+    ref = orc.matmul_q8_from_f32(14, raw, K, N, xs)
+    try:
+        for splitk in (1, 0, 3):
+            accel.tune("gemm_splitk", splitk)
+            ys = {}
+            for height in (0, 128, 256):
+                accel.tune("gemm_tile_m", height)
+                ys[height] = accel.prefill_q8_gemm("t.wide", xs, m, N)
+                assert relerr(ys[height], ref) <= TOL, (splitk, height)
+            if splitk == 1:
+                assert np.array_equal(ys[128], ys[256]) and np.array_equal(ys[0], ys[256])
+        accel.tune("gemm_splitk", 0)
+        for narrow in (2, 4):   # strips of 96 rows as well
+            accel.tune("gemm_narrow", narrow)
+            assert relerr(accel.prefill_q8_gemm("t.wide", xs, m, N), ref) <= TOL, narrow
+    finally:
+        for knob in ("gemm_tile_m", "gemm_splitk", "gemm_narrow"):
+            accel.tune(knob, 0)
+    accel.evict("t.wide")
