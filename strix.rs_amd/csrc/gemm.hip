@@ -8,7 +8,8 @@
 //   * workgroup tile 128 tokens x 128 rows, 4 waves, each wave 32 tokens x 128 rows;
 //   * K advances 4 blocks (128 bytes per row, one full cache line) per stage, double-buffered
 //     through LDS in MFMA-fragment order so every fragment read is one conflict-free 128-bit load;
-//   * Q4_0 nibbles are widened to signed int8 (nibble - 8) while being staged (kernels.rs:458-462);
+//   * Q4_0 nibbles are widened to signed int8 while being staged (kernels.rs:458-462), to 16 (nibble - 8): three operations per
+//     eight of them (nine for nibble - 8); the block scale takes the sixteenth, which is exact.  2048 x 15360 x 3840 319 -> 306 us;
 //   * per block and output: acc += dx * (dw * I).  The MFMA accumulates onto the constant
 //     0x4B400000 so its i32 result, read as a float, is 12582912 + I exactly; one FMA with the
 //     exactly representable -dw*12582912 (dw is an f16 value) gives fl(dw*I) with no int->float
@@ -94,7 +95,7 @@ __global__ __launch_bounds__(64 * NW, 2) void gemm_i8_kernel(GemmArgs p) {
     // contiguous bytes), threads 128..255 the four fp32 scales of token tid - 128 (16 contiguous bytes): one load per thread.
     const bool role_w = wave < 2, role_x = !role_w;   // scalar: waves 0, 1 carry the weights' scales, 2, 3 the activations'
     const int role_r = tid & 127;
-    const bool w_valid = row0 + role_r < N_end, x_valid = tok0 + role_r < M_end;
+    const bool x_valid = tok0 + role_r < M_end;
     const unsigned scw_base = (unsigned)min(row0 + role_r, N_end - 1) * (unsigned)p.nb;   // below 2^26
     unsigned scx_base;
     {
@@ -144,26 +145,32 @@ __global__ __launch_bounds__(64 * NW, 2) void gemm_i8_kernel(GemmArgs p) {
                 const int r = (ps * NW + wave) * 16 + q_rowlo;
                 const int off = (r >> 3) * GRP + (r & 7) * 128;  // + slot * 16
                 const uint4 q = rb[ps];
-                uint4 lo, hi;
-                lo.x = sub8(q.x & 0x0f0f0f0fu); hi.x = sub8((q.x >> 4) & 0x0f0f0f0fu);
-                lo.y = sub8(q.y & 0x0f0f0f0fu); hi.y = sub8((q.y >> 4) & 0x0f0f0f0fu);
-                lo.z = sub8(q.z & 0x0f0f0f0fu); hi.z = sub8((q.z >> 4) & 0x0f0f0f0fu);
-                lo.w = sub8(q.w & 0x0f0f0f0fu); hi.w = sub8((q.w >> 4) & 0x0f0f0f0fu);
+                const uint4 lo = make_uint4(nib16(q.x << 4), nib16(q.y << 4), nib16(q.z << 4), nib16(q.w << 4));
+                const uint4 hi = make_uint4(nib16(q.x), nib16(q.y), nib16(q.z), nib16(q.w));
                 *(uint4*)(sB + off + ((2 * q_bi + r) & 7) * 16) = lo;      // elements 0..15 of the block
                 *(uint4*)(sB + off + ((2 * q_bi + 1 + r) & 7) * 16) = hi;  // elements 16..31
             }
         }
+        const int live = p.nb - blk0;   // blocks of the stage that lie within K (scalar); the scales of the others are zero
         if (role_w) {   // the four block scales of a row side by side: one 16-byte write here, one 16-byte read per row tile and stage
             const unsigned h[4] = {rsv.x & 0xffffu, rsv.x >> 16, rsv.y & 0xffffu, rsv.y >> 16};
-            float v[KB];
+            float v[KB];   // (a row past the tile's end has its last one's; nothing of it is stored)
 #pragma unroll
-            for (int j = 0; j < KB; j++) v[j] = (w_valid && blk0 + j < p.nb) ? h2f_((uint16_t)h[j]) : 0.f;
+            for (int j = 0; j < KB; j++) v[j] = h2f_((uint16_t)h[j]) * (Q4 ? 0.0625f : 1.f);   // nib16: sixteen times the quants
+            if (live < KB) {
+#pragma unroll
+                for (int j = 1; j < KB; j++) v[j] = j < live ? v[j] : 0.f;
+            }
             *(float4*)(sdw + role_r * 4) = make_float4(v[0], v[1], v[2], v[3]);
         }
         if (role_x) {
-            const unsigned v[4] = {rsv.x, rsv.y, rsv.z, rsv.w};
+            float v[KB] = {__uint_as_float(rsv.x), __uint_as_float(rsv.y), __uint_as_float(rsv.z), __uint_as_float(rsv.w)};
+            if (live < KB) {
 #pragma unroll
-            for (int j = 0; j < KB; j++) sdx[j * BM + role_r] = (x_valid && blk0 + j < p.nb) ? __uint_as_float(v[j]) : 0.f;
+                for (int j = 1; j < KB; j++) v[j] = j < live ? v[j] : 0.f;
+            }
+#pragma unroll
+            for (int j = 0; j < KB; j++) sdx[j * BM + role_r] = x_valid ? v[j] : 0.f;   // (zeros cost the matrix loop less power than repeated rows)
         }
     };
 
@@ -239,7 +246,7 @@ __global__ __launch_bounds__(64 * NW, 2) void gemm_i8_kernel(GemmArgs p) {
 #pragma unroll
                 for (int i = 0; i < 16; i++) {
                     const int tok = tok0 + tw * 32 + (i >> 2) * 8 + half * 4 + (i & 3);
-                    if (tok < M_end && row < N_end && blk < p.nb) p.dump[((size_t)tok * p.N + row) * p.nb + blk] = dn[i] - MAGIC_I;
+                    if (tok < M_end && row < N_end && blk < p.nb) p.dump[((size_t)tok * p.N + row) * p.nb + blk] = (dn[i] - MAGIC_I) / (Q4 ? 16 : 1);
                 }
             }
             if (!LAST && bi == 3) read_scales(nt, nbuf);

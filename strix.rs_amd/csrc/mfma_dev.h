@@ -16,8 +16,8 @@ constexpr float MAGIC_F = 12582912.f;  // 1.5 * 2^23
 constexpr int MAGIC_I = 0x4B400000;
 
 __device__ __forceinline__ float h2f_(uint16_t h) { return __half2float(__ushort_as_half(h)); }
-// four nibbles (one per byte) -> four signed bytes nibble - 8 (kernels.rs:458-462)
-__device__ __forceinline__ unsigned sub8(unsigned x) { return ((x | 0x80808080u) - 0x08080808u) ^ 0x80808080u; }
+// the high nibbles of four bytes -> four signed bytes 16 (nibble - 8): with its top bit turned over a nibble is nibble - 8 in two's complement
+__device__ __forceinline__ unsigned nib16(unsigned x) { return (x ^ 0x80808080u) & 0xf0f0f0f0u; }
 
 // 64 lanes x 16 bytes from global memory straight into LDS (no register round trip): lane i's
 // bytes land at LDS byte address lds_base + 16 * i; lds_base is wave-uniform (M0).  Completion is

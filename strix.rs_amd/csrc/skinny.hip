@@ -65,7 +65,9 @@ struct SkinnyArgs {
 };
 
 __device__ __forceinline__ float h2f_s(uint16_t h) { return __half2float(__ushort_as_half(h)); }
-__device__ __forceinline__ unsigned sub8s(unsigned x) { return ((x | 0x80808080u) - 0x08080808u) ^ 0x80808080u; }
+// the high nibbles of four bytes -> four signed bytes 16 (nibble - 8): with its top bit turned over a nibble is nibble - 8 in two's
+// complement; the block scale takes the sixteenth, which is exact (9728 x 2560, 6 rows 8.9 -> 8.7 us, 30 rows 10.9 -> 10.6)
+__device__ __forceinline__ unsigned nib16_s(unsigned x) { return (x ^ 0x80808080u) & 0xf0f0f0f0u; }
 
 #define SMX_SK_FMAC(I)                                                                      \
     asm("v_fmac_f32_dpp %0, %1, %2 row_newbcast:" #I " row_mask:0xf bank_mask:0xf" : "+v"(av[I]) : "v"(dxv), "v"(t[I]))
@@ -261,11 +263,8 @@ __global__ __launch_bounds__(64 * NW) void skinny_kernel(const SkinnyArgs p) {
             for (int j = 0; j < 2; j++) {
                 const int row = j * 16 + (lane >> 2), bi = lane & 3;
                 const uint4 q = *(const uint4*)(raw + j * 1024 + lane * 16);
-                uint4 lo, hi;
-                lo.x = sub8s(q.x & 0x0f0f0f0fu); hi.x = sub8s((q.x >> 4) & 0x0f0f0f0fu);
-                lo.y = sub8s(q.y & 0x0f0f0f0fu); hi.y = sub8s((q.y >> 4) & 0x0f0f0f0fu);
-                lo.z = sub8s(q.z & 0x0f0f0f0fu); hi.z = sub8s((q.z >> 4) & 0x0f0f0f0fu);
-                lo.w = sub8s(q.w & 0x0f0f0f0fu); hi.w = sub8s((q.w >> 4) & 0x0f0f0f0fu);
+                const uint4 lo = make_uint4(nib16_s(q.x << 4), nib16_s(q.y << 4), nib16_s(q.z << 4), nib16_s(q.w << 4));
+                const uint4 hi = make_uint4(nib16_s(q.x), nib16_s(q.y), nib16_s(q.z), nib16_s(q.w));
                 *(uint4*)(wide + row * 128 + ((2 * bi + row) & 7) * 16) = lo;       // elements 0..15 of the block
                 *(uint4*)(wide + row * 128 + ((2 * bi + 1 + row) & 7) * 16) = hi;   // elements 16..31
             }
@@ -324,14 +323,14 @@ __global__ __launch_bounds__(64 * NW) void skinny_kernel(const SkinnyArgs p) {
                 const v4i afrag = ALDS ? *(const v4i*)(mine_a + ((bi * 2 + half) * p.tslots + min(col, p.tslots - 1)) * 16)
                                        : (bi == 0 ? r.a0 : (bi == 1 ? r.a1 : (bi == 2 ? r.a2 : r.a3)));
                 const v16i d = __builtin_amdgcn_mfma_i32_32x32x32_i8(afrag, bfrag, cmagic, 0, 0, 0);
-                const float dw = live ? h2f_s((uint16_t)dwh[bi]) : 0.f;
+                const float dw = live ? h2f_s((uint16_t)dwh[bi]) * (Q4 ? 0.0625f : 1.f) : 0.f;
                 rescale(acc, d, dw, dxv);
                 if (DUMP) {
                     const int row = r0 + col;
 #pragma unroll
                     for (int i = 0; i < NACC; i++) {
                         const int tok = (i >> 2) * 8 + half * 4 + (i & 3);
-                        if (live && tok < p.m && row <= r_last) p.dump[((size_t)tok * p.N + row) * p.nb + blk0 + bi] = d[i] - kMagicI;
+                        if (live && tok < p.m && row <= r_last) p.dump[((size_t)tok * p.N + row) * p.nb + blk0 + bi] = (d[i] - kMagicI) / (Q4 ? 16 : 1);
                     }
                 }
                 if constexpr (TT == 2) {   // the second token tile on the same weight fragment
@@ -344,7 +343,7 @@ __global__ __launch_bounds__(64 * NW) void skinny_kernel(const SkinnyArgs p) {
 #pragma unroll
                         for (int i = 0; i < 16; i++) {
                             const int tok = 32 + (i >> 2) * 8 + half * 4 + (i & 3);
-                            if (live && tok < p.m && row <= r_last) p.dump[((size_t)tok * p.N + row) * p.nb + blk0 + bi] = d1[i] - kMagicI;
+                            if (live && tok < p.m && row <= r_last) p.dump[((size_t)tok * p.N + row) * p.nb + blk0 + bi] = (d1[i] - kMagicI) / (Q4 ? 16 : 1);
                         }
                     }
                 }
