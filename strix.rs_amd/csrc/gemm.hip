@@ -5,7 +5,8 @@
 //   * v_mfma_i32_32x32x32_i8: K = 32 is exactly one quant block, so each MFMA yields the exact
 //     i32 block dots of a 32-token x 32-row tile (tokens on the A side, weight rows on the B side:
 //     a lane then owns one weight row and 16 tokens, and stores are 128-byte row segments);
-//   * workgroup tile 128 tokens x 128 rows, 4 waves, each wave 32 tokens x 128 rows;
+//   * workgroup tile 128 tokens x 128 rows, 4 waves, two workgroups per CU; or (NW = 8) 256 tokens, 8 waves, one per CU; each
+//     wave 32 tokens x 128 rows;
 //   * K advances 4 blocks (128 bytes per row, one full cache line) per stage, double-buffered
 //     through LDS in MFMA-fragment order so every fragment read is one conflict-free 128-bit load;
 //   * Q4_0 nibbles are widened to signed int8 while being staged (kernels.rs:458-462), to 16 (nibble - 8): three operations per
@@ -31,7 +32,7 @@
 
 namespace smx {
 
-constexpr int STAGE_BYTES = A_BYTES + B_BYTES + KB * 128 * 4 + KB * BM * 4;
+constexpr int stage_bytes(int nw) { return 4 * nw * GRP + B_BYTES + KB * 128 * 4 + KB * 32 * nw * 4; }
 
 // Operand fragments on their way from LDS to the matrix cores.  The weight fragments of several row tiles are not
 // double-buffered: a row tile's registers are refilled for the next block as soon as its MFMA has been issued (a single row
@@ -43,9 +44,10 @@ struct GemmFrag {
     float4 dw[4];     // weight scales of this lane's row in each row tile, the four blocks of the stage
 };
 
-template <bool Q4, bool DUMP>
+template <bool Q4, bool DUMP, int NW>
 __global__ __launch_bounds__(64 * NW, 2) void gemm_i8_kernel(GemmArgs p) {
     SMX_GEMM_T0;
+    constexpr int BM = 32 * NW, A_BYTES = 4 * NW * GRP, STAGE_BYTES = stage_bytes(NW);
     constexpr int BG = 16 / NW;  // 8-row groups of B each wave stages
     extern __shared__ __align__(16) char smem[];
     const int tid = threadIdx.x, lane = tid & 63;
@@ -54,7 +56,7 @@ __global__ __launch_bounds__(64 * NW, 2) void gemm_i8_kernel(GemmArgs p) {
     const unsigned smem_base = lds_addr(smem);
 
     const TileAt at = gemm_tile_at(p);
-    const WaveRole role = gemm_wave_role(at, wave);
+    const WaveRole role = gemm_wave_role(at, wave, NW);
     const int tok0 = at.tok0, row0 = at.row0, M_end = at.M_end, N_end = at.N_end;
     const int live_tok = role.live_tok, live_rows = role.live_rows, tw = role.tw, nt_cnt = role.nt_cnt, nt_base = role.nt_base;
     const GemmOperand op = p.op[at.op_i];
@@ -93,8 +95,8 @@ __global__ __launch_bounds__(64 * NW, 2) void gemm_i8_kernel(GemmArgs p) {
     }
     // scales of a stage (4 blocks): threads 0..127 carry the four f16 scales of weight row tid (8
     // contiguous bytes), threads 128..255 the four fp32 scales of token tid - 128 (16 contiguous bytes): one load per thread.
-    const bool role_w = wave < 2, role_x = !role_w;   // scalar: waves 0, 1 carry the weights' scales, 2, 3 the activations'
-    const int role_r = tid & 127;
+    const bool role_w = wave < 2, role_x = NW == 4 ? !role_w : wave >= NW / 2;   // scalar: waves 0, 1 carry the weights' scales, the second half the activations'
+    const int role_r = NW > 4 && role_w ? tid : tid & (BM - 1);
     const bool x_valid = tok0 + role_r < M_end;
     const unsigned scw_base = (unsigned)min(row0 + role_r, N_end - 1) * (unsigned)p.nb;   // below 2^26
     unsigned scx_base;
@@ -291,9 +293,14 @@ __global__ __launch_bounds__(64 * NW, 2) void gemm_i8_kernel(GemmArgs p) {
         for (int s = s_begin; s < s_end; s++) {
             const int buf = (s - s_begin) & 1;
             if constexpr (NT > 0) {
+                // eight waves that meet once a stage: of a SIMD's two the one that is behind goes first (see gemm_q6_kernel)
+                if constexpr (NW == 8) __builtin_amdgcn_s_setprio(3);
                 compute(ntc, I0(), F(), s, buf);
+                if constexpr (NW == 8) __builtin_amdgcn_s_setprio(2);
                 compute(ntc, I1(), F(), s, buf);
+                if constexpr (NW == 8) __builtin_amdgcn_s_setprio(1);
                 compute(ntc, I2(), F(), s, buf);
+                if constexpr (NW == 8) __builtin_amdgcn_s_setprio(0);
             }
             if (s + 1 == s_end) break;
             finish_stage(buf ^ 1, s + 1);
@@ -362,7 +369,7 @@ __global__ __launch_bounds__(64 * NW, 2) void gemm_i8_kernel(GemmArgs p) {
             buf = buf == 2 ? 0 : buf + 1;
         }
     };
-    if constexpr (!Q4 && !DUMP) {
+    if constexpr (!Q4 && !DUMP && NW == 4) {
         if (live_tok <= 32 && (p.nb & (KB - 1)) == 0) {   // workgroup-uniform
             sparse_loop();
             gemm_store(p, op, at, role, acc, lane);
@@ -401,28 +408,32 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float4* __rest
 }
 
 // Tile height and K slices.  The reference splits only the long-K shapes (in_dim >= 12288, decode.rs:5658) to fill its grid.  Here the
-// launch that is estimated to take least, among tiles of 64 (Q8_0, Q4_0) and 128 tokens and every number of whole-stage slices
+// launch that is estimated to take least, among tiles of 64 (Q8_0, Q4_0), 128 and 256 tokens and every number of whole-stage slices
 // whose workgroups fit the chip's slots in ONE round (a second, partly filled round costs more than shorter slices save): a
 // workgroup's stages one after the other, at the time a stage takes with the CU to itself or shared with a second
-// workgroup, plus the launch that adds up the slices' partials, 3.5 us and 5 MB of them per us.  Tiles that need several rounds: one slice, 128
-// tokens or (Q6_K) 256, whichever's rounds take less.
-// The stage times are measured (us): 64 tokens 1.05 alone / 1.46 shared, 128 tokens 1.55 / 2.7, Q6_K 2.75 / 4.3, its 256-token tiles (one
-// workgroup per CU) 3.9.  Per call against a
-// rule of at least 6 stages per slice and 128-token tiles: Q8_0 200 x 2560 x 2560 23.5 -> 19 us, 300 x 9728 x 2560 41.2 -> 36.8,
+// workgroup, plus the launch that adds up the slices' partials, 3.5 us and 5 MB of them per us.  Tiles that need several rounds: one
+// slice, 128 or 256 tokens, whichever's rounds take less.
+// The stage times are measured (us): 64 tokens 1.05 alone / 1.46 shared, 128 tokens 1.55 / 2.7, Q6_K 2.75 / 4.3; 256 tokens (one workgroup
+// per CU) 2.35, Q6_K 3.85.  Over 200 shapes of 129..2048 tokens the choice takes 0.6 % more than the best of the three
+// heights, 11 % at worst.  Per call against a rule of at least 6 stages per slice and 128-token tiles: Q8_0 200 x 2560 x 2560 23.5 -> 19 us, 300 x 9728 x 2560 41.2 -> 36.8,
 // 333 x 2560 x 9728 43.8 -> 41.2 (Q4_0 44.5 -> 42.9), Q4_0 103 x 1088 x 1024 15.5 -> 12.0, Q6_K 72 x 2208 x 3328 28.9 -> 21.2, 600 x 2560 x
 // 2560 44.0 -> 37.5; Q8_0 500 and 1000 x 2560 x 9728 keep 128-token tiles (64: 52.8 for 52.1, 109 for 87.4).
 struct Tiling { int bm, slices; };
-static Tiling pick_tiling(int num_cu, bool q6, int M, int N, int nstages, bool split, bool dump) {
-    Tiling best = {128, 1};
+static Tiling pick_tiling(int num_cu, bool q6, int M, int N, int nstages, bool split, int only) {
+    Tiling best = {only ? only : 128, 1};
     double least = 1e30;
     for (int bm : {64, 128, 256}) {
-        if (bm == 64 ? q6 || M <= 64 : bm == 128 ? !q6 && M > 64 && M <= 128 : !q6 || M <= 128 || dump) continue;   // (65..128 tokens: as two rows of tiles)
+        if (only ? bm != only : bm == 64 ? q6 || M <= 64 : bm == 128 ? !q6 && M > 64 && M <= 128 : M <= 128) continue;   // (65..128 tokens: as two rows of tiles)
         const int T = (M + bm - 1) / bm * ((N + BN - 1) / BN), slots = bm == 256 ? num_cu : 2 * num_cu;
         const bool low = bm == 64 || M <= 64;
-        const double alone = bm == 256 ? 3.9 : q6 ? 2.75 : low ? 1.05 : 1.55, shared = bm == 256 ? 3.9 : q6 ? 4.3 : low ? 1.46 : 2.7;
+        const double alone = bm == 256 ? (q6 ? 3.85 : 2.35) : q6 ? 2.75 : low ? 1.05 : 1.55;
+        const double shared = bm == 256 ? alone : q6 ? 4.3 : low ? 1.46 : 2.7;
+        // a stage of `n` workgroups side by side
+        const auto stage = [&](int n) {
+            return n == 0 ? 0.0 : n <= num_cu ? alone : std::max(alone, shared * (0.93 + 0.07 * (n - num_cu) / num_cu));
+        };
         if (T > slots) {   // whole rounds and the rest
-            const int rest = T % slots;
-            const double us = nstages * (T / slots * shared + (rest > num_cu ? shared : rest > 0 ? alone : 0.0));
+            const double us = nstages * (T / slots * shared + stage(T % slots));
             if (bm >= 128 && us < least) {
                 least = us;
                 best = {bm, 1};
@@ -433,7 +444,7 @@ static Tiling pick_tiling(int num_cu, bool q6, int M, int N, int nstages, bool s
         for (int z = 1; z <= zmax; z++) {
             const int stages = (nstages + z - 1) / z;
             if (z > 1 && stages == (nstages + z - 2) / (z - 1)) continue;   // the same slices as with one fewer
-            const double us = stages * (T * z > num_cu ? shared : alone) + (z > 1 ? 3.5 + (double)z * M * N * 4 / 5e6 : 0.0);
+            const double us = stages * stage(T * z) + (z > 1 ? 3.5 + (double)z * M * N * 4 / 5e6 : 0.0);
             if (us < least) {
                 least = us;
                 best = {bm, z};
@@ -454,8 +465,9 @@ static int launch_gemm_variant(smx_ctx* c, Kernel k, size_t lds, const GemmArgs&
 static int launch_gemm_type(smx_ctx* c, QType type, bool dump, const GemmArgs& p, dim3 grid) {
     if (type == kQ6_K && p.tile_m == 256) return launch_gemm_variant(c, gemm_q6_kernel<false, 8>, q6_lds_bytes(8), p, grid, 8);
     if (type == kQ6_K) return launch_gemm_variant(c, dump ? gemm_q6_kernel<true, NW> : gemm_q6_kernel<false, NW>, q6_lds_bytes(NW), p, grid);
-    if (type == kQ4_0) return launch_gemm_variant(c, dump ? gemm_i8_kernel<true, true> : gemm_i8_kernel<true, false>, 2 * STAGE_BYTES, p, grid);
-    return launch_gemm_variant(c, dump ? gemm_i8_kernel<false, true> : gemm_i8_kernel<false, false>, 2 * STAGE_BYTES, p, grid);
+    if (p.tile_m == 256) return launch_gemm_variant(c, type == kQ4_0 ? gemm_i8_kernel<true, false, 8> : gemm_i8_kernel<false, false, 8>, 2 * stage_bytes(8), p, grid, 8);
+    if (type == kQ4_0) return launch_gemm_variant(c, dump ? gemm_i8_kernel<true, true, NW> : gemm_i8_kernel<true, false, NW>, 2 * stage_bytes(NW), p, grid);
+    return launch_gemm_variant(c, dump ? gemm_i8_kernel<false, true, NW> : gemm_i8_kernel<false, false, NW>, 2 * stage_bytes(NW), p, grid);
 }
 
 GemmOperand gemm_operand(const Weight& w, float* out) {
@@ -484,20 +496,24 @@ int launch_gemm(smx_ctx* c, const Weight& w, const int8_t* xq, const float* xd, 
     p.N = (int)w.N;
     p.ldo = (int)w.N;
     p.nb = (int)(w.K / 32);
-    // 128 x 128 tiles, two 4-wave workgroups per CU (Q6_K from 129 tokens on also 256 x 128, gemm_q6.h).  Measured alternatives for
-    // Q8_0 and Q4_0, all slower on every shape tried (M 512..4096 of both FFN shapes, grouped MoE tiles): 256 x 128 tiles with one 8-wave workgroup per CU
-    // (-7 %); three workgroups per CU with 2-block stages, every operand and scale staged LDS-direct and the
-    // LDS reads software-pipelined (-5..-10 %: the third wave per SIMD raises the instruction issue rate,
-    // and the clock the chip sustains drops by as much).
+    // 128 x 128 tiles, two 4-wave workgroups per CU, or 256 x 128, one 8-wave workgroup per CU.  Loading, widening and scaling weights
+    // is what the larger tile does half as often (loads alone cost the Q8_0 kernel 13 % of its time, the scales 5 %, Q4_0's nibbles
+    // 4 %); all eight waves meeting at the barriers costs some of it back.  Without the priorities of the main loop the larger
+    // tile loses (-7 %).  Per call, 128 -> 256 tokens: 2048 x 15360 x 3840 Q8_0 316 -> 308 us, Q4_0 323 -> 306; 2048 x 3840 x 15360 328 -> 310,
+    // 334 -> 304; Q8_0 512 x 15360 x 3840 84.8 -> 79.4, Q4_0 512 x 9728 x 2560 58.1 -> 50.6; but Q8_0 1000 x 9728 x 2560 (304 tiles for
+    // 256 CUs) 88 -> 101.  Measured and slower on every shape tried (M 512..4096 of both FFN shapes, grouped MoE tiles): three
+    // workgroups per CU with 2-block stages, every operand and scale staged LDS-direct and the LDS reads software-pipelined
+    // (-5..-10 %: the third wave per SIMD raises the instruction issue rate, and the clock the chip sustains drops by as much).
     p.tiles_n = (p.N + BN - 1) / BN;
     const int nstages = (p.nb + KB - 1) / KB;
     const bool may_split = dump == nullptr && (m * w.N) % 4 == 0;
-    const Tiling tiling = pick_tiling(c->num_cu, w.type == kQ6_K, p.M, p.N, nstages, may_split && c->tune_gemm_splitk == 0, dump != nullptr);
+    // (the kernels that write the block dots out have four waves)
+    const int only = c->tune_gemm_tile_m == 256 && dump ? 128 : c->tune_gemm_tile_m != 0 ? c->tune_gemm_tile_m : dump && p.M > 128 ? 128 : 0;
+    const Tiling tiling = pick_tiling(c->num_cu, w.type == kQ6_K, p.M, p.N, nstages, may_split && c->tune_gemm_splitk == 0, only);
     // 65..128 tokens are always two rows of 64-token tiles (in one row of 128 half the waves of a workgroup may idle): Q8_0
     // 2560 x 9728 and 9728 x 2560 at 96 / 128 tokens 28.2 / 29.4 -> 25.4 / 26.7 us and 25.9 / 27.3 -> 22.9 / 24.7 us.
     int bm = tiling.bm;
-    if (p.M > 64 && p.M <= 128 && w.type != kQ6_K) bm = 64;   // (also when they need several rounds)
-    if (c->tune_gemm_tile_m != 0) bm = c->tune_gemm_tile_m == 256 && (w.type != kQ6_K || dump) ? 128 : c->tune_gemm_tile_m;
+    if (p.M > 64 && p.M <= 128 && w.type != kQ6_K && only == 0) bm = 64;   // (also when they need several rounds)
     const int slots = c->num_cu * (bm == 256 ? 1 : 2);   // workgroups the chip holds
     p.tile_m = bm;
     p.tiles_m = (p.M + bm - 1) / bm;

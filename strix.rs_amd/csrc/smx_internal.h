@@ -243,7 +243,7 @@ struct GemmArgs {
     int* dump;              // optional [M][N][nb] (Q6_K: [M][N][2 * nb], one per 16-element sub-block)
     int M, N, nb, ldo;
     int tiles_m, tiles_n;
-    int tile_m;             // dense tiling: tokens per tile, 128, 64 or (Q6_K) 256 (a 64-token tile's waves pair up on two row tiles each)
+    int tile_m;             // dense tiling: tokens per tile, 256, 128 or 64 (a 64-token tile's waves pair up on two row tiles each)
     int stages_per_slice;   // stages (of 4 blocks) each grid.z slice covers
     int xcd_remap;
     int walk_gm;            // dense tiling: token tiles per group of the tile walk (see launch_gemm)

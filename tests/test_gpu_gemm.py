@@ -232,14 +232,17 @@ def test_gemm_tile_heights_agree(accel, orc, synth, relerr, ty, m, N, K):
     accel.evict("t.th")
 
 
+@pytest.mark.parametrize("ty", [14, 8, 2])
 @pytest.mark.parametrize("m,N,K", [(129, 130, 256), (257, 300, 768), (290, 96, 2560), (511, 1000, 512), (640, 15000, 256), (1000, 416, 4096)])
-def test_gemm_q6_k_wide_tiles(accel, orc, synth, relerr, m, N, K):
-    """256-token tiles of a Q6_K weight: last tiles of 1, 34, 128 and all but one tokens, strips that end inside a row tile, one
+def test_gemm_wide_tiles(accel, orc, synth, relerr, ty, m, N, K):
+    """256-token tiles: last tiles of 1, 34, 128 and all but one tokens, strips that end inside a row tile, one
     stage pair and many, several rounds of workgroups, K slices.  Unsplit they give the bits of 128-token tiles."""
-    raw = synth.make_weight(14, N, K, seed=N)
+    if ty != 14:
+        K += 32 * (m % 4)   # rows that are no whole number of stages
+    raw = synth.make_weight(ty, N, K, seed=N)
     xs = synth.make_acts(m, K, seed=m)
-    assert accel.upload_q6_k("t.wide", raw, K, N)
-    ref = orc.matmul_q8_from_f32(14, raw, K, N, xs)
+    assert getattr(accel, UPLOAD[ty])("t.wide", raw, K, N)
+    ref = orc.matmul_q8_from_f32(ty, raw, K, N, xs)
     try:
         for splitk in (1, 0, 3):
             accel.tune("gemm_splitk", splitk)
