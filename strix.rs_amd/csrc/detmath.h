@@ -49,6 +49,20 @@ __device__ __forceinline__ float det_gelu_tanh(float x) {
     return 0.5f * x * (1.0f + det_tanhf(inner));
 }
 
+// (the threads' sums of squares -> the scale; see rms_scale)
+__device__ __forceinline__ float rms_scale_of(char* scratch, double ss, int n, float eps) {
+#pragma clang fp contract(off)
+    for (int off = 32; off > 0; off >>= 1) ss += __shfl_xor(ss, off);
+    double* red = (double*)scratch;
+    const int nwaves = blockDim.x >> 6;
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ss;
+    __syncthreads();
+    double tot = 0.0;
+    for (int w = 0; w < nwaves; w++) tot += red[w];
+    __syncthreads();  // the caller overwrites the scratch next
+    return (float)(1.0 / sqrt(tot / (double)n + (double)eps));
+}
+
 // 1/sqrt(mean(x^2) + eps) of one row for the rmsnorm producer (kernels.rs:101-113).  The squares are
 // summed in double by the whole workgroup (per thread, per wave, then over the waves in index order)
 // and the scale is rounded to fp32 once, so it does not depend on the workgroup's shape.  `scratch`
@@ -63,15 +77,21 @@ __device__ __forceinline__ float rms_scale(char* scratch, const float* x, int n,
         ss += (double)v.z * (double)v.z;
         ss += (double)v.w * (double)v.w;
     }
-    for (int off = 32; off > 0; off >>= 1) ss += __shfl_xor(ss, off);
-    double* red = (double*)scratch;
-    const int nwaves = blockDim.x >> 6;
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ss;
-    __syncthreads();
-    double tot = 0.0;
-    for (int w = 0; w < nwaves; w++) tot += red[w];
-    __syncthreads();  // the caller overwrites the scratch next
-    return (float)(1.0 / sqrt(tot / (double)n + (double)eps));
+    return rms_scale_of(scratch, ss, n, eps);
+}
+// The same for a row that the workgroup holds: thread t's items t, t + blockDim.x, ... (zeros past the row).
+template <int IT>
+__device__ __forceinline__ float rms_scale_held(char* scratch, const float4 (&v)[IT], int n, float eps) {
+#pragma clang fp contract(off)
+    double ss = 0.0;
+#pragma unroll
+    for (int j = 0; j < IT; j++) {
+        ss += (double)v[j].x * (double)v[j].x;
+        ss += (double)v[j].y * (double)v[j].y;
+        ss += (double)v[j].z * (double)v[j].z;
+        ss += (double)v[j].w * (double)v[j].w;
+    }
+    return rms_scale_of(scratch, ss, n, eps);
 }
 
 }  // namespace smx
