@@ -8,8 +8,8 @@
 //   * v_dot4_i32_i8 integer block dots, exact i32 per block, then acc += (dw*dx)*float(isum);
 //   * cross-lane (DPP) combination of lanes that share a block and of the lanes of a row.
 // Two forms (gemv_body.h): the flat form (activation requested before the weights, a workgroup's rows
-// walked as one sequence of 64-unit loads, no conditional loads) for every shape whose rows are a whole
-// number of unit groups, and the persistent row-per-wave form for the rest.
+// walked as one sequence of 64-unit loads, no conditional loads) for rows of up to 16384 elements, and the
+// persistent row-per-wave form for longer ones.
 // HBM-bound: algorithmic bytes per row are K/32 * {18, 34} (Q4_0, Q8_0) or K/256 * 210 (Q6_K).
 #include <algorithm>
 #include <cstddef>
@@ -178,7 +178,7 @@ struct Geom {
     bool prod = false;  // an activation producer runs in the staging
     bool preq = false;  // the (single) activation row arrives quantised
     bool rowsf = false; // 2..4 fp32 activation rows are quantised inside the flat kernel
-    int flat = 0;       // flat form: lanes per group (16 or 8), 0 = not used
+    int flat = 0;       // flat form: lanes per group (16, 8 or kFlatLeast), 0 = not used
     int flat_pre = 0;   // its loads per round
     int rpw, pre, ks, lpr, nt;
     unsigned grid;
@@ -247,6 +247,10 @@ int launch_flat_fq(smx_ctx* c, const Geom& g, const GemvJobs& J, int njobs, int 
     return fail(c, SMX_ERR_ARG, "gemv: several activation rows take one job per launch");
 }
 
+// Lanes per group of the flat form where a row's units are no multiple of 8: what any row of the format is a whole number of.
+template <class Ops>
+constexpr int kFlatLeast = std::is_same<Ops, OpsQ6_K>::value ? 4 : (std::is_same<Ops, OpsQ8_0>::value ? 2 : 1);
+
 template <class Ops, int MT>
 int launch_flat(smx_ctx* c, const Geom& g, const GemvJobs& J, int njobs, int nblk, int m, int* dump = nullptr,
                 int dump_per_row = 0) {
@@ -260,7 +264,7 @@ int launch_flat(smx_ctx* c, const Geom& g, const GemvJobs& J, int njobs, int nbl
         return launch_flat_fq<Ops, 1, PRE, GL, 1>(c, g, J, njobs, nblk, m);                          \
     }
         if constexpr (std::is_same<Ops, OpsQ4_0>::value || std::is_same<Ops, OpsQ8_0>::value) {
-            SMX_FLAT(3, 16) SMX_FLAT(3, 8) SMX_FLAT(2, 16) SMX_FLAT(4, 16)
+            SMX_FLAT(3, 16) SMX_FLAT(3, 8) SMX_FLAT(2, 16) SMX_FLAT(4, 16) SMX_FLAT(3, kFlatLeast<Ops>)
         } else if constexpr (kQ6) {
             SMX_FLAT(1, 16) SMX_FLAT(1, 8) SMX_FLAT(1, 4)
         }
@@ -278,6 +282,9 @@ int launch_flat(smx_ctx* c, const Geom& g, const GemvJobs& J, int njobs, int nbl
                 if (g.rowsf) {   // fp32 rows, quantised by the kernel
                     if (g.flat == 16) return launch_flat_fq<Ops, MT, PRE, 16, 1>(c, g, J, njobs, nblk, m);
                     if (g.flat == 8) return launch_flat_fq<Ops, MT, PRE, 8, 1>(c, g, J, njobs, nblk, m);
+                    if constexpr (!kQ6) {
+                        if (g.flat == kFlatLeast<Ops>) return launch_flat_fq<Ops, MT, PRE, kFlatLeast<Ops>, 1>(c, g, J, njobs, nblk, m);
+                    }
                     if constexpr (kQ6) {
                         if (g.flat == 4) return launch_flat_fq<Ops, MT, PRE, 4, 1>(c, g, J, njobs, nblk, m);
                     }
@@ -285,6 +292,9 @@ int launch_flat(smx_ctx* c, const Geom& g, const GemvJobs& J, int njobs, int nbl
             }
             if (g.flat == 16) return launch_flat_fq<Ops, MT, PRE, 16, 0>(c, g, J, njobs, nblk, m);
             if (g.flat == 8) return launch_flat_fq<Ops, MT, PRE, 8, 0>(c, g, J, njobs, nblk, m);
+            if constexpr (!kQ6 && MT <= 4) {
+                if (g.flat == kFlatLeast<Ops>) return launch_flat_fq<Ops, MT, PRE, kFlatLeast<Ops>, 0>(c, g, J, njobs, nblk, m);
+            }
             if constexpr (kQ6) {
                 if (g.flat == 4) return launch_flat_fq<Ops, MT, PRE, 4, 0>(c, g, J, njobs, nblk, m);
             }
@@ -370,15 +380,7 @@ static Geom pick_geom(const smx_ctx* c, QType type, size_t N, size_t nblk, int m
     g.ks = 1;
     const size_t cus = std::max<size_t>(1, (size_t)c->num_cu / njobs);  // this job's share of the chip
     const size_t waves = cus * 16;
-    // lanes per row: fewest wasted lanes, whole-wave rows on ties (short rows, one activation row only)
-    if (mt == 1 && units < 256) {
-        size_t best = ((units + 63) / 64) * 64;
-        for (int lpr : {32, 16}) {
-            const size_t slots = ((units + lpr - 1) / lpr) * lpr;
-            // measured: with equal waste, rows of fewer than 128 units run best two to a wave
-            if (slots < best || (slots == best && lpr == 32 && units < 128)) { best = slots; g.lpr = lpr; }
-        }
-    }
+    if (mt == 1 && units == 1) g.lpr = 16;   // the only short rows that come here: four to a wave
     if (c->tune_gemv_lpr > 0 && mt == 1) g.lpr = c->tune_gemv_lpr;
     const int P = (int)((units + g.lpr - 1) / g.lpr);
     if (g.lpr == 64) {
@@ -421,15 +423,22 @@ static Geom pick_geom(const smx_ctx* c, QType type, size_t N, size_t nblk, int m
         if (dump) wpc = 8;
         g.grid = (unsigned)std::min<size_t>(wgs, cus * wpc);
     }
-    // Flat form: one activation row of up to 16384 elements and rows of a whole number of unit groups.
+    // Flat form: rows of up to 16384 elements.
     // Measured against the persistent form above: Q4_0 9728 x 2560 6.8 -> 5.4 us, eight of them in one
     // launch 24.8 -> 22.4 us, Q6_K 262144 x 3840 159 -> 144 us.
+    // Rows whose units are no multiple of 8 have groups of 1 lane (Q4_0, and Q8_0 by whole blocks) or 2 (Q8_0): eight to sixteen
+    // times the group sums, and still ahead of the persistent form, whose waves have lanes without a unit in every row's last
+    // pass: one row, Q4_0 9728 x 2592 6.4 -> 4.5 us, 2560 x 9760 8.1 -> 5.0, Q8_0 9728 x 2592 7.9 -> 6.0, 2560 x 9760 8.2 -> 6.4;
+    // three rows, Q4_0 131 x 2208 8.0 -> 3.4, Q8_0 13696 x 800 9.0 -> 4.3; four rows, Q8_0 2560 x 9760 9.9 -> 9.3.  Two things
+    // stay with the persistent form: eight activation rows (their sums of single units would be eight to a lane), and rows of one
+    // unit (the division by the units per row has no 32-bit constant for 1).
     // The block-dot dump of the parity tests runs in whichever form the shape gets.
-    if (!(type == kQ6_K && mt == 8) && (units % (type == kQ6_K ? 4 : 8)) == 0 &&
+    const int least = type == kQ6_K ? 4 : (type == kQ8_0 && units == nblk * 2 ? 2 : 1);   // (kFlatLeast)
+    if (!(type == kQ6_K && mt == 8) && (units % 8 == 0 || type == kQ6_K || (mt <= 4 && units > 1)) &&
         nblk * (type == kQ6_K ? 256 : 32) <= 16384) {  // the row is held in registers while the weights are requested
         // a workgroup's units are indexed with 16 bits and its group sums live in LDS: whole further
         // rounds of workgroups when a CU's share of the rows is too large for either
-        g.flat = (units % 16) == 0 ? 16 : ((units % 8) == 0 ? 8 : 4);
+        g.flat = (units % 16) == 0 ? 16 : ((units % 8) == 0 ? 8 : least);
         const size_t share = (N + cus - 1) / cus * units;   // units of a CU's share of the rows
         size_t rounds = share < 65536 ? 1 : (share + 59999) / 60000;   // margin for the rounding of rows per workgroup
         size_t fwgs, rows, lds;

@@ -20,6 +20,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <type_traits>
 
 #include "../../include/strix_mi355.h"
 #include "detmath.h"
@@ -615,10 +616,10 @@ __device__ __forceinline__ void gemv_body(const GemvW W, const GemvX X, float* _
     SMX_STAMP_FLUSH();
 }
 
-// Sum over groups of GL = 2, 4, 8 or 16 adjacent lanes (all lanes of a group end up with the total).
+// Sum over groups of GL = 1, 2, 4, 8 or 16 adjacent lanes (all lanes of a group end up with the total).
 template <int GL>
 __device__ __forceinline__ float small_group_sum(float v) {
-    v += dpp_f<0xB1>(v);
+    if (GL >= 2) v += dpp_f<0xB1>(v);
     if (GL >= 4) v += dpp_f<0x4E>(v);
     if (GL >= 8) v += dpp_f<0x141>(v);
     if (GL >= 16) v += dpp_f<0x140>(v);
@@ -857,7 +858,8 @@ struct FlatXRowsF {
     }
 };
 
-// Flat form for weight rows that are a whole number of GL-lane groups (GL = 16, 8 or 4 units).  Rows are contiguous in the planar layout, so the units of a workgroup's rows [r0, r1) are
+// Flat form for weight rows that are a whole number of GL-lane groups (GL = 16, 8, 4, 2 or 1 units: any row; with 1 every unit's
+// sum goes to LDS by itself).  Rows are contiguous in the planar layout, so the units of a workgroup's rows [r0, r1) are
 // one flat sequence: a wave load covers 64 consecutive units of it (1 KB of quants, whatever the row
 // length), wave w takes loads w, w + 16, ...  Every GL-lane group lies inside one row; its sum goes
 // to LDS, and after a barrier the groups of a row are added in ascending order.  All waves of a
@@ -982,14 +984,26 @@ __device__ __forceinline__ void gemv_body_flat(const GemvW W, const GemvX X, flo
         }
         return;
     }
-    for (int i8 = threadIdx.x; i8 < (r1 - r0) * MT * 8; i8 += 1024) {   // 1024: the form's workgroup size
-        const int i = i8 >> 3, l = i8 & 7;
-        const int r = i / MT, t = i % MT;
-        float s = 0.f;
-        for (int j = l; j < G; j += 8) s += part[(r * G + j) * MT + t];
-        s = small_group_sum<8>(s);
-        if (l == 0 && t < m) y[(size_t)t * ldy + r0 + r] = s;
-    }
+    // Rows of many sums (GL 1 or 2 and at least 64 of them) take 16 lanes, four of whose reads are in flight at a time: Q4_0
+    // 2560 x 9760 5.8 -> 5.0 us; on rows of fewer sums 8 lanes are ahead (Q8_0 13696 x 800, three tokens 4.4 us against 4.6).
+    auto finish = [&](auto lanes) __attribute__((always_inline)) {
+        constexpr int LP = decltype(lanes)::value;
+        for (int i8 = threadIdx.x; i8 < (r1 - r0) * MT * LP; i8 += 1024) {   // 1024: the form's workgroup size
+            const int i = i8 / LP, l = i8 % LP;
+            const int r = i / MT, t = i % MT;
+            float s = 0.f;
+            if constexpr (LP == 16) {
+#pragma unroll 4
+                for (int j = l; j < G; j += LP) s += part[(r * G + j) * MT + t];
+            } else {
+                for (int j = l; j < G; j += LP) s += part[(r * G + j) * MT + t];
+            }
+            s = small_group_sum<LP>(s);
+            if (l == 0 && t < m) y[(size_t)t * ldy + r0 + r] = s;
+        }
+    };
+    if (GL <= 2 && G >= 64) finish(std::integral_constant<int, 16>());
+    else finish(std::integral_constant<int, 8>());
 }
 
 }  // namespace smx

@@ -5,13 +5,12 @@
 // fp32 activation staged in LDS.  The decode path proper is the Q8-activation GEMV (gemv.hip); this
 // form serves callers that hold the accelerator to the CPU result at fp32 accuracy.
 //
-// Two kernels.  gemv_f32_flat_kernel (rows of up to 16384 elements that are a whole number of unit groups: every shape
-// of the models) has the memory side of the flat Q8-activation GEMV: the activation row is requested first, a
+// Two kernels.  gemv_f32_flat_kernel (rows of up to 16384 elements) has the memory side of the flat Q8-activation GEMV: the activation row is requested first, a
 // workgroup's rows are one flat sequence of 64-unit loads, three loads per wave in flight, group sums through LDS.
 // A weight element costs two vector operations: one conversion (v_cvt_f32_ubyteN on the unsigned quants of Q4_0 and
 // Q6_K, the sign-extending byte select on Q8_0) and one FMA; the offsets (q - 8, q - 32) are taken out per
 // 16-element half through the sums of the activation that the staging leaves in LDS.
-// gemv_f32_kernel (any other shape up to 32768 elements): a wave serves RPW rows at a time, one load per row and lane
+// gemv_f32_kernel (longer rows, up to 32768 elements, and rows of one unit): a wave serves RPW rows at a time, one load per row and lane
 // in flight, DPP reduction per row.
 // HBM-bound by bytes.
 #include <algorithm>
@@ -278,13 +277,23 @@ __device__ __forceinline__ void f32_flat_body(const GemvW W, const float* __rest
     __syncthreads();
     // a row's G group sums: 8 lanes take them in ascending order, then a fixed DPP tree
     const int G = U / GL;
-    for (int i8 = threadIdx.x; i8 < (r1 - r0) * 8; i8 += 1024) {
-        const int r = i8 >> 3, l = i8 & 7;
-        float s = 0.f;
-        for (int j = l; j < G; j += 8) s += part[r * G + j];
-        s = small_group_sum<8>(s);
-        if (l == 0) y[r0 + r] = s;
-    }
+    auto finish = [&](auto lanes) __attribute__((always_inline)) {   // (16 lanes for rows of many sums, as in gemv_body_flat)
+        constexpr int LP = decltype(lanes)::value;
+        for (int i8 = threadIdx.x; i8 < (r1 - r0) * LP; i8 += 1024) {
+            const int r = i8 / LP, l = i8 % LP;
+            float s = 0.f;
+            if constexpr (LP == 16) {
+#pragma unroll 4
+                for (int j = l; j < G; j += LP) s += part[r * G + j];
+            } else {
+                for (int j = l; j < G; j += LP) s += part[r * G + j];
+            }
+            s = small_group_sum<LP>(s);
+            if (l == 0) y[r0 + r] = s;
+        }
+    };
+    if (GL <= 2 && G >= 64) finish(std::integral_constant<int, 16>());
+    else finish(std::integral_constant<int, 8>());
 }
 
 // Every argument lies in the first 64-byte line of the kernel-argument segment.
@@ -323,15 +332,21 @@ __global__ __launch_bounds__(1024) void gemv_f32_group_kernel(const F32Jobs J) {
     f32_flat_body<Ops, PRE, GL>(jb.W, jb.x, jb.y, J.nblk, jb.N, blockIdx.x - w0, w1 - w0, J.magic_u);
 }
 
+// Lanes per group where a row's units are no multiple of 8: what any row of the format is a whole number of.
+template <class Ops>
+constexpr int kF32Least = std::is_same<Ops, OpsQ6_K>::value ? 4 : (std::is_same<Ops, OpsQ8_0>::value ? 2 : 1);
+
 // The flat form's geometry (as for the Q8-activation GEMV): whole further rounds of workgroups when a CU's share of
-// the rows is too large for the 16-bit unit index or for LDS.  Returns false when the shape is not served.
+// the rows is too large for the 16-bit unit index or for LDS.  Returns false when the shape is not served: longer rows, and rows
+// of one unit (the division by the units per row has no 32-bit constant for 1).
+// Rows whose units are no multiple of 8, against gemv_f32_kernel: Q8_0 4900 x 6880 21.5 -> 19.6 us a host call, a batch of seven
+// with 576-long rows 41 -> 16.2 (one launch for each weight's items instead of one per item).
 struct F32Flat { int gl; unsigned grid, magic; size_t lds; };
 static bool f32_flat_geom(const smx_ctx* c, const Weight& w, F32Flat& g) {
     const size_t upb = w.type == kQ6_K ? 4 : (w.type == kQ8_0 ? 2 : 1);
     const size_t units = w.nblk * upb, nb32 = w.K / 32;
-    if (w.K > 16384 || units == 0) return false;
-    g.gl = units % 16 == 0 ? 16 : (units % 8 == 0 ? 8 : (w.type == kQ6_K && units % 4 == 0 ? 4 : 0));
-    if (!g.gl) return false;
+    if (w.K > 16384 || units < 2) return false;
+    g.gl = units % 16 == 0 ? 16 : (units % 8 == 0 ? 8 : (w.type == kQ6_K ? 4 : (w.type == kQ8_0 ? 2 : 1)));   // (kF32Least)
     const size_t cus = (size_t)c->num_cu, xbytes = nb32 * (36 + 2) * 4;
     const size_t share = (w.N + cus - 1) / cus * units;
     size_t rounds = share < 65536 ? 1 : (share + 59999) / 60000;
@@ -361,9 +376,7 @@ static int launch_f32_flat(smx_ctx* c, const Weight& w, const float* x, float* y
     };
     if (g.gl == 16) return go(gemv_f32_flat_kernel<Ops, PRE, 16>);
     if (g.gl == 8) return go(gemv_f32_flat_kernel<Ops, PRE, 8>);
-    if constexpr (std::is_same<Ops, OpsQ6_K>::value) {
-        if (g.gl == 4) return go(gemv_f32_flat_kernel<Ops, PRE, 4>);
-    }
+    if (g.gl == kF32Least<Ops>) return go(gemv_f32_flat_kernel<Ops, PRE, kF32Least<Ops>>);
     return fail(c, SMX_ERR_ARG, "gemv_f32: no flat variant for %d-unit groups", g.gl);
 }
 
@@ -378,9 +391,7 @@ static int launch_f32_group_type(smx_ctx* c, const F32Jobs& J, int gl, size_t ld
     };
     if (gl == 16) return go(gemv_f32_group_kernel<Ops, PRE, 16>);
     if (gl == 8) return go(gemv_f32_group_kernel<Ops, PRE, 8>);
-    if constexpr (std::is_same<Ops, OpsQ6_K>::value) {
-        if (gl == 4) return go(gemv_f32_group_kernel<Ops, PRE, 4>);
-    }
+    if (gl == kF32Least<Ops>) return go(gemv_f32_group_kernel<Ops, PRE, kF32Least<Ops>>);
     return fail(c, SMX_ERR_ARG, "gemv_f32: no group variant for %d-unit groups", gl);
 }
 

@@ -211,6 +211,37 @@ def test_gemv_rows_long_k_batched(accel, orc, synth, relerr):
     accel.evict("t.long")
 
 
+# rows whose units are no multiple of 8: two blocks (the shortest), odd block counts on both sides of 64 and 128 sums per row, an
+# activation loaded before the weights (257 blocks), the longest such row (511 blocks), several rounds of workgroups, fewer rows
+# than compute units; rows of one unit and longer ones stay with the row-per-wave kernel
+@pytest.mark.parametrize("ty,N,K", [(2, 3001, 64), (2, 700, 32 * 63), (2, 3000, 32 * 65), (8, 300, 32 * 33), (8, 70, 32 * 127), (2, 7, 32 * 257),
+                                    (8, 1500, 32 * 511), (2, 2500, 32 * 511), (8, 3001, 96), (2, 3001, 32), (8, 3001, 32), (2, 300, 32 * 513)])
+def test_gemv_rows_of_any_block_count(accel, orc, synth, relerr, ty, N, K):
+    raw = synth.make_weight(ty, N, K, seed=N + K)
+    _up(accel, ty, "t.any", raw, K, N)
+    xs = synth.make_acts(5, K, seed=K)
+    ref = orc.matmul_q8_from_f32(ty, raw, K, N, xs)
+    xq, _, _ = orc.actquant(xs[:1], K)
+    assert np.array_equal(accel.gemv_block_dots("t.any", xs[0], N, K // 32), orc.block_dots(ty, raw, K, N, xq[0]))
+    assert relerr(accel.gemv("t.any", xs[0], N), ref[0]) <= TOL
+    for m in (2, 3, 4, 5):
+        assert relerr(accel.gemv_rows("t.any", xs[:m], N), ref[:m]) <= TOL, m
+    short = raw[:(N // 3 + 1) * (len(raw) // N)]          # a group whose second job has fewer rows
+    _up(accel, ty, "t.any2", short, K, N // 3 + 1)
+    calls, dims = [("t.any", xs[0]), ("t.any2", xs[1])], [N, N // 3 + 1]
+    for f32 in (False, True):
+        out = accel.gemv_batch(calls, dims, f32=f32)
+        want = (lambda w, n, i: orc.matmul_f32(ty, w, K, n, xs[i:i + 1], order=1)[0]) if f32 else (lambda w, n, i: ref[i][:n])
+        assert relerr(out[0], want(raw, N, 0)) <= 1e-5 and relerr(out[1], want(short, N // 3 + 1, 1)) <= 1e-5
+    if K > 16384:                                          # the launch knobs of the row-per-wave kernel
+        for knob, v in (("gemv_lpr", 16), ("gemv_lpr", 32), ("gemv_rpw", 4), ("gemv_ks", 4)):
+            accel.tune(knob, v)
+            assert relerr(accel.gemv("t.any", xs[0], N), ref[0]) <= TOL, knob
+            accel.tune(knob, 0)
+    accel.evict("t.any")
+    accel.evict("t.any2")
+
+
 def test_gemv_batch_and_declines(accel, orc, synth, relerr, pkg):
     K, N = 256, 64
     raws = [synth.make_weight(ty, N, K, seed=ty) for ty in (2, 8, 14)]
