@@ -266,7 +266,7 @@ void smx_graph_destroy(smx_ctx* ctx, smx_graph* g);
 /* Measurement hook, not part of the operator surface (no counterpart in the reference; a binding has no reason to
  * call it): launch-geometry overrides for sweeps; value 0 restores the built-in choice.  They shape
  * a kernel's launch, never which kernel a shape is served by.
- * Knobs: "gemm_splitk" (K slices of the GEMM), "gemm_tile_m" (tokens per GEMM tile: 64, 128 or 256), "gemm_walk" (token-tile
+ * Knobs: "gemm_splitk" (K slices of the GEMM and of the grouped gate and up products), "gemm_tile_m" (tokens per GEMM tile: 64, 128 or 256), "gemm_walk" (token-tile
  * groups of the GEMM's tile walk), "gemm_narrow" (1: every weight strip of the GEMM 128 rows; 1 + n: the first n strips 96 rows);
  * for rows of more than 16384 elements, which the row-per-wavefront GEMV serves: "gemv_rpw" (rows per wavefront: 1, 2, 4),
  * "gemv_ks" (wavefronts sharing a row: 1, 2, 4), "gemv_lpr" (lanes per row: 16, 32, 64), "gemv_wpc" (workgroups per CU);

@@ -606,16 +606,31 @@ int launch_gemm(smx_ctx* c, const Weight& w, const int8_t* xq, const float* xd, 
     return SMX_OK;
 }
 
+// A grouped launch with fewer workgroups than the chip has slots leaves CUs idle while each workgroup walks its K stages alone:
+// K slices, up to four of at least two stages, as long as all workgroups run in one round.  Over 90 drawn layers (8..64 experts, 512..4096
+// wide, 256..1536 inner, 8..640 tokens, Q8_0 and Q6_K) the call gains 7 % on average and never loses; the best number of slices
+// for each would gain 9 %.  A second round of workgroups (768 allowed) loses up to 3 %, six and eight slices are
+// ahead of four on two shapes and cost scratch and traffic.  Q6_K, 22 stages: 72 workgroups 65 -> 25 us, 112 workgroups and 244 tokens 109 -> 71 us
+// a call; Q8_0, 138 workgroups, 152 tokens 56 -> 45.
+int gemm_grouped_slices(const smx_ctx* c, size_t K, size_t ntiles, int nops) {
+    const size_t stages = (K / 32 + KB - 1) / KB;
+    const size_t wgs = std::max<size_t>(1, ntiles * (size_t)nops);
+    size_t z = std::max<size_t>(1, std::min({size_t(4), stages / 2, 2 * (size_t)c->num_cu / wgs}));
+    if (c->tune_gemm_splitk > 0) z = std::min<size_t>((size_t)c->tune_gemm_splitk, stages);
+    const size_t per_slice = (stages + z - 1) / z;
+    return (int)((stages + per_slice - 1) / per_slice);   // (no empty slices)
+}
+
 // Grouped GEMM over a tile table (MoE prefill): one launch covers every expert; a tile's workgroups serve
 // one of `nops` weight/output pairs each that share the activation rows (gate and up).  The caller has
 // checked the shape (moe_check_shape: the kernels' offsets into the expert tensors are 32 bits wide).
-int launch_gemm_grouped(smx_ctx* c, QType type, const GemmArgs& args, int ntiles, int nops, const char* name) {
+int launch_gemm_grouped(smx_ctx* c, QType type, const GemmArgs& args, int ntiles, int nops, int slices, const char* name) {
     if (ntiles <= 0) return SMX_OK;
     ProfScope ps(c, name);
-    const dim3 grid((unsigned)(ntiles * nops), 1, 1);
-    GemmArgs p = args;   // one K slice: every stage
+    const dim3 grid((unsigned)(ntiles * nops), 1, (unsigned)slices);
+    GemmArgs p = args;
     p.nops = nops;
-    p.stages_per_slice = (p.nb + KB - 1) / KB;
+    p.stages_per_slice = ((p.nb + KB - 1) / KB + slices - 1) / slices;
     if (type == kQ6_K || type == kQ8_0) return launch_gemm_type(c, type, false, p, grid);
     return fail(c, SMX_ERR_ARG, "grouped gemm: weight type %d not supported", (int)type);
 }

@@ -34,22 +34,27 @@ __device__ __forceinline__ float4 silu_mul4(float4 g, float4 u) {
 }
 __device__ __forceinline__ void silu_mul_quant4(float4 gv, float4 uv, int* packed, float* scale) { quant4(silu_mul4(gv, uv), packed, scale); }
 
-// g, u [items / 8 blocks of 32] -> quantised silu(g)*u; 8 lanes per 32-block, two items per thread (one: 0.6 us longer
-// on 4096 x 768).
-__global__ __launch_bounds__(256) void silu_mul_quant_kernel(const float4* __restrict__ g, const float4* __restrict__ u, int* __restrict__ xq4,
-                                                             float* __restrict__ xd, size_t items) {
-    constexpr int IT = 2;
-    const size_t i0 = (size_t)blockIdx.x * (256 * IT) + threadIdx.x;
-    const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
-    float4 gv[IT], uv[IT];
-#pragma unroll
-    for (int j = 0; j < IT; j++) {
-        const size_t i = i0 + j * 256;
-        gv[j] = i < items ? g[i] : zero;
-        uv[j] = i < items ? u[i] : zero;
+// g, u [items / 8 blocks of 32] -> quantised silu(g)*u; 8 lanes per 32-block, one item per thread.  Lanes past the end read the last
+// item: with a select for each load the two were waited for one after the other (4096 x 768: 8.4 against 6.8 us; two items
+// per thread 8.2).
+// SPLIT: g and u arrive as `slices` planes of partial sums, added here in ascending order (keep: the sums replace the first planes).
+template <bool SPLIT>
+__global__ __launch_bounds__(256) void silu_mul_quant_kernel(float4* __restrict__ g, float4* __restrict__ u, int* __restrict__ xq4,
+                                                             float* __restrict__ xd, size_t items, int slices, bool keep) {
+    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x, ic = min(i, items - 1);
+    float4 gv = g[ic], uv = u[ic];
+    if constexpr (SPLIT) {
+        for (int z = 1; z < slices; z++) {
+            const float4 gz = g[z * items + ic], uz = u[z * items + ic];
+            gv.x += gz.x; gv.y += gz.y; gv.z += gz.z; gv.w += gz.w;
+            uv.x += uz.x; uv.y += uz.y; uv.z += uz.z; uv.w += uz.w;
+        }
+        if (keep && i < items) {
+            g[i] = gv;
+            u[i] = uv;
+        }
     }
-#pragma unroll
-    for (int j = 0; j < IT; j++) put_quant4(quantize4(silu_mul4(gv[j], uv[j])), i0 + j * 256 < items, i0 + j * 256, xq4, xd, nullptr);
+    put_quant4(quantize4(silu_mul4(gv, uv)), i < items, i, xq4, xd, nullptr);
 }
 
 // Routed expert ids and weights travel as kernel arguments (no table upload on the decode path), or,
@@ -440,11 +445,11 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(const float* __restric
     }
 }
 
-static int silu_mul_quant(smx_ctx* c, const float* g, const float* u, size_t rows, size_t eff, int8_t* xq, float* xd) {
+static int silu_mul_quant(smx_ctx* c, float* g, float* u, size_t rows, size_t eff, int8_t* xq, float* xd, int slices = 1, bool keep = false) {
     const size_t items = rows * eff / 4;
     ProfScope ps(c, "silu_mul_quant");
-    hipLaunchKernelGGL(silu_mul_quant_kernel, dim3((unsigned)((items + 511) / 512)), dim3(256), 0, c->stream, (const float4*)g, (const float4*)u,
-                       (int*)xq, xd, items);
+    auto kern = slices > 1 ? silu_mul_quant_kernel<true> : silu_mul_quant_kernel<false>;
+    hipLaunchKernelGGL(kern, dim3((unsigned)((items + 255) / 256)), dim3(256), 0, c->stream, (float4*)g, (float4*)u, (int*)xq, xd, items, slices, keep);
     SMX_HIP(c, hipGetLastError());
     return SMX_OK;
 }
@@ -953,7 +958,8 @@ int smx_moe_shexp_dev(smx_ctx* c, size_t layer, float sgate, const float* x_dev,
 
 // The grouped expert FFN over a slot table: quantise the m activation rows, gate and up of every
 // expert group in one GEMM launch (slot s reads activation row rowmap[s], or row s when rowmap is
-// null), silu(g)*u re-quantised, down in a second GEMM launch.  dy[slots][hidden] is left in c->work.
+// null), over slices_gu K slices whose sums the next launch adds up (keep_gu: and leaves in g and u), silu(g)*u re-quantised,
+// down in a second GEMM launch.  dy[slots][hidden] is left in c->work.
 // The two tile tables (device pointers) are those of build_tiles over the plan for eff and hidden rows.
 struct SlotScratch {
     float *g, *u;   // [slots][eff] gate and up outputs
@@ -962,14 +968,15 @@ struct SlotScratch {
     float* dy;      // [slots][hidden] unweighted down outputs
 };
 static int moe_slots_enqueue(smx_ctx* c, const MoeLayer& L, const float* x_dev, size_t m, const int* rowmap_dev, size_t slots,
-                             const GemmTile* tiles_gu, size_t n_gu, const GemmTile* tiles_dn, size_t n_dn, SlotScratch* out) {
+                             const GemmTile* tiles_gu, size_t n_gu, int slices_gu, const GemmTile* tiles_dn, size_t n_dn, bool keep_gu,
+                             SlotScratch* out) {
     const size_t hidden = L.hidden, eff = L.eff, nb = hidden / 32, enb = eff / 32;
     int rc;
     if ((rc = ensure(c, c->xq, m * hidden + kReadSlack)) != SMX_OK) return rc;
     if ((rc = ensure(c, c->xd, m * nb * 4 + kReadSlack)) != SMX_OK) return rc;
     if ((rc = ensure(c, c->xs, m * nb * 4)) != SMX_OK) return rc;
     Carver cv;
-    const size_t o_g = cv.take(slots * eff * 4), o_u = cv.take(slots * eff * 4), o_aq = cv.take(slots * eff),
+    const size_t o_g = cv.take(slices_gu * slots * eff * 4), o_u = cv.take(slices_gu * slots * eff * 4), o_aq = cv.take(slots * eff),
                  o_ad = cv.take(slots * enb * 4), o_dy = cv.take(slots * hidden * 4);
     if ((rc = ensure(c, c->work, cv.off)) != SMX_OK) return rc;
     float* g = (float*)(c->work.p + o_g);
@@ -991,11 +998,10 @@ static int moe_slots_enqueue(smx_ctx* c, const MoeLayer& L, const float* x_dev, 
         p.N = (int)eff;
         p.nb = (int)nb;
         p.ldo = (int)eff;
-        p.stages_per_slice = (int)((nb + 3) / 4);
-        rc = launch_gemm_grouped(c, L.type, p, (int)n_gu, 2, "moe_gemm_gate_up");
+        rc = launch_gemm_grouped(c, L.type, p, (int)n_gu, 2, slices_gu, "moe_gemm_gate_up");
         if (rc != SMX_OK) return rc;
     }
-    rc = silu_mul_quant(c, g, u, slots, eff, aq, ad);
+    rc = silu_mul_quant(c, g, u, slots, eff, aq, ad, slices_gu, keep_gu);
     if (rc != SMX_OK) return rc;
     {
         GemmArgs p = {};
@@ -1008,8 +1014,7 @@ static int moe_slots_enqueue(smx_ctx* c, const MoeLayer& L, const float* x_dev, 
         p.N = (int)hidden;
         p.nb = (int)enb;
         p.ldo = (int)hidden;
-        p.stages_per_slice = (int)((enb + 3) / 4);
-        rc = launch_gemm_grouped(c, L.type, p, (int)n_dn, 1, "moe_gemm_down");
+        rc = launch_gemm_grouped(c, L.type, p, (int)n_dn, 1, 1, "moe_gemm_down");
         if (rc != SMX_OK) return rc;
     }
     *out = SlotScratch{g, u, aq, ad, dy};
@@ -1104,6 +1109,7 @@ static int moe_layer_impl(smx_ctx* c, size_t layer, const float* xs, size_t m, c
     std::vector<GemmTile> tiles_gu, tiles_dn;
     build_tiles(plan, nplan, L.eff, &tiles_gu);
     build_tiles(plan, nplan, hidden, &tiles_dn);
+    const int slices_gu = gemm_grouped_slices(c, hidden, tiles_gu.size(), 2);
     TableBlob tb;
     const size_t o_st = tb.add(slot_tok, slots * 4), o_ws = tb.add(wslot, slots * 4), o_tp = tb.add(tok_ptr.data(), (m + 1) * 4),
                  o_ts = tb.add(tok_slots.data(), slots * 4), o_t1 = tb.add(tiles_gu.data(), tiles_gu.size() * sizeof(GemmTile)),
@@ -1115,7 +1121,7 @@ static int moe_layer_impl(smx_ctx* c, size_t layer, const float* xs, size_t m, c
         int rc = tb.upload(c);
         if (rc != SMX_OK) return rc;
         rc = moe_slots_enqueue(c, L, x_dev, m, (const int*)(c->tab.p + o_st), slots, (const GemmTile*)(c->tab.p + o_t1), tiles_gu.size(),
-                               (const GemmTile*)(c->tab.p + o_t2), tiles_dn.size(), &ss);
+                               slices_gu, (const GemmTile*)(c->tab.p + o_t2), tiles_dn.size(), stages != nullptr, &ss);
         if (rc != SMX_OK) return rc;
         float* dy = ss.dy;
         ProfScope ps(c, "moe_combine");
@@ -1178,6 +1184,7 @@ int smx_moe_layer_ffn(smx_ctx* c, size_t layer, const int32_t* plan, size_t npla
     std::vector<GemmTile> tiles_gu, tiles_dn;
     build_tiles(plan3.data(), nplan, L.eff, &tiles_gu);
     build_tiles(plan3.data(), nplan, hidden, &tiles_dn);
+    const int slices_gu = gemm_grouped_slices(c, hidden, tiles_gu.size(), 2);
     TableBlob tb;
     const size_t o_t1 = tb.add(tiles_gu.data(), tiles_gu.size() * sizeof(GemmTile)),
                  o_t2 = tb.add(tiles_dn.data(), tiles_dn.size() * sizeof(GemmTile));
@@ -1188,7 +1195,7 @@ int smx_moe_layer_ffn(smx_ctx* c, size_t layer, const int32_t* plan, size_t npla
     if ((rc = host_send(c, c->xf32.p, xs, rows * hidden * 4, true, dy, rows * hidden * 4, &hp, &x_dev)) != SMX_OK) return rc;
     SlotScratch ss = {};
     rc = moe_slots_enqueue(c, L, x_dev, rows, nullptr, rows, (const GemmTile*)(c->tab.p + o_t1), tiles_gu.size(),
-                           (const GemmTile*)(c->tab.p + o_t2), tiles_dn.size(), &ss);
+                           slices_gu, (const GemmTile*)(c->tab.p + o_t2), tiles_dn.size(), false, &ss);
     rc = host_receive(c, dy, ss.dy, rows * hidden * 4, hp, rc);
     return rc == SMX_OK ? call.done() : rc;
     });

@@ -145,6 +145,22 @@ def test_moe_layer_q6k_stagewise(accel, orc, synth, moe_stagewise, ne, hidden, e
     assert np.array_equal(y, accel.moe_layer_q8_dev(17, xs, m, plan, slot_tok, wslot))
 
 
+# gate and up over K slices, by the rule and forced: a last stage of 3 blocks and a last slice of fewer stages (1120 wide: 9 stages), slices
+# that begin inside a superblock (2816 wide Q6_K: 22 stages), as many slices as stages (512 wide), one slice
+@pytest.mark.parametrize("ty,ne,hidden,eff,k,m", [(8, 5, 1120, 160, 2, 40), (14, 6, 2816, 256, 3, 60), (14, 3, 512, 256, 2, 200)])
+def test_moe_layer_k_slices(accel, orc, synth, moe_stagewise, ty, ne, hidden, eff, k, m):
+    gate, up, down = (synth.make_moe_q8 if ty == 8 else synth.make_moe_q6)(ne, hidden, eff, seed=hidden)
+    assert (accel.upload_moe_q8 if ty == 8 else accel.upload_moe_q6)(18, gate, up, down, hidden, eff, ne)
+    ids, w = synth.zipf_routing(m, ne, k, seed=21)
+    xs = synth.make_acts(m, hidden, seed=22)
+    plan, slot_tok, wslot = synth.group_by_expert(ids, w, ne)
+    for slices in (0, 1, 4, 5):
+        accel.tune("gemm_splitk", slices)
+        y, worst = moe_stagewise(accel, orc, 18, ty, gate, up, down, ne, hidden, eff, xs, plan, slot_tok, wslot)
+        assert np.array_equal(y, accel.moe_layer_q8_dev(18, xs, m, plan, slot_tok, wslot)), slices
+    accel.tune("gemm_splitk", 0)
+
+
 @pytest.mark.parametrize("ne,hidden,eff,k,m", [(4, 64, 32, 2, 5), (8, 256, 160, 3, 37), (16, 512, 256, 4, 300)])
 def test_moe_layer_matches_decode_path(accel, orc, synth, relerr, ne, hidden, eff, k, m):
     gate, up, down = _layer(accel, synth, 7, ne, hidden, eff, seed=hidden + m)
