@@ -42,34 +42,27 @@ __global__ __launch_bounds__(256) void actprod_quant_kernel(const ProdRows R, in
     put_quant4(quantize4(w), live, (size_t)j * nb32 * 8 + gid, xq4, xd, xs);
 }
 
-// m rows through an activation producer and the quantiser: the prefill form of the producers (kernels.rs:101-147
-// rmsnorm_xquant per row, :1174-1187 silu_quant_rows).  b: rmsnorm weight [K] (or null) shared by the rows
-// (b_stride 0), or the second operand [m][K] of silu / gelu.  Workgroup (row, part) takes the slices part, part + gridDim.y, ... of
-// 256 * IT items of its row: rmsnorm needs the whole row's sum of squares and runs one workgroup per
-// row; the exp-based producers have independent blocks and spread a row over one workgroup per slice (a single
-// workgroup per 9728-element row left 64 rows on 64 of the 256 CUs, ten exp-heavy rounds each).
-// rmsnorm rows of up to 256 * IT items (IT = 4: 4096 values) stay in registers between the two passes over them: 2048 x 3840
+// m rmsnorm rows through the quantiser (kernels.rs:101-147 rmsnorm_xquant per row), one workgroup per row.  b: the rmsnorm weight [K] or
+// null.  Rows of up to 256 * IT items (4096 values) stay in registers between the two passes over them: 2048 x 3840
 // 16.2 -> 13.1 us, and of a dense FFN of 100 tokens (2560 <-> 9728), where the second pass is one more trip to memory, 76.7 -> 74.0.
-template <int IT>
-__global__ __launch_bounds__(256) void rows_prod_quant_kernel(const float* __restrict__ a, const float* __restrict__ b,
-                                                              size_t b_stride, int kind, float eps, int* __restrict__ xq4,
-                                                              float* __restrict__ xd, int* __restrict__ xs, int nb32) {
+__global__ __launch_bounds__(256) void rmsnorm_quant_kernel(const float* __restrict__ a, const float* __restrict__ b, float eps,
+                                                            int* __restrict__ xq4, float* __restrict__ xd, int* __restrict__ xs, int nb32) {
 #pragma clang fp contract(off)
+    constexpr int IT = 4;
     __shared__ double red[4];
     const size_t row = blockIdx.x;
     const float* ar = a + row * (size_t)nb32 * 32;
-    const float* br = b ? b + row * b_stride : nullptr;
     const int items = nb32 * 8;
     float rs = 1.f;
-    const bool held = kind == SMX_ACT_RMSNORM && items <= 256 * IT;
-    if (kind == SMX_ACT_RMSNORM && !held) rs = rms_scale((char*)red, ar, nb32 * 32, eps);
-    for (int i0 = blockIdx.y * 256 * IT; i0 < items; i0 += gridDim.y * 256 * IT) {  // whole 8-lane groups stay together: items % 8 == 0
+    const bool held = items <= 256 * IT;
+    if (!held) rs = rms_scale((char*)red, ar, nb32 * 32, eps);
+    for (int i0 = 0; i0 < items; i0 += 256 * IT) {  // whole 8-lane groups stay together: items % 8 == 0
         float4 v[IT], g[IT];
 #pragma unroll
         for (int j = 0; j < IT; j++) {
             const int i = i0 + j * 256 + threadIdx.x;
             v[j] = i < items ? ((const float4*)ar)[i] : make_float4(0.f, 0.f, 0.f, 0.f);
-            g[j] = br && i < items ? ((const float4*)br)[i] : make_float4(1.f, 1.f, 1.f, 1.f);
+            g[j] = b && i < items ? ((const float4*)b)[i] : make_float4(1.f, 1.f, 1.f, 1.f);
         }
         if (held) rs = rms_scale_held<IT>((char*)red, v, nb32 * 32, eps);
 #pragma unroll
@@ -77,34 +70,10 @@ __global__ __launch_bounds__(256) void rows_prod_quant_kernel(const float* __res
             const int i = i0 + j * 256 + threadIdx.x;
             if (i0 + j * 256 >= items) break;   // the whole workgroup
             const float4 x = v[j], y = g[j];
-            float4 w;
-            if (kind == SMX_ACT_RMSNORM) {
-                w.x = (x.x * rs) * y.x; w.y = (x.y * rs) * y.y; w.z = (x.z * rs) * y.z; w.w = (x.w * rs) * y.w;
-            } else if (kind == SMX_ACT_SILU_MUL) {
-                w.x = det_silu(x.x) * y.x; w.y = det_silu(x.y) * y.y; w.z = det_silu(x.z) * y.z; w.w = det_silu(x.w) * y.w;
-            } else {
-                w.x = det_gelu_tanh(x.x) * y.x; w.y = det_gelu_tanh(x.y) * y.y;
-                w.z = det_gelu_tanh(x.z) * y.z; w.w = det_gelu_tanh(x.w) * y.w;
-            }
+            const float4 w = make_float4((x.x * rs) * y.x, (x.y * rs) * y.y, (x.z * rs) * y.z, (x.w * rs) * y.w);
             put_quant4(quantize4(w), i < items, row * (size_t)items + i, xq4, xd, xs);
         }
     }
-}
-
-int launch_rows_prod_quant(smx_ctx* c, int kind, const float* a, const float* b, size_t m, size_t K, float eps, int8_t* xq,
-                           float* xd, int32_t* xs) {
-    if (K % 32 != 0 || m == 0 || m > 0x7fffffffu) return fail(c, SMX_ERR_ARG, "producer quantiser: %zu rows of %zu", m, K);
-    if (kind != SMX_ACT_RMSNORM && kind != SMX_ACT_SILU_MUL && kind != SMX_ACT_GEGLU)
-        return fail(c, SMX_ERR_ARG, "producer quantiser: kind %d", kind);
-    ProfScope ps(c, "rows_prod_quant");
-    const bool norm = kind == SMX_ACT_RMSNORM;
-    constexpr int IT = 2;   // items per thread of the exp-based producers
-    const unsigned parts = norm ? 1u : (unsigned)std::min<size_t>((K / 4 + 256 * IT - 1) / (256 * IT), 65535);
-    const auto kern = norm ? rows_prod_quant_kernel<4> : rows_prod_quant_kernel<IT>;
-    hipLaunchKernelGGL(kern, dim3((unsigned)m, parts), dim3(256), 0, c->stream, a, b, norm ? (size_t)0 : K, kind, eps, (int*)xq, xd, (int*)xs,
-                       (int)(K / 32));
-    SMX_HIP(c, hipGetLastError());
-    return SMX_OK;
 }
 
 int launch_actprod_quant(smx_ctx* c, int kind, const float* const* as, const float* const* bs, int n, size_t K,
@@ -120,6 +89,29 @@ int launch_actprod_quant(smx_ctx* c, int kind, const float* const* as, const flo
     ProfScope ps(c, "actprod_quant");
     hipLaunchKernelGGL(actprod_quant_kernel, dim3((unsigned)((nb32 * 8 + 255) / 256), (unsigned)n), dim3(256), 0, c->stream, R,
                        kind, (int*)xq, xd, (int*)xs, nb32);
+    SMX_HIP(c, hipGetLastError());
+    return SMX_OK;
+}
+
+// The prefill form of the producers (rmsnorm: above; kernels.rs:1174-1187 silu_quant_rows).  The exp-based ones have independent blocks and
+// [m][K] operands: their m rows are one long row of actprod_quant_kernel, an item per thread.  Against a workgroup per 512 items of a row
+// in a loop over its parts: 2048 x 15360 50.8 -> 45.2 us (283 MB: the memory's rate), 400 x 5888 8.0 -> 6.5, 40 x 3072 3.6 -> 2.9.
+int launch_rows_prod_quant(smx_ctx* c, int kind, const float* a, const float* b, size_t m, size_t K, float eps, int8_t* xq,
+                           float* xd, int32_t* xs) {
+    if (K % 32 != 0 || m == 0 || m > 0x7fffffffu) return fail(c, SMX_ERR_ARG, "producer quantiser: %zu rows of %zu", m, K);
+    if (kind != SMX_ACT_RMSNORM && kind != SMX_ACT_SILU_MUL && kind != SMX_ACT_GEGLU)
+        return fail(c, SMX_ERR_ARG, "producer quantiser: kind %d", kind);
+    ProfScope ps(c, "rows_prod_quant");
+    if (kind != SMX_ACT_RMSNORM) {
+        if (m * K / 4 > 0x7fffff00u) return fail(c, SMX_ERR_LIMIT, "producer quantiser: %zu rows of %zu exceed the launch limits", m, K);
+        ProdRows R = {};
+        R.a[0] = (const float4*)a;
+        R.b[0] = (const float4*)b;
+        hipLaunchKernelGGL(actprod_quant_kernel, dim3((unsigned)((m * K / 4 + 255) / 256)), dim3(256), 0, c->stream, R, kind, (int*)xq, xd, (int*)xs,
+                           (int)(m * K / 32));
+    } else {
+        hipLaunchKernelGGL(rmsnorm_quant_kernel, dim3((unsigned)m), dim3(256), 0, c->stream, a, b, eps, (int*)xq, xd, (int*)xs, (int)(K / 32));
+    }
     SMX_HIP(c, hipGetLastError());
     return SMX_OK;
 }
