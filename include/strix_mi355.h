@@ -101,8 +101,8 @@ int smx_gemv_f32(smx_ctx* ctx, const char* key, const float* x, size_t in_len, f
 int smx_gemv_f32_dev(smx_ctx* ctx, const char* key, const float* x_dev, float* y_dev);
 /* Small batches, m <= SMX_GEMV_ROWS_MAX rows against one weight read once (kernels.rs:1605-1632 q8_gemm_rows,
  * :830-857 q8_gemm_rows32, :1016-1045 q8i_gemm_rows32; the n-gram verify step and short prefill chunks):
- * xs[m][in_dim] -> y[m][out_dim].  Up to 4 rows run in the dot4 GEMV; 5..32 rows of a Q8_0 / Q4_0 weight (17..32 rows:
- * weights of up to 32768 rows) and 5..16 rows of a Q6_K weight in the small-batch kernel on the matrix cores; every other
+ * xs[m][in_dim] -> y[m][out_dim].  Up to 4 rows run in the dot4 GEMV; 5..32 rows (17..32:
+ * of weights of up to 32768 rows) in the small-batch kernel on the matrix cores; every other
  * case in the tiled GEMM.  The integer block dots do not depend on which, the fp32 sums agree within 1e-5. */
 #define SMX_GEMV_MAX_M 8
 #define SMX_GEMV_ROWS_MAX 32

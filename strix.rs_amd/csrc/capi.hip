@@ -93,8 +93,8 @@ static int launch_argmax_rows(smx_ctx* c, const float* y, size_t m, size_t N, vo
 }
 
 // quantise m device rows and run the right matmul kernel into y_dev
-// Which kernel serves m rows: the small-batch MFMA kernel for 5..32 rows of a Q8_0 / Q4_0 weight (17..32 rows: weights of up
-// to 32768 rows) and 5..16 rows of a Q6_K weight (skinny_serves); otherwise the dot4 GEMV up to SMX_GEMV_MAX_M rows (4 of a
+// Which kernel serves m rows: the small-batch MFMA kernel for 5..64 rows (17 and more: weights of up to 32768 rows, 33 and more of a
+// Q6_K weight: 10240 and 40 Mi elements; skinny_serves); otherwise the dot4 GEMV up to SMX_GEMV_MAX_M rows (4 of a
 // Q6_K weight), the tiled GEMM beyond.
 }  // namespace
 

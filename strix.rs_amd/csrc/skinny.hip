@@ -1,4 +1,4 @@
-// Small-batch matmul on the matrix cores: 5..32 activation rows against one resident Q8_0 / Q4_0 weight
+// Small-batch matmul on the matrix cores: 5..64 activation rows against one resident weight
 // that is streamed from HBM exactly once.  Stands in for the reference's token-tile kernels
 // (crates/strix-backend-rocm/src/kernels.rs:1605-1632 q8_gemm_rows, :830-857 q8_gemm_rows32, :1016-1045
 // q8i_gemm_rows32; dispatch decode.rs:1742-1766): the n-gram verify step and short prefill chunks.
@@ -114,20 +114,21 @@ struct PieceRegs {
 // ALDS (8 or 16 token slots): the activation fragments of a piece, tslots * 128 contiguous bytes, go global -> LDS
 // directly in one or two instructions and every lane reads its own from there, instead of four register loads in
 // which most lanes fetch a copy (the kernel is bound by the number of vector-memory instructions).
-// Q6_K (always with ALDS, so up to 16 rows): a piece is half a superblock; its ql and qh bytes land as they are (3 LDS-direct
+// Q6_K: a piece is half a superblock; its ql and qh bytes land as they are (3 LDS-direct
 // instructions), the wave widens them to signed int8 in operand order (thread = [row:5][p:1] makes the 16-byte chunks 2j + p,
-// ggml_quant.rs:417-426), and a 32-block is two v_mfma_i32_32x32x16_i8, one per 16-element sub-block with its own d * sc.
+// ggml_quant.rs:417-426), and a 32-block is two v_mfma_i32_32x32x16_i8, one per 16-element sub-block with its own d * sc.  Beyond 16 rows the activation fragments come through registers as for the other formats, 16 bytes of
+// sub-block `half` per lane, and v_permlane32_swap trades them into 8 bytes of either.  Per call of 17..32 rows against the tiled GEMM:
+// 2560 x 9728 22 -> 13.8 us, 9728 x 2560 20.5 -> 14.3, 4096 x 4096 20 -> 9.4, 168 x 11264 20 -> 13.6, 512 x 512 10 -> 6.6.
 // NACC: accumulators per lane that hold live tokens (accumulator i of lane half h is token (i / 4) * 8 + 4 h + i % 4: 4 for up
 // to 8 token slots, 8 for 16); only those are rescaled -- with all 16 the Q6_K variant would be bound by its vector ALU work,
 // and Q4_0 9728 x 2560 takes 1.3 us longer at 5..16 rows.
-// TT = 2 (33..64 rows of a Q8_0 / Q4_0 weight): two 32-token tiles share every weight piece -- two MFMAs per block on the same
+// TT = 2 (33..64 rows): two 32-token tiles share every weight piece -- two MFMAs per block on the same
 // weight fragment, 32 accumulators per lane -- so the weight is still read once (the tiled GEMM takes 22 us where 32 rows
 // take 14: 128-row strips leave it 20 tiles to split over K, and a reduction launch behind them).
 template <int FMT, bool DUMP, int NW, bool ALDS, int NACC = 16, int TT = 1>
 __global__ __launch_bounds__(64 * NW) void skinny_kernel(const SkinnyArgs p) {
     constexpr bool Q4 = FMT == FMT_Q4, Q6 = FMT == FMT_Q6;
-    static_assert(!Q6 || ALDS, "the Q6_K variant reads its activation fragments from LDS");
-    static_assert(TT == 1 || (!ALDS && !Q6 && NACC == 16), "two token tiles: fragments through registers, all accumulators live");
+    static_assert(TT == 1 || (!ALDS && NACC == 16), "two token tiles: fragments through registers, all accumulators live");
     constexpr int kWaves = NW;
     constexpr int kWaveLds = wave_lds(FMT, ALDS);
     extern __shared__ __align__(16) char smem[];
@@ -300,10 +301,20 @@ __global__ __launch_bounds__(64 * NW) void skinny_kernel(const SkinnyArgs p) {
             const float dxv = __uint_as_float(dxs[bi]);
             if constexpr (Q6) {
                 const float d6 = h2f_s(r.d6), d6m128 = -128.f * d6;
+                // register fragments: lane half h holds sub-block h; the halves trade so that each holds 8 elements of either
+                long ar[2], cr[2];
+                const auto by_half = [](const v4i& a, long (&o)[2]) {
+                    const auto xz = __builtin_amdgcn_permlane32_swap((unsigned)a.x, (unsigned)a.z, false, false);
+                    const auto yw = __builtin_amdgcn_permlane32_swap((unsigned)a.y, (unsigned)a.w, false, false);
+                    o[0] = (long)(((unsigned long)yw[0] << 32) | xz[0]);
+                    o[1] = (long)(((unsigned long)yw[1] << 32) | xz[1]);
+                };
+                if constexpr (!ALDS) by_half(bi == 0 ? r.a0 : (bi == 1 ? r.a1 : (bi == 2 ? r.a2 : r.a3)), ar);
+                if constexpr (TT == 2) by_half(bi == 0 ? r.c0 : (bi == 1 ? r.c1 : (bi == 2 ? r.c2 : r.c3)), cr);
 #pragma unroll
                 for (int jj = 0; jj < 2; jj++) {   // sub-block jj: chunk 2 bi + jj; a lane holds bytes 8 half .. + 7 of it on both sides
                     const long bw = *(const long*)(buf + col * 128 + ((2 * bi + jj + col) & 7) * 16 + half * 8);
-                    const long aw = *(const long*)(mine_a + ((bi * 2 + jj) * p.tslots + min(col, p.tslots - 1)) * 16 + half * 8);
+                    const long aw = ALDS ? *(const long*)(mine_a + ((bi * 2 + jj) * p.tslots + min(col, p.tslots - 1)) * 16 + half * 8) : ar[jj];
                     const v16i d = __builtin_amdgcn_mfma_i32_32x32x16_i8(aw, bw, cmagic, 0, 0, 0);
                     // d * sc, exact in fp32 (11 x 8 significant bits): sc + 128 as an unsigned byte -> float, then one FMA
                     const unsigned scw = ((2 * bi + jj) < 4 ? r.dw.x : r.dw.y) ^ 0x80808080u;
@@ -315,6 +326,19 @@ __global__ __launch_bounds__(64 * NW) void skinny_kernel(const SkinnyArgs p) {
                         for (int i = 0; i < NACC; i++) {
                             const int tok = (i >> 2) * 8 + half * 4 + (i & 3);
                             if (tok < p.m && row <= r_last) p.dump[((size_t)tok * p.N + row) * (2 * p.nb) + 2 * (blk0 + bi) + jj] = d[i] - kMagicI;
+                        }
+                    }
+                    if constexpr (TT == 2) {   // the second token tile on the same weight fragment
+                        const v16i d1 = __builtin_amdgcn_mfma_i32_32x32x16_i8(cr[jj], bw, cmagic, 0, 0, 0);
+                        const unsigned dxs1[4] = {r.dx1.x, r.dx1.y, r.dx1.z, r.dx1.w};
+                        rescale(acc1, d1, dw, __uint_as_float(dxs1[bi]));
+                        if (DUMP) {
+                            const int row = r0 + col;
+#pragma unroll
+                            for (int i = 0; i < 16; i++) {
+                                const int tok = 32 + (i >> 2) * 8 + half * 4 + (i & 3);
+                                if (tok < p.m && row <= r_last) p.dump[((size_t)tok * p.N + row) * (2 * p.nb) + 2 * (blk0 + bi) + jj] = d1[i] - kMagicI;
+                            }
                         }
                     }
                 }
@@ -452,9 +476,10 @@ bool skinny_serves(const Weight& w, size_t m) {
     // 17..32 rows of a very tall weight: the tiled GEMM is ahead (Q8_0 65536 x 3840 at 32 rows 61.6 against 70.7 us; at 16 rows
     // 58.3 / 61.8, at 8 rows the dot4 GEMV 68.2 / 57.6 us; 262144 x 2560: 174.5 / 169.6, 159.2 / 155.5, 171.6 / 139.0 us)
     if (m < SMX_SKINNY_MIN_M || m > SMX_SKINNY_MAX_M || w.K < 128) return false;
-    if (w.type == kQ6_K) return m <= 16;   // its activation fragments travel through LDS: up to 16 token slots
-    // 33..64 rows: two token tiles per weight piece
-    return (w.type == kQ8_0 || w.type == kQ4_0) && (m <= 16 || w.N <= 32768);
+    // 33..64 rows of a Q6_K weight, whose 32 accumulators are rescaled twice per block: 4096 x 4096 23 -> 12.7 us, 2560 x 9728 25.8 -> 21.8,
+    // 9728 x 2560 24.6 -> 22.5; but 6254 x 9216 37.2 -> 37.8, 15360 x 3840 35.6 -> 36.0, 32000 x 1792 34.2 -> 38.8
+    if (w.type == kQ6_K && m > 32) return w.N <= 10240 && w.N * w.K <= size_t(40) << 20;
+    return m <= 16 || w.N <= 32768;
 }
 
 static size_t skinny_slots(size_t m) { return m <= 8 ? 8 : (m <= 16 ? 16 : (m <= 32 ? 32 : 64)); }   // 64: two tiles of 32
@@ -523,17 +548,15 @@ int launch_skinny(smx_ctx* c, const Weight& w, const float* x, size_t m, float* 
         return SMX_OK;
     };
 #define SMX_SK_GO(F_, NW_, AL_, NA_) (dump ? go(skinny_kernel<F_, true, NW_, AL_, NA_>) : go(skinny_kernel<F_, false, NW_, AL_, NA_>))
-    if (fmt == FMT_Q6) {
-        if (nw == 16) return p.tslots == 8 ? SMX_SK_GO(FMT_Q6, 16, true, 4) : SMX_SK_GO(FMT_Q6, 16, true, 8);
-        return p.tslots == 8 ? SMX_SK_GO(FMT_Q6, 8, true, 4) : SMX_SK_GO(FMT_Q6, 8, true, 8);
-    }
     // live accumulators per lane: 4 with up to 8 token slots, 8 with 16, all 16 with 32
 #define SMX_SK_ROWS(F_, NW_)                                                                      \
     (p.tslots == 8 ? SMX_SK_GO(F_, NW_, true, 4) : (p.tslots == 16 ? SMX_SK_GO(F_, NW_, true, 8) : SMX_SK_GO(F_, NW_, false, 16)))
     if (ntiles == 2) {
+        if (fmt == FMT_Q6) return dump ? go(skinny_kernel<FMT_Q6, true, 8, false, 16, 2>) : go(skinny_kernel<FMT_Q6, false, 8, false, 16, 2>);
         if (fmt == FMT_Q4) return dump ? go(skinny_kernel<FMT_Q4, true, 8, false, 16, 2>) : go(skinny_kernel<FMT_Q4, false, 8, false, 16, 2>);
         return dump ? go(skinny_kernel<FMT_Q8, true, 8, false, 16, 2>) : go(skinny_kernel<FMT_Q8, false, 8, false, 16, 2>);
     }
+    if (fmt == FMT_Q6) return nw == 16 ? SMX_SK_ROWS(FMT_Q6, 16) : SMX_SK_ROWS(FMT_Q6, 8);
     if (nw == 16) return fmt == FMT_Q4 ? SMX_SK_ROWS(FMT_Q4, 16) : SMX_SK_ROWS(FMT_Q8, 16);
     return fmt == FMT_Q4 ? SMX_SK_ROWS(FMT_Q4, 8) : SMX_SK_ROWS(FMT_Q8, 8);
 #undef SMX_SK_ROWS

@@ -317,7 +317,7 @@ int launch_gemv_dual(smx_ctx* c, const Weight* const* wg, const Weight* const* w
 int launch_gemm(smx_ctx* c, const Weight& w, const int8_t* xq, const float* xd, size_t m, float* y,
                 int32_t* dump);
 
-// Small-batch matmul on the matrix cores (skinny.hip): m <= SMX_SKINNY_MAX_M fp32 rows against a Q8_0 / Q4_0
+// Small-batch matmul on the matrix cores (skinny.hip): m <= SMX_SKINNY_MAX_M fp32 rows against a
 // weight read once (its own quantiser launch + the matmul launch).  dump (optional): out[m][N][K/32] i32.
 #define SMX_SKINNY_MAX_M 64
 #define SMX_SKINNY_MIN_M 5

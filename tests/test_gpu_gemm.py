@@ -162,6 +162,21 @@ def test_small_batch_matches_oracle(accel, orc, synth, relerr, ty, N, K):
     accel.evict("t.sb")
 
 
+# Q6_K beyond 16 rows: both sides of the weight heights up to which 17..32 and 33..64 rows run there, a ragged height, an odd number of
+# superblocks, outputs whose count is no multiple of 4 (one K slice)
+@pytest.mark.parametrize("N,K", [(10240, 256), (10241, 256), (32768, 256), (32769, 256), (77, 2304), (4097, 1024)])
+def test_small_batch_q6k_beyond_16_rows(accel, orc, synth, relerr, N, K):
+    raw = synth.make_weight(14, N, K, seed=N + K)
+    assert accel.upload_q6_k("t.sb6", raw, K, N)
+    for m in (17, 18, 31, 33, 50):
+        xs = synth.make_acts(m, K, seed=m + N)
+        y = accel.prefill_q8_gemm("t.sb6", xs, m, N)
+        assert relerr(y, orc.matmul_q8_from_f32(14, raw, K, N, xs)) <= TOL, m
+        if m <= 32:
+            assert np.array_equal(accel.gemv_rows("t.sb6", xs, N), y)
+    accel.evict("t.sb6")
+
+
 @pytest.mark.parametrize("ty", [8, 2])
 def test_small_batch_ignores_stale_scales_past_k(accel, orc, synth, relerr, ty):
     """The activation scales of a call's last 4-block piece have slots past K when K is not a multiple of 128.  An earlier
