@@ -11,7 +11,8 @@
 //   * a wave's piece (rows x 128 B) goes global -> LDS directly into the wave's own corner of LDS (no
 //     registers, no workgroup barrier); LDS turns "lane = 16 bytes of one row" into the MFMA operand
 //     "lane = row, k-half", chunk-rotated so the transposed reads spread over the banks (Q4_0 nibbles land
-//     raw and are widened to int8 in a second step).  One piece per wave is in flight: the kernel is bound by
+//     raw; both lane halves read a row's 16 bytes of a block and widen theirs, the low nibbles or the high.  Through a widened copy in
+//     LDS: 9728 x 2560, 6 rows 8.75 against 8.35 us, 12 rows 9.4 / 9.05, 2560 x 9728 8.8 / 8.5).  One piece per wave is in flight: the kernel is bound by
 //     the number of vector-memory instructions a CU can take, not by bytes, and a ring of several pieces per wave
 //     costs re-requested pieces at the end of every run (measured: four in flight 16.4 us, two 14.3, one 13.8 on
 //     Q8_0 2560 x 9728 at 16 rows); the other waves of the CU cover a wave's wait;
@@ -39,13 +40,12 @@ namespace {
 constexpr int kMagicI = 0x4B400000;       // float 12582912 = 1.5 * 2^23: adding an i32 |I| < 2^22 to its bits adds I to its value
 constexpr float kMagicF = 12582912.f;
 constexpr int kPiece = 32 * 128;          // LDS bytes of one piece: 32 rows x 4 blocks of int8
-// LDS bytes per wave: the landing area of its piece (Q8_0: 4 KB, already in operand order; Q4_0: 2 KB of raw
-// nibbles and the 4 KB area the widened piece is built in)
-// and, when the activation fragments travel through LDS too (ALDS, up to 16 token slots), 2 KB for those of a piece
-// Q6_K: 2 KB of ql + 1 KB of qh as they are, and the 4 KB widened area.
+// LDS bytes per wave: the landing area of its piece (Q8_0: 4 KB, already in operand order; Q4_0: 2 KB of nibbles, widened on their way
+// out; Q6_K: 2 KB of ql + 1 KB of qh as they are, and the 4 KB widened area) and, when the activation fragments travel through LDS
+// too (ALDS, up to 16 token slots), 1 or 2 KB for those of a piece
 constexpr int FMT_Q8 = 0, FMT_Q4 = 1, FMT_Q6 = 2;
-constexpr int weight_lds(int fmt) { return fmt == FMT_Q4 ? 2048 + kPiece : (fmt == FMT_Q6 ? 3072 + kPiece : kPiece); }
-constexpr int wave_lds(int fmt, bool alds) { return weight_lds(fmt) + (alds ? 2048 : 0); }
+constexpr int weight_lds(int fmt) { return fmt == FMT_Q4 ? 2048 : (fmt == FMT_Q6 ? 3072 + kPiece : kPiece); }
+constexpr int wave_lds(int fmt, bool alds, int nacc) { return weight_lds(fmt) + (alds ? (nacc == 4 ? 1024 : 2048) : 0); }
 
 struct SkinnyArgs {
     const uint16_t* wscales;  // f16 [N][nb]; Q6_K: d [N][K / 256]
@@ -130,7 +130,11 @@ __global__ __launch_bounds__(64 * NW) void skinny_kernel(const SkinnyArgs p) {
     constexpr bool Q4 = FMT == FMT_Q4, Q6 = FMT == FMT_Q6;
     static_assert(TT == 1 || (!ALDS && NACC == 16), "two token tiles: fragments through registers, all accumulators live");
     constexpr int kWaves = NW;
-    constexpr int kWaveLds = wave_lds(FMT, ALDS);
+    // Up to 8 rows of a Q4_0 weight: the MFMA starts from zero and the four live results are converted, which frees the registers of the
+    // constant and lets a CU hold more waves (233361 x 672, 7 rows 50 -> 42 us; Q8_0 and Q6_K 150000 x 3840 lose 3 % by it)
+    constexpr bool kConvert = Q4 && NACC == 4;
+    constexpr int kStart = kConvert ? 0 : kMagicI;
+    constexpr int kWaveLds = wave_lds(FMT, ALDS, NACC);
     extern __shared__ __align__(16) char smem[];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int col = lane & 31, half = lane >> 5;
@@ -155,7 +159,6 @@ __global__ __launch_bounds__(64 * NW) void skinny_kernel(const SkinnyArgs p) {
     const int dx_slot = ((lane & 15) >> 2) * 8 + half * 4 + (lane & 3);
     const int dx_tok = min(dx_slot, m0 - 1);   // token of accumulator lane % 16 in this lane half
     const int dx_tok1 = min(dx_slot, max(m1, 1) - 1);
-    const bool vec_sc = (p.nb & 3) == 0;
     // Q8_0 landing: lane = [row:3][slot:3] of an 8-row group; the lane fetches chunk (slot - row) % 8 of its row, so
     // chunk c of row r sits in slot (c + r) % 8 and the transposed fragment reads spread over the banks
     const int g_rowlo = lane >> 3, g_chunk = ((lane & 7) - g_rowlo) & 7;
@@ -190,12 +193,15 @@ __global__ __launch_bounds__(64 * NW) void skinny_kernel(const SkinnyArgs p) {
             const size_t sb = (size_t)wrow * (p.nb >> 3) + (piece >> 1);
             r.d6 = p.wscales[sb];
             r.dw = *(const uint2*)(p.wsc + sb * 16 + (piece & 1) * 8);
-        } else if (vec_sc) {
+        } else if (TT == 2 && (p.nb & 3) == 0) {   // (Q8_0 2560 x 9728, 48 rows: 14.4 us, 14.6 through the general form)
             r.dw = *(const uint2*)(ws + blk0);
-        } else {   // (the scalar form costs more loads; the waits below are then over-conservative, never too lax)
-            const int last = p.nb - 1;
-            r.dw.x = (unsigned)ws[min(blk0, last)] | ((unsigned)ws[min(blk0 + 1, last)] << 16);
-            r.dw.y = (unsigned)ws[min(blk0 + 2, last)] | ((unsigned)ws[min(blk0 + 3, last)] << 16);
+        } else {   // four scales in one load at any alignment (four of 2 bytes: Q8_0 2560 x 9760, 24 rows 12.4 -> 11.7 us, Q4_0 211582 x 2528,
+                   // 6 rows 106 -> 95); of a last piece of fewer blocks the four that end the row, moved down
+            const int b = min(blk0, p.nb - 4);
+            uint64_t v;
+            __builtin_memcpy(&v, ws + b, 8);
+            v >>= 16 * (blk0 - b);
+            r.dw = make_uint2((unsigned)v, (unsigned)(v >> 32));
         }
         if (Q6) {   // ql: lane = [row:4][chunk:2], 64 bytes per row and half superblock; qh: lane = [row:5][chunk:1], 32 bytes
             const int nsb = p.nb >> 3, sbi = piece >> 1, hs = piece & 1;
@@ -206,8 +212,8 @@ __global__ __launch_bounds__(64 * NW) void skinny_kernel(const SkinnyArgs p) {
                                   mine_lds + j * 1024);
             load_to_lds16((const char*)p.wqh + ((size_t)min(r0 + (lane >> 1), r_last) * nsb + sbi) * 64 + hs * 32 + (lane & 1) * 16,
                           mine_lds + 2048);
-        } else if (Q4) {   // lane = [row:4][block:2]: 64 contiguous bytes of nibbles per row, landing as they are
-            const int b = min(blk0 + (lane & 3), p.nb - 1);
+        } else if (Q4) {   // lane = [row:4][slot:2]: 64 contiguous bytes of nibbles per row, landing as they are; block b in slot (b + row / 2) % 4
+            const int b = min(blk0 + (((lane & 3) - (lane >> 3)) & 3), p.nb - 1);
 #pragma unroll
             for (int j = 0; j < 2; j++)
                 if (j * 16 < nrows)   // wave-uniform
@@ -231,7 +237,7 @@ __global__ __launch_bounds__(64 * NW) void skinny_kernel(const SkinnyArgs p) {
     for (int i = 0; i < (TT == 2 ? 16 : 1); i++) acc1[i] = 0.f;
     v16i cmagic;
 #pragma unroll
-    for (int i = 0; i < 16; i++) cmagic[i] = kMagicI;
+    for (int i = 0; i < 16; i++) cmagic[i] = kStart;
 
     auto consume = [&](const PieceRegs r, int piece) {
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the piece's LDS-direct loads (the compiler does not see them)
@@ -257,27 +263,11 @@ __global__ __launch_bounds__(64 * NW) void skinny_kernel(const SkinnyArgs p) {
             __builtin_amdgcn_wave_barrier();
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
             buf = wide;
-        } else if (Q4) {   // widen the raw nibbles (lane = [row:4][block:2]) into the operand-order area
-            char* wide = mine + 2048;
-            const char* raw = mine;
-#pragma unroll
-            for (int j = 0; j < 2; j++) {
-                const int row = j * 16 + (lane >> 2), bi = lane & 3;
-                const uint4 q = *(const uint4*)(raw + j * 1024 + lane * 16);
-                const uint4 lo = make_uint4(nib16_s(q.x << 4), nib16_s(q.y << 4), nib16_s(q.z << 4), nib16_s(q.w << 4));
-                const uint4 hi = make_uint4(nib16_s(q.x), nib16_s(q.y), nib16_s(q.z), nib16_s(q.w));
-                *(uint4*)(wide + row * 128 + ((2 * bi + row) & 7) * 16) = lo;       // elements 0..15 of the block
-                *(uint4*)(wide + row * 128 + ((2 * bi + 1 + row) & 7) * 16) = hi;   // elements 16..31
-            }
-            // the wave's own LDS writes above are read back by other lanes of the same wave below
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-            buf = wide;
         } else {
             buf = mine;
         }
         const int blk0 = piece * 4;
+        const int q4_shift = half ? 0 : 4;
         const unsigned dwh[4] = {r.dw.x & 0xffffu, r.dw.x >> 16, r.dw.y & 0xffffu, r.dw.y >> 16};
         const unsigned dxs[4] = {r.dx.x, r.dx.y, r.dx.z, r.dx.w};
         // acc[i] += dx(token of accumulator i) * fl(dw * I) for the live accumulators, I the exact i32 of MFMA result d
@@ -285,7 +275,7 @@ __global__ __launch_bounds__(64 * NW) void skinny_kernel(const SkinnyArgs p) {
             const float ndw = -dw * kMagicF;   // exact: dw has at most 18 significant bits (f16, or f16 x int8)
             float t[16];
 #pragma unroll
-            for (int i = 0; i < NACC; i++) t[i] = fmaf(dw, __int_as_float(d[i]), ndw);
+            for (int i = 0; i < NACC; i++) t[i] = kConvert ? dw * (float)d[i] : fmaf(dw, __int_as_float(d[i]), ndw);
             SMX_SK_FMAC(0); SMX_SK_FMAC(1); SMX_SK_FMAC(2); SMX_SK_FMAC(3);
             if constexpr (NACC > 4) { SMX_SK_FMAC(4); SMX_SK_FMAC(5); SMX_SK_FMAC(6); SMX_SK_FMAC(7); }
             if constexpr (NACC > 8) {
@@ -325,7 +315,7 @@ __global__ __launch_bounds__(64 * NW) void skinny_kernel(const SkinnyArgs p) {
 #pragma unroll
                         for (int i = 0; i < NACC; i++) {
                             const int tok = (i >> 2) * 8 + half * 4 + (i & 3);
-                            if (tok < p.m && row <= r_last) p.dump[((size_t)tok * p.N + row) * (2 * p.nb) + 2 * (blk0 + bi) + jj] = d[i] - kMagicI;
+                            if (tok < p.m && row <= r_last) p.dump[((size_t)tok * p.N + row) * (2 * p.nb) + 2 * (blk0 + bi) + jj] = d[i] - kStart;
                         }
                     }
                     if constexpr (TT == 2) {   // the second token tile on the same weight fragment
@@ -337,13 +327,19 @@ __global__ __launch_bounds__(64 * NW) void skinny_kernel(const SkinnyArgs p) {
 #pragma unroll
                             for (int i = 0; i < 16; i++) {
                                 const int tok = 32 + (i >> 2) * 8 + half * 4 + (i & 3);
-                                if (tok < p.m && row <= r_last) p.dump[((size_t)tok * p.N + row) * (2 * p.nb) + 2 * (blk0 + bi) + jj] = d1[i] - kMagicI;
+                                if (tok < p.m && row <= r_last) p.dump[((size_t)tok * p.N + row) * (2 * p.nb) + 2 * (blk0 + bi) + jj] = d1[i] - kStart;
                             }
                         }
                     }
                 }
             } else {
-                const v4i bfrag = *(const v4i*)(buf + col * 128 + ((2 * bi + half + col) & 7) * 16);
+                v4i bfrag;
+                if constexpr (Q4) {   // the row's 16 bytes of the block: low nibbles are elements 0..15 (lane half 0), high ones 16..31
+                    const uint4 q = *(const uint4*)(buf + col * 64 + ((bi + (col >> 1)) & 3) * 16);
+                    bfrag = v4i{(int)nib16_s(q.x << q4_shift), (int)nib16_s(q.y << q4_shift), (int)nib16_s(q.z << q4_shift), (int)nib16_s(q.w << q4_shift)};
+                } else {
+                    bfrag = *(const v4i*)(buf + col * 128 + ((2 * bi + half + col) & 7) * 16);
+                }
                 const v4i afrag = ALDS ? *(const v4i*)(mine_a + ((bi * 2 + half) * p.tslots + min(col, p.tslots - 1)) * 16)
                                        : (bi == 0 ? r.a0 : (bi == 1 ? r.a1 : (bi == 2 ? r.a2 : r.a3)));
                 const v16i d = __builtin_amdgcn_mfma_i32_32x32x32_i8(afrag, bfrag, cmagic, 0, 0, 0);
@@ -354,7 +350,7 @@ __global__ __launch_bounds__(64 * NW) void skinny_kernel(const SkinnyArgs p) {
 #pragma unroll
                     for (int i = 0; i < NACC; i++) {
                         const int tok = (i >> 2) * 8 + half * 4 + (i & 3);
-                        if (live && tok < p.m && row <= r_last) p.dump[((size_t)tok * p.N + row) * p.nb + blk0 + bi] = (d[i] - kMagicI) / (Q4 ? 16 : 1);
+                        if (live && tok < p.m && row <= r_last) p.dump[((size_t)tok * p.N + row) * p.nb + blk0 + bi] = (d[i] - kStart) / (Q4 ? 16 : 1);
                     }
                 }
                 if constexpr (TT == 2) {   // the second token tile on the same weight fragment
@@ -367,7 +363,7 @@ __global__ __launch_bounds__(64 * NW) void skinny_kernel(const SkinnyArgs p) {
 #pragma unroll
                         for (int i = 0; i < 16; i++) {
                             const int tok = 32 + (i >> 2) * 8 + half * 4 + (i & 3);
-                            if (live && tok < p.m && row <= r_last) p.dump[((size_t)tok * p.N + row) * p.nb + blk0 + bi] = (d1[i] - kMagicI) / (Q4 ? 16 : 1);
+                            if (live && tok < p.m && row <= r_last) p.dump[((size_t)tok * p.N + row) * p.nb + blk0 + bi] = (d1[i] - kStart) / (Q4 ? 16 : 1);
                         }
                     }
                 }
@@ -389,19 +385,19 @@ __global__ __launch_bounds__(64 * NW) void skinny_kernel(const SkinnyArgs p) {
     }
 
     // the waves' partial tiles, added in wave order (one token tile after the other through the same LDS)
-    float* red = (float*)smem;   // [wave][16][64]
+    float* red = (float*)smem;   // [wave][NACC][64]
 #pragma unroll
     for (int tile = 0; tile < TT; tile++) {
         __syncthreads();
         const float* av = (TT == 2 && tile == 1) ? acc1 : acc;
 #pragma unroll
-        for (int i = 0; i < NACC; i++) red[(wave * 16 + i) * 64 + lane] = av[i];
+        for (int i = 0; i < NACC; i++) red[(wave * NACC + i) * 64 + lane] = av[i];
         __syncthreads();
 #pragma unroll
         for (int i = wave; i < NACC; i += kWaves) {   // accumulator index; lane as above
             float s = 0.f;
 #pragma unroll
-            for (int w = 0; w < kWaves; w++) s += red[(w * 16 + i) * 64 + lane];
+            for (int w = 0; w < kWaves; w++) s += red[(w * NACC + i) * 64 + lane];
             const int tok = tile * 32 + (i >> 2) * 8 + half * 4 + (i & 3), row = r0 + col;
             if (tok < p.m && row <= r_last) {
                 float* o = p.y + (size_t)tok * p.N + row;
@@ -537,7 +533,8 @@ int launch_skinny(smx_ctx* c, const Weight& w, const float* x, size_t m, float* 
     const int nwg = nrg * ksplit;
     const int nw = (nwg <= c->num_cu && ntiles == 1) ? 16 : 8;   // waves per workgroup (see the kernel; two token tiles: 32 more accumulators per lane)
     const bool alds = p.tslots <= 16;
-    const size_t lds = (size_t)nw * wave_lds(fmt, alds);   // the reduction reuses the first nw * 4 KB
+    const int nacc = p.tslots / 2 < 16 ? p.tslots / 2 : 16;   // live accumulators per lane
+    const size_t lds = (size_t)nw * std::max(wave_lds(fmt, alds, nacc), nacc * 256);   // (the reduction: nw * nacc * 256 bytes)
     const dim3 grid((unsigned)nwg);
     ProfScope ps(c, fmt == FMT_Q4 ? "skinny_q4_0" : (fmt == FMT_Q6 ? "skinny_q6_k" : "skinny_q8_0"));
     auto go = [&](auto kern) -> int {

@@ -162,6 +162,23 @@ def test_small_batch_matches_oracle(accel, orc, synth, relerr, ty, N, K):
     accel.evict("t.sb")
 
 
+# rows of no whole pieces: 1, 2 and 3 blocks in the last one, of fewer and more pieces than waves, row scales at every alignment
+@pytest.mark.parametrize("ty", [2, 8])
+@pytest.mark.parametrize("N,K", [(75, 32 * 7), (33, 32 * 5), (300, 32 * 6), (9, 32 * 79), (1000, 32 * 81), (70, 32 * 66)])
+def test_small_batch_any_block_count(accel, orc, synth, relerr, ty, N, K):
+    raw = synth.make_weight(ty, N, K, seed=N + K)
+    assert getattr(accel, UPLOAD[ty])("t.sbk", raw, K, N)
+    for m in (5, 8, 12, 20, 40):
+        xs = synth.make_acts(m, K, seed=m + N)
+        assert relerr(accel.prefill_q8_gemm("t.sbk", xs, m, N), orc.matmul_q8_from_f32(ty, raw, K, N, xs)) <= TOL, m
+        if N <= 75:
+            xq, _, _ = orc.actquant(xs, K)
+            dots = accel.gemm_block_dots("t.sbk", xs, m, N, K // 32)
+            for i in range(m):
+                assert np.array_equal(dots[i], orc.block_dots(ty, raw, K, N, xq[i])), (m, i)
+    accel.evict("t.sbk")
+
+
 # Q6_K beyond 16 rows: both sides of the weight heights up to which 17..32 and 33..64 rows run there, a ragged height, an odd number of
 # superblocks, outputs whose count is no multiple of 4 (one K slice)
 @pytest.mark.parametrize("N,K", [(10240, 256), (10241, 256), (32768, 256), (32769, 256), (77, 2304), (4097, 1024)])
