@@ -425,6 +425,10 @@ static Tiling pick_tiling(int num_cu, bool q6, int M, int N, int nstages, bool s
     for (int bm : {64, 128, 256}) {
         if (only ? bm != only : bm == 64 ? q6 || M <= 64 : bm == 128 ? !q6 && M > 64 && M <= 128 : M <= 128) continue;   // (65..128 tokens: as two rows of tiles)
         const int T = (M + bm - 1) / bm * ((N + BN - 1) / BN), slots = bm == 256 ? num_cu : 2 * num_cu;
+        // A last row of tiles of up to 32 tokens is over early: where the tiles are up to a tenth more than the CUs, its do not count as
+        // neighbours of the others (Q6_K 1565 x 2544 x 2816, 240 + 20 tiles of 128 tokens: 75 us, where 280 full ones take 97 and 140 of
+        // 256 tokens 92; 1289 x 3088 x 1024, 250 + 25: 34.7 against 39; but 648 x 6464 x 768, 255 + 51: 34.8 against 31.1)
+        const int light = bm == 128 && M > bm && M % bm != 0 && M % bm <= 32 && T <= num_cu + num_cu / 10 ? (N + BN - 1) / BN : 0;
         const bool low = bm == 64 || M <= 64;
         const double alone = bm == 256 ? (q6 ? 3.85 : 2.35) : q6 ? 2.75 : low ? 1.05 : 1.55;
         const double shared = bm == 256 ? alone : q6 ? 4.3 : low ? 1.46 : 2.7;
@@ -444,7 +448,7 @@ static Tiling pick_tiling(int num_cu, bool q6, int M, int N, int nstages, bool s
         for (int z = 1; z <= zmax; z++) {
             const int stages = (nstages + z - 1) / z;
             if (z > 1 && stages == (nstages + z - 2) / (z - 1)) continue;   // the same slices as with one fewer
-            const double us = stages * stage(T * z) + (z > 1 ? 3.5 + (double)z * M * N * 4 / 5e6 : 0.0);
+            const double us = stages * stage(z == 1 ? T - light : T * z) + (z > 1 ? 3.5 + (double)z * M * N * 4 / 5e6 : 0.0);
             if (us < least) {
                 least = us;
                 best = {bm, z};
