@@ -411,7 +411,8 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float4* __rest
 // launch that is estimated to take least, among tiles of 64 (Q8_0, Q4_0), 128 and 256 tokens and every number of whole-stage slices
 // whose workgroups fit the chip's slots in ONE round (a second, partly filled round costs more than shorter slices save): a
 // workgroup's stages one after the other, at the time a stage takes with the CU to itself or shared with a second
-// workgroup, plus the launch that adds up the slices' partials, 3.5 us and 5 MB of them per us.  Tiles that need several rounds: one
+// workgroup and one more for its first loads, plus the launch that adds up the slices' partials, 2.3 us, 0.3 a slice and 5 MB of them per us
+// (without the one more and the 0.3, slices of a single stage: Q4_0 37 x 2816 x 2048 17.4 against 15.9 us, Q8_0 110 x 1104 x 1472 14.5 / 12.9).  Tiles that need several rounds: one
 // slice, 128 or 256 tokens, whichever's rounds take less.
 // The stage times are measured (us): 64 tokens 1.05 alone / 1.46 shared, 128 tokens 1.55 / 2.7, Q6_K 2.75 / 4.3; 256 tokens (one workgroup
 // per CU) 2.35, Q6_K 3.85.  Over 200 shapes of 129..2048 tokens the choice takes 0.6 % more than the best of the three
@@ -437,7 +438,7 @@ static Tiling pick_tiling(int num_cu, bool q6, int M, int N, int nstages, bool s
             return n == 0 ? 0.0 : n <= num_cu ? alone : std::max(alone, shared * (0.93 + 0.07 * (n - num_cu) / num_cu));
         };
         if (T > slots) {   // whole rounds and the rest
-            const double us = nstages * (T / slots * shared + stage(T % slots));
+            const double us = (nstages + 1) * (T / slots * shared + stage(T % slots));
             if (bm >= 128 && us < least) {
                 least = us;
                 best = {bm, 1};
@@ -448,7 +449,7 @@ static Tiling pick_tiling(int num_cu, bool q6, int M, int N, int nstages, bool s
         for (int z = 1; z <= zmax; z++) {
             const int stages = (nstages + z - 1) / z;
             if (z > 1 && stages == (nstages + z - 2) / (z - 1)) continue;   // the same slices as with one fewer
-            const double us = stages * stage(z == 1 ? T - light : T * z) + (z > 1 ? 3.5 + (double)z * M * N * 4 / 5e6 : 0.0);
+            const double us = (stages + 1) * stage(z == 1 ? T - light : T * z) + (z > 1 ? 2.3 + 0.3 * z + (double)z * M * N * 4 / 5e6 : 0.0);
             if (us < least) {
                 least = us;
                 best = {bm, z};
