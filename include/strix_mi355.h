@@ -144,7 +144,10 @@ int smx_moe_ffn(smx_ctx* ctx, size_t layer, const int32_t* ids, const float* wex
  * moe_expert_ffn / moe_expert_queue + flush, accel.rs:220-262, which are this call with one group).
  * xs[rows][hidden] holds the rows of every expert group back to back (gathered by the caller),
  * plan[nplan][2] = (expert, rows of the group); dy[rows][hidden] = the unweighted expert outputs,
- * for the caller's weighted scatter.  Q8_0 and Q6_K expert layers. */
+ * for the caller's weighted scatter.  Q8_0 and Q6_K expert layers.
+ * Summation order of the layer calls: gate and up are summed over one to four K slices, whose number follows from the sizes
+ * alone (the layer's dimensions and expert count, the rows of the call, one group for moe_expert_ffn).  A row's result does not
+ * depend on the other rows' values or experts; calls of other sizes may differ from it in the last bits of those sums. */
 int smx_moe_layer_ffn(smx_ctx* ctx, size_t layer, const int32_t* plan, size_t nplan, const float* xs,
                       size_t rows, float* dy, size_t dy_cap);
 int smx_moe_expert_ffn(smx_ctx* ctx, size_t layer, size_t expert, const float* xs, size_t m, float* y,

@@ -612,15 +612,21 @@ int launch_gemm(smx_ctx* c, const Weight& w, const int8_t* xq, const float* xd, 
 }
 
 // A grouped launch with fewer workgroups than the chip has slots leaves CUs idle while each workgroup walks its K stages alone:
-// K slices, up to four of at least two stages, as long as all workgroups run in one round.  Over 90 drawn layers (8..64 experts, 512..4096
-// wide, 256..1536 inner, 8..640 tokens, Q8_0 and Q6_K) the call gains 7 % on average and never loses; the best number of slices
-// for each would gain 9 %.  A second round of workgroups (768 allowed) loses up to 3 %, six and eight slices are
-// ahead of four on two shapes and cost scratch and traffic.  Q6_K, 22 stages: 72 workgroups 65 -> 25 us, 112 workgroups and 244 tokens 109 -> 71 us
-// a call; Q8_0, 138 workgroups, 152 tokens 56 -> 45.
-int gemm_grouped_slices(const smx_ctx* c, size_t K, size_t ntiles, int nops) {
+// K slices, up to four, as long as all workgroups run in about one round.  The number follows from the sizes alone: a row's sums
+// must not depend on where the router sent the other rows of the call (taken from the tile table they did).  What tiles to expect:
+// the rows in whole tiles and, for the groups' ends, 0.8 tiles a group there may be, 0.5 for Q6_K, whose stages take three times
+// as long and gain where a second round has begun; slices of only two stages where a tile for every group fits 7/8 of the slots.
+// Over 456 calls (44 layers of 8..64 experts, 512..4096 wide, 256..1536 inner, 4..2000 tokens, Zipf and even routing) against one
+// slice: Q8_0 -3.4 %, at worst +1.8 %, Q6_K -11.2 %, +0.2 %; taken from the table -3.8 %, +3.8 % and -10.2 %, 0.  Taken from the
+// layer alone, so that calls of every size agreed, +14 % at 2000 tokens: a slice is 8 bytes a row and inner column, written and
+// read again.  Q6_K, 22 stages: 72 workgroups 65 -> 25 us; Q8_0, 152 tokens 56 -> 45 a call.
+int gemm_grouped_slices(const smx_ctx* c, QType type, size_t K, size_t N, size_t groups, size_t rows, int nops) {
     const size_t stages = (K / 32 + KB - 1) / KB;
-    const size_t wgs = std::max<size_t>(1, ntiles * (size_t)nops);
-    size_t z = std::max<size_t>(1, std::min({size_t(4), stages / 2, 2 * (size_t)c->num_cu / wgs}));
+    const double ends = (double)std::min(groups, rows), whole = (double)rows / BM, per_tile = (double)((N + BN - 1) / BN) * nops;
+    const double slots = 2.0 * c->num_cu;
+    const size_t z3 = std::min(stages / 3, (size_t)(slots / ((ends * (type == kQ6_K ? 0.5 : 0.8) + whole) * per_tile)));
+    const size_t z2 = std::min(stages / 2, (size_t)(0.875 * slots / ((ends + whole) * per_tile)));
+    size_t z = std::max<size_t>(1, std::min<size_t>(4, std::max(z3, z2)));
     if (c->tune_gemm_splitk > 0) z = std::min<size_t>((size_t)c->tune_gemm_splitk, stages);
     const size_t per_slice = (stages + z - 1) / z;
     return (int)((stages + per_slice - 1) / per_slice);   // (no empty slices)

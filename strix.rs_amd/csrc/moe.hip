@@ -1109,7 +1109,7 @@ static int moe_layer_impl(smx_ctx* c, size_t layer, const float* xs, size_t m, c
     std::vector<GemmTile> tiles_gu, tiles_dn;
     build_tiles(plan, nplan, L.eff, &tiles_gu);
     build_tiles(plan, nplan, hidden, &tiles_dn);
-    const int slices_gu = gemm_grouped_slices(c, hidden, tiles_gu.size(), 2);
+    const int slices_gu = gemm_grouped_slices(c, L.type, hidden, L.eff, L.ne, slots, 2);
     TableBlob tb;
     const size_t o_st = tb.add(slot_tok, slots * 4), o_ws = tb.add(wslot, slots * 4), o_tp = tb.add(tok_ptr.data(), (m + 1) * 4),
                  o_ts = tb.add(tok_slots.data(), slots * 4), o_t1 = tb.add(tiles_gu.data(), tiles_gu.size() * sizeof(GemmTile)),
@@ -1155,8 +1155,9 @@ static int moe_layer_impl(smx_ctx* c, size_t layer, const float* xs, size_t m, c
 // WeightAccel::moe_layer_ffn (accel.rs:238-246, decode.rs:3552-3629): xs holds the rows of every
 // expert group back to back (expert-major, already gathered by the caller), plan = (expert, rows)
 // pairs; returns the unweighted expert outputs dy[rows][hidden] for the caller's weighted scatter.
-int smx_moe_layer_ffn(smx_ctx* c, size_t layer, const int32_t* plan, size_t nplan, const float* xs, size_t rows, float* dy,
-                      size_t dy_cap) {
+// one_expert: the entry point for the rows of a single expert, whose K slices are chosen for one group.
+static int moe_layer_ffn_impl(smx_ctx* c, size_t layer, const int32_t* plan, size_t nplan, const float* xs, size_t rows, float* dy,
+                              size_t dy_cap, bool one_expert) {
     if (!c) return SMX_ERR_ARG;
     if (!plan || !xs || !dy) return fail(c, SMX_ERR_ARG, "moe_layer_ffn: null argument");
     return guarded(c, "moe_layer_ffn", [&]() -> int {
@@ -1184,7 +1185,7 @@ int smx_moe_layer_ffn(smx_ctx* c, size_t layer, const int32_t* plan, size_t npla
     std::vector<GemmTile> tiles_gu, tiles_dn;
     build_tiles(plan3.data(), nplan, L.eff, &tiles_gu);
     build_tiles(plan3.data(), nplan, hidden, &tiles_dn);
-    const int slices_gu = gemm_grouped_slices(c, hidden, tiles_gu.size(), 2);
+    const int slices_gu = gemm_grouped_slices(c, L.type, hidden, L.eff, one_expert ? 1 : L.ne, rows, 2);
     TableBlob tb;
     const size_t o_t1 = tb.add(tiles_gu.data(), tiles_gu.size() * sizeof(GemmTile)),
                  o_t2 = tb.add(tiles_dn.data(), tiles_dn.size() * sizeof(GemmTile));
@@ -1201,11 +1202,16 @@ int smx_moe_layer_ffn(smx_ctx* c, size_t layer, const int32_t* plan, size_t npla
     });
 }
 
+int smx_moe_layer_ffn(smx_ctx* c, size_t layer, const int32_t* plan, size_t nplan, const float* xs, size_t rows, float* dy,
+                      size_t dy_cap) {
+    return moe_layer_ffn_impl(c, layer, plan, nplan, xs, rows, dy, dy_cap, false);
+}
+
 // WeightAccel::moe_expert_ffn (accel.rs:220-223): one expert's FFN for m grouped rows, one sync.
 int smx_moe_expert_ffn(smx_ctx* c, size_t layer, size_t expert, const float* xs, size_t m, float* y, size_t y_cap) {
     if (expert > 0x7fffffffu || m > 0x7fffffffu) return c ? fail(c, SMX_ERR_ARG, "moe_expert_ffn: expert %zu, %zu rows", expert, m) : SMX_ERR_ARG;
     const int32_t plan[2] = {(int32_t)expert, (int32_t)m};
-    return smx_moe_layer_ffn(c, layer, plan, 1, xs, m, y, y_cap);
+    return moe_layer_ffn_impl(c, layer, plan, 1, xs, m, y, y_cap, true);
 }
 
 int smx_moe_layer(smx_ctx* c, size_t layer, const float* xs, size_t m, const size_t* plan, size_t nplan,

@@ -327,8 +327,9 @@ size_t skinny_xq_bytes(size_t m, size_t K);
 size_t skinny_xd_bytes(size_t m, size_t K);   // of sc.xd (block scales, piece-major)
 int launch_skinny(smx_ctx* c, const Weight& w, const float* x, size_t m, float* y, int32_t* dump, const ActScratch& sc);
 
-// K slices worth making of a grouped launch of ntiles * nops workgroups (the consumer adds up the planes they leave at op.out).
-int gemm_grouped_slices(const smx_ctx* c, size_t K, size_t ntiles, int nops);
+// K slices worth making of a grouped launch: `rows` rows in up to `groups` expert groups against nops weights [N][K] (the consumer adds
+// up the planes they leave at op.out).
+int gemm_grouped_slices(const smx_ctx* c, QType type, size_t K, size_t N, size_t groups, size_t rows, int nops);
 int launch_gemm_grouped(smx_ctx* c, QType type, const GemmArgs& args, int ntiles, int nops, int slices, const char* name);
 // the weight planes of w as a GEMM operand writing to out
 GemmOperand gemm_operand(const Weight& w, float* out);

@@ -161,6 +161,31 @@ def test_moe_layer_k_slices(accel, orc, synth, moe_stagewise, ty, ne, hidden, ef
     accel.tune("gemm_splitk", 0)
 
 
+@pytest.mark.parametrize("ty,ne,hidden,eff,m", [(8, 48, 1024, 256, 96), (14, 40, 1536, 256, 64)])
+def test_moe_layer_rows_do_not_depend_on_the_others(accel, synth, ty, ne, hidden, eff, m):
+    """The first rows of two calls of the same sizes are the same, with the same experts; the other rows go to all experts in
+    one call and to the same two in the other, which is a fifth of the tiles.  The first rows' results are the same bits."""
+    gate, up, down = (synth.make_moe_q8 if ty == 8 else synth.make_moe_q6)(ne, hidden, eff, seed=hidden)
+    assert (accel.upload_moe_q8 if ty == 8 else accel.upload_moe_q6)(19, gate, up, down, hidden, eff, ne)
+    few, w = 8, np.full((m, 2), 0.5, np.float32)
+    even = np.array([[(2 * t) % ne, (2 * t + 1) % ne] for t in range(m)], np.int32)
+    one = np.tile(np.array([[0, 1]], np.int32), (m, 1))
+    xa, xb = synth.make_acts(m, hidden, seed=23), synth.make_acts(m, hidden, seed=24)
+    xb[:few] = xa[:few]
+    one[:few] = even[:few]
+    plans = [synth.group_by_expert(ids, w, ne) for ids in (even, one)]
+    ya, yb = (accel.moe_layer_q8_dev(19, x, m, *p) for x, p in zip((xa, xb), plans))
+    assert np.array_equal(ya[:few], yb[:few])
+    outs = []   # the same through the expert-major call
+    for x, (plan, slot_tok, _) in zip((xa, xb), plans):
+        rows = np.ascontiguousarray(x[slot_tok])
+        dy = accel.moe_layer_ffn(19, [(int(e), int(n)) for e, _, n in np.asarray(plan).reshape(-1, 3)], rows, len(slot_tok))
+        outs.append({(int(t), int(e)): dy[o + i] for e, o, n in np.asarray(plan).reshape(-1, 3) for i, t in enumerate(np.asarray(slot_tok)[o:o + n])})
+    for t in range(few):
+        for e in even[t]:
+            assert np.array_equal(outs[0][t, int(e)], outs[1][t, int(e)]), (t, e)
+
+
 @pytest.mark.parametrize("ne,hidden,eff,k,m", [(4, 64, 32, 2, 5), (8, 256, 160, 3, 37), (16, 512, 256, 4, 300)])
 def test_moe_layer_matches_decode_path(accel, orc, synth, relerr, ne, hidden, eff, k, m):
     gate, up, down = _layer(accel, synth, 7, ne, hidden, eff, seed=hidden + m)
