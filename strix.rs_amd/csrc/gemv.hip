@@ -264,7 +264,7 @@ int launch_flat(smx_ctx* c, const Geom& g, const GemvJobs& J, int njobs, int nbl
         return launch_flat_fq<Ops, 1, PRE, GL, 1>(c, g, J, njobs, nblk, m);                          \
     }
         if constexpr (std::is_same<Ops, OpsQ4_0>::value || std::is_same<Ops, OpsQ8_0>::value) {
-            SMX_FLAT(3, 16) SMX_FLAT(3, 8) SMX_FLAT(2, 16) SMX_FLAT(4, 16) SMX_FLAT(3, kFlatLeast<Ops>)
+            SMX_FLAT(3, 16) SMX_FLAT(3, 8) SMX_FLAT(2, 16) SMX_FLAT(4, 16) SMX_FLAT(3, kFlatLeast<Ops>) SMX_FLAT(2, kFlatLeast<Ops>)
         } else if constexpr (kQ6) {
             SMX_FLAT(1, 16) SMX_FLAT(1, 8) SMX_FLAT(1, 4)
         }
@@ -368,6 +368,13 @@ static int pick_flat_pre(size_t units_per_wg) {
     if (L % 3 == 2) return 3;
     return L >= 7 ? 4 : 3;   // 7 = 4 + 3; a single load either way
 }
+// The same for the groups of 1 or 2 lanes: three loads where that is all a wave has, else two.  Cold, ten to fifteen GEMVs, 3 / 2 / 4 per
+// round: Q8_0 16000 x 992 (L = 4) 60.4 / 55.1 / 59.2 us, 60000 x 2016 (29) 42.7 / 40.5 / 43.1, 16000 x 1504 (6) 61.5 / 58.9 / 63.5; Q4_0
+// 16000 x 2016 (4) 38.3 / 35.1 / 37.3, 60000 x 4064 (30) 22.6 / 22.0 / 23.5, 60000 x 800 (6) 31.7 / 32.2 / 33.3; L = 3: Q4_0 16000 x 1504
+// 44.3 / 46.8 / 44.9, Q8_0 16000 x 544 44.5 / 44.7 / 44.6.  The row-per-wave form takes 58.9, 40.8, 65.8, 41.4, 24.0 and 38.0 on the first six.
+static int pick_flat_pre_least(size_t units_per_wg) {
+    return ((units_per_wg + 63) / 64 + 15) / 16 == 3 ? 3 : 2;
+}
 
 static Geom pick_geom(const smx_ctx* c, QType type, size_t N, size_t nblk, int mt, bool dump, int njobs) {
     Geom g;
@@ -454,6 +461,7 @@ static Geom pick_geom(const smx_ctx* c, QType type, size_t N, size_t nblk, int m
             // eight rows on Q8_0 2560 x 9728 14.1-14.6 / 14.8 / 15.8 us with 1 / 2 / 3
             g.flat_pre = type == kQ6_K ? 1 : (mt == 1 ? 3 : 1);
             if (mt == 1 && type != kQ6_K && g.flat == 16) g.flat_pre = pick_flat_pre(rows * units);
+            if (mt == 1 && type != kQ6_K && g.flat < 8) g.flat_pre = pick_flat_pre_least(rows * units);
             g.nt = 1024;
             g.grid = (unsigned)fwgs;
             g.lds = lds;
