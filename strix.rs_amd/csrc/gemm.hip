@@ -407,18 +407,26 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float4* __rest
     y[i] = s;
 }
 
+// Token tiles that are walked together (see launch_gemm): the largest divisor of their number up to 8.
+static int walk_group(int tiles_m) {
+    int gm = std::min(tiles_m, 8);
+    while (tiles_m % gm != 0) gm--;   // whole groups
+    return gm;
+}
+
 // Tile height and K slices.  The reference splits only the long-K shapes (in_dim >= 12288, decode.rs:5658) to fill its grid.  Here the
 // launch that is estimated to take least, among tiles of 64 (Q8_0, Q4_0), 128 and 256 tokens and every number of whole-stage slices
 // whose workgroups fit the chip's slots in ONE round (a second, partly filled round costs more than shorter slices save): a
 // workgroup's stages one after the other, at the time a stage takes with the CU to itself or shared with a second
-// workgroup and one more for its first loads, plus the launch that adds up the slices' partials, 2.3 us, 0.3 a slice and 5 MB of them per us
-// (without the one more and the 0.3, slices of a single stage: Q4_0 37 x 2816 x 2048 17.4 against 15.9 us, Q8_0 110 x 1104 x 1472 14.5 / 12.9).  Tiles that need several rounds: one
-// slice, 128 or 256 tokens, whichever's rounds take less.
+// workgroup and one more for its first loads, plus the launch that adds up the slices' partials, 1.9 us, 0.3 a slice and 5 MB of them per us.
+// Tiles that need several rounds: one slice, 128 or 256 tokens, whichever's rounds take less; there the first loads and the stores of
+// two workgroups on a CU hide behind each other's arithmetic (half a stage a round), those of one on its own do not (one and a half).
 // The stage times are measured (us): 64 tokens 1.05 alone / 1.46 shared, 128 tokens 1.55 / 2.7, Q6_K 2.75 / 4.3; 256 tokens (one workgroup
-// per CU) 2.35, Q6_K 3.85.  Over 200 shapes of 129..2048 tokens the choice takes 0.6 % more than the best of the three
-// heights, 11 % at worst.  Per call against a rule of at least 6 stages per slice and 128-token tiles: Q8_0 200 x 2560 x 2560 23.5 -> 19 us, 300 x 9728 x 2560 41.2 -> 36.8,
-// 333 x 2560 x 9728 43.8 -> 41.2 (Q4_0 44.5 -> 42.9), Q4_0 103 x 1088 x 1024 15.5 -> 12.0, Q6_K 72 x 2208 x 3328 28.9 -> 21.2, 600 x 2560 x
-// 2560 44.0 -> 37.5; Q8_0 500 and 1000 x 2560 x 9728 keep 128-token tiles (64: 52.8 for 52.1, 109 for 87.4).
+// per CU) 2.35, Q6_K 3.85.  Over 252 shapes of 65..2048 tokens (512..15360 rows and columns) the choice takes 0.7 % more than the best of
+// all heights and up to 16 slices, 15 % at worst (Q8_0 180 x 2384 x 15328: 44.0 us, twelve slices of one 256-token tile 38.4).  Constants fitted
+// to half of the shapes do no better on the other half.  The choice of 64- and 128-token tiles without the first loads takes 4.9 % more than
+// the best; it is ahead of this one by more than 2 % on three of 312 shapes: Q8_0 539 x 1264 x 960 (15.2 against 15.9), Q6_K 592 x 960 x 4096 (31.5 /
+// 32.8), Q4_0 134 x 1072 x 14464 (28.0 / 28.7).
 struct Tiling { int bm, slices; };
 static Tiling pick_tiling(int num_cu, bool q6, int M, int N, int nstages, bool split, int only) {
     Tiling best = {only ? only : 128, 1};
@@ -426,10 +434,13 @@ static Tiling pick_tiling(int num_cu, bool q6, int M, int N, int nstages, bool s
     for (int bm : {64, 128, 256}) {
         if (only ? bm != only : bm == 64 ? q6 || M <= 64 : bm == 128 ? !q6 && M > 64 && M <= 128 : M <= 128) continue;   // (65..128 tokens: as two rows of tiles)
         const int T = (M + bm - 1) / bm * ((N + BN - 1) / BN), slots = bm == 256 ? num_cu : 2 * num_cu;
-        // A last row of tiles of up to 32 tokens is over early: where the tiles are up to a tenth more than the CUs, its do not count as
-        // neighbours of the others (Q6_K 1565 x 2544 x 2816, 240 + 20 tiles of 128 tokens: 75 us, where 280 full ones take 97 and 140 of
-        // 256 tokens 92; 1289 x 3088 x 1024, 250 + 25: 34.7 against 39; but 648 x 6464 x 768, 255 + 51: 34.8 against 31.1)
-        const int light = bm == 128 && M > bm && M % bm != 0 && M % bm <= 32 && T <= num_cu + num_cu / 10 ? (N + BN - 1) / BN : 0;
+        // A last row of tiles of up to 64 tokens that is dispatched behind all others (tiles walked one row after the other, no remap over
+        // the XCDs) does not count as their neighbours where the rest fits the CUs: every wave of it has one or two row tiles and the
+        // tile is over early.  1536-long rows, 128- against 256-token tiles: Q6_K 13 rows of 20 tiles 46.4 / 55.5 us (last row of 8 tokens), 49.3 /
+        // 55.6 (64), 58.7 / 55.8 (128); 11 rows of 25 Q8_0 29.9 / 35.2 (8), 30.1 / 35.4 (64), 37.6 / 35.6 (128).  Walked in groups the row's tiles
+        // start among the others: 12 rows of 23 58.5 / 55.0 (8), 3 rows of 86 55.6 / 53.1.
+        const int tiles_m = (M + bm - 1) / bm, last = M - (tiles_m - 1) * bm;
+        const int light = bm == 128 && tiles_m > 1 && last <= 64 && walk_group(tiles_m) == 1 && T % 8 != 0 && T - T / tiles_m <= num_cu ? T / tiles_m : 0;
         const bool low = bm == 64 || M <= 64;
         const double alone = bm == 256 ? (q6 ? 3.85 : 2.35) : q6 ? 2.75 : low ? 1.05 : 1.55;
         const double shared = bm == 256 ? alone : q6 ? 4.3 : low ? 1.46 : 2.7;
@@ -438,7 +449,7 @@ static Tiling pick_tiling(int num_cu, bool q6, int M, int N, int nstages, bool s
             return n == 0 ? 0.0 : n <= num_cu ? alone : std::max(alone, shared * (0.93 + 0.07 * (n - num_cu) / num_cu));
         };
         if (T > slots) {   // whole rounds and the rest
-            const double us = (nstages + 1) * (T / slots * shared + stage(T % slots));
+            const double us = (nstages + (q6 ? 1.0 : bm == 256 ? 1.5 : 0.5)) * (T / slots * shared + stage(T % slots));
             if (bm >= 128 && us < least) {
                 least = us;
                 best = {bm, 1};
@@ -449,7 +460,7 @@ static Tiling pick_tiling(int num_cu, bool q6, int M, int N, int nstages, bool s
         for (int z = 1; z <= zmax; z++) {
             const int stages = (nstages + z - 1) / z;
             if (z > 1 && stages == (nstages + z - 2) / (z - 1)) continue;   // the same slices as with one fewer
-            const double us = (stages + 1) * stage(z == 1 ? T - light : T * z) + (z > 1 ? 2.3 + 0.3 * z + (double)z * M * N * 4 / 5e6 : 0.0);
+            const double us = (stages + 1) * stage(z == 1 ? T - light : T * z) + (z > 1 ? 1.9 + 0.3 * z + (double)z * M * N * 4 / 5e6 : 0.0);
             if (us < least) {
                 least = us;
                 best = {bm, z};
@@ -532,9 +543,11 @@ int launch_gemm(smx_ctx* c, const Weight& w, const int8_t* xq, const float* xd, 
     // of 8; groups of 4: 360 / 363 MB; of 1 (ffn_down): 947 MB.  The launch time does not move (the kernel is bound by
     // instruction issue, and these fetches are served by the Infinity Cache).
     {
-        int gm = std::min(p.tiles_m, 8);
-        if (c->tune_gemm_walk > 0) gm = std::max(1, p.tiles_m / c->tune_gemm_walk);
-        while (p.tiles_m % gm != 0) gm--;   // whole groups
+        int gm = walk_group(p.tiles_m);
+        if (c->tune_gemm_walk > 0) {
+            gm = std::max(1, p.tiles_m / c->tune_gemm_walk);
+            while (p.tiles_m % gm != 0) gm--;
+        }
         p.walk_gm = gm;
     }
     int Z = !may_split ? 1 : c->tune_gemm_splitk > 0 ? std::min(c->tune_gemm_splitk, nstages) : T <= slots ? std::min(tiling.slices, std::max(1, slots / T)) : 1;
