@@ -94,7 +94,7 @@ static int launch_argmax_rows(smx_ctx* c, const float* y, size_t m, size_t N, vo
 
 // quantise m device rows and run the right matmul kernel into y_dev
 // Which kernel serves m rows: the small-batch MFMA kernel for 5..64 rows (17 and more: weights of up to 32768 rows, 33 and more of a
-// Q6_K weight: 10240 and 40 Mi elements; skinny_serves); otherwise the dot4 GEMV up to SMX_GEMV_MAX_M rows (4 of a
+// Q6_K weight: up to 4096, of shorter rows up to 16384; skinny_serves); otherwise the dot4 GEMV up to SMX_GEMV_MAX_M rows (4 of a
 // Q6_K weight), the tiled GEMM beyond.
 }  // namespace
 

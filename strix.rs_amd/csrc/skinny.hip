@@ -472,9 +472,13 @@ bool skinny_serves(const Weight& w, size_t m) {
     // 17..32 rows of a very tall weight: the tiled GEMM is ahead (Q8_0 65536 x 3840 at 32 rows 61.6 against 70.7 us; at 16 rows
     // 58.3 / 61.8, at 8 rows the dot4 GEMV 68.2 / 57.6 us; 262144 x 2560: 174.5 / 169.6, 159.2 / 155.5, 171.6 / 139.0 us)
     if (m < SMX_SKINNY_MIN_M || m > SMX_SKINNY_MAX_M || w.K < 128) return false;
-    // 33..64 rows of a Q6_K weight, whose 32 accumulators are rescaled twice per block: 4096 x 4096 23 -> 12.7 us, 2560 x 9728 25.8 -> 21.8,
-    // 9728 x 2560 24.6 -> 22.5; but 6254 x 9216 37.2 -> 37.8, 15360 x 3840 35.6 -> 36.0, 32000 x 1792 34.2 -> 38.8
-    if (w.type == kQ6_K && m > 32) return w.N <= 10240 && w.N * w.K <= size_t(40) << 20;
+    // 33..64 rows of a Q6_K weight, whose 32 accumulators are rescaled twice per block: the more rounds of 256 workgroups of 32 weight rows
+    // (in two K slices), the shorter the rows up to which this kernel is ahead of the tiled one, which cuts K for itself.  Time of the tiled
+    // GEMM over this kernel's at 33 / 64 rows: one round (up to 4096 weight rows) 1.1-1.7 up to 12288 columns, 1.0 at 15360; two
+    // rounds (8192) 1.03 / 1.05 and up to 5120 columns 1.1, 0.97-1.0 / 1.0 at 6144, 0.87 at 9728; up to four (16384) 1.02 / 1.07 and up to 2560
+    // columns 1.1-1.3, 0.9-1.0 / 0.95-1.04 at 3072, 0.84 / 0.87 at 4096; beyond 0.74 (32768 x 512) to 1.07 (20480 x 1024).
+    if (w.type == kQ6_K && m > 32) return w.N <= 4096 || (w.N <= 8192 && w.K < 6144) || (w.N <= 16384 && w.K < 3072);
+    // (17..32 rows of a Q6_K weight: 1.16-1.9 up to 32768 weight rows)
     return m <= 16 || w.N <= 32768;
 }
 

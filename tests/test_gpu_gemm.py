@@ -181,7 +181,8 @@ def test_small_batch_any_block_count(accel, orc, synth, relerr, ty, N, K):
 
 # Q6_K beyond 16 rows: both sides of the weight heights up to which 17..32 and 33..64 rows run there, a ragged height, an odd number of
 # superblocks, outputs whose count is no multiple of 4 (one K slice)
-@pytest.mark.parametrize("N,K", [(10240, 256), (10241, 256), (32768, 256), (32769, 256), (77, 2304), (4097, 1024)])
+@pytest.mark.parametrize("N,K", [(10240, 256), (10241, 256), (32768, 256), (32769, 256), (77, 2304), (4097, 1024),
+                                 (16384, 512), (16385, 256), (4097, 5888), (4097, 6144), (8193, 2816), (8193, 3072)])
 def test_small_batch_q6k_beyond_16_rows(accel, orc, synth, relerr, N, K):
     raw = synth.make_weight(14, N, K, seed=N + K)
     assert accel.upload_q6_k("t.sb6", raw, K, N)
