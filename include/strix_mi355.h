@@ -271,8 +271,8 @@ void smx_graph_destroy(smx_ctx* ctx, smx_graph* g);
  * a kernel's launch, never which kernel a shape is served by.
  * Knobs: "gemm_splitk" (K slices of the GEMM and of the grouped gate and up products), "gemm_tile_m" (tokens per GEMM tile: 64, 128 or 256), "gemm_walk" (token-tile
  * groups of the GEMM's tile walk), "gemm_narrow" (1: every weight strip of the GEMM 128 rows; 1 + n: the first n strips 96 rows);
- * for rows of more than 16384 elements, which the row-per-wavefront GEMV serves: "gemv_rpw" (rows per wavefront: 1, 2, 4),
- * "gemv_ks" (wavefronts sharing a row: 1, 2, 4), "gemv_lpr" (lanes per row: 16, 32, 64), "gemv_wpc" (workgroups per CU);
+ * for rows of more than 16384 elements, which the row-per-wavefront GEMV serves: "gemv_ks" (wavefronts sharing a row: 1, 2, 4, of a
+ * single activation row), "gemv_wpc" (workgroups per CU); "gemv_rpw" (1, 2, 4) and "gemv_lpr" (16, 32, 64) are taken and have no effect;
  * "host_io" (host-pointer GEMV calls: 0 = the kernels read and write the context's
  * pinned staging buffers themselves where that is the rule, 1 = a copy command each way, 2 = a copy command in, the result
  * written by the kernel).  Results do not depend on them beyond fp32 summation order. */

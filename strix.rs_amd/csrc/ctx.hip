@@ -594,14 +594,12 @@ int smx_tune(smx_ctx* c, const char* knob, int value) {
     if (value < 0) return fail(c, SMX_ERR_ARG, "tune: negative value for %s", knob);
     const std::string k = knob;
     if (k == "gemv_rpw") {
-        if (value != 0 && value != 1 && value != 2 && value != 4) return fail(c, SMX_ERR_ARG, "tune: gemv_rpw must be 0, 1, 2 or 4");
-        c->tune_gemv_rpw = value;
+        if (value != 0 && value != 1 && value != 2 && value != 4) return fail(c, SMX_ERR_ARG, "tune: gemv_rpw must be 0, 1, 2 or 4");   // (no variants left to choose from)
     } else if (k == "gemv_ks") {
         if (value != 0 && value != 1 && value != 2 && value != 4) return fail(c, SMX_ERR_ARG, "tune: gemv_ks must be 0, 1, 2 or 4");
         c->tune_gemv_ks = value;
     } else if (k == "gemv_lpr") {
-        if (value != 0 && value != 16 && value != 32 && value != 64) return fail(c, SMX_ERR_ARG, "tune: gemv_lpr must be 0, 16, 32 or 64");
-        c->tune_gemv_lpr = value;
+        if (value != 0 && value != 16 && value != 32 && value != 64) return fail(c, SMX_ERR_ARG, "tune: gemv_lpr must be 0, 16, 32 or 64");   // (the same)
     } else if (k == "gemv_wpc") {
         if (value > 32) return fail(c, SMX_ERR_ARG, "tune: gemv_wpc must be 0..32");
         c->tune_gemv_wpc = value;

@@ -173,23 +173,28 @@ namespace {
 // Row length from which silu / gelu producers run in their own launch (measured on 2560 <- 9728).
 constexpr size_t kProducerSplitK = 4096;
 
-// Launch geometry: slots per wave, pipeline depth, K-split, lanes per row, threads per workgroup.
+// Launch geometry: rows per wave, K-split, lanes per row, threads per workgroup.
 struct Geom {
     bool prod = false;  // an activation producer runs in the staging
     bool preq = false;  // the (single) activation row arrives quantised
     bool rowsf = false; // 2..4 fp32 activation rows are quantised inside the flat kernel
     int flat = 0;       // flat form: lanes per group (16, 8 or kFlatLeast), 0 = not used
     int flat_pre = 0;   // its loads per round
-    int rpw, pre, ks, lpr, nt;
+    int rpw, ks, lpr, nt;
     unsigned grid;
     size_t lds;
 };
 
+// Experts chosen on the device: Q8_0 and Q6_K layers, one fp32 row per job; an activation producer (the down projections of a Q6_K
+// layer) runs in the staging on rows of the flat form only.
+template <class Ops, int MT, int FQ, bool DUMP, bool FLAT>
+constexpr bool kRouted = MT == 1 && !DUMP && (FQ == 1 ? !std::is_same<Ops, OpsQ4_0>::value : FQ == 2 && FLAT && std::is_same<Ops, OpsQ6_K>::value);
+
 template <class Ops, int MT, int RPW, int PRE, int KS, int LPR, int FQ, bool DUMP, int NT>
 int launch_fq(smx_ctx* c, const Geom& g, const GemvJobs& J, int njobs, int nblk, int m, int* dump, int dump_per_row) {
     auto k = gemv_kernel<Ops, MT, RPW, PRE, KS, LPR, FQ, DUMP, NT>;
-    if (J.ids) {   // experts chosen on the device: one fp32 activation row per job, no dump
-        if constexpr (MT == 1 && FQ != 0 && !DUMP) k = gemv_kernel<Ops, MT, RPW, PRE, KS, LPR, FQ, DUMP, NT, true>;
+    if (J.ids) {
+        if constexpr (kRouted<Ops, MT, FQ, DUMP, false>) k = gemv_kernel<Ops, MT, RPW, PRE, KS, LPR, FQ, DUMP, NT, true>;
         else return fail(c, SMX_ERR_ARG, "gemv: device-routed experts take one fp32 activation row per job");
     }
     int rc = set_dyn_lds(c, k, g.lds);
@@ -232,8 +237,8 @@ int launch_flat_fq(smx_ctx* c, const Geom& g, const GemvJobs& J, int njobs, int 
     }
     if constexpr (MT == 1) {
         auto k = gemv_flat_kernel<Ops, MT, PRE, GL, FQ, DUMP>;
-        if (J.ids) {   // experts chosen on the device: one fp32 activation row per job, no dump
-            if constexpr (FQ != 0 && !DUMP) k = gemv_flat_kernel<Ops, MT, PRE, GL, FQ, DUMP, true>;
+        if (J.ids) {
+            if constexpr (kRouted<Ops, MT, FQ, DUMP, true>) k = gemv_flat_kernel<Ops, MT, PRE, GL, FQ, DUMP, true>;
             else return fail(c, SMX_ERR_ARG, "gemv: device-routed experts take one fp32 activation row per job");
         }
         int rc = set_dyn_lds(c, k, g.lds);
@@ -303,50 +308,58 @@ int launch_flat(smx_ctx* c, const Geom& g, const GemvJobs& J, int njobs, int nbl
     return fail(c, SMX_ERR_ARG, "gemv: no flat variant for this geometry");
 }
 
-// The compiled variants (RPW, PRE, KS, LPR):
-//   whole-wave rows   (4,2,1,64) (2,2,1,64) (1,4,1,64) (1,2,2,64) (1,2,4,64)
-//   sub-wave rows     (2,2,1,32) (1,2,1,32) (2,2,1,16) (1,2,1,16)        [one activation row only]
+// The row-per-wave variants (RPW, PRE, KS, LPR) and what they serve:
+//   (1,4,1,64) (1,2,2,64) (1,2,4,64)  rows of more than 16384 elements, the last two one activation row over few weight rows
+//   (1,4,1,64)                        eight activation rows over units that are no multiple of 8, or too long for the flat form's LDS
+//   (2,2,1,64)                        2..4 activation rows over rows of one unit
+//   (1,6,1,16) (2,3,1,16)             one activation row over such rows, which are Q4_0's of 32 elements (Q8_0 has two units in them)
 template <class Ops, int MT>
 int launch_variant(smx_ctx* c, const Geom& g, const GemvJobs& J, int njobs, int nblk, int m) {
-    // sub-wave rows: the pipeline is deep enough to put a whole short row set in flight before the
-    // activation is staged (Q6_K units are three times as wide, so half the depth)
     constexpr bool kWide = sizeof(typename Ops::Regs) > 32;
     if (g.flat) return launch_flat<Ops, MT>(c, g, J, njobs, nblk, m);
-    if (MT == 1 && g.lpr == 32) {
-        if (g.rpw == 2) return launch_one<Ops, 1, 2, kWide ? 2 : 3, 1, 32, false, 1024>(c, g, J, njobs, nblk, m, nullptr, 0);
-        return launch_one<Ops, 1, 1, kWide ? 2 : 4, 1, 32, false, 1024>(c, g, J, njobs, nblk, m, nullptr, 0);
+    if constexpr (MT == 3) return fail(c, SMX_ERR_ARG, "gemv: no variant for three rows of this geometry");   // (see launch_gemv)
+    else {
+        if constexpr (MT == 1) {
+            if constexpr (std::is_same<Ops, OpsQ4_0>::value) {
+                if (g.lpr == 16 && g.rpw == 2) return launch_one<Ops, 1, 2, 3, 1, 16, false, 1024>(c, g, J, njobs, nblk, m, nullptr, 0);
+                if (g.lpr == 16) return launch_one<Ops, 1, 1, 6, 1, 16, false, 1024>(c, g, J, njobs, nblk, m, nullptr, 0);
+            }
+            if (g.ks == 4) return launch_one<Ops, 1, 1, 2, 4, 64, false, 1024>(c, g, J, njobs, nblk, m, nullptr, 0);
+            if (g.ks == 2) return launch_one<Ops, 1, 1, 2, 2, 64, false, 1024>(c, g, J, njobs, nblk, m, nullptr, 0);
+        } else if constexpr (MT <= 4 && !kWide) {
+            if (g.rpw == 2) return launch_one<Ops, MT, 2, 2, 1, 64, false, 1024>(c, g, J, njobs, nblk, m, nullptr, 0);
+        }
+        // 8 activation rows (4 with Q6_K's wide units): a ring of 4 units spills (128 registers per lane at
+        // 16 waves), and the scratch traffic costs more than the shallower pipeline: 2 fit
+        return launch_one<Ops, MT, 1, (MT == 8 || (kWide && MT == 4)) ? 2 : 4, 1, 64, false, 1024>(c, g, J, njobs, nblk, m, nullptr, 0);
     }
-    if (MT == 1 && g.lpr == 16) {
-        if (g.rpw == 2) return launch_one<Ops, 1, 2, kWide ? 2 : 3, 1, 16, false, 1024>(c, g, J, njobs, nblk, m, nullptr, 0);
-        return launch_one<Ops, 1, 1, kWide ? 4 : 6, 1, 16, false, 1024>(c, g, J, njobs, nblk, m, nullptr, 0);
-    }
-    if (g.ks == 4) return launch_one<Ops, MT, 1, 2, 4, 64, false, 1024>(c, g, J, njobs, nblk, m, nullptr, 0);
-    if (g.ks == 2) return launch_one<Ops, MT, 1, 2, 2, 64, false, 1024>(c, g, J, njobs, nblk, m, nullptr, 0);
-    // 8 activation rows (4 with Q6_K's wide units): a ring of 4 units spills (128 registers per lane at
-    // 16 waves), and the scratch traffic costs more than the shallower pipeline: 2 fit
-    constexpr int kPre1 = (MT == 8 || (kWide && MT == 4)) ? 2 : 4;
-    if (g.rpw == 1) return launch_one<Ops, MT, 1, kPre1, 1, 64, false, 1024>(c, g, J, njobs, nblk, m, nullptr, 0);
-    if (g.rpw == 4 && MT == 1) return launch_one<Ops, 1, 4, 2, 1, 64, false, 1024>(c, g, J, njobs, nblk, m, nullptr, 0);
-    return launch_one<Ops, MT, 2, 2, 1, 64, false, 1024>(c, g, J, njobs, nblk, m, nullptr, 0);
 }
 
+// mt: rows the kernel is compiled for.  Half blocks of Q8_0 serve one and two rows, whole blocks three and more (launch_jobs); Q6_K
+// has four at most.
 template <class Ops>
 int launch_type(smx_ctx* c, const Geom& g, const GemvJobs& J, int njobs, int nblk, int m, int mt,
                 int* dump, int dump_per_row) {
-    if (dump && g.flat) return launch_flat<Ops, 1>(c, g, J, njobs, nblk, m, dump, dump_per_row);
-    if (dump) {
-        if (g.lpr == 16) return launch_one<Ops, 1, 1, 2, 1, 16, true, 256>(c, g, J, njobs, nblk, m, dump, dump_per_row);
-        return launch_one<Ops, 1, 1, 4, 1, 64, true, 256>(c, g, J, njobs, nblk, m, dump, dump_per_row);
+    constexpr bool kHalf = std::is_same<Ops, OpsQ8_0>::value, kWhole = std::is_same<Ops, OpsQ8_0W>::value, kQ6 = std::is_same<Ops, OpsQ6_K>::value;
+    if constexpr (!kWhole) {
+        if (dump && g.flat) return launch_flat<Ops, 1>(c, g, J, njobs, nblk, m, dump, dump_per_row);
+        if (dump) {
+            if constexpr (std::is_same<Ops, OpsQ4_0>::value) {
+                if (g.lpr == 16) return launch_one<Ops, 1, 1, 2, 1, 16, true, 256>(c, g, J, njobs, nblk, m, dump, dump_per_row);
+            }
+            return launch_one<Ops, 1, 1, 4, 1, 64, true, 256>(c, g, J, njobs, nblk, m, dump, dump_per_row);
+        }
+        if (mt == 1) return launch_variant<Ops, 1>(c, g, J, njobs, nblk, m);
+        if (mt == 2) return launch_variant<Ops, 2>(c, g, J, njobs, nblk, m);
     }
-    switch (mt) {
-        case 1: return launch_variant<Ops, 1>(c, g, J, njobs, nblk, m);
-        case 2: return launch_variant<Ops, 2>(c, g, J, njobs, nblk, m);
-        case 3:   // the flat form only (see launch_gemv)
-            if (g.flat) return launch_flat<Ops, 3>(c, g, J, njobs, nblk, m);
-            return fail(c, SMX_ERR_ARG, "gemv: no variant for three rows of this geometry");
-        case 4: return launch_variant<Ops, 4>(c, g, J, njobs, nblk, m);
-        default: return launch_variant<Ops, 8>(c, g, J, njobs, nblk, m);
+    if constexpr (!kHalf) {
+        if (mt == 3) return launch_variant<Ops, 3>(c, g, J, njobs, nblk, m);
+        if (mt == 4) return launch_variant<Ops, 4>(c, g, J, njobs, nblk, m);
+        if constexpr (!kQ6) {
+            if (mt == 8) return launch_variant<Ops, 8>(c, g, J, njobs, nblk, m);
+        }
     }
+    return fail(c, SMX_ERR_ARG, "gemv: no variant for %d rows of this weight", mt);
 }
 
 }  // namespace
@@ -385,39 +398,22 @@ static Geom pick_geom(const smx_ctx* c, QType type, size_t N, size_t nblk, int m
     g.nt = 1024;
     g.lpr = 64;
     g.ks = 1;
+    g.rpw = 1;
     const size_t cus = std::max<size_t>(1, (size_t)c->num_cu / njobs);  // this job's share of the chip
     const size_t waves = cus * 16;
-    if (mt == 1 && units == 1) g.lpr = 16;   // the only short rows that come here: four to a wave
-    if (c->tune_gemv_lpr > 0 && mt == 1) g.lpr = c->tune_gemv_lpr;
-    const int P = (int)((units + g.lpr - 1) / g.lpr);
-    if (g.lpr == 64) {
-        // K-split pays for a single activation row only (batched rows are bound by their own arithmetic)
-        if (mt == 1 && P >= 4 && N * 2 <= waves) g.ks = (P >= 8 && N * 4 <= waves) ? 4 : 2;
-        else if (mt == 1 && P >= 4 && N <= waves) g.ks = 2;  // more wave-tasks than one round of waves: extra workgroups queue
-        if (g.ks > 1) { g.rpw = 1; g.pre = 2; }
-        else if (P >= 4) { g.rpw = 1; g.pre = 4; }
-        else if (mt == 1 && type != kQ6_K && P <= 2 && N >= waves * 4) { g.rpw = 4; g.pre = 2; }
-        else { g.rpw = 2; g.pre = 2; }
-        if (c->tune_gemv_rpw > 0 || c->tune_gemv_ks > 0) {
-            const int ks = c->tune_gemv_ks > 0 ? c->tune_gemv_ks : 1;
-            const int rpw = c->tune_gemv_rpw > 0 ? c->tune_gemv_rpw : 1;
-            if (ks > 1) { g.ks = ks; g.rpw = 1; g.pre = 2; }
-            else if (rpw == 1) { g.ks = 1; g.rpw = 1; g.pre = 4; }
-            else if (rpw == 4 && mt == 1) { g.ks = 1; g.rpw = 4; g.pre = 2; }
-            else { g.ks = 1; g.rpw = 2; g.pre = 2; }
-        }
-        // register budget of the 16-wave workgroup (128 VGPRs): Q6_K units are wide, batched rows multiply accumulators
-        if (g.ks == 1 && g.rpw > 1 && ((type == kQ6_K && (g.rpw > 2 || mt > 1)) || mt == 8)) {
-            g.rpw = (type == kQ6_K && mt == 1) ? 2 : 1;
-            g.pre = g.rpw == 1 ? 4 : 2;
-        }
-    } else {
-        const size_t rows_per_slot = 64 / g.lpr;
-        g.pre = 2;
-        g.rpw = (N / rows_per_slot >= waves * 2 && type != kQ6_K) ? 2 : 1;
-        if (c->tune_gemv_rpw > 0) g.rpw = c->tune_gemv_rpw >= 2 && type != kQ6_K ? 2 : 1;
+    if (mt == 1 && units == 1) {   // the only short rows that come here: four to a wave
+        g.lpr = 16;
+        if (!dump && N / 4 >= waves * 2) g.rpw = 2;
+    } else if (mt == 1) {
+        const int P = (int)((units + 63) / 64);
+        if (P >= 4 && N * 2 <= waves) g.ks = (P >= 8 && N * 4 <= waves) ? 4 : 2;
+        else if (P >= 4 && N <= waves) g.ks = 2;  // more wave-tasks than one round of waves: extra workgroups queue
+        if (c->tune_gemv_ks > 0) g.ks = c->tune_gemv_ks;
+        if (dump) g.ks = 1;
+    } else if (mt <= 4 && units == 1) {
+        g.rpw = 2;
     }
-    if (dump) { g.rpw = 1; g.pre = g.lpr == 16 ? 2 : 4; g.ks = 1; g.nt = 256; if (g.lpr == 32) g.lpr = 64; }
+    if (dump) g.nt = 256;
     const int nw = g.nt / 64;
     const size_t rc = (size_t)g.rpw * (64 / g.lpr);
     g.lds = tokb * (size_t)mt + (g.ks > 1 ? (size_t)nw * rc * mt * 4 : 0);
@@ -665,10 +661,14 @@ int launch_gemv_dual(smx_ctx* c, const Weight* const* wg, const Weight* const* w
         *served = true;
         return SMX_OK;
     };
+    if (ind && w0.type == kQ4_0) return fail(c, SMX_ERR_ARG, "paired gemv: expert layers are Q8_0 or Q6_K");
 #define SMX_DUAL(OPS, PRE, GL)                                                                                  \
-    if (g.flat_pre == PRE && g.flat == GL)                                                                      \
-        return ind ? (ind->logits ? go(gemv_flat_dual_kernel<OPS, PRE, GL, 1, 2>) : go(gemv_flat_dual_kernel<OPS, PRE, GL, 1, 1>)) \
-                   : (norm ? go(gemv_flat_dual_kernel<OPS, PRE, GL, 2>) : go(gemv_flat_dual_kernel<OPS, PRE, GL, 1>));
+    if (g.flat_pre == PRE && g.flat == GL) {                                                                    \
+        if constexpr (!std::is_same<OPS, OpsQ4_0>::value) {                                                     \
+            if (ind) return ind->logits ? go(gemv_flat_dual_kernel<OPS, PRE, GL, 1, 2>) : go(gemv_flat_dual_kernel<OPS, PRE, GL, 1, 1>); \
+        }                                                                                                       \
+        return norm ? go(gemv_flat_dual_kernel<OPS, PRE, GL, 2>) : go(gemv_flat_dual_kernel<OPS, PRE, GL, 1>);  \
+    }
     if (w0.type == kQ4_0) { SMX_DUAL(OpsQ4_0, 3, 16) SMX_DUAL(OpsQ4_0, 3, 8) SMX_DUAL(OpsQ4_0, 2, 16) SMX_DUAL(OpsQ4_0, 4, 16) }
     else if (w0.type == kQ8_0) { SMX_DUAL(OpsQ8_0, 3, 16) SMX_DUAL(OpsQ8_0, 3, 8) SMX_DUAL(OpsQ8_0, 2, 16) SMX_DUAL(OpsQ8_0, 4, 16) }
     else { SMX_DUAL(OpsQ6_K, 1, 16) SMX_DUAL(OpsQ6_K, 1, 8) SMX_DUAL(OpsQ6_K, 1, 4) }

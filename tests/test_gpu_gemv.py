@@ -215,7 +215,7 @@ def test_gemv_rows_long_k_batched(accel, orc, synth, relerr):
 # activation loaded before the weights (257 blocks), the longest such row (511 blocks), several rounds of workgroups, fewer rows
 # than compute units; rows of one unit and longer ones stay with the row-per-wave kernel
 @pytest.mark.parametrize("ty,N,K", [(2, 3001, 64), (2, 700, 32 * 63), (2, 3000, 32 * 65), (8, 300, 32 * 33), (8, 70, 32 * 127), (2, 7, 32 * 257),
-                                    (8, 1500, 32 * 511), (2, 2500, 32 * 511), (8, 3001, 96), (2, 3001, 32), (8, 3001, 32), (2, 300, 32 * 513),
+                                    (8, 1500, 32 * 511), (2, 2500, 32 * 511), (8, 3001, 96), (2, 3001, 32), (2, 33001, 32), (8, 3001, 32), (2, 300, 32 * 513),
                                     # two loads a round over four, five and six loads of a wave, the last round whole, single or cut; and three
                                     (8, 16000, 992), (8, 16000, 1056), (2, 16000, 2016), (8, 16000, 1504), (2, 16000, 1504)])
 def test_gemv_rows_of_any_block_count(accel, orc, synth, relerr, ty, N, K):
