@@ -185,17 +185,17 @@ struct Geom {
     size_t lds;
 };
 
-// Experts chosen on the device: Q8_0 and Q6_K layers, one fp32 row per job; an activation producer (the down projections of a Q6_K
-// layer) runs in the staging on rows of the flat form only.
+// Experts chosen on the device: Q8_0 and Q6_K layers, one row per job.  The down projections of a Q6_K layer have an activation producer
+// in front: in the staging on rows of the flat form, or, from kProducerSplitK on, in a launch that leaves the rows quantised.
 template <class Ops, int MT, int FQ, bool DUMP, bool FLAT>
-constexpr bool kRouted = MT == 1 && !DUMP && (FQ == 1 ? !std::is_same<Ops, OpsQ4_0>::value : FQ == 2 && FLAT && std::is_same<Ops, OpsQ6_K>::value);
+constexpr bool kRouted = MT == 1 && !DUMP && (FQ == 1 ? !std::is_same<Ops, OpsQ4_0>::value : std::is_same<Ops, OpsQ6_K>::value && (FQ == 0 || FLAT));
 
 template <class Ops, int MT, int RPW, int PRE, int KS, int LPR, int FQ, bool DUMP, int NT>
 int launch_fq(smx_ctx* c, const Geom& g, const GemvJobs& J, int njobs, int nblk, int m, int* dump, int dump_per_row) {
     auto k = gemv_kernel<Ops, MT, RPW, PRE, KS, LPR, FQ, DUMP, NT>;
     if (J.ids) {
         if constexpr (kRouted<Ops, MT, FQ, DUMP, false>) k = gemv_kernel<Ops, MT, RPW, PRE, KS, LPR, FQ, DUMP, NT, true>;
-        else return fail(c, SMX_ERR_ARG, "gemv: device-routed experts take one fp32 activation row per job");
+        else return fail(c, SMX_ERR_ARG, "gemv: no device-routed variant of this form");
     }
     int rc = set_dyn_lds(c, k, g.lds);
     if (rc != SMX_OK) return rc;
@@ -239,7 +239,7 @@ int launch_flat_fq(smx_ctx* c, const Geom& g, const GemvJobs& J, int njobs, int 
         auto k = gemv_flat_kernel<Ops, MT, PRE, GL, FQ, DUMP>;
         if (J.ids) {
             if constexpr (kRouted<Ops, MT, FQ, DUMP, true>) k = gemv_flat_kernel<Ops, MT, PRE, GL, FQ, DUMP, true>;
-            else return fail(c, SMX_ERR_ARG, "gemv: device-routed experts take one fp32 activation row per job");
+            else return fail(c, SMX_ERR_ARG, "gemv: no device-routed variant of this form");
         }
         int rc = set_dyn_lds(c, k, g.lds);
         if (rc != SMX_OK) return rc;

@@ -345,6 +345,25 @@ def test_moe_decode_graph_serves_each_tokens_own_routing(accel, orc, synth, ty):
     assert accel.moe_ffn_routed_dev(999, idd, wd, k, xd, yd) is False
 
 
+@pytest.mark.parametrize("ne,hidden,eff,k", [(6, 256, 4096, 5), (6, 256, 3840, 5), (3, 256, 16640, 2)])
+def test_moe_ffn_routed_long_inner_rows(accel, synth, ne, hidden, eff, k):
+    """Q6_K experts whose k inner rows are too long for one workgroup's LDS run their down projections as a grouped GEMV, from
+    4096 elements on behind a quantiser launch of its own: the device-routed call has the host-routed one's bits."""
+    gate, up, down = synth.make_moe_q6(ne, hidden, eff, seed=eff)
+    assert accel.upload_moe_q6(46, gate, up, down, hidden, eff, ne)
+    x = synth.make_acts(1, hidden, seed=7)[0]
+    ids, w = synth.zipf_routing(1, ne, k, seed=8)
+    want = accel.moe_ffn(46, ids[0], w[0], x)
+    xd, yd, idd, wd = (accel.dev_alloc(n * 4) for n in (hidden, hidden, k, k))
+    accel.h2d(xd, x)
+    accel.h2d(idd, ids[0])
+    accel.h2d(wd, w[0])
+    assert accel.moe_ffn_routed_dev(46, idd, wd, k, xd, yd)
+    assert np.array_equal(accel.d2h(np.empty(hidden, np.float32), yd), want)
+    for p in (xd, yd, idd, wd):
+        accel.dev_free(p)
+
+
 @pytest.mark.parametrize("ty,ne,hidden,eff,k", [(8, 64, 2048, 768, 8), (8, 16, 512, 256, 4), (14, 16, 512, 256, 4), (8, 64, 512, 256, 12),
                                                 (8, 128, 256, 128, 6), (8, 8, 256, 96, 2), (8, 5, 256, 64, 5)])
 def test_moe_ffn_from_router_logits(accel, orc, synth, ty, ne, hidden, eff, k):
