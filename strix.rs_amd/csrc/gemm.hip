@@ -471,19 +471,24 @@ static Tiling pick_tiling(int num_cu, bool q6, int M, int N, int nstages, bool s
 }
 
 template <class Kernel>
-static int launch_gemm_variant(smx_ctx* c, Kernel k, size_t lds, const GemmArgs& p, dim3 grid, int nw = NW) {
+static int launch_gemm_variant(smx_ctx* c, Kernel k, size_t lds, const GemmArgs& p, dim3 grid, int nw) {
     int rc = set_dyn_lds(c, k, lds);
     if (rc != SMX_OK) return rc;
     hipLaunchKernelGGL(k, grid, dim3(64 * nw), lds, c->stream, p);
     SMX_HIP(c, hipGetLastError());
     return SMX_OK;
 }
+// The kernel of a format and tile height, with or without the block dots written out.
+template <int WAVES>
+static int launch_gemm_waves(smx_ctx* c, QType type, bool dump, const GemmArgs& p, dim3 grid) {
+    const size_t lds = type == kQ6_K ? q6_lds_bytes(WAVES) : 2 * stage_bytes(WAVES);
+    const auto go = [&](auto kern) { return launch_gemm_variant(c, kern, lds, p, grid, WAVES); };
+    if (type == kQ6_K) return dump ? go(gemm_q6_kernel<true, WAVES>) : go(gemm_q6_kernel<false, WAVES>);
+    if (type == kQ4_0) return dump ? go(gemm_i8_kernel<true, true, WAVES>) : go(gemm_i8_kernel<true, false, WAVES>);
+    return dump ? go(gemm_i8_kernel<false, true, WAVES>) : go(gemm_i8_kernel<false, false, WAVES>);
+}
 static int launch_gemm_type(smx_ctx* c, QType type, bool dump, const GemmArgs& p, dim3 grid) {
-    if (type == kQ6_K && p.tile_m == 256) return launch_gemm_variant(c, gemm_q6_kernel<false, 8>, q6_lds_bytes(8), p, grid, 8);
-    if (type == kQ6_K) return launch_gemm_variant(c, dump ? gemm_q6_kernel<true, NW> : gemm_q6_kernel<false, NW>, q6_lds_bytes(NW), p, grid);
-    if (p.tile_m == 256) return launch_gemm_variant(c, type == kQ4_0 ? gemm_i8_kernel<true, false, 8> : gemm_i8_kernel<false, false, 8>, 2 * stage_bytes(8), p, grid, 8);
-    if (type == kQ4_0) return launch_gemm_variant(c, dump ? gemm_i8_kernel<true, true, NW> : gemm_i8_kernel<true, false, NW>, 2 * stage_bytes(NW), p, grid);
-    return launch_gemm_variant(c, dump ? gemm_i8_kernel<false, true, NW> : gemm_i8_kernel<false, false, NW>, 2 * stage_bytes(NW), p, grid);
+    return p.tile_m == 256 ? launch_gemm_waves<8>(c, type, dump, p, grid) : launch_gemm_waves<NW>(c, type, dump, p, grid);
 }
 
 GemmOperand gemm_operand(const Weight& w, float* out) {
@@ -523,8 +528,7 @@ int launch_gemm(smx_ctx* c, const Weight& w, const int8_t* xq, const float* xd, 
     p.tiles_n = (p.N + BN - 1) / BN;
     const int nstages = (p.nb + KB - 1) / KB;
     const bool may_split = dump == nullptr && (m * w.N) % 4 == 0;
-    // (the kernels that write the block dots out have four waves)
-    const int only = c->tune_gemm_tile_m == 256 && dump ? 128 : c->tune_gemm_tile_m != 0 ? c->tune_gemm_tile_m : dump && p.M > 128 ? 128 : 0;
+    const int only = c->tune_gemm_tile_m;
     const Tiling tiling = pick_tiling(c->num_cu, w.type == kQ6_K, p.M, p.N, nstages, may_split && c->tune_gemm_splitk == 0, only);
     // 65..128 tokens are always two rows of 64-token tiles (in one row of 128 half the waves of a workgroup may idle): Q8_0
     // 2560 x 9728 and 9728 x 2560 at 96 / 128 tokens 28.2 / 29.4 -> 25.4 / 26.7 us and 25.9 / 27.3 -> 22.9 / 24.7 us.

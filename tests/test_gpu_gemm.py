@@ -294,3 +294,23 @@ def test_gemm_wide_tiles(accel, orc, synth, relerr, ty, m, N, K):
         for knob in ("gemm_tile_m", "gemm_splitk", "gemm_narrow"):
             accel.tune(knob, 0)
     accel.evict("t.wide")
+
+
+@pytest.mark.parametrize("ty", [14, 8, 2])
+@pytest.mark.parametrize("m,N,K", [(257, 130, 256), (300, 97, 1280)])
+def test_gemm_wide_tile_block_dots(accel, orc, synth, ty, m, N, K):
+    """The integers of 256-token tiles: a last tile of one token, waves without tokens, strips of one to four row tiles."""
+    if ty != 14:
+        K += 96   # a stage of three blocks
+    raw = synth.make_weight(ty, N, K, seed=N)
+    xs = synth.make_acts(m, K, seed=m)
+    assert getattr(accel, UPLOAD[ty])("t.wd", raw, K, N)
+    xq, _, _ = orc.actquant(xs, K)
+    try:
+        accel.tune("gemm_tile_m", 256)
+        dots = accel.gemm_block_dots("t.wd", xs, m, N, K // (16 if ty == 14 else 32))
+    finally:
+        accel.tune("gemm_tile_m", 0)
+    for t in (0, 31, 32, 127, 128, 255, 256, m - 1):
+        assert np.array_equal(dots[t], orc.block_dots(ty, raw, K, N, xq[t])), t
+    accel.evict("t.wd")
