@@ -558,45 +558,42 @@ int launch_gemm(smx_ctx* c, const Weight& w, const int8_t* xq, const float* xd, 
     p.stages_per_slice = (nstages + Z - 1) / Z;
     Z = (nstages + p.stages_per_slice - 1) / p.stages_per_slice;
     // Mixed strips.  When the tiles need several rounds of the chip's workgroup slots and the last round is partly filled,
-    // its idle slots cost up to a whole tile's time.  A tile of 96 weight rows runs three of the four row tiles (about 0.8
+    // its idle slots cost up to a whole tile's time.  A Q6_K tile of 96 weight rows runs three of the four row tiles (about 0.8
     // of the time), so with the first `narrow` strips of N cut at 96 rows and dispatched last, the last round can be made
-    // of shorter tiles on more slots: 15360 rows x 2048 tokens = 1920 tiles = 3.75 rounds of 512 becomes 1536 tiles of
-    // 128 rows (3 rounds) and one round of 512 tiles of 96.  Chosen by the estimated makespan; taken when it saves 3 %, for
-    // Q6_K weights only: measured at that shape Q6_K 598 -> 575 us per launch, Q8_0 339.6 -> 337 and Q4_0 350.7 -> 349 (inside
-    // the spread between machines, with 2.5 % more vector instructions per launch: a partly filled round runs faster
-    // already, a workgroup alone on a CU has its SIMDs to itself).  The knob forces any number of strips for any format.
+    // of shorter tiles on more slots: 15360 rows x 2048 tokens = 960 tiles of 256 tokens = 3.75 rounds of 256 becomes 768 tiles of
+    // 128 rows (3 rounds) and one round of 256 tiles of 96.  Chosen by the estimated makespan, taken when it saves 3 %.  What is left
+    // of the 128-token tiles, two to a CU, for a last round takes 0.64 of the time if every CU gets one at most: 700 x 15360 x 3840 (208
+    // tiles left, 280 narrow ones with strips) 211 us without strips, 241 with; 2048 x 10240 x 2560 237 / 256.  Tiles that end early
+    // fill no round: a last row of up to 64 tokens that starts behind others (1680 x 4656 x 1024 53 / 60, 1293 x 6336 x 4096 183 / 206), a
+    // last strip of up to 64 rows (1672 x 13984 x 1280 150 / 162), narrow ones of up to 32 tokens (798 x 12912 x 1536 with 98.6 -> 92.3).
+    // Where strips are taken: 1650 x 6208 x 4608 258 -> 237, 1871 x 5280 x 4352 248 -> 214, 1073 x 9360 x 768 56 -> 49, 2048 x 15360 x 3840 498
+    // -> 490; over 106 shapes of more than one round -3.1 %, 58 gain, four lose 1-5 % (786 x 10432 x 1280 71.5 -> 75.0).  The Q8_0 and Q4_0
+    // kernel has no loop for three row tiles and computes the fourth of such a strip as well: no rule for them.  The knob forces any number of strips for any format.
     if (Z == 1 && bm >= 128 && !dump && c->tune_gemm_narrow != 1) {
-        const auto makespan = [&](int b) -> double {   // in 128-row tile times; -1: N does not split that way
-            if (96 * b > p.N) return -1.0;
-            const int a = (p.N - 96 * b + BN - 1) / BN;
-            const long full = (long)a * p.tiles_m, nar = (long)b * p.tiles_m;
-            const double c96 = 0.80;
-            const long q = full / slots, r = full % slots;
-            if (nar == 0) return (double)(q + (r ? 1 : 0));
-            // narrow tiles go to the slots that are free at q first, then in turn to whichever frees first
-            double t_a = (double)q, t_b = (double)q + 1.0;   // slots - r slots free at t_a, r slots at t_b
-            long n_a = slots - r, n_b = r, left = nar;
-            double end = r ? t_b : t_a;
-            while (left > 0) {
-                const bool use_a = n_b == 0 || (n_a > 0 && t_a <= t_b);
-                const long n = std::min(left, use_a ? n_a : n_b);
-                double& tt = use_a ? t_a : t_b;
-                if (n < (use_a ? n_a : n_b)) { end = std::max(end, tt + c96); break; }   // the rest of this group stays free
-                tt += c96;
-                end = std::max(end, tt);
-                left -= n;
-            }
-            return end;
-        };
         int best_b = 0;
+        const int last = p.M - (p.tiles_m - 1) * bm, row = T / p.tiles_m;
         if (c->tune_gemm_narrow > 1) {
             best_b = std::min(c->tune_gemm_narrow - 1, p.N / 96);
-        } else if (T > slots && w.type == kQ6_K) {
-            double best = makespan(0);
-            const double need = 0.97 * best;
-            for (int b = 1; (long)b * p.tiles_m <= slots && 96 * b <= p.N; b++) {
+        } else if (T > slots && w.type == kQ6_K &&
+                   !(last <= 64 && p.walk_gm < p.tiles_m && T - (p.walk_gm == 1 ? row : row * 2 / 3) <= T / slots * slots)) {
+            const double c96 = 0.80, one = 0.64;   // of a 128-row tile's time: a 96-row tile; either with the CU to itself
+            const bool two = bm == 128;            // slots per CU
+            const auto part = [&](int n, double len) { return n == 0 ? 0.0 : two && n <= c->num_cu ? one * len : len; };
+            const auto makespan = [&](int b) {     // in 128-row tile times
+                const int full = (p.N - 96 * b + (b == 0 ? 63 : BN - 1)) / BN * p.tiles_m, nar = b * p.tiles_m;   // nar <= slots
+                const int early = last <= 32 && p.walk_gm == p.tiles_m ? b : 0;
+                const int q = full / slots, r = full % slots, free = slots - r;
+                if (nar == 0) return q + part(r, 1.0);
+                if (r == 0) return q + part(nar - early, c96);
+                if (nar <= free) return q + part(r + nar, 1.0);
+                if (nar <= 2 * free) return q + 1 + part(nar - free, 2 * c96 - 1);   // behind the narrow tiles beside the last full ones
+                return q + 1 + part(nar - free - early, c96);
+            };
+            const double plain = makespan(0);
+            double best = plain;
+            for (int b = 1; b * p.tiles_m <= slots && 96 * b <= p.N; b++) {
                 const double t = makespan(b);
-                if (t > 0 && t < best && t <= need) { best = t; best_b = b; }
+                if (t < best && t <= 0.97 * plain) { best = t; best_b = b; }
             }
         }
         if (best_b > 0) {
