@@ -420,7 +420,7 @@ static int walk_group(int tiles_m) {
 // workgroup's stages one after the other, at the time a stage takes with the CU to itself or shared with a second
 // workgroup and one more for its first loads, plus the launch that adds up the slices' partials, 1.9 us, 0.3 a slice and 5 MB of them per us.
 // Tiles that need several rounds: one slice, 128 or 256 tokens, whichever's rounds take less; there the first loads and the stores of
-// two workgroups on a CU hide behind each other's arithmetic (half a stage a round), those of one on its own do not (one and a half).
+// two workgroups on a CU hide behind each other's arithmetic (half a stage a round, 0.8 of Q6_K's), those of one on its own do not (1.5, 1.2).
 // The stage times are measured (us): 64 tokens 1.05 alone / 1.46 shared, 128 tokens 1.55 / 2.7, Q6_K 2.75 / 4.3; 256 tokens (one workgroup
 // per CU) 2.35, Q6_K 3.85.  Over 252 shapes of 65..2048 tokens (512..15360 rows and columns) the choice takes 0.7 % more than the best of
 // all heights and up to 16 slices, 15 % at worst (Q8_0 180 x 2384 x 15328: 44.0 us, twelve slices of one 256-token tile 38.4).  Constants fitted
@@ -449,7 +449,7 @@ static Tiling pick_tiling(int num_cu, bool q6, int M, int N, int nstages, bool s
             return n == 0 ? 0.0 : n <= num_cu ? alone : std::max(alone, shared * (0.93 + 0.07 * (n - num_cu) / num_cu));
         };
         if (T > slots) {   // whole rounds and the rest
-            const double us = (nstages + (q6 ? 1.0 : bm == 256 ? 1.5 : 0.5)) * (T / slots * shared + stage(T % slots));
+            const double us = (nstages + (q6 ? (bm == 256 ? 1.2 : 0.8) : bm == 256 ? 1.5 : 0.5)) * (T / slots * shared + stage(T % slots));
             if (bm >= 128 && us < least) {
                 least = us;
                 best = {bm, 1};
