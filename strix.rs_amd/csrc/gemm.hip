@@ -108,7 +108,8 @@ __global__ __launch_bounds__(64 * NW, 2) void gemm_i8_kernel(GemmArgs p) {
     uint4 rsv = {0, 0, 0, 0};  // the thread's four raw scales: f16 pairs in .x .y (weights) or four fp32 (activations)
 
     // all global reads of stage s (issuing them piecemeal between the blocks measures slower); the register-staged parts are
-    // written by finish_stage.  full: more than 64 live tokens, every 8-row group is fetched
+    // written by finish_stage.  full (waves with all four row tiles): every 8-row group is fetched, those past the tile's end as
+    // copies of its last row; of four waves' tiles that is more than 64 live tokens, of eight waves' any number
     auto issue_stage = [&](auto full, int buf, int s) __attribute__((always_inline)) {
         const unsigned sA = __builtin_amdgcn_readfirstlane(smem_base + buf * STAGE_BYTES + wave * GRP);
         const int blk0 = s * KB;
@@ -381,7 +382,7 @@ __global__ __launch_bounds__(64 * NW, 2) void gemm_i8_kernel(GemmArgs p) {
     else if (nt_cnt == 4) main_loop(std::integral_constant<int, 4>(), T());
     else if (nt_cnt == 2) main_loop(std::integral_constant<int, 2>(), F());
     else if (nt_cnt == 1) main_loop(std::integral_constant<int, 1>(), F());
-    else main_loop(std::integral_constant<int, 4>(), F());   // three, or the end of N: what is past it is not written
+    else main_loop(std::integral_constant<int, 4>(), F());   // three: there is no loop for them, the fourth is computed and not written
 
     gemm_store(p, op, at, role, acc, lane);
     SMX_GEMM_T1(live_tok, at.op_i);

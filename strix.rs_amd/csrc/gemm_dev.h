@@ -73,10 +73,11 @@ __device__ __forceinline__ TileAt gemm_tile_at(const GemmArgs& p) {
 struct WaveRole {
     int live_tok, live_rows;
     int tw;        // token sub-tile
-    int nt_cnt;    // row tiles of this wave; a tile at the end of N, or a 96-row strip: only the row tiles that exist
+    int nt_cnt;    // row tiles of this wave; a tile at the end of N, or a 96-row strip: only those that exist (gemm_i8_kernel computes four for three)
     int nt_base;
 };
-// A workgroup of eight waves (256 tokens): 32 tokens a wave, all of the row tiles.
+// A workgroup of eight waves (256 tokens): 32 tokens a wave, all of the row tiles; of a ragged last tile the waves past its end only stage
+// (77 live tokens: three of eight waves compute), and its time is that of a whole one (pick_tiling prices it so).
 __device__ __forceinline__ WaveRole gemm_wave_role(const TileAt& t, int wave, int nw = NW) {
     WaveRole r;
     r.live_tok = t.M_end - t.tok0;
