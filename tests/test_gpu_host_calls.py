@@ -171,7 +171,7 @@ def test_large_expert_ffn_equals_its_groups(accel, synth, hidden, rows):
     got = accel.moe_layer_ffn(9, plan, xs, sum(rows))
     o = 0
     for e, n in plan:
-        for a in range(0, n, 128):   # whole tiles: the same sums
+        for a in range(0, n, 128):   # whole tiles, and sizes that take the same number of K slices: the same sums
             part = xs[o + a:o + min(n, a + 128)]
             assert np.array_equal(got[o + a:o + min(n, a + 128)], accel.moe_expert_ffn(9, e, part, part.shape[0])), (e, a)
         o += n
